@@ -111,9 +111,8 @@ def _config(c):
                            act_bf16=c["dtype"] == "bf16", bias_zipf=c["zipf"])
 
 
-def _layer(hip, c, g):
-    """A layer's weights as a loader leaves them: MXFP4 codes and scales made on the device, packed where the
-    matrix-core modes take the shape, in the checkpoint layout where they do not."""
+def _tensors(hip, c, g):
+    """A layer's weights in the checkpoint layout: MXFP4 codes and scales made on the device."""
     cfg = _config(c)
     E, H, I, S = cfg.n_experts, cfg.hidden, cfg.inter, cfg.shared_inter
     dev = hip.device
@@ -136,6 +135,13 @@ def _layer(hip, c, g):
     t["down_w"], t["down_s"] = codes(E, H, I // 2), scales(E, H, I // 32)
     if S:
         t["sh_down_w"], t["sh_down_s"] = codes(1, H, S // 2), scales(1, H, S // 32)
+    return t
+
+
+def _layer(hip, c, g):
+    """The layer as a loader leaves it: packed where the matrix-core modes take the shape, in the checkpoint layout
+    where they do not."""
+    cfg, t, dev = _config(c), _tensors(hip, c, g), hip.device
     layer = backend.MoeLayer(cfg, t, None)
     nbytes = hip.lib.ferrite_moe_packed_bytes(ctypes.byref(layer.shape))
     if nbytes == 0:
@@ -287,3 +293,82 @@ def tolerance(case):
     if case["mode"] == "fp8x2":
         return {"rel": 1e-2, "max": 6e-2}   # bf16 outputs or expert outputs: 2.6e-3, 1.5e-2
     return {"rel": 1e-2, "max": 1.5e-1}     # an e4m3 code of three mantissa bits that falls to its neighbour: 2.6e-3, 3.5e-2
+
+
+def _values(codes, scales):
+    """MXFP4 codes (low nibble = even column) and e8m0 scales of one matrix as 64-bit values."""
+    mags = [0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0]
+    table = torch.tensor(mags + [-m for m in mags], dtype=torch.float64, device=codes.device)
+    v = torch.stack([table[(codes & 15).long()], table[(codes >> 4).long()]], dim=-1).reshape(codes.shape[0], -1, 32)
+    return (v * torch.exp2(scales.double() - 127.0).unsqueeze(-1)).reshape(codes.shape[0], -1)
+
+
+def _swiglu64(gate, up, limit):
+    gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+    return gate * torch.sigmoid(gate) * up
+
+
+def _norm64(x, w):
+    return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + EPS) * w.double()
+
+
+def _route64(logits, bias, topk, n_group, topk_group, scaling):
+    sig = torch.sigmoid(logits)
+    choice = sig + bias.double()
+    if n_group > 1 and topk_group < n_group:
+        groups = choice.reshape(choice.shape[0], n_group, -1)
+        score = groups.topk(min(2, groups.shape[-1]), -1).values.sum(-1)
+        keep = torch.zeros_like(score).scatter_(1, score.topk(topk_group, -1).indices, 1.0) > 0
+        choice = torch.where(keep.unsqueeze(-1), groups, -math.inf).reshape(choice.shape)
+    ids = choice.topk(topk, -1).indices
+    w = sig.gather(1, ids)
+    return ids, w / (w.sum(-1, keepdim=True) + 2.0 ** -23) * scaling
+
+
+def _ffn64(cfg, t, x):
+    """The layer on x [n, H] with nothing quantised but its weights."""
+    ids, w = _route64(x @ t["router_w"].double().T, t["router_bias"], cfg.topk, cfg.n_group, cfg.topk_group, cfg.routed_scaling)
+
+    def expert(prefix, e, rows):
+        gate, up, down = (_values(t[prefix + m + "_w"][e], t[prefix + m + "_s"][e]) for m in ("gate", "up", "down"))
+        return _swiglu64(rows @ gate.T, rows @ up.T, cfg.swiglu_limit) @ down.T
+
+    out = expert("sh_", 0, x) if cfg.shared_inter else torch.zeros_like(x)
+    for e in range(cfg.n_experts):
+        tok, slot = (ids == e).nonzero(as_tuple=True)
+        if len(tok):
+            out.index_add_(0, tok, expert("", e, x[tok]) * w[tok, slot].unsqueeze(-1))
+    return out
+
+
+def _hc_post64(x, s):
+    return s.post.double().unsqueeze(-1) * x.unsqueeze(1) + s.comb.double().transpose(1, 2) @ s.residual.double()
+
+
+def exact(case, seed):
+    """What run() returns, in 64 bits.  The engine's ids and tables and an ingest's bytes are whole numbers: none here."""
+    kind, n, H = case["kind"], case["n"], case["hidden"]
+    if kind == "ingest":
+        return None
+    hip = _hip()
+    g = torch.Generator(device=hip.device).manual_seed(seed)
+    if kind == "ops":
+        s = prepare(case, seed)
+        h = _norm64(s.x.double(), s.norm_w)
+        logits = h @ s.router_w.double().T
+        probs = _route64(logits, s.bias, case["topk"], case["n_group"], case["topk_group"], 2.5)[1]
+        gate, up = (h @ s.gate_up_w.double().T).chunk(2, -1)
+        out = _hc_post64(_swiglu64(gate, up, 10.0) @ s.down_w.double().T, s)
+        return [out, logits, probs, None, None]
+    x = torch.randn(n, H, device=hip.device, generator=g).to(DTYPES[case["dtype"]]).double()
+    if kind == "step":
+        weights = [_tensors(hip, case, g) for _ in range(case["layers"])]
+        norm_ws = [torch.rand(H, device=hip.device, generator=g) + 0.5 for _ in weights]
+        xs = torch.randn(case["layers"], n, H, device=hip.device, generator=g)
+        return torch.stack([_ffn64(_config(case), t, _norm64(xl.double(), w)) for t, w, xl in zip(weights, norm_ws, xs)])
+    t = _tensors(hip, case, g)
+    if kind == "layer":
+        return _ffn64(_config(case), t, x)
+    s = _State(hip, case)
+    _streams(case, g, hip.device, s)
+    return _hc_post64(_ffn64(_config(case), t, _norm64(x, s.norm_w)), s)
