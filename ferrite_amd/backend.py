@@ -271,16 +271,32 @@ class HipBackend:
             raise InvalidArg(f"{what} must be contiguous")
         return t
 
-    def _enter(self):
+    def _enter(self, mark=None):
         """Make this backend's stream wait for work already queued on torch's current stream (not while a
-        capture is open: the capture must stay on one stream)."""
+        capture is open: the capture must stay on one stream), or for what was queued there at `mark`."""
         if not self._capturing:
-            self.stream.wait_stream(torch.cuda.current_stream(self.device))
+            if mark is None:
+                self.stream.wait_stream(torch.cuda.current_stream(self.device))
+            else:
+                self.stream.wait_event(mark)
 
     def _leave(self):
         """Make torch's current stream wait for what was just enqueued, so torch ops on the outputs are ordered."""
         if not self._capturing:
             torch.cuda.current_stream(self.device).wait_stream(self.stream)
+
+    def _mark_and_leave(self):
+        """What a call on caller-allocated buffers starts with: the point of torch's current stream that its launches
+        have to wait for (the argument of _enter), taken before that stream is made to wait for this backend's earlier
+        work.  Taken after it, the mark would be reached only once that earlier work has ended, and every call of a
+        back-to-back sequence would begin with two cross-queue signals on an idle GPU: 21 us between the last kernel
+        of one call and the first of the next (32 tokens, H 4096: 244 us a call, 234 us this way).  The backend's
+        earlier work is on its own stream, so waiting for it there adds no ordering."""
+        if self._capturing:
+            return None
+        mark = torch.cuda.current_stream(self.device).record_event()
+        self._leave()
+        return mark
 
     def sync(self):
         self.stream.synchronize()
@@ -301,7 +317,7 @@ class HipBackend:
     def matmul(self, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor):
         """lib.rs:73 / cpu.rs:82-122 (recorded twice, like the reference: cpu.rs:89-90)."""
         self.recorder.record("matmul")
-        self._leave()
+        mark = self._mark_and_leave()
         self.recorder.record("matmul")
         if x.dim() != 2 or w.dim() != 2:
             raise InvalidArg("matmul operands must be 2-d")
@@ -316,21 +332,21 @@ class HipBackend:
             self._dev(bias, torch.float32, "bias")
             if bias.numel() != o:
                 raise InvalidArg("matmul bias shape")
-        self._enter()
+        self._enter(mark)
         self._ck(self.lib.ferrite_matmul_f32(x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(),
                                              out.data_ptr(), n, k, o, self._st()), "matmul")
 
     def rmsnorm(self, x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor):
         """lib.rs:76 / cpu.rs:124-143: x, out [..., dim] f32, w [dim] f32."""
         self.recorder.record("rmsnorm")
-        self._leave()
+        mark = self._mark_and_leave()
         if x.dim() < 1:
             raise InvalidArg("rmsnorm rank 0")
         dim = x.shape[-1]
         if w.numel() != dim or tuple(out.shape) != tuple(x.shape):
             raise InvalidArg("rmsnorm shape mismatch")
         self._dev(x, torch.float32, "x"); self._dev(w, torch.float32, "w"); self._dev(out, torch.float32, "out")
-        self._enter()
+        self._enter(mark)
         self._ck(self.lib.ferrite_rmsnorm_f32(x.data_ptr(), w.data_ptr(), eps, out.data_ptr(), x.numel() // dim, dim,
                                               self._st()), "rmsnorm")
 
@@ -355,7 +371,7 @@ class HipBackend:
     def swiglu_limited(self, gate_up: torch.Tensor, limit: float, out: torch.Tensor):
         """lib.rs:83-85 / cpu.rs:178-203"""
         self.recorder.record("swiglu")
-        self._leave()
+        mark = self._mark_and_leave()
         if gate_up.dim() != 2:
             raise InvalidArg("swiglu input must be 2-d")
         n, two_i = gate_up.shape
@@ -364,7 +380,7 @@ class HipBackend:
         if tuple(out.shape) != (n, two_i // 2):
             raise InvalidArg(f"swiglu out {tuple(out.shape)} != [{n},{two_i // 2}]")
         self._dev(gate_up, torch.float32, "gate_up"); self._dev(out, torch.float32, "out")
-        self._enter()
+        self._enter(mark)
         self._ck(self.lib.ferrite_swiglu_limited_f32(gate_up.data_ptr(), limit, out.data_ptr(), n, two_i // 2,
                                                      self._st()), "swiglu")
 
@@ -373,7 +389,7 @@ class HipBackend:
                   ids_i32: Optional[torch.Tensor] = None):
         """lib.rs:194-206 / cpu.rs:528-572; ids is an f32 tensor as in the reference."""
         self.recorder.record("moe_route")
-        self._leave()
+        mark = self._mark_and_leave()
         self.recorder.record("moe_route")
         if logits.dim() != 2:
             raise InvalidArg("logits must be 2-d")
@@ -386,7 +402,7 @@ class HipBackend:
         self._dev(probs, torch.float32, "probs"); self._dev(ids, torch.float32, "ids")
         if ids_i32 is not None:
             self._dev(ids_i32, torch.int32, "ids_i32")
-        self._enter()
+        self._enter(mark)
         self._ck(self.lib.ferrite_moe_route(logits.data_ptr(), bias.data_ptr(), n, e, topk, n_group, topk_group,
                                             routed_scaling, probs.data_ptr(), ids.data_ptr(),
                                             None if ids_i32 is None else ids_i32.data_ptr(), self._st()), "moe_route")
@@ -564,7 +580,7 @@ class HipBackend:
         """The whole layer on the device: router GEMM -> route -> permute -> experts -> combine (+shared).
         x [n, H] f32 or bf16, out [n, H] f32 or bf16, both pre-allocated device tensors."""
         self.recorder.record("moe_layer_mxfp4")
-        self._leave()
+        mark = self._mark_and_leave()
         cfg = layer.cfg
         if x.dim() != 2 or x.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"x {tuple(x.shape)} vs hidden {cfg.hidden}")
@@ -578,7 +594,7 @@ class HipBackend:
         if mode != MODE_F32_CHECK and layer.packed is None:
             raise InvalidArg("layer has no packed weights")
         ws = workspace if workspace is not None else self.workspace(layer, n, mode)
-        self._enter()
+        self._enter(mark)
         args = (C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
                 x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, ws.data_ptr(), ws.numel(),
                 self._st())
@@ -592,7 +608,7 @@ class HipBackend:
     def moe_layer_dev_mxfp4_static(self, layer: MoeLayer, x: torch.Tensor, out: torch.Tensor, mode: int = MODE_MFMA_FP8):
         """The same layer on the library's built-in workspace: nothing is allocated, here or in the library."""
         self.recorder.record("moe_layer_mxfp4")
-        self._leave()
+        mark = self._mark_and_leave()
         cfg = layer.cfg
         if x.dim() != 2 or x.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"x {tuple(x.shape)} vs hidden {cfg.hidden}")
@@ -602,7 +618,7 @@ class HipBackend:
         dts = {torch.float32: DT_F32, torch.bfloat16: DT_BF16}
         if x.dtype not in dts or out.dtype not in dts or not x.is_contiguous() or not out.is_contiguous():
             raise InvalidArg("x/out must be contiguous f32 or bf16 device tensors")
-        self._enter()
+        self._enter(mark)
         rc = self.lib.ferrite_moe_layer_mxfp4_static(
             C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
             x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, self._st())
@@ -632,7 +648,7 @@ class HipBackend:
         li [n,H] f32, residual/out [n,nh,H] f32, post [n,nh], comb [n,nh,nh].  residual None: rmsnorm -> MoE FFN
         only, out [n,H]."""
         self.recorder.record("moe_block_mxfp4")
-        self._leave()
+        mark = self._mark_and_leave()
         cfg = layer.cfg
         if li.dim() != 2 or li.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"li {tuple(li.shape)} vs hidden {cfg.hidden}")
@@ -656,7 +672,7 @@ class HipBackend:
         ws = workspace if workspace is not None else self.block_workspace(layer, n, mode)
         ptr = lambda t: None if t is None else t.data_ptr()
         blk = MoeBlockArgs(norm_w.data_ptr(), eps, ptr(residual), ptr(post), ptr(comb), nh)
-        self._enter()
+        self._enter(mark)
         self._ck(self.lib.ferrite_moe_block_mxfp4(C.byref(layer.shape), C.byref(layer.weights),
                                                   None if layer.packed is None else layer.packed.data_ptr(),
                                                   li.data_ptr(), C.byref(blk), n, out.data_ptr(), mode, ws.data_ptr(),
