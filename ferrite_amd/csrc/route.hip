@@ -8,124 +8,272 @@ namespace fe {
 
 // ------------------------------------------------------------------------------------------------
 // x . w^T with the reference's arithmetic (crates/ferrite-kernel/src/cpu.rs:106-111): for every output one
-// chain s = 0; s = fl(s + fl(x[l] * w[l])) in ascending l.  The chain cannot be re-associated, so the
-// kernel gives every output its own lane and only organises the operand traffic: a block owns 4 rows of x
-// and 64 rows of w, stages 64-wide k-chunks of both through LDS (w transposed so that a lane reads four
-// consecutive k of its own row with one 128-bit LDS read), and double-buffers the staging.
+// chain s = 0; s = fl(s + fl(x[l] * w[l])) in ascending l.  The chain cannot be re-associated, its adds stay on the
+// vector ALU.  Two kernels; both stage x and w through LDS as f32 in chunks of 64 k, with the fetches of several chunks
+// in flight in registers and one barrier per chunk.
+//
+// chain_mfma_kernel, for enough chains: the products come from the matrix cores (an f32 MFMA on a zero accumulator
+// gives the correctly rounded product; -0 comes out as +0, which a chain that starts at +0 cannot see).  A wave owns
+// 16 tokens x 16 outputs.  v_mfma_f32_16x16x1_4b is four outer products of 16 x 16, and its four blocks take the same
+// tokens and outputs at four different k: lane l = (q = l / 16, r = l % 16) holds x[t0 + r] and w[o0 + r] at
+// k = 16 s + 4 q .. + 3, the MFMA of component c leaves in register 4 b + v the product of token 4 q + v, output r at
+// k = 16 s + 4 b + c.  A step of 16 k is two 16-byte LDS reads per lane, four MFMAs and 64 adds (four chains per lane);
+// the products of step s + 1 are made while the adds of step s run.  Bound by the matrix pipe (66 cycles per MFMA) and
+// the adds, which overlap between the waves of a SIMD only.
+//
+// chain_valu_kernel, for few chains, where a chain's own length is the time: one chain per lane (8 tokens x 8 outputs per
+// wave), multiply and add on the vector ALU.  A lone wave issues one instruction per four cycles.
+//
+// us:                                                   before    mfma    valu
+//   router 8192 tokens x 256, H 7168 (bf16 x)              735     648     -       (valu, 4 x 4 chains per lane: 620)
+//   router 4096 x 128, H 4096 (bf16 x)                     149     105     -       (2 x 2 chains per lane: 125)
+//   router 2047 x 128, H 4096 (f32 x)                      146      76     -       (2 x 2: 101)
+//   router 509 x 128, H 4096 (bf16 x)                       47      50     42
+//   100 x 3072, k 4096 / 100 x 4096, k 1536             168 / 78   91 / 40  -      (2 x 2: 109 / 47)
+//   100 x 128, k 4096 / 27 x 32, k 2080                  70 / 37   46 / 25  35 / 20
+// Also built: x through DPP broadcasts or v_readlane instead of LDS (161 and 177 us for the second line: both instructions
+// cost several plain ones); operands read from memory in MFMA order without LDS (64 requests per load to the address
+// unit: 121 us for 100 x 3072); one chunk in flight instead of three (51 against 46 us for 100 x 128).
 // ------------------------------------------------------------------------------------------------
-constexpr int MM_TT = 4;    // x rows per block (one per wave)
-constexpr int MM_TO = 64;   // w rows per block (one per lane)
-constexpr int MM_KC = 64;   // k chunk
-constexpr int MM_WPAD = MM_TO + 1;
+typedef float ch_f16 __attribute__((ext_vector_type(16)));
+typedef float ch_f4 __attribute__((ext_vector_type(4)));
+typedef ch_f4 ch_f4u __attribute__((aligned(4)));   // x of the stand-alone op may be aligned to its elements only
+typedef unsigned int ch_u2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float load_x(const float* p, size_t i) { return p[i]; }
-__device__ __forceinline__ float load_x(const uint16_t* p, size_t i) { return u2f((uint32_t)p[i] << 16); }
+constexpr int CH_T = 16;              // rows of x and of w per staged tile
+constexpr int CH_KC = 64;             // k per chunk
+constexpr int CH_PIECES = CH_KC / 4;  // 16-byte pieces of a row's chunk
+constexpr int CH_TILE = CH_T * CH_PIECES;
 
-template <typename XT>
-__global__ __launch_bounds__(256) void matmul_exact_kernel(const XT* __restrict__ x, const float* __restrict__ w,
-                                                           const float* __restrict__ bias, float* __restrict__ out,
-                                                           int n, int k, int o) {
-    __shared__ float4 w_lds[2][MM_KC / 4][MM_WPAD];
-    __shared__ float4 x_lds[2][MM_TT][MM_KC / 4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int o0 = blockIdx.x * MM_TO, t0 = blockIdx.y * MM_TT;
-    const int nchunk = (k + MM_KC - 1) / MM_KC;
+struct ChainArgs {
+    const void* x;       // [n][k]
+    const float* w;      // [o][k], or the k-blocked transpose [k/4][w_pitch][4] of the packed router weight
+    const float* bias;   // [o] or NULL
+    float* out;          // [n][o]
+    int n, k, o, w_pitch;
+    int x_major;         // which operand's tiles are dealt to the XCDs
+};
 
-    // staging assignment: 64 w rows x 16 float4 per chunk = 1024 float4 -> 4 per thread; x: 4 x 16 = 64 float4
-    float4 wreg[4];
-    float4 xreg;
-    auto fetch = [&](int c) {
-        const int kb = c * MM_KC;
+// Block -> (token tile of 16, output group of OT tiles).  Hardware deals consecutive blocks round-robin over the 8 XCDs,
+// so the blocks that read the same tile of the larger operand (x of thousands of tokens, or the weight of a wide matmul)
+// get block numbers 8 apart: one L2 fetches that tile once.  Returns false for blocks without work.
+template <int OT>
+__device__ __forceinline__ bool chain_block(const ChainArgs& a, int& t0, int& o0) {
+    const int tg = (a.n + CH_T - 1) / CH_T, og = (a.o + OT * CH_T - 1) / (OT * CH_T);
+    const int minor = a.x_major ? og : tg, majors = a.x_major ? tg : og;
+    const int slot = blockIdx.x >> 3;
+    const int mj = (slot / minor) * 8 + (blockIdx.x & 7), mn = slot % minor;
+    t0 = (a.x_major ? mj : mn) * CH_T;
+    o0 = (a.x_major ? mn : mj) * OT * CH_T;
+    return mj < majors;
+}
+
+// A thread's part of the block's staging: one piece of x and WN of w per chunk.  Of a row-major operand 16 lanes fetch
+// the 16 pieces of a row, of the transposed weight 16 rows of a piece (256 contiguous bytes either way); w tile `tile`
+// of the block, its rows or pieces group * 4 * WN .. are fetched by the calling wave.  Piece j of row r sits at slot
+// 16 r + (j ^ r) of its tile: the sixteen neighbouring lanes of a write and of a read touch different banks.  Rows past
+// the end repeat the last one, pieces past K are zero (they add +0 to the chains).
+template <typename XT, bool kPackedW, int WN>
+struct ChainFetch {
+    const XT* xrow;
+    const float* wrow[WN];
+    int xslot, wslot[WN], pj, K, nchunk, w_pitch;
+    struct Set {
+        ch_f4 x, w[WN];
+    };
+    __device__ __forceinline__ ChainFetch(const ChainArgs& a, int t0, int o_tile, int group) : pj(threadIdx.x & 15), K(a.k) {
+        const int pr = threadIdx.x >> 4, r = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+        nchunk = (K + CH_KC - 1) / CH_KC;
+        w_pitch = a.w_pitch;
+        xrow = static_cast<const XT*>(a.x) + (size_t)min(t0 + pr, a.n - 1) * K;
+        xslot = pr * CH_PIECES + (pj ^ pr);
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            int idx = tid + p * 256;
-            int r = idx >> 4, c4 = idx & 15;
-            int col = kb + c4 * 4;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (o0 + r < o) {
-                const float* src = w + (size_t)(o0 + r) * k + col;
-                if (col + 3 < k) v = *reinterpret_cast<const float4*>(src);
-                else {
-                    if (col < k) v.x = src[0];
-                    if (col + 1 < k) v.y = src[1];
-                    if (col + 2 < k) v.z = src[2];
+        for (int i = 0; i < WN; ++i) {
+            const int m = (group * WN + i) * 4 + q;
+            if constexpr (kPackedW) {
+                wrow[i] = a.w + ((size_t)m * a.w_pitch + min(o_tile + r, a.w_pitch - 1)) * 4;
+                wslot[i] = r * CH_PIECES + (m ^ r);
+            } else {
+                wrow[i] = a.w + (size_t)min(o_tile + m, a.o - 1) * K;
+                wslot[i] = m * CH_PIECES + (r ^ m);
+            }
+        }
+    }
+    __device__ __forceinline__ void load(Set& f, int c) const {   // past the end the last chunk again, never used
+        c = min(c, nchunk - 1);
+        const int k = min(c * CH_KC + pj * 4, K - 4);
+        if constexpr (sizeof(XT) == 4) {
+            f.x = *reinterpret_cast<const ch_f4u*>(xrow + k);
+        } else {
+            const ch_u2 v = *reinterpret_cast<const ch_u2*>(xrow + k);
+            f.x[0] = u2f(v[0]);
+            f.x[1] = u2f(v[1]);
+        }
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+            f.w[i] = *reinterpret_cast<const ch_f4*>(wrow[i] + (kPackedW ? (size_t)c * CH_PIECES * 4 * w_pitch : (size_t)k));
+    }
+    __device__ __forceinline__ void store(const Set& f, int c, ch_f4* xs, ch_f4* ws) const {
+        const bool in = min(c, nchunk - 1) * CH_KC + pj * 4 < K;   // the transposed weight comes with K % 64 == 0
+        const ch_f4 zero = {0.f, 0.f, 0.f, 0.f};
+        ch_f4 xv = f.x;
+        if constexpr (sizeof(XT) == 2) {
+            const uint32_t lo = f2u(xv[0]), hi = f2u(xv[1]);
+            xv = (ch_f4){u2f(lo << 16), u2f(lo & 0xffff0000u), u2f(hi << 16), u2f(hi & 0xffff0000u)};
+        }
+        xs[xslot] = in ? xv : zero;
+#pragma unroll
+        for (int i = 0; i < WN; ++i) ws[wslot[i]] = (kPackedW || in) ? f.w[i] : zero;
+    }
+};
+
+// Block = 4 waves: 16 tokens x 64 outputs.  Chunks c and c + 1 are readable while chunk c is walked, chunk c + 2 is
+// written at its start; three more chunks are on their way.
+template <typename XT, bool kPackedW>
+__global__ __launch_bounds__(256, 2) void chain_mfma_kernel(ChainArgs a) {
+    __shared__ ch_f4 xs[3][CH_TILE];
+    __shared__ ch_f4 ws[4][3][CH_TILE];
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int t0, o0;
+    if (!chain_block<4>(a, t0, o0)) return;   // the whole block
+    o0 += wave * CH_T;                        // may lie past o: such a wave works on the last row
+    const ChainFetch<XT, kPackedW, 4> src(a, t0, o0, 0);
+    const int nchunk = src.nchunk;
+    ch_f4 xo[2], wo[2];
+    auto read = [&](int at, int u, int to) {
+        xo[to] = xs[at][r * CH_PIECES + ((4 * u + q) ^ r)];
+        wo[to] = ws[wave][at][r * CH_PIECES + ((4 * u + q) ^ r)];
+    };
+    ch_f16 p[2][4];
+    const ch_f16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+
+    typename ChainFetch<XT, kPackedW, 4>::Set f[3];   // f[c % 3]: chunk c
+    src.load(f[0], 0);
+    src.load(f[1], 1);
+    src.load(f[2], 2);
+    src.store(f[0], 0, xs[0], ws[wave][0]);
+    src.load(f[0], 3);
+    src.store(f[1], 1, xs[1], ws[wave][1]);
+    src.load(f[1], 4);
+    __syncthreads();
+    read(0, 0, 0);
+    read(0, 1, 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) p[0][c] = __builtin_amdgcn_mfma_f32_16x16x1f32(xo[0][c], wo[0][c], zero, 0, 0, 0);
+#pragma unroll 1
+    for (int c0 = 0; c0 < nchunk; c0 += 3) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if (c0 + j >= nchunk) break;   // uniform
+            const int c = c0 + j, at = j, at1 = (j + 1) % 3, at2 = (j + 2) % 3;   // slots of chunks c, c + 1, c + 2
+            if (c) __syncthreads();   // chunk c + 1 is complete; nobody reads the slot of chunk c - 1 any more
+            src.store(f[at2], c + 2, xs[at2], ws[wave][at2]);
+            __builtin_amdgcn_sched_barrier(0);
+            src.load(f[at2], c + 5);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                // adds of step 4 c + u, products of the next one, operands of the one after
+                read(u < 2 ? at : at1, (u + 2) & 3, u & 1);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    p[(u + 1) & 1][b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xo[(u + 1) & 1][b], wo[(u + 1) & 1][b], zero, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) acc[v] = fadd(acc[v], p[u & 1][cc][4 * b + v]);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            wreg[p] = v;
         }
-        if (tid < MM_TT * (MM_KC / 4)) {
-            int r = tid >> 4, c4 = tid & 15;
-            int col = kb + c4 * 4;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (t0 + r < n) {
-                size_t base = (size_t)(t0 + r) * k + col;
-                if (col < k) v.x = load_x(x, base);
-                if (col + 1 < k) v.y = load_x(x, base + 1);
-                if (col + 2 < k) v.z = load_x(x, base + 2);
-                if (col + 3 < k) v.w = load_x(x, base + 3);
-            }
-            xreg = v;
-        }
-    };
-    auto stash = [&](int buf) {
+    }
+    const int col = o0 + r;
+    if (col < a.o) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            int idx = tid + p * 256;
-            int r = idx >> 4, c4 = idx & 15;
-            w_lds[buf][c4][r] = wreg[p];
+        for (int v = 0; v < 4; ++v) {
+            const int t = t0 + 4 * q + v;
+            if (t < a.n) a.out[(size_t)t * a.o + col] = a.bias ? fadd(acc[v], a.bias[col]) : acc[v];
         }
-        if (tid < MM_TT * (MM_KC / 4)) x_lds[buf][tid >> 4][tid & 15] = xreg;
-    };
+    }
+}
 
-    float s = 0.0f;
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int c = 0; c < nchunk; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nchunk) fetch(c + 1);
-        const int klen = min(MM_KC, k - c * MM_KC);
-        const int full4 = klen >> 2;
-        for (int c4 = 0; c4 < full4; ++c4) {
-            float4 wv = w_lds[buf][c4][lane];
-            float4 xv = x_lds[buf][wave][c4];
-            s = fadd(s, fmul(xv.x, wv.x));
-            s = fadd(s, fmul(xv.y, wv.y));
-            s = fadd(s, fmul(xv.z, wv.z));
-            s = fadd(s, fmul(xv.w, wv.w));
+// Block = 4 waves, two by two: 16 tokens x 16 outputs.  Chunk c + 1 is written while chunk c is walked; three more are
+// on their way.
+template <typename XT, bool kPackedW>
+__global__ __launch_bounds__(256, 2) void chain_valu_kernel(ChainArgs a) {
+    constexpr int FD = 4;   // even: a register set's LDS slot is a constant
+    __shared__ ch_f4 xs[2][CH_TILE], ws[2][CH_TILE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int t0, o0;
+    if (!chain_block<1>(a, t0, o0)) return;   // the whole block
+    const ChainFetch<XT, kPackedW, 1> src(a, t0, o0, wave);
+    const int nchunk = src.nchunk;
+    const int xr = (wave >> 1) * 8 + (lane >> 3), wr = (wave & 1) * 8 + (lane & 7);
+    float acc = 0.0f;
+    typename ChainFetch<XT, kPackedW, 1>::Set f[FD];   // f[c % FD]: chunk c
+#pragma unroll
+    for (int i = 0; i < FD; ++i) src.load(f[i], i);
+    src.store(f[0], 0, xs[0], ws[0]);
+    src.load(f[0], FD);
+#pragma unroll 1
+    for (int c0 = 0; c0 < nchunk; c0 += FD) {
+#pragma unroll
+        for (int h = 0; h < FD; ++h) {
+            const int c = c0 + h;
+            if (c >= nchunk) break;   // uniform
+            __syncthreads();   // chunk c is complete; nobody reads the slot of chunk c - 1 any more
+            src.store(f[(h + 1) % FD], c + 1, xs[(h + 1) & 1], ws[(h + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            src.load(f[(h + 1) % FD], c + 1 + FD);
+            __builtin_amdgcn_sched_barrier(0);
+            ch_f4 xv[2], wv[2];
+            auto read = [&](int p, int to) {
+                xv[to] = xs[h & 1][xr * CH_PIECES + (p ^ xr)];
+                wv[to] = ws[h & 1][wr * CH_PIECES + (p ^ wr)];
+            };
+            read(0, 0);
+#pragma unroll
+            for (int p = 0; p < CH_PIECES; ++p) {
+                if (p + 1 < CH_PIECES) read(p + 1, (p + 1) & 1);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc = fadd(acc, fmul(xv[p & 1][q], wv[p & 1][q]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        if (klen & 3) {
-            float4 wv = w_lds[buf][full4][lane];
-            float4 xv = x_lds[buf][wave][full4];
-            int rem = klen & 3;
-            s = fadd(s, fmul(xv.x, wv.x));
-            if (rem > 1) s = fadd(s, fmul(xv.y, wv.y));
-            if (rem > 2) s = fadd(s, fmul(xv.z, wv.z));
-        }
-        if (c + 1 < nchunk) stash(buf ^ 1);
-        __syncthreads();
     }
-    const int t = t0 + wave, j = o0 + lane;
-    if (t < n && j < o) {
-        if (bias) s = fadd(s, bias[j]);
-        out[(size_t)t * o + j] = s;
-    }
+    const int t = t0 + xr, col = o0 + wr;
+    if (t < a.n && col < a.o) a.out[(size_t)t * a.o + col] = a.bias ? fadd(acc, a.bias[col]) : acc;
+}
+
+// The line between the two: 512 tiles of 16 x 16 chains are two waves of the one-chain-per-lane kernel for each of the
+// chip's 1024 SIMDs; beyond that its LDS reads bound it, and below that the matrix-core kernel leaves SIMDs idle.
+template <typename XT, bool kPackedW>
+static int launch_chain(ChainArgs a, hipStream_t st) {
+    const long tg = ((long)a.n + CH_T - 1) / CH_T, ot = ((long)a.o + CH_T - 1) / CH_T;
+    const bool mfma = tg * ot > 512;
+    const long og = mfma ? (ot + 3) / 4 : ot;
+    a.x_major = (size_t)a.n * sizeof(XT) >= (size_t)a.o * sizeof(float);
+    const long blocks = ((a.x_major ? tg : og) + 7) / 8 * 8 * (a.x_major ? og : tg);
+    if (blocks > 0x7fffffffL) return FERRITE_DECLINED;
+    if (mfma) chain_mfma_kernel<XT, kPackedW><<<(unsigned)blocks, 256, 0, st>>>(a);
+    else chain_valu_kernel<XT, kPackedW><<<(unsigned)blocks, 256, 0, st>>>(a);
+    return check_launch("chain");
 }
 
 int launch_matmul_exact(const void* x, int x_dtype, const float* w, const float* bias, float* out, int n, int k,
                         int o, hipStream_t st) {
     if (n < 0 || k < 0 || o < 0) return FERRITE_ERR_INVALID_ARG;
     if (n == 0 || o == 0) return FERRITE_OK;
-    dim3 grid((o + MM_TO - 1) / MM_TO, (n + MM_TT - 1) / MM_TT);
-    // the staging reads w with 128-bit loads: row starts must be 16-byte aligned
-    if ((k & 3) != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0) return FERRITE_DECLINED;
-    if (x_dtype == FERRITE_DT_F32)
-        matmul_exact_kernel<float><<<grid, 256, 0, st>>>((const float*)x, w, bias, out, n, k, o);
-    else if (x_dtype == FERRITE_DT_BF16)
-        matmul_exact_kernel<uint16_t><<<grid, 256, 0, st>>>((const uint16_t*)x, w, bias, out, n, k, o);
-    else
-        return FERRITE_ERR_INVALID_ARG;
-    return check_launch("matmul_exact");
+    // four consecutive k per load: the weight's rows are whole, 16-byte aligned pieces of four
+    if (k < 4 || (k & 3) != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0) return FERRITE_DECLINED;
+    ChainArgs a{x, w, bias, out, n, k, o, 0, 0};
+    if (x_dtype == FERRITE_DT_F32) return launch_chain<float, false>(a, st);
+    if (x_dtype == FERRITE_DT_BF16) return launch_chain<uint16_t, false>(a, st);
+    return FERRITE_ERR_INVALID_ARG;
 }
 
 // Any-k variant: one lane per output straight from global memory (small or unaligned problems).
@@ -560,7 +708,7 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(PermArgs a, const 
 }
 
 // ------------------------------------------------------------------------------------------------
-// The head of the layer as ONE launch (decode-sized batches), or the router GEMM alone (kFused = false).
+// The head of the layer as ONE launch (decode-sized batches).
 // Workgroups have eight waves.
 //   blocks (eb, tg), eb < eblocks: router logits of the tokens of group tg for experts [64 eb, 64 eb + 64): the reference's
 //                                  sequential chain, one lane of wave 0 per expert.  A lone wave issues one
@@ -788,7 +936,7 @@ __device__ __forceinline__ void head_bystander(int nk4, const HeadNorm& nm) {
     }
 }
 
-template <typename XT, bool kFused, int T, int W>
+template <typename XT, int T, int W>
 __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
     extern __shared__ __align__(16) unsigned char head_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -868,7 +1016,7 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
     }
     // From here on wave 0 works alone (LDS is free for its scratch); with a fused permutation the other waves wait
     // at the barrier below and join in if this block turns out to be the one that routed the last token.
-    const bool block_perm = kFused && a.fuse_perm;
+    const bool block_perm = a.fuse_perm;
     if (wave != 0 && !block_perm) return;
     __shared__ int perm_here;
     int do_perm = 0;
@@ -879,29 +1027,27 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
             const int t = t0 + ti;
             if (t >= a.n) break;
             if (e < a.E) a.logits[(size_t)t * a.E + e] = s[ti];
-            if constexpr (kFused) {
-                // arrival: the stores above are made visible before the counter moves
-                __threadfence();
-                int last = 0;
-                if (lane == 0) last = atomicAdd(&a.counters[1 + t], 1) == eblocks - 1;
-                last = __shfl(last, 0, 64);
-                if (!last) continue;
-                __threadfence();
-                wave_sync();
-                RouteScratch& sc = *reinterpret_cast<RouteScratch*>(head_lds);
-                route_wave<true>(a.logits + (size_t)t * a.E, a.bias, true, a.E, a.topk, a.n_group, a.topk_group,
-                                 a.scaling, sc, a.probs + (size_t)t * a.topk, a.ids_f32 + (size_t)t * a.topk,
-                                 a.ids + (size_t)t * a.topk);
-                __threadfence();
-                last = 0;
-                if (lane == 0) last = atomicAdd(&a.counters[0], 1) == a.n - 1;
-                last = __shfl(last, 0, 64);
-                if (!last) continue;
-                __threadfence();
-                wave_sync();
-                do_perm = 1;
-                for (int i = lane; i < a.n + 1; i += 64) a.counters[i] = 0;
-            }
+            // arrival: the stores above are made visible before the counter moves
+            __threadfence();
+            int last = 0;
+            if (lane == 0) last = atomicAdd(&a.counters[1 + t], 1) == eblocks - 1;
+            last = __shfl(last, 0, 64);
+            if (!last) continue;
+            __threadfence();
+            wave_sync();
+            RouteScratch& sc = *reinterpret_cast<RouteScratch*>(head_lds);
+            route_wave<true>(a.logits + (size_t)t * a.E, a.bias, true, a.E, a.topk, a.n_group, a.topk_group,
+                             a.scaling, sc, a.probs + (size_t)t * a.topk, a.ids_f32 + (size_t)t * a.topk,
+                             a.ids + (size_t)t * a.topk);
+            __threadfence();
+            last = 0;
+            if (lane == 0) last = atomicAdd(&a.counters[0], 1) == a.n - 1;
+            last = __shfl(last, 0, 64);
+            if (!last) continue;
+            __threadfence();
+            wave_sync();
+            do_perm = 1;
+            for (int i = lane; i < a.n + 1; i += 64) a.counters[i] = 0;
         }
         if (lane == 0) perm_here = do_perm;
     }
@@ -922,14 +1068,12 @@ static HeadShape head_shape(int n, int eblocks) {
     return {2, 32};
 }
 
-static size_t head_lds_bytes(int n, int H, int E, bool fused) {
+static size_t head_lds_bytes(int n, int H, int E) {
     const HeadShape hs = head_shape(n, (E + 63) / 64);
     size_t b = 2 * (size_t)hs.W * 1024 + (size_t)hs.T * H * 4 + 64;   // ring, x rows, the rows' 1/rms
-    if (fused) {
-        if (b < sizeof(RouteScratch)) b = sizeof(RouteScratch);
-        size_t p = perm_block_lds_bytes(n, E);
-        if (p > b) b = p;
-    }
+    if (b < sizeof(RouteScratch)) b = sizeof(RouteScratch);
+    const size_t p = perm_block_lds_bytes(n, E);
+    if (p > b) b = p;
     return b;
 }
 
@@ -944,24 +1088,24 @@ bool head_norm_supported(int n, int H, int E) {
 }
 
 bool head_supported(int n, int H, int E) {
-    return n <= HEAD_MAX_N && E <= RT_MAX_E && (H % 128) == 0 && head_lds_bytes(n, H, E, true) <= 160 * 1024 - 64;   // 64: the kernel's static LDS
+    return n <= HEAD_MAX_N && E <= RT_MAX_E && (H % 128) == 0 && head_lds_bytes(n, H, E) <= 160 * 1024 - 64;   // 64: the kernel's static LDS
 }
 
-template <typename XT, bool kFused, int T, int W>
+template <typename XT, int T, int W>
 static int launch_head_tt(const HeadArgs& a, int quant, size_t lds, hipStream_t st) {
-    int rc = LdsLimit<&moe_head_kernel<XT, kFused, T, W>>::ensure(lds);
+    int rc = LdsLimit<&moe_head_kernel<XT, T, W>>::ensure(lds);
     if (rc) return rc;
     dim3 grid(a.Epad / 64 + quant, (a.n + T - 1) / T);
-    moe_head_kernel<XT, kFused, T, W><<<grid, 512, lds, st>>>(a);
+    moe_head_kernel<XT, T, W><<<grid, 512, lds, st>>>(a);
     return check_launch("moe_head");
 }
 
-template <typename XT, bool kFused>
+template <typename XT>
 static int launch_head_t(const HeadArgs& a, int quant, size_t lds, hipStream_t st) {
     const HeadShape hs = head_shape(a.n, a.Epad / 64);
-    if (hs.T == 2) return launch_head_tt<XT, kFused, 2, 32>(a, quant, lds, st);
-    if (hs.W == 16) return launch_head_tt<XT, kFused, 1, 16>(a, quant, lds, st);
-    return launch_head_tt<XT, kFused, 1, 32>(a, quant, lds, st);
+    if (hs.T == 2) return launch_head_tt<XT, 2, 32>(a, quant, lds, st);
+    if (hs.W == 16) return launch_head_tt<XT, 1, 16>(a, quant, lds, st);
+    return launch_head_tt<XT, 1, 32>(a, quant, lds, st);
 }
 
 int launch_moe_head(const void* x, int x_dtype, const float* router_t, const float* bias, const ferrite_moe_shape& s,
@@ -988,9 +1132,9 @@ int launch_moe_head(const void* x, int x_dtype, const float* router_t, const flo
         p.unit_first = units->unit_first; p.unit_count = units->unit_count;
         p.n_units = units->n_units; p.unit_cap = units->unit_rows_cap; p.max_units = units->max_units;
     }
-    const size_t lds = head_lds_bytes(n, s.hidden, s.n_experts, true);
-    if (x_dtype == FERRITE_DT_F32) return launch_head_t<float, true>(a, xq.q ? 1 : 0, lds, st);
-    if (x_dtype == FERRITE_DT_BF16) return launch_head_t<uint16_t, true>(a, xq.q ? 1 : 0, lds, st);
+    const size_t lds = head_lds_bytes(n, s.hidden, s.n_experts);
+    if (x_dtype == FERRITE_DT_F32) return launch_head_t<float>(a, xq.q ? 1 : 0, lds, st);
+    if (x_dtype == FERRITE_DT_BF16) return launch_head_t<uint16_t>(a, xq.q ? 1 : 0, lds, st);
     return FERRITE_ERR_INVALID_ARG;
 }
 
@@ -1008,273 +1152,28 @@ int check_routing_params(int e, int topk, int n_group, int topk_group) {
     return FERRITE_OK;
 }
 
-template <typename XT, bool kFused>
+template <typename XT>
 static int warmup_head() {
     const size_t cap = kLdsCap - 64;   // 64: the kernel's static LDS
     int rc;
-    if ((rc = LdsLimit<&moe_head_kernel<XT, kFused, 1, 32>>::ensure(cap))) return rc;
-    if ((rc = LdsLimit<&moe_head_kernel<XT, kFused, 1, 16>>::ensure(cap))) return rc;
-    return LdsLimit<&moe_head_kernel<XT, kFused, 2, 32>>::ensure(cap);
+    if ((rc = LdsLimit<&moe_head_kernel<XT, 1, 32>>::ensure(cap))) return rc;
+    if ((rc = LdsLimit<&moe_head_kernel<XT, 1, 16>>::ensure(cap))) return rc;
+    return LdsLimit<&moe_head_kernel<XT, 2, 32>>::ensure(cap);
 }
-
-template <typename XT> __global__ __launch_bounds__(256) void router_lds_kernel(const XT*, const float4*, int, int, int, int, float*);
 
 int warmup_route() {
     int rc;
-    if ((rc = LdsLimit<&router_lds_kernel<float>>::ensure(70 * 1024))) return rc;
-    if ((rc = LdsLimit<&router_lds_kernel<uint16_t>>::ensure(70 * 1024))) return rc;
-    if ((rc = warmup_head<float, true>())) return rc;
-    if ((rc = warmup_head<uint16_t, true>())) return rc;
-    if ((rc = warmup_head<float, false>())) return rc;
-    return warmup_head<uint16_t, false>();
-}
-
-// Router GEMM for many tokens: the same sequential chain (cpu.rs:82-122), register tiled.  A wave owns 64 experts
-// (one per lane, weights from the k-blocked transpose: one coalesced float4 per lane and four k) x T tokens whose
-// activations are wave-uniform and therefore come through scalar loads; every (token, expert) pair still sees
-// acc = acc + x*w for k ascending with separately rounded multiply and add.  T independent chains per lane cover
-// the VALU latency.  grid (Epad/64, ceil(n / (4*T))), 4 waves per block on the same experts.
-// One macro step = KM groups of four k: 16 k for bf16 activations, 8 k for f32, i.e. 32 bytes per token and step.
-template <typename XT>
-struct RouterStep {
-    static constexpr int KM = sizeof(XT) == 4 ? 2 : 4;
-};
-
-template <typename XT, int T, int TE>
-struct RouterSet {
-    uint4 x[T][2];                            // 32 bytes of each token as loaded; wave-uniform -> scalar registers
-    float4 w[RouterStep<XT>::KM][TE];
-};
-
-// Loads only: the bf16 -> f32 shifts happen at the use, so nothing here waits for the data.
-template <typename XT, int T, int TE>
-__device__ __forceinline__ void router_load(RouterSet<XT, T, TE>& r, const XT* const (&xr)[T], const float4* wp,
-                                            int Epad, int step) {
-    constexpr int KM = RouterStep<XT>::KM;
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-        const uint4* p = reinterpret_cast<const uint4*>(xr[i]) + (size_t)step * 2;
-        r.x[i][0] = p[0];
-        r.x[i][1] = p[1];
-    }
-#pragma unroll
-    for (int q = 0; q < KM; ++q)
-#pragma unroll
-        for (int j = 0; j < TE; ++j) r.w[q][j] = wp[(size_t)(step * KM + q) * Epad + j * 64];
-}
-
-template <typename XT, int T, int TE>
-__device__ __forceinline__ void router_chain(float (&acc)[TE][T], const RouterSet<XT, T, TE>& r) {
-    constexpr int KM = RouterStep<XT>::KM;
-#pragma unroll
-    for (int q = 0; q < KM; ++q) {
-#pragma unroll
-        for (int i = 0; i < T; ++i) {
-            float x0, x1, x2, x3;
-            if constexpr (sizeof(XT) == 4) {
-                const uint4 v = r.x[i][q];
-                x0 = u2f(v.x); x1 = u2f(v.y); x2 = u2f(v.z); x3 = u2f(v.w);
-            } else {
-                const uint4 v = r.x[i][q >> 1];
-                const uint32_t lo = (q & 1) ? v.z : v.x, hi = (q & 1) ? v.w : v.y;
-                x0 = u2f(lo << 16); x1 = u2f(lo & 0xffff0000u); x2 = u2f(hi << 16); x3 = u2f(hi & 0xffff0000u);
-            }
-#pragma unroll
-            for (int j = 0; j < TE; ++j) {
-                float a = acc[j][i];
-                a = fadd(a, fmul(x0, r.w[q][j].x));
-                a = fadd(a, fmul(x1, r.w[q][j].y));
-                a = fadd(a, fmul(x2, r.w[q][j].z));
-                a = fadd(a, fmul(x3, r.w[q][j].w));
-                acc[j][i] = a;
-            }
-        }
-    }
-}
-
-// TE blocks of 64 experts (lane = expert within the block) x T tokens per wave.
-template <typename XT, int T, int TE>
-__global__ __launch_bounds__(256) void router_tile_kernel(const XT* __restrict__ x, const float4* __restrict__ wt,
-                                                          int n, int H, int E, int Epad, float* __restrict__ logits) {
-    constexpr int KM = RouterStep<XT>::KM;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t0 = (blockIdx.y * 4 + wave) * T;
-    if (t0 >= n) return;
-    const int e0 = blockIdx.x * 64 * TE + lane;
-    const float4* wp = wt + e0;
-    const XT* xr[T];
-#pragma unroll
-    for (int i = 0; i < T; ++i) xr[i] = x + (size_t)min(t0 + i, n - 1) * H;
-    float acc[TE][T];
-#pragma unroll
-    for (int j = 0; j < TE; ++j)
-#pragma unroll
-        for (int i = 0; i < T; ++i) acc[j][i] = 0.0f;
-    const int nsteps = H / (4 * KM);   // even: H % 128 == 0
-    RouterSet<XT, T, TE> sa, sb;
-    router_load(sa, xr, wp, Epad, 0);
-    // Two register sets alternate: the loads of one are issued before the chains over the other.  Scalar loads
-    // return out of order, so any wait on them is a wait for all of them: the set about to be used is waited
-    // for BEFORE the other set's loads are issued (0xC07F: lgkmcnt 0, vmcnt and expcnt untouched).
-    for (int st = 0; st < nsteps; st += 2) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        router_load(sb, xr, wp, Epad, st + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        router_chain(acc, sa);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        router_load(sa, xr, wp, Epad, min(st + 2, nsteps - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        router_chain(acc, sb);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int j = 0; j < TE; ++j) {
-        const int e = e0 + j * 64;
-        if (e < E) {
-#pragma unroll
-            for (int i = 0; i < T; ++i)
-                if (t0 + i < n) logits[(size_t)(t0 + i) * E + e] = acc[j][i];
-        }
-    }
-}
-
-// The same chain for batches of a few hundred tokens, where the kernel above leaves SIMDs idle (four tokens per
-// wave: 160 waves at 320 tokens x 128 experts, 115 us) or, with one token per wave, pulls every wave's own copy of
-// the router weights through the vector memory path (1 KiB per wave and four k: 79 us, bound by the 64 bytes per
-// clock a CU's address unit handles).  Here the four waves of a block work on four tokens against the same 64
-// experts and share the weights through LDS: a chunk of RL_KC k (all 64 experts) is fetched once per block into a
-// two-slot ring, a chunk ahead of its use, each wave stages its own token's activations (as f32) beside it, and a
-// lane reads its expert's float4 and the token's float4 (a broadcast) per four k.  One barrier per chunk.
-typedef float rl_f4 __attribute__((ext_vector_type(4)));
-constexpr int RL_KC = 128;                                   // k per chunk
-constexpr int RL_W_SLOT = RL_KC / 4 * 64;                    // float4 of weights per slot (32 KiB)
-constexpr int RL_X_SLOT = 4 * RL_KC / 4;                     // float4 of activations per slot: 4 tokens x RL_KC f32
-constexpr size_t RL_LDS_BYTES = 2 * (size_t)(RL_W_SLOT + RL_X_SLOT) * 16;
-
-// A thread's share of chunk c: weight rows wave + 4 i of the chunk for expert e0 + lane, and two activations of the
-// wave's token.
-template <typename XT>
-__device__ __forceinline__ void rl_fetch(rl_f4 (&wr)[RL_KC / 16], float (&xv)[2], const rl_f4* __restrict__ wt,
-                                         const XT* __restrict__ xrow, int Epad, int col, int wave, int lane, int c) {
-    const rl_f4* src = wt + (size_t)(c * (RL_KC / 4) + wave) * Epad + col;
-#pragma unroll
-    for (int i = 0; i < RL_KC / 16; ++i) wr[i] = src[(size_t)(4 * i) * Epad];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const XT v = xrow[c * RL_KC + i * 64 + lane];
-        if constexpr (sizeof(XT) == 4) xv[i] = v; else xv[i] = u2f((uint32_t)v << 16);
-    }
-}
-
-__device__ __forceinline__ void rl_stash(rl_f4* slot, const rl_f4 (&wr)[RL_KC / 16], const float (&xv)[2], int wave,
-                                         int lane) {
-#pragma unroll
-    for (int i = 0; i < RL_KC / 16; ++i) slot[(wave + 4 * i) * 64 + lane] = wr[i];
-    float* xs = reinterpret_cast<float*>(slot + RL_W_SLOT) + wave * RL_KC;
-    xs[lane] = xv[0];
-    xs[64 + lane] = xv[1];
-}
-
-template <typename XT>
-__global__ __launch_bounds__(256) void router_lds_kernel(const XT* __restrict__ x, const float4* __restrict__ wt,
-                                                         int n, int H, int E, int Epad, float* __restrict__ logits) {
-    extern __shared__ __align__(16) unsigned char rl_raw[];
-    rl_f4* lds = reinterpret_cast<rl_f4*>(rl_raw);
-    const rl_f4* wt4 = reinterpret_cast<const rl_f4*>(wt);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int t = blockIdx.y * 4 + wave;
-    const int col = blockIdx.x * 64 + lane;
-    const XT* xrow = x + (size_t)min(t, n - 1) * H;
-    const int nchunk = H / RL_KC;
-    // One register set: chunk c + 1 is in flight while chunk c is walked.  What bounds a block is LDS bandwidth:
-    // four waves read 1 KiB of weights each per four k, eight cycles per k, and with the chains' own instructions
-    // on top a block takes 46-48 us at H 4096 (31 us with the multiplies compiled out).  Measured and not kept: a
-    // second register set, a chunk fetched two chunk times ahead (67 us); the next group's LDS reads issued before
-    // the current group's chain (46 us); the activations taken with v_readlane from registers instead of broadcast
-    // LDS reads (50 us).
-    rl_f4 wr[RL_KC / 16];
-    float xv[2];
-    float acc = 0.0f;
-    rl_fetch(wr, xv, wt4, xrow, Epad, col, wave, lane, 0);
-    rl_stash(lds, wr, xv, wave, lane);
-    rl_fetch(wr, xv, wt4, xrow, Epad, col, wave, lane, min(1, nchunk - 1));
-    for (int c = 0; c < nchunk; ++c) {
-        __syncthreads();   // slot c % 2 is complete; nobody reads slot (c + 1) % 2 any more
-        // past the last chunk both lines repeat it into the slot nobody reads any more: no branch around loads
-        rl_stash(lds + ((c + 1) & 1) * (RL_W_SLOT + RL_X_SLOT), wr, xv, wave, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        rl_fetch(wr, xv, wt4, xrow, Epad, col, wave, lane, min(c + 2, nchunk - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        const rl_f4* w = lds + (c & 1) * (RL_W_SLOT + RL_X_SLOT);
-        const rl_f4* xs = w + RL_W_SLOT + wave * (RL_KC / 4);
-#pragma unroll 8
-        for (int q = 0; q < RL_KC / 4; ++q) {
-            const rl_f4 wq = w[q * 64 + lane], xq = xs[q];
-            acc = fadd(acc, fmul(xq[0], wq[0]));
-            acc = fadd(acc, fmul(xq[1], wq[1]));
-            acc = fadd(acc, fmul(xq[2], wq[2]));
-            acc = fadd(acc, fmul(xq[3], wq[3]));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (t < n && col < E) logits[(size_t)t * E + col] = acc;
-}
-
-template <typename XT, int T>
-static int launch_router_tile_t(const XT* xp, const float4* wp, int n, int H, int E, int Epad, float* logits,
-                                hipStream_t st) {
-    dim3 grid(1, (n + 4 * T - 1) / (4 * T));
-    // two expert blocks per wave halve the weight traffic, but only when enough waves remain to hide latency
-    if (Epad % 128 == 0 && (long)(Epad / 128) * grid.y * 4 >= 4096) {
-        grid.x = Epad / 128;
-        router_tile_kernel<XT, T, 2><<<grid, 256, 0, st>>>(xp, wp, n, H, E, Epad, logits);
-    } else {
-        grid.x = Epad / 64;
-        router_tile_kernel<XT, T, 1><<<grid, 256, 0, st>>>(xp, wp, n, H, E, Epad, logits);
-    }
-    return check_launch("router_tile");
-}
-
-// Four tokens per wave in registers for thousands of tokens, two for a thousand or two (more waves), and the
-// LDS-sharing kernel below that.
-template <typename XT>
-static int launch_router_tile(const void* x, const float* router_t, int n, int H, int E, float* logits, hipStream_t st) {
-    const int Epad = (E + 63) / 64 * 64;
-    const XT* xp = static_cast<const XT*>(x);
-    const float4* wp = reinterpret_cast<const float4*>(router_t);
-    const long groups = Epad / 64;
-    // measured at 128 experts, H 4096: 320 / 512 / 767 / 1024 tokens 48 / 49 / 61 / 63 us with the LDS-sharing kernel
-    // (79 / 80 / 85 / 86 us with one token per wave of the register-tiled kernel, 115 us with four); 1536 / 2048
-    // tokens 97 / 98 us with two tokens per wave (101 / 117 us LDS-sharing, 115 / 116 us with four)
-    if (groups * n <= 2048) {
-        int rc = LdsLimit<&router_lds_kernel<XT>>::ensure(RL_LDS_BYTES);
-        if (rc) return rc;
-        dim3 grid((unsigned)groups, (n + 3) / 4);
-        router_lds_kernel<XT><<<grid, 256, RL_LDS_BYTES, st>>>(xp, wp, n, H, E, Epad, logits);
-        return check_launch("router_lds");
-    }
-    if (groups * n <= 4096) return launch_router_tile_t<XT, 2>(xp, wp, n, H, E, Epad, logits, st);
-    return launch_router_tile_t<XT, 4>(xp, wp, n, H, E, Epad, logits, st);
+    if ((rc = warmup_head<float>())) return rc;
+    return warmup_head<uint16_t>();
 }
 
 // Router GEMM alone from the transposed weight (any n): logits only.
 int launch_router_chain(const void* x, int x_dtype, const float* router_t, int n, int H, int E, float* logits,
                         hipStream_t st) {
     if (H % 128 != 0 || n <= 0 || n > 65535) return FERRITE_DECLINED;
-    if (n >= 64) {
-        if (x_dtype == FERRITE_DT_F32) return launch_router_tile<float>(x, router_t, n, H, E, logits, st);
-        if (x_dtype == FERRITE_DT_BF16) return launch_router_tile<uint16_t>(x, router_t, n, H, E, logits, st);
-        return FERRITE_ERR_INVALID_ARG;
-    }
-    if (head_lds_bytes(n, H, E, false) > 160 * 1024 - 64) return FERRITE_DECLINED;   // 64: the kernel's static LDS
-    HeadArgs a{};
-    a.x = x; a.wt = router_t; a.n = n; a.H = H; a.E = E; a.Epad = (E + 63) / 64 * 64; a.logits = logits;
-    const size_t lds = head_lds_bytes(n, H, E, false);
-    if (x_dtype == FERRITE_DT_F32) return launch_head_t<float, false>(a, 0, lds, st);
-    if (x_dtype == FERRITE_DT_BF16) return launch_head_t<uint16_t, false>(a, 0, lds, st);
+    ChainArgs a{x, router_t, nullptr, logits, n, H, E, (E + 63) / 64 * 64, 0};
+    if (x_dtype == FERRITE_DT_F32) return launch_chain<float, true>(a, st);
+    if (x_dtype == FERRITE_DT_BF16) return launch_chain<uint16_t, true>(a, st);
     return FERRITE_ERR_INVALID_ARG;
 }
 
@@ -1356,7 +1255,7 @@ extern "C" int ferrite_matmul_f32(const float* x, const float* w, const float* b
     if (n == 0 || o == 0) return FERRITE_OK;
     if ((n > 0 && !x) || !w || !out) return FERRITE_ERR_INVALID_ARG;
     hipStream_t st = as_stream(stream);
-    if ((k & 3) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (size_t)n * o >= 1024)
+    if (k > 0 && (k & 3) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (size_t)n * o >= 1024)
         return launch_matmul_exact(x, FERRITE_DT_F32, w, bias, out, n, k, o, st);
     size_t total = (size_t)n * o;
     matmul_exact_simple_kernel<<<(unsigned)((total + 63) / 64), 64, 0, st>>>(x, w, bias, out, n, k, o);

@@ -42,6 +42,25 @@ def test_matmul_bit_exact_vs_oracle(hip, oracle, n, k, o):
     assert np.array_equal(host(hip, out), oracle.matmul(x, w, b))
 
 
+# tile edges (16 rows, 16 outputs, 64 outputs a block), k remainders of the 16-wide steps and of the rounds of four,
+# both kernels (the line is 512 tiles of 16 x 16), rows that are only 4-byte aligned, values whose products are denormal or -0
+@pytest.mark.parametrize("n,k,o", [(1, 4, 1024), (15, 12, 80), (16, 16, 64), (17, 20, 65), (33, 52, 31), (64, 64, 16), (31, 68, 129),
+                                   (100, 132, 3072), (7, 736, 2080), (1030, 100, 272), (257, 260, 1041)])
+def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o):
+    rng = np.random.default_rng(n * 1000 + k)
+    x = rng.normal(0, 1, (n, k)).astype(np.float32)
+    w = rng.normal(0, 0.02, (o, k)).astype(np.float32)
+    x[0], w[0] = x[0] * np.float32(1e-30), w[0] * np.float32(1e-10)   # denormal products and sums
+    x[n // 2, ::3] = -0.0
+    w[o // 2, ::2] = 0.0
+    xbuf = torch.empty(n * k + 1, device=hip.device)
+    xd = xbuf[1:].view(n, k)
+    xd.copy_(torch.from_numpy(x))
+    out = torch.full((n, o), -1.0, device=hip.device)
+    hip.matmul(xd, dev(hip, w), None, out)
+    assert np.array_equal(host(hip, out), oracle.matmul(x, w))
+
+
 def test_matmul_shape_errors(hip):
     z = lambda *s: torch.zeros(*s, device=hip.device)
     with pytest.raises(ShapeMismatch):
