@@ -97,11 +97,11 @@ int launch_router_chain(const void* x, int x_dtype, const float* router_t, int n
 int launch_router_transpose(const float* w, int E, int H, float* dst, hipStream_t st);
 int launch_zero_i32(int32_t* p, int count, hipStream_t st);
 
-// experts_f32.hip (check mode)
+// experts_f32.hip
 int launch_gate_up_f32(const ferrite_moe_shape& s, const ferrite_moe_weights& w, const float* x, int n,
-                       const int32_t* ids, const int32_t* gather_src, float* act, hipStream_t st);
+                       const int32_t* gather_src, const UnitTables& units, float* act, hipStream_t st);
 int launch_down_f32(const ferrite_moe_shape& s, const ferrite_moe_weights& w, const float* act, int n,
-                    const int32_t* ids, const int32_t* gather_src, float* y, hipStream_t st);
+                    const UnitTables& units, float* y, hipStream_t st);
 // The hyper-connection update behind the layer, for a combine that applies it on the way out (f32 output only):
 // residual [n, nh, H], post [n, nh], comb [n, nh, nh]; out is then [n, nh, H].
 struct HcPostArgs {

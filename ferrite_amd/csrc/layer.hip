@@ -357,9 +357,9 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
     // 4-5. expert FFNs in grouped order, shared expert as the trailing rows
     if (mode == FERRITE_MODE_F32_CHECK) {
         float* act = reinterpret_cast<float*>(b + w.act);
-        if ((rc = launch_gate_up_f32(s, *wts, static_cast<const float*>(x), n, ids, gather_src, act, st))) return rc;
+        if ((rc = launch_gate_up_f32(s, *wts, static_cast<const float*>(x), n, gather_src, units, act, st))) return rc;
         if ((rc = mark(ev, 5, st))) return rc;
-        if ((rc = launch_down_f32(s, *wts, act, n, ids, gather_src, static_cast<float*>(y), st))) return rc;
+        if ((rc = launch_down_f32(s, *wts, act, n, units, static_cast<float*>(y), st))) return rc;
     } else {
         const ActPlanes act{at(w.act), at(w.act_s), x2 ? at(w.act2) : nullptr, x2 ? at(w.act_s2) : nullptr};
         if ((rc = launch_gate_up_mfma(s, packed, xq, n, gather_src, units, act, st,

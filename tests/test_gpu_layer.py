@@ -116,6 +116,23 @@ def test_layer_small_shapes_all_modes(hip, oracle, seed, n):
     check_mfma(hip, oracle, layer, inp, MODE_MFMA_FP8_X2, ref32)
 
 
+@pytest.mark.parametrize("n,hidden,inter,shared", [(1, 32, 32, 0), (5, 544, 96, 64), (40, 1056, 736, 32), (3, 2080, 1120, 736),
+                                                   (130, 480, 160, 320)])
+def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared):
+    """The f32 mode on sizes that are multiples of 32 only: reductions shorter than a block of 128, longer than the
+    activation window and ragged in both, odd numbers of row tiles, units of 1..16 rows, weights shared out to one wave
+    per pair of tiles or to four; zero scales."""
+    cfg = synth.MoeConfig(n, hidden, 8, 3, inter, shared, 4, 2)
+    inp = synth.make_inputs(cfg, seed=n + hidden)
+    inp.gate_s.reshape(-1)[::7] = 0
+    inp.down_s.reshape(-1)[::5] = 0
+    layer = hip.load_moe_layer(inp, pack=False)
+    ref = oracle.moe_ffn_mxfp4(inp, n_threads=8)
+    out, v = run_layer(hip, layer, inp.x, MODE_F32_CHECK)
+    check_routing(v, ref, oracle, cfg)
+    assert max_abs_rel(out, ref["out"]) <= TOL_F32
+
+
 @pytest.mark.parametrize("n,hidden,inter,shared", [(24, 2304, 2304, 2304), (19, 2176, 128, 2432), (5, 4096, 256, 0)])
 def test_two_term_long_reductions_stream_their_activations_in_windows(hip, oracle, n, hidden, inter, shared):
     """Two-term activations of a reduction longer than 2048 do not stay in LDS whole: they pass through a ring of
