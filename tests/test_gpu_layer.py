@@ -741,3 +741,16 @@ def test_layer_c3_skewed_scale(hip, oracle):
     counts = np.sort(v["counts"])[::-1]
     top = counts[: cfg.n_experts // 10].sum() / counts.sum()
     assert 0.35 <= top <= 0.65, top
+
+
+@pytest.mark.parametrize("mode", [MODE_MFMA_FP8, MODE_MFMA_FP8_X2])
+@pytest.mark.parametrize("n,hidden,inter,shared", [(1, 4096, 1536, 1536), (4, 640, 1152, 512), (3, 2176, 512, 2432), (2, 1024, 2048, 0),
+                                                   (5, 1024, 1024, 512)])
+def test_few_tokens_share_items_among_waves(hip, oracle, n, hidden, inter, shared, mode):
+    """A few tokens with a few hundred items: the waves of a block split an item's reduction.  Groups that do not divide
+    among the waves, last groups of less than four k steps, routed and shared reductions of different lengths; five
+    tokens do not split."""
+    cfg = synth.MoeConfig(n, hidden, 8, 4, inter, shared, 4, 2)
+    inp = synth.make_inputs(cfg, seed=n)
+    layer = hip.load_moe_layer(inp)
+    check_mfma(hip, oracle, layer, inp, mode)
