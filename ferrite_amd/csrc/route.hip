@@ -796,8 +796,8 @@ __device__ __forceinline__ void head_pmul(const HeadSet<T, W>& st, const float4*
 
 // rmsnorm of the block's token(s) in place of the first barrier ("x is in LDS") of every wave's role.  On entry
 // every thread has staged its share of the raw rows in xl and of their squares (each rounded once) in sq.  The
-// reference sums the squares of a row left to right in f32 (cpu.rs:124-143): a serial chain, walked by wave 0 with
-// 16-byte broadcast reads in counted batches, while the producer waves' first weight loads are already in flight.
+// reference sums the squares of a row left to right in f32 (cpu.rs:124-143): a serial chain, which wave 0 works out
+// (sumsq_walk) while the producer waves' first weight loads are already in flight.
 // Then all waves scale xl to (x * inv) * w, which is what the router chain and the quantisation see.
 struct HeadNorm {
     const float* w;
@@ -944,12 +944,13 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
     const int eb = blockIdx.x, t0 = blockIdx.y * T;
     const int eblocks = a.Epad >> 6;
     const int H = a.H;
+    constexpr bool kNorm = sizeof(XT) == 4 && T == 1 && W == 32;   // see head_norm_supported
     if (eb == eblocks) {
         for (int ti = 0; ti < T; ++ti) {
             const int t = t0 + ti;
             if (t >= a.n) break;
             const XT* xrow = static_cast<const XT*>(a.x) + (size_t)t * H;
-            if constexpr (sizeof(XT) == 4) {
+            if constexpr (kNorm) {
                 if (a.norm_w) {
                     // normalise the row in LDS first (the same three steps as in the logits blocks), quantise from there
                     float4* row = reinterpret_cast<float4*>(head_lds + HeadCfg<T, W>::RING_BYTES);
@@ -993,11 +994,11 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
             v = make_float4(u2f(q.x << 16), u2f(q.x & 0xffff0000u), u2f(q.y << 16), u2f(q.y & 0xffff0000u));
         }
         xl[i] = v;
-        if constexpr (sizeof(XT) == 4) {
+        if constexpr (kNorm) {
             if (a.norm_w) ring[i] = make_float4(fmul(v.x, v.x), fmul(v.y, v.y), fmul(v.z, v.z), fmul(v.w, v.w));
         }
     }
-    const HeadNorm nm{sizeof(XT) == 4 ? a.norm_w : nullptr, a.eps, xl, ring,
+    const HeadNorm nm{kNorm ? a.norm_w : nullptr, a.eps, xl, ring,
                       reinterpret_cast<float*>(head_lds + HeadCfg<T, W>::RING_BYTES + (size_t)T * H * 4), nk4, T};
     // wave 0 chains; wave 4 would share its SIMD (and its VALU issue slots) and only keeps the barriers company; the
     // others produce

@@ -69,6 +69,44 @@ def test_matmul_shape_errors(hip):
         hip.matmul(z(2, 3), z(4, 3), None, z(2, 2))
 
 
+# ---- the sum of squares behind rmsnorm: the serial chain's bits whichever part of it is walked in parallel ----
+def _sumsq_rows(dim, rng):
+    rows = [rng.normal(0, s, dim) for s in (1.0, 1e-3, 1e4, 1e-18, 1e-23, 1e17)]
+    rows += [np.sqrt(rng.integers(0, 1 << b, dim) * 2.0 ** -b) for b in (1, 3, 6, 10)]
+    rows += [rng.integers(-4, 5, dim) * 0.5, rng.integers(0, 64, dim) / 8.0,           # squares of few bits: exact ties
+             np.full(dim, 1.0), np.full(dim, 0.1), np.full(dim, 3.0 * 2.0 ** -12), np.zeros(dim)]
+    rows += [np.exp(np.linspace(-20, 20, dim)), np.exp(np.linspace(20, -20, dim))]       # a binade every few values / one
+    spike = rng.normal(0, 1, dim)
+    spike[dim // 2], spike[dim // 3] = 4096.0, 64.0
+    late = np.zeros(dim)
+    late[-3:] = [1e-30, 1e-12, 3.0]
+    rng_ties = 2.0 ** rng.integers(-13, 1, dim)                                           # halves of the running sum's ulp
+    rng_ties[0] = 4096.0
+    rows += [spike, late, rng_ties, -np.abs(rng.normal(0, 1, dim))]
+    return np.stack(rows).astype(np.float32)
+
+
+@pytest.mark.parametrize("dim", [4, 60, 64, 256, 260, 1000, 4096, 5120, 7168, 8192, 12296])
+def test_rmsnorm_sum_of_squares_is_the_serial_chain(hip, oracle, dim):
+    rng = np.random.default_rng(dim)
+    x = _sumsq_rows(dim, rng)
+    x = np.concatenate([x, x * np.float32(1.3), rng.normal(0, 1, (40, dim)).astype(np.float32)])
+    w = rng.normal(1, 0.1, dim).astype(np.float32)
+    out = torch.empty(x.shape, device=hip.device)
+    hip.rmsnorm(dev(hip, x), dev(hip, w), 1e-6, out)
+    assert np.array_equal(host(hip, out), oracle.rmsnorm(x, w, 1e-6))
+    # more rows than the four-waves-per-row kernel takes
+    many = np.tile(x, (1100 // len(x) + 1, 1))
+    out = torch.empty(many.shape, device=hip.device)
+    hip.rmsnorm(dev(hip, many), dev(hip, w), 1e-6, out)
+    assert np.array_equal(host(hip, out)[:len(x)], oracle.rmsnorm(x, w, 1e-6))
+    bad = x[:3].copy()
+    bad[0, dim // 2], bad[1, dim - 1], bad[2, 0] = np.inf, np.nan, 3e38
+    out = torch.empty(bad.shape, device=hip.device)
+    hip.rmsnorm(dev(hip, bad), dev(hip, w), 1e-6, out)
+    assert np.array_equal(host(hip, out), oracle.rmsnorm(bad, w, 1e-6), equal_nan=True)
+
+
 # ---- swiglu ----
 def test_swiglu_bit_exact_vs_oracle(hip, oracle):  # golden.rs:44-55 values included
     rng = np.random.default_rng(1)
