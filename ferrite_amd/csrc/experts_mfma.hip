@@ -115,6 +115,14 @@ __global__ __launch_bounds__(256) void pack_scales_kernel(PackSrc s, int n_exper
 template <int NR>
 __device__ __forceinline__ int b_lane(int lane) { return NR == 16 ? lane : (lane >> 4) * NR + (lane & (NR - 1)); }
 
+// Slot of the 16-byte piece (k step ktw, half h, quarter g) of row c in the operand image.  The row is XORed with the
+// piece's number, so that the pieces of one row, which neighbouring lanes write when the image is filled, land in
+// different banks; for the lanes of a read it is a permutation of neighbouring slots.
+template <int NR>
+__device__ __forceinline__ int b_slot(int ktw, int h, int g, int c) {
+    return ((ktw * 2 + h) * 4 + g) * NR + (c ^ (((ktw & 1) * 8 + h * 4 + g) & (NR - 1)));
+}
+
 struct BWindow {
     const u4v* bq;
     const u4v* bq2;
@@ -124,11 +132,12 @@ struct BWindow {
 
 template <int Q, bool kX2, int NR>
 __device__ __forceinline__ void mfma_step(const u4v (&a)[4], const u4v& sc, const BWindow& b, uint32_t bs, uint32_t bs2,
-                                          int ktw, int bl, v4f (&acc)[4]) {
+                                          int ktw, int lane, v4f (&acc)[4]) {
+    const int bg = lane >> 4, bc = lane & (NR - 1);
     const uint32_t scs[4] = {sc[0], sc[1], sc[2], sc[3]};
     {
-        const u4v b0 = b.bq[(ktw * 2 + 0) * (4 * NR) + bl];
-        const u4v b1 = b.bq[(ktw * 2 + 1) * (4 * NR) + bl];
+        const u4v b0 = b.bq[b_slot<NR>((ktw & ~3) | Q, 0, bg, bc)];
+        const u4v b1 = b.bq[b_slot<NR>((ktw & ~3) | Q, 1, bg, bc)];
         const v8i bv = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -138,8 +147,8 @@ __device__ __forceinline__ void mfma_step(const u4v (&a)[4], const u4v& sc, cons
         }
     }
     if constexpr (kX2) {
-        const u4v b0 = b.bq2[(ktw * 2 + 0) * (4 * NR) + bl];
-        const u4v b1 = b.bq2[(ktw * 2 + 1) * (4 * NR) + bl];
+        const u4v b0 = b.bq2[b_slot<NR>((ktw & ~3) | Q, 0, bg, bc)];
+        const u4v b1 = b.bq2[b_slot<NR>((ktw & ~3) | Q, 1, bg, bc)];
         const v8i bv = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -186,10 +195,10 @@ __device__ __forceinline__ void stream_group(const StreamRegs& r, const BWindow&
     uint32_t bs2 = 0;
     if constexpr (kX2) bs2 = b.bsc2[g4w * (4 * NR) + bl];
     const int kt = g4 * 4, ktw = g4w * 4;
-    mfma_step<0, kX2, NR>(r.a[BUF][0], r.sc[BUF], b, bs, bs2, ktw, bl, acc);
-    if (kt + 1 < KT) mfma_step<1, kX2, NR>(r.a[BUF][1], r.sc[BUF], b, bs, bs2, ktw + 1, bl, acc);
-    if (kt + 2 < KT) mfma_step<2, kX2, NR>(r.a[BUF][2], r.sc[BUF], b, bs, bs2, ktw + 2, bl, acc);
-    if (kt + 3 < KT) mfma_step<3, kX2, NR>(r.a[BUF][3], r.sc[BUF], b, bs, bs2, ktw + 3, bl, acc);
+    mfma_step<0, kX2, NR>(r.a[BUF][0], r.sc[BUF], b, bs, bs2, ktw, lane, acc);
+    if (kt + 1 < KT) mfma_step<1, kX2, NR>(r.a[BUF][1], r.sc[BUF], b, bs, bs2, ktw + 1, lane, acc);
+    if (kt + 2 < KT) mfma_step<2, kX2, NR>(r.a[BUF][2], r.sc[BUF], b, bs, bs2, ktw + 2, lane, acc);
+    if (kt + 3 < KT) mfma_step<3, kX2, NR>(r.a[BUF][3], r.sc[BUF], b, bs, bs2, ktw + 3, lane, acc);
 }
 
 // Groups [g_lo, g_hi) of the item against the window in LDS (whose first group is g_lo).  Group g_lo must already
@@ -241,9 +250,7 @@ struct BPlanes {
     __device__ __forceinline__ BWindow window() const { return BWindow{bq, bq2, bsc, bsc2}; }
 };
 
-// One 16-byte chunk / one scale word of a window: where it comes from and which slot of the B operand it fills.
-// row_src(r) gives the source row of unit row r (or -1).  Source rows are `pitch` bytes apart; scale rows are in
-// operand order (scale_pos), `spitch` bytes apart.
+// Source rows are `pitch` bytes apart; scale rows are in operand order (scale_pos), `spitch` bytes apart.
 template <bool kX2>
 struct BSource {
     ActPlanes src;
@@ -251,51 +258,57 @@ struct BSource {
     int spitch, nrows;
 };
 
-template <bool kX2, int NR, typename RowFn>
-__device__ __forceinline__ int b_chunk(const BSource<kX2>& s, RowFn row_src, int kt0, int wkt, int idx, u4v& v) {
-    const int chunks = wkt * 8;   // 16-byte chunks per row and plane in the window
-    const int p = idx / (s.nrows * chunks), rem = idx - p * (s.nrows * chunks);
-    const int c = rem / chunks, j = rem % chunks;
-    const int r = row_src(c);
-    const uint8_t* plane = p ? s.src.q2 : s.src.q;
-    v = (u4v){0u, 0u, 0u, 0u};
-    if (r >= 0) v = *reinterpret_cast<const u4v*>(plane + (size_t)r * s.pitch + (size_t)kt0 * 128 + (size_t)j * 16);
-    const int ktw = j >> 3, within = (j & 7) * 16;
-    const int half = within >> 6, g = (within & 63) >> 4;
-    return (p << 30) | ((ktw * 2 + half) * (4 * NR) + g * NR + c);
-}
-
-template <bool kX2, int NR, typename RowFn>
-__device__ __forceinline__ int b_scale_word(const BSource<kX2>& s, RowFn row_src, int kt0, int wkt, int idx, uint32_t& v) {
-    const int wg = (wkt + 3) / 4;
-    const int p = idx / (wg * 4 * NR), rem = idx - p * (wg * 4 * NR);
-    const int k4 = rem / (4 * NR), l = rem % (4 * NR), c = l % NR, g = l / NR;
-    v = 0x7f7f7f7fu;
-    if (c < s.nrows) {
-        const int r = row_src(c);
-        const uint8_t* plane = p ? s.src.s2 : s.src.s;
-        if (r >= 0) v = *reinterpret_cast<const uint32_t*>(plane + (size_t)r * s.spitch + (kt0 / 4 + k4) * 16 + g * 4);
-    }
-    return (p << 30) | rem;
-}
-
-// Copies k steps [kt0, kt0 + wkt) of the unit's rows into LDS in B-operand order and builds the packed scale words
-// (any window length; loads and stores alternate).
+// Copies k steps [kt0, kt0 + wkt) of the unit's rows into LDS in B-operand order and builds the packed scale words.
+// row_src(r) gives the source row of unit row r (or -1: zeros).  Work is dealt in pieces of 512 bytes (four k steps of one
+// row and plane), two to a wave's load; four loads are in flight.
+// At 192 tokens (two terms, 12 rows a unit) the gate/up kernel takes 168 us, 175 us with a loop of one load and one store
+// at a time, an integer division per 16 bytes and sixteen lanes of a store on the same banks (down, half as much per block, 92.9 -> 95.5).
 template <bool kX2, int NR = 16, typename RowFn>
 __device__ __forceinline__ void fill_b_window(const BSource<kX2>& s, RowFn row_src, int kt0, int wkt,
                                               const BPlanes<kX2, NR>& d) {
-    constexpr int NP = kX2 ? 2 : 1;
-    const int total = NP * s.nrows * wkt * 8;
-    for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-        u4v v;
-        const int slot = b_chunk<kX2, NR>(s, row_src, kt0, wkt, idx, v);
-        ((slot >> 30) ? d.bq2 : d.bq)[slot & 0x3fffffff] = v;
+    constexpr int NP = kX2 ? 2 : 1, BATCH = 4;
+    const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int chunks = wkt * 8, segs = (wkt + 3) / 4;   // 16-byte chunks of a row's window, pieces of 32 chunks
+    const int rows = s.nrows * NP;                      // (row, plane) pairs, planes of a row together
+    const int ids = (lane & 15) < s.nrows ? row_src(lane & 15) : -1;   // the unit's rows, one per lane
+    int rp = 0, seg = 2 * wave;                         // of the wave's first piece; the second is the one behind it
+    while (seg >= segs) { seg -= segs; ++rp; }
+    while (rp < rows) {
+        u4v v[BATCH];
+        int slot[BATCH];
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            slot[b] = -1;
+            v[b] = (u4v){0u, 0u, 0u, 0u};
+            if (rp < rows) {   // wave-uniform
+                const bool wrap = seg + 1 >= segs;
+                const int rp1 = min(rp + (wrap ? 1 : 0), rows - 1), seg1 = wrap ? 0 : seg + 1;
+                const int r0 = __builtin_amdgcn_readlane(ids, rp / NP), r1 = __builtin_amdgcn_readlane(ids, rp1 / NP);
+                const bool second = lane >= 32;
+                const int rpl = second ? rp1 : rp, r = second ? r1 : r0;
+                const int c = rpl / NP, p = rpl % NP, j = (second ? seg1 : seg) * 32 + (lane & 31);
+                if (j < chunks && !(second && wrap && rp + 1 >= rows)) {
+                    const uint8_t* plane = p ? s.src.q2 : s.src.q;
+                    if (r >= 0) v[b] = *reinterpret_cast<const u4v*>(plane + (size_t)r * s.pitch + (size_t)kt0 * 128 + (size_t)j * 16);
+                    slot[b] = (p << 30) | b_slot<NR>(j >> 3, (j >> 2) & 1, j & 3, c);
+                }
+                seg += 2 * waves;
+                while (seg >= segs) { seg -= segs; ++rp; }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b)
+            if (slot[b] >= 0) ((slot[b] >> 30) ? d.bq2 : d.bq)[slot[b] & 0x3fffffff] = v[b];
     }
     const int wg = (wkt + 3) / 4;
-    for (int idx = threadIdx.x; idx < NP * wg * 4 * NR; idx += blockDim.x) {
-        uint32_t v;
-        const int slot = b_scale_word<kX2, NR>(s, row_src, kt0, wkt, idx, v);
-        ((slot >> 30) ? d.bsc2 : d.bsc)[slot & 0x3fffffff] = v;
+    const int c = threadIdx.x % NR, g = (threadIdx.x / NR) & 3;
+    const int r = c < s.nrows ? row_src(c) : -1;
+    for (int t = threadIdx.x / (4 * NR); t < NP * wg; t += blockDim.x / (4 * NR)) {
+        const int p = t >= wg ? 1 : 0, k4 = t - p * wg;
+        uint32_t v = 0x7f7f7f7fu;
+        if (r >= 0) v = *reinterpret_cast<const uint32_t*>((p ? s.src.s2 : s.src.s) + (size_t)r * s.spitch + (kt0 / 4 + k4) * 16 + g * 4);
+        (p ? d.bsc2 : d.bsc)[k4 * (4 * NR) + g * NR + c] = v;
     }
 }
 
