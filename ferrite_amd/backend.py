@@ -9,11 +9,17 @@ subclasses (never a crash), exactly as the reference returns `Err` for shape pro
 
 torch is used for device memory and streams only.  There is no CPU fallback: if the shared library is missing
 or no GPU is present the constructor raises.
+
+Calls run on torch's current stream, like torch's own ops: what was queued there before a call has run when the call
+reads its inputs, what is queued there after it sees its outputs, and a tensor freed after the call is not reused before
+the call has run.  Calls of one backend run one after the other whatever streams and threads they come from, because they
+share workspaces and graphs.  `stream` is a stream of the backend's own, for captures.
 """
 from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 from dataclasses import dataclass
 from typing import Dict, List, Optional
 
@@ -230,6 +236,40 @@ class MoeLayer:
         self._ws: Dict[tuple, torch.Tensor] = {}
 
 
+class _Launch:
+    """`with backend._launch() as st:` - st is the stream that the call's launches go to (HipBackend._begin_call)."""
+    __slots__ = ("be", "stream", "device")
+
+    def __init__(self, be: "HipBackend"):
+        self.be = be
+
+    def __enter__(self):
+        be = self.be
+        self.device = torch.cuda.current_device()
+        be._turn.acquire()
+        try:
+            if self.device != be.device.index:   # a handle of 0 means the current device's default stream
+                torch.cuda.set_device(be.device)
+            self.stream = be._begin_call()
+        except BaseException:
+            self._restore()
+            raise
+        return C.c_void_p(self.stream.cuda_stream)
+
+    def __exit__(self, *exc):
+        try:
+            self.be._end_call(self.stream)
+        finally:
+            self._restore()
+
+    def _restore(self):
+        try:
+            if self.device != self.be.device.index:
+                torch.cuda.set_device(self.device)
+        finally:
+            self.be._turn.release()
+
+
 class HipBackend:
     def __init__(self, so_path: Optional[str] = None, device: int = 0):
         self.lib = load_library(so_path)
@@ -237,7 +277,10 @@ class HipBackend:
             raise FerriteError("no GPU visible: HipBackend has no CPU path")
         self.device = torch.device("cuda", device)
         torch.cuda.set_device(self.device)
-        self.stream = torch.cuda.Stream(device=self.device)   # one stream per backend (cuda.rs:996)
+        self._own = torch.cuda.Stream(device=self.device)   # what captures record on (cuda.rs:996)
+        self._turn = threading.RLock()   # one call at a time, from the choice of its stream to its last launch
+        self._last = None                # the stream of the latest call
+        self._done = torch.cuda.Event()  # behind the latest call, see _end_call
         self.recorder = Recorder()
         self._capturing = False
         self._graphs: Dict[str, int] = {}
@@ -249,9 +292,6 @@ class HipBackend:
     @property
     def build_id(self) -> str:
         return self.lib.ferrite_kernel_build_id().decode()
-
-    def _st(self):
-        return C.c_void_p(self.stream.cuda_stream)
 
     def _ck(self, rc: int, what: str):
         if rc == OK:
@@ -271,35 +311,60 @@ class HipBackend:
             raise InvalidArg(f"{what} must be contiguous")
         return t
 
-    def _enter(self, mark=None):
-        """Make this backend's stream wait for work already queued on torch's current stream (not while a
-        capture is open: the capture must stay on one stream), or for what was queued there at `mark`."""
-        if not self._capturing:
-            if mark is None:
-                self.stream.wait_stream(torch.cuda.current_stream(self.device))
-            else:
-                self.stream.wait_event(mark)
+    def _launch(self) -> _Launch:
+        return _Launch(self)
 
-    def _leave(self):
-        """Make torch's current stream wait for what was just enqueued, so torch ops on the outputs are ordered."""
-        if not self._capturing:
-            torch.cuda.current_stream(self.device).wait_stream(self.stream)
-
-    def _mark_and_leave(self):
-        """What a call on caller-allocated buffers starts with: the point of torch's current stream that its launches
-        have to wait for (the argument of _enter), taken before that stream is made to wait for this backend's earlier
-        work.  Taken after it, the mark would be reached only once that earlier work has ended, and every call of a
-        back-to-back sequence would begin with two cross-queue signals on an idle GPU: 21 us between the last kernel
-        of one call and the first of the next (32 tokens, H 4096: 244 us a call, 234 us this way).  The backend's
-        earlier work is on its own stream, so waiting for it there adds no ordering."""
+    def _begin_call(self):
+        """The stream a call runs on: torch's current one, behind the backend's earlier calls; the backend's own while its
+        capture is open (a capture stays on one stream)."""
         if self._capturing:
-            return None
-        mark = torch.cuda.current_stream(self.device).record_event()
-        self._leave()
-        return mark
+            return self._own
+        cur = torch.cuda.current_stream(self.device)
+        if torch.cuda.is_current_stream_capturing():
+            # another capture orders nothing against this backend's other calls, and a workspace made inside it would
+            # belong to its graph
+            if cur != self._own:
+                raise FerriteError("a capture that this backend has not begun is open on torch's current stream")
+        elif cur != self._last:
+            self._follow(cur)
+        return cur
+
+    def _end_call(self, stream):
+        # The default stream and the backend's own outlive every call, so the event is recorded on them only when another
+        # stream has to wait for it; any other stream may be gone by then.
+        if stream.cuda_stream != 0 and stream != self._own:
+            self._done.record(stream)
+
+    def _follow(self, stream):
+        """Make `stream` the next to run calls: it waits for the latest call."""
+        last = self._last
+        if last is not None and last != stream:
+            if last.cuda_stream == 0 or last == self._own:
+                self._done.record(last)
+            stream.wait_event(self._done)
+        self._last = stream
+
+    @property
+    def stream(self):
+        """The backend's own stream.  Work that a program queues on it after this access runs behind the calls made
+        before the access and ahead of the calls made after that work was queued."""
+        with self._turn:
+            own_capture = self._capturing or (torch.cuda.current_stream(self.device) == self._own
+                                              and torch.cuda.is_current_stream_capturing())
+            if not own_capture and self._last != self._own:
+                self._follow(self._own)
+        return self._own
 
     def sync(self):
-        self.stream.synchronize()
+        """Wait for every call made so far and for the backend's own stream."""
+        self._own.synchronize()
+        last = self._last
+        if last is None or last == self._own:
+            return
+        if last.cuda_stream == 0:
+            last.synchronize()
+        else:
+            self._done.synchronize()
 
     def set_override(self, which: int, value: int):
         """Process-wide test hook of the library (token tile of the expert GEMMs, f32 expert outputs).  Changes the
@@ -317,7 +382,6 @@ class HipBackend:
     def matmul(self, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor):
         """lib.rs:73 / cpu.rs:82-122 (recorded twice, like the reference: cpu.rs:89-90)."""
         self.recorder.record("matmul")
-        mark = self._mark_and_leave()
         self.recorder.record("matmul")
         if x.dim() != 2 or w.dim() != 2:
             raise InvalidArg("matmul operands must be 2-d")
@@ -332,28 +396,26 @@ class HipBackend:
             self._dev(bias, torch.float32, "bias")
             if bias.numel() != o:
                 raise InvalidArg("matmul bias shape")
-        self._enter(mark)
-        self._ck(self.lib.ferrite_matmul_f32(x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(),
-                                             out.data_ptr(), n, k, o, self._st()), "matmul")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_matmul_f32(x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(),
+                                                 out.data_ptr(), n, k, o, st), "matmul")
 
     def rmsnorm(self, x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor):
         """lib.rs:76 / cpu.rs:124-143: x, out [..., dim] f32, w [dim] f32."""
         self.recorder.record("rmsnorm")
-        mark = self._mark_and_leave()
         if x.dim() < 1:
             raise InvalidArg("rmsnorm rank 0")
         dim = x.shape[-1]
         if w.numel() != dim or tuple(out.shape) != tuple(x.shape):
             raise InvalidArg("rmsnorm shape mismatch")
         self._dev(x, torch.float32, "x"); self._dev(w, torch.float32, "w"); self._dev(out, torch.float32, "out")
-        self._enter(mark)
-        self._ck(self.lib.ferrite_rmsnorm_f32(x.data_ptr(), w.data_ptr(), eps, out.data_ptr(), x.numel() // dim, dim,
-                                              self._st()), "rmsnorm")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_rmsnorm_f32(x.data_ptr(), w.data_ptr(), eps, out.data_ptr(), x.numel() // dim, dim, st),
+                     "rmsnorm")
 
     def hc_post(self, x: torch.Tensor, residual: torch.Tensor, post: torch.Tensor, comb: torch.Tensor) -> torch.Tensor:
         """lib.rs:256 / cpu.rs:788-807: x [s,h], residual [s,nh,h], post [s,nh], comb [s,nh,nh] -> new [s,nh,h]."""
         self.recorder.record("hc_post")
-        self._leave()
         if x.dim() != 2 or residual.dim() != 3:
             raise InvalidArg("hc_post expects x [s,h] and residual [s,nh,h]")
         s, h = x.shape
@@ -363,15 +425,14 @@ class HipBackend:
         for t, nm in ((x, "x"), (residual, "residual"), (post, "post"), (comb, "comb")):
             self._dev(t, torch.float32, nm)
         out = torch.empty_like(residual)
-        self._enter()
-        self._ck(self.lib.ferrite_hc_post_f32(x.data_ptr(), residual.data_ptr(), post.data_ptr(), comb.data_ptr(),
-                                              out.data_ptr(), s, nh, h, self._st()), "hc_post")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_hc_post_f32(x.data_ptr(), residual.data_ptr(), post.data_ptr(), comb.data_ptr(),
+                                                  out.data_ptr(), s, nh, h, st), "hc_post")
         return out
 
     def swiglu_limited(self, gate_up: torch.Tensor, limit: float, out: torch.Tensor):
         """lib.rs:83-85 / cpu.rs:178-203"""
         self.recorder.record("swiglu")
-        mark = self._mark_and_leave()
         if gate_up.dim() != 2:
             raise InvalidArg("swiglu input must be 2-d")
         n, two_i = gate_up.shape
@@ -380,16 +441,14 @@ class HipBackend:
         if tuple(out.shape) != (n, two_i // 2):
             raise InvalidArg(f"swiglu out {tuple(out.shape)} != [{n},{two_i // 2}]")
         self._dev(gate_up, torch.float32, "gate_up"); self._dev(out, torch.float32, "out")
-        self._enter(mark)
-        self._ck(self.lib.ferrite_swiglu_limited_f32(gate_up.data_ptr(), limit, out.data_ptr(), n, two_i // 2,
-                                                     self._st()), "swiglu")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_swiglu_limited_f32(gate_up.data_ptr(), limit, out.data_ptr(), n, two_i // 2, st), "swiglu")
 
     def moe_route(self, logits: torch.Tensor, bias: torch.Tensor, topk: int, routed_scaling: float,
                   probs: torch.Tensor, ids: torch.Tensor, n_group: int = 1, topk_group: int = 1,
                   ids_i32: Optional[torch.Tensor] = None):
         """lib.rs:194-206 / cpu.rs:528-572; ids is an f32 tensor as in the reference."""
         self.recorder.record("moe_route")
-        mark = self._mark_and_leave()
         self.recorder.record("moe_route")
         if logits.dim() != 2:
             raise InvalidArg("logits must be 2-d")
@@ -402,10 +461,10 @@ class HipBackend:
         self._dev(probs, torch.float32, "probs"); self._dev(ids, torch.float32, "ids")
         if ids_i32 is not None:
             self._dev(ids_i32, torch.int32, "ids_i32")
-        self._enter(mark)
-        self._ck(self.lib.ferrite_moe_route(logits.data_ptr(), bias.data_ptr(), n, e, topk, n_group, topk_group,
-                                            routed_scaling, probs.data_ptr(), ids.data_ptr(),
-                                            None if ids_i32 is None else ids_i32.data_ptr(), self._st()), "moe_route")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_moe_route(logits.data_ptr(), bias.data_ptr(), n, e, topk, n_group, topk_group,
+                                                routed_scaling, probs.data_ptr(), ids.data_ptr(),
+                                                None if ids_i32 is None else ids_i32.data_ptr(), st), "moe_route")
 
     # ---- inherent ops ----
     def moe_permute(self, ids: torch.Tensor, n_experts: int) -> Dict[str, torch.Tensor]:
@@ -419,12 +478,12 @@ class HipBackend:
                  active=mk(n_experts), n_active=mk(1))
         sb = self.lib.ferrite_moe_permute_scratch_bytes(n, topk, n_experts)
         scratch = torch.empty(max(sb, 16), dtype=torch.uint8, device=self.device)
-        self._enter()
-        self._ck(self.lib.ferrite_moe_permute(ids.data_ptr(), n, topk, n_experts, t["counts"].data_ptr(),
-                                              t["starts"].data_ptr(), t["perm_map"].data_ptr(),
-                                              t["gather_src"].data_ptr(), t["active"].data_ptr(),
-                                              t["n_active"].data_ptr(), scratch.data_ptr(), sb, self._st()),
-                 "moe_permute")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_moe_permute(ids.data_ptr(), n, topk, n_experts, t["counts"].data_ptr(),
+                                                  t["starts"].data_ptr(), t["perm_map"].data_ptr(),
+                                                  t["gather_src"].data_ptr(), t["active"].data_ptr(),
+                                                  t["n_active"].data_ptr(), scratch.data_ptr(), sb, st),
+                     "moe_permute")
         self.sync()   # scratch goes out of scope
         return t
 
@@ -435,10 +494,9 @@ class HipBackend:
         if scale.numel() != rows * (cols // 32):
             raise ShapeMismatch("scale shape")
         out = torch.empty(tuple(w.shape[:-1]) + (cols,), dtype=torch.float32, device=self.device)
-        self._enter()
-        self._ck(self.lib.ferrite_mxfp4_dequant(w.data_ptr(), scale.data_ptr(), rows, cols, out.data_ptr(),
-                                                self._st()), "mxfp4_dequant")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_mxfp4_dequant(w.data_ptr(), scale.data_ptr(), rows, cols, out.data_ptr(), st),
+                     "mxfp4_dequant")
         return out
 
     def mxfp4_quant(self, x: torch.Tensor):
@@ -451,10 +509,9 @@ class HipBackend:
         self._dev(x, x.dtype, "x")
         codes = torch.empty((rows, cols // 2), dtype=torch.uint8, device=self.device)
         s = torch.empty((rows, cols // 32), dtype=torch.uint8, device=self.device)
-        self._enter()
-        self._ck(self.lib.ferrite_mxfp4_quant(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
-                                              cols, codes.data_ptr(), s.data_ptr(), self._st()), "mxfp4_quant")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_mxfp4_quant(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
+                                                  cols, codes.data_ptr(), s.data_ptr(), st), "mxfp4_quant")
         return codes, s
 
     def pack_expert(self, layer: MoeLayer, expert: int, gate=None, up=None, down=None, gate_up_scale_pitch: int = 0,
@@ -471,10 +528,9 @@ class HipBackend:
             setattr(src, key + "_w", w.data_ptr()); setattr(src, key + "_s", s.data_ptr())
             keep += [w, s]
         src.gate_up_scale_pitch, src.down_scale_pitch = gate_up_scale_pitch, down_scale_pitch
-        self._enter()
-        self._ck(self.lib.ferrite_moe_pack_expert(C.byref(layer.shape), expert, C.byref(src), layer.packed.data_ptr(),
-                                                  self._st()), "pack_expert")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_moe_pack_expert(C.byref(layer.shape), expert, C.byref(src), layer.packed.data_ptr(), st),
+                     "pack_expert")
 
     def act_quant_fp8(self, x: torch.Tensor):
         if x.dtype not in (torch.float32, torch.bfloat16) or x.dim() != 2 or not x.is_contiguous():
@@ -484,10 +540,9 @@ class HipBackend:
             raise InvalidArg("cols must be a multiple of 32")
         q = torch.empty((rows, cols), dtype=torch.uint8, device=self.device)
         s = torch.empty((rows, cols // 32), dtype=torch.uint8, device=self.device)
-        self._enter()
-        self._ck(self.lib.ferrite_act_quant_fp8(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
-                                                cols, q.data_ptr(), s.data_ptr(), self._st()), "act_quant_fp8")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_act_quant_fp8(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
+                                                    cols, q.data_ptr(), s.data_ptr(), st), "act_quant_fp8")
         return q, s
 
     def act_quant_fp8_x2(self, x: torch.Tensor):
@@ -499,11 +554,10 @@ class HipBackend:
             raise InvalidArg("cols must be a multiple of 32")
         mk = lambda c: torch.empty((rows, c), dtype=torch.uint8, device=self.device)
         q1, s1, q2, s2 = mk(cols), mk(cols // 32), mk(cols), mk(cols // 32)
-        self._enter()
-        self._ck(self.lib.ferrite_act_quant_fp8_x2(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
-                                                   cols, q1.data_ptr(), s1.data_ptr(), q2.data_ptr(), s2.data_ptr(),
-                                                   self._st()), "act_quant_fp8_x2")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_act_quant_fp8_x2(x.data_ptr(), DT_F32 if x.dtype == torch.float32 else DT_BF16, rows,
+                                                       cols, q1.data_ptr(), s1.data_ptr(), q2.data_ptr(), s2.data_ptr(),
+                                                       st), "act_quant_fp8_x2")
         return q1, s1, q2, s2
 
     # ---- the fused layer ----
@@ -517,9 +571,9 @@ class HipBackend:
             if nbytes == 0:
                 raise Declined("shape not supported by the MFMA path")
             layer.packed = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            self._enter()
-            self._ck(self.lib.ferrite_moe_pack_weights(C.byref(layer.shape), C.byref(layer.weights),
-                                                       layer.packed.data_ptr(), self._st()), "pack_weights")
+            with self._launch() as st:
+                self._ck(self.lib.ferrite_moe_pack_weights(C.byref(layer.shape), C.byref(layer.weights),
+                                                           layer.packed.data_ptr(), st), "pack_weights")
             self.sync()
         if not keep_checkpoint_layout:
             for k in _WEIGHT_FIELDS[2:]:
@@ -533,10 +587,9 @@ class HipBackend:
         inter = cfg.shared_inter if expert == cfg.n_experts else cfg.inter
         rows, cols = (cfg.hidden, inter) if which == 2 else (inter, cfg.hidden)
         out = torch.empty((rows, cols), dtype=torch.float32, device=self.device)
-        self._enter()
-        self._ck(self.lib.ferrite_moe_packed_dequant(C.byref(layer.shape), layer.packed.data_ptr(), expert, which,
-                                                     out.data_ptr(), self._st()), "packed_dequant")
-        self._leave()
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_moe_packed_dequant(C.byref(layer.shape), layer.packed.data_ptr(), expert, which,
+                                                         out.data_ptr(), st), "packed_dequant")
         return out
 
     def effective_mode(self, layer: MoeLayer, n: int, mode: int) -> int:
@@ -563,12 +616,18 @@ class HipBackend:
             if nbytes == 0:
                 raise InvalidArg("unsupported shape / mode")
             ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            self._enter()
-            self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
-                                                               self._st()), "workspace_init")
-            self._leave()
+            with self._launch() as st:
+                self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
+                                                                   st), "workspace_init")
             layer._ws[key] = ws
-        return layer._ws[key]
+        return self._on_this_stream(layer._ws[key])
+
+    def _on_this_stream(self, ws: torch.Tensor) -> torch.Tensor:
+        """A cached workspace may be dropped with its layer while a call on another stream than the one it was allocated
+        on still uses it."""
+        if not self._capturing:
+            ws.record_stream(torch.cuda.current_stream(self.device))
+        return ws
 
     def unit_rows(self, layer: MoeLayer, n: int, mode: int = MODE_MFMA_FP8) -> int:
         """Token tile of the expert GEMMs for such a call: 16 (streaming kernels), or the tiled kernels' 128 (one-term
@@ -580,7 +639,6 @@ class HipBackend:
         """The whole layer on the device: router GEMM -> route -> permute -> experts -> combine (+shared).
         x [n, H] f32 or bf16, out [n, H] f32 or bf16, both pre-allocated device tensors."""
         self.recorder.record("moe_layer_mxfp4")
-        mark = self._mark_and_leave()
         cfg = layer.cfg
         if x.dim() != 2 or x.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"x {tuple(x.shape)} vs hidden {cfg.hidden}")
@@ -594,21 +652,19 @@ class HipBackend:
         if mode != MODE_F32_CHECK and layer.packed is None:
             raise InvalidArg("layer has no packed weights")
         ws = workspace if workspace is not None else self.workspace(layer, n, mode)
-        self._enter(mark)
-        args = (C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
-                x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, ws.data_ptr(), ws.numel(),
-                self._st())
-        if stage_events is None:
-            self._ck(self.lib.ferrite_moe_layer_mxfp4(*args), "moe_layer_mxfp4")
-        else:
-            if len(stage_events) != STAGE_EVENTS:
-                raise InvalidArg(f"stage_events must hold {STAGE_EVENTS} event handles")
-            self._ck(self.lib.ferrite_moe_layer_mxfp4_timed(*args, stage_events), "moe_layer_mxfp4")
+        if stage_events is not None and len(stage_events) != STAGE_EVENTS:
+            raise InvalidArg(f"stage_events must hold {STAGE_EVENTS} event handles")
+        with self._launch() as st:
+            args = (C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
+                    x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, ws.data_ptr(), ws.numel(), st)
+            if stage_events is None:
+                self._ck(self.lib.ferrite_moe_layer_mxfp4(*args), "moe_layer_mxfp4")
+            else:
+                self._ck(self.lib.ferrite_moe_layer_mxfp4_timed(*args, stage_events), "moe_layer_mxfp4")
 
     def moe_layer_dev_mxfp4_static(self, layer: MoeLayer, x: torch.Tensor, out: torch.Tensor, mode: int = MODE_MFMA_FP8):
         """The same layer on the library's built-in workspace: nothing is allocated, here or in the library."""
         self.recorder.record("moe_layer_mxfp4")
-        mark = self._mark_and_leave()
         cfg = layer.cfg
         if x.dim() != 2 or x.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"x {tuple(x.shape)} vs hidden {cfg.hidden}")
@@ -618,10 +674,10 @@ class HipBackend:
         dts = {torch.float32: DT_F32, torch.bfloat16: DT_BF16}
         if x.dtype not in dts or out.dtype not in dts or not x.is_contiguous() or not out.is_contiguous():
             raise InvalidArg("x/out must be contiguous f32 or bf16 device tensors")
-        self._enter(mark)
-        rc = self.lib.ferrite_moe_layer_mxfp4_static(
-            C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
-            x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, self._st())
+        with self._launch() as st:
+            rc = self.lib.ferrite_moe_layer_mxfp4_static(
+                C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
+                x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, st)
         if rc == ERR_WORKSPACE:
             raise FerriteError(self.lib.ferrite_hip_last_error().decode())
         self._ck(rc, "moe_layer_mxfp4_static")
@@ -634,12 +690,11 @@ class HipBackend:
             if nbytes == 0:
                 raise InvalidArg("unsupported shape / mode")
             ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            self._enter()
-            self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
-                                                               self._st()), "workspace_init")
-            self._leave()
+            with self._launch() as st:
+                self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
+                                                                   st), "workspace_init")
             layer._ws[key] = ws
-        return layer._ws[key]
+        return self._on_this_stream(layer._ws[key])
 
     def moe_block_mxfp4(self, layer: MoeLayer, li: torch.Tensor, norm_w: torch.Tensor, eps: float,
                         residual: Optional[torch.Tensor], post: Optional[torch.Tensor], comb: Optional[torch.Tensor],
@@ -648,7 +703,6 @@ class HipBackend:
         li [n,H] f32, residual/out [n,nh,H] f32, post [n,nh], comb [n,nh,nh].  residual None: rmsnorm -> MoE FFN
         only, out [n,H]."""
         self.recorder.record("moe_block_mxfp4")
-        mark = self._mark_and_leave()
         cfg = layer.cfg
         if li.dim() != 2 or li.shape[1] != cfg.hidden:
             raise ShapeMismatch(f"li {tuple(li.shape)} vs hidden {cfg.hidden}")
@@ -672,11 +726,11 @@ class HipBackend:
         ws = workspace if workspace is not None else self.block_workspace(layer, n, mode)
         ptr = lambda t: None if t is None else t.data_ptr()
         blk = MoeBlockArgs(norm_w.data_ptr(), eps, ptr(residual), ptr(post), ptr(comb), nh)
-        self._enter(mark)
-        self._ck(self.lib.ferrite_moe_block_mxfp4(C.byref(layer.shape), C.byref(layer.weights),
-                                                  None if layer.packed is None else layer.packed.data_ptr(),
-                                                  li.data_ptr(), C.byref(blk), n, out.data_ptr(), mode, ws.data_ptr(),
-                                                  ws.numel(), self._st()), "moe_block_mxfp4")
+        with self._launch() as st:
+            self._ck(self.lib.ferrite_moe_block_mxfp4(C.byref(layer.shape), C.byref(layer.weights),
+                                                      None if layer.packed is None else layer.packed.data_ptr(),
+                                                      li.data_ptr(), C.byref(blk), n, out.data_ptr(), mode, ws.data_ptr(),
+                                                      ws.numel(), st), "moe_block_mxfp4")
 
     def workspace_view(self, layer: MoeLayer, n: int, mode: int,
                        workspace: Optional[torch.Tensor] = None) -> Dict[str, torch.Tensor]:
@@ -712,15 +766,16 @@ class HipBackend:
     def begin_capture(self):
         """Start stream capture; ops issued until end_capture are recorded into a graph, not executed."""
         self.recorder.begin_capture()
-        self._enter()
-        self._ck(self.lib.ferrite_graph_begin(self._st()), "graph_begin")
-        self._capturing = True
+        with self._turn:
+            self._ck(self.lib.ferrite_graph_begin(C.c_void_p(self.stream.cuda_stream)), "graph_begin")
+            self._capturing = True
 
     def end_capture(self) -> OpTrace:
         """End capture and instantiate.  The returned trace carries the op names and the graph handle."""
         exec_ = C.c_void_p()
-        self._capturing = False
-        rc = self.lib.ferrite_graph_end(self._st(), C.byref(exec_))
+        with self._turn:
+            self._capturing = False
+            rc = self.lib.ferrite_graph_end(C.c_void_p(self._own.cuda_stream), C.byref(exec_))
         trace = self.recorder.end_capture()
         if rc != OK:
             raise FerriteError(f"graph capture failed: {self.lib.ferrite_hip_last_error().decode()}")
@@ -731,8 +786,8 @@ class HipBackend:
         """Replay launch of the captured graph into the same static buffers."""
         if trace.graph_exec is None:
             raise InvalidArg("trace holds no graph")
-        self._enter()
-        rc = self.lib.ferrite_graph_launch(C.c_void_p(trace.graph_exec), self._st())
+        with self._launch() as st:
+            rc = self.lib.ferrite_graph_launch(C.c_void_p(trace.graph_exec), st)
         self._verify_ok = rc == OK
 
     def end_verify(self) -> bool:

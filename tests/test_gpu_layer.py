@@ -754,3 +754,57 @@ def test_few_tokens_share_items_among_waves(hip, oracle, n, hidden, inter, share
     inp = synth.make_inputs(cfg, seed=n)
     layer = hip.load_moe_layer(inp)
     check_mfma(hip, oracle, layer, inp, mode)
+
+
+def test_calls_are_ordered_with_torch_ops_on_any_stream(hip):
+    """No synchronisation by the program: inputs made by torch ops just before a call, outputs read by torch ops just
+    behind it, temporaries dropped at once, calls and graph replays of one layer and workspace on alternating streams.
+    The same bits as one call at a time with a synchronisation around each."""
+    cfg = synth.CONFIGS["c0"].with_tokens(24)
+    layer = hip.load_moe_layer(synth.make_inputs(cfg, seed=31))
+    ws = hip.block_workspace(layer, 24, MODE_MFMA_FP8)
+    w = torch.rand(cfg.hidden, device=hip.device) + 0.5
+    xs, outs = torch.zeros(24, cfg.hidden, device=hip.device), torch.zeros(24, cfg.hidden, device=hip.device)
+
+    def call(x, out):
+        hip.moe_block_mxfp4(layer, x, w, 1e-6, None, None, None, out, MODE_MFMA_FP8, workspace=ws)
+
+    call(xs, outs)
+    hip.begin_capture()
+    call(xs, outs)
+    trace = hip.end_capture()
+    base = torch.randn(24, cfg.hidden, device=hip.device)
+    torch.cuda.synchronize()
+
+    want = []
+    for i in range(40):
+        x, out, h = base * (i + 1) - 3.0, torch.empty_like(base), torch.empty_like(base)
+        torch.cuda.synchronize()
+        call(x, out)
+        hip.sync()
+        hip.rmsnorm(out, w, 1e-6, h)
+        hip.sync()
+        want.append(h * 2.0)
+    torch.cuda.synchronize()
+
+    streams = [torch.cuda.default_stream(hip.device), torch.cuda.Stream(hip.device), hip.stream, torch.cuda.Stream(hip.device)]
+    got, replay_done = [], None
+    for i in range(40):
+        with torch.cuda.stream(streams[i % 4]):
+            h = torch.empty_like(base)
+            if i % 3 == 1:
+                if replay_done is not None:
+                    replay_done.wait()   # the replay's buffers are the program's own
+                xs.copy_(base * (i + 1) - 3.0)
+                hip.begin_verify(trace)
+                hip.rmsnorm(outs, w, 1e-6, h)
+                replay_done = torch.cuda.current_stream().record_event()
+            else:
+                out = torch.empty_like(base)
+                call(base * (i + 1) - 3.0, out)
+                hip.rmsnorm(out, w, 1e-6, h)
+                del out
+            got.append(h * 2.0)
+    torch.cuda.synchronize()
+    hip.graph_destroy(trace)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
