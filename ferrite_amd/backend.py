@@ -277,7 +277,8 @@ class HipBackend:
             raise FerriteError("no GPU visible: HipBackend has no CPU path")
         self.device = torch.device("cuda", device)
         torch.cuda.set_device(self.device)
-        self._own = torch.cuda.Stream(device=self.device)   # what captures record on (cuda.rs:996)
+        # what captures record on (cuda.rs:996); streams are compared by their handles (torch's `stream != None` is False)
+        self._own = torch.cuda.Stream(device=self.device)
         self._turn = threading.RLock()   # one call at a time, from the choice of its stream to its last launch
         self._last = None                # the stream of the latest call
         self._done = torch.cuda.Event()  # behind the latest call, see _end_call
@@ -323,23 +324,28 @@ class HipBackend:
         if torch.cuda.is_current_stream_capturing():
             # another capture orders nothing against this backend's other calls, and a workspace made inside it would
             # belong to its graph
-            if cur != self._own:
+            if cur.cuda_stream != self._own.cuda_stream:
                 raise FerriteError("a capture that this backend has not begun is open on torch's current stream")
-        elif cur != self._last:
+        else:
             self._follow(cur)
         return cur
+
+    def _outlives_calls(self, stream):
+        return stream.cuda_stream in (0, self._own.cuda_stream)
 
     def _end_call(self, stream):
         # The default stream and the backend's own outlive every call, so the event is recorded on them only when another
         # stream has to wait for it; any other stream may be gone by then.
-        if stream.cuda_stream != 0 and stream != self._own:
+        if not self._outlives_calls(stream):
             self._done.record(stream)
 
     def _follow(self, stream):
         """Make `stream` the next to run calls: it waits for the latest call."""
         last = self._last
-        if last is not None and last != stream:
-            if last.cuda_stream == 0 or last == self._own:
+        if last is not None:
+            if last.cuda_stream == stream.cuda_stream:
+                return
+            if self._outlives_calls(last):
                 self._done.record(last)
             stream.wait_event(self._done)
         self._last = stream
@@ -349,9 +355,8 @@ class HipBackend:
         """The backend's own stream.  Work that a program queues on it after this access runs behind the calls made
         before the access and ahead of the calls made after that work was queued."""
         with self._turn:
-            own_capture = self._capturing or (torch.cuda.current_stream(self.device) == self._own
-                                              and torch.cuda.is_current_stream_capturing())
-            if not own_capture and self._last != self._own:
+            own_is_current = torch.cuda.current_stream(self.device).cuda_stream == self._own.cuda_stream
+            if not (self._capturing or (own_is_current and torch.cuda.is_current_stream_capturing())):
                 self._follow(self._own)
         return self._own
 
@@ -359,12 +364,8 @@ class HipBackend:
         """Wait for every call made so far and for the backend's own stream."""
         self._own.synchronize()
         last = self._last
-        if last is None or last == self._own:
-            return
-        if last.cuda_stream == 0:
-            last.synchronize()
-        else:
-            self._done.synchronize()
+        if last is not None:
+            (last if self._outlives_calls(last) else self._done).synchronize()
 
     def set_override(self, which: int, value: int):
         """Process-wide test hook of the library (token tile of the expert GEMMs, f32 expert outputs).  Changes the

@@ -808,3 +808,45 @@ def test_calls_are_ordered_with_torch_ops_on_any_stream(hip):
     torch.cuda.synchronize()
     hip.graph_destroy(trace)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_sync_waits_and_a_call_on_another_stream_follows(hip):
+    """About 4 ms of calls are queued on one stream: sync() returns behind them, and a call on another stream, which the
+    program orders with nothing, reads what the last of them wrote."""
+    x = torch.randn(4000, 4096, device=hip.device)
+    w = torch.rand(4096, device=hip.device) + 0.5
+    bufs, h = [torch.empty_like(x) for _ in range(2)], torch.empty_like(x)
+    streams = [torch.cuda.default_stream(hip.device), torch.cuda.Stream(hip.device), hip.stream]
+
+    def work():
+        src = x
+        for i in range(100):
+            hip.rmsnorm(src, w, 1e-6, bufs[i & 1])
+            src = bufs[i & 1]
+        return src
+
+    last = work()
+    hip.rmsnorm(last, w, 1e-6, h)
+    torch.cuda.synchronize()
+    want = h.clone()
+    for busy in streams:
+        for other in streams:
+            bufs[0].zero_(); bufs[1].zero_(); h.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(busy):
+                last = work()
+                assert not busy.query()
+            with torch.cuda.stream(other):
+                hip.rmsnorm(last, w, 1e-6, h)
+            hip.sync()
+            assert busy.query() and other.query()
+            assert torch.equal(h, want)
+    hip.begin_capture()
+    work()
+    trace = hip.end_capture()
+    for s in streams:
+        with torch.cuda.stream(s):
+            hip.begin_verify(trace)
+        hip.sync()
+        assert s.query()
+    hip.graph_destroy(trace)

@@ -27,6 +27,11 @@ class Stream:
         self.before, self.capturing = set(), False
         Sim.streams[self.cuda_stream] = self
 
+    def __eq__(self, other):
+        raise TypeError("streams are compared by their handles: torch's `stream != None` is False")
+
+    __ne__ = __eq__
+
     def record_event(self, event=None):
         event = event or Event()
         event.record(self)
