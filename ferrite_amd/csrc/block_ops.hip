@@ -13,8 +13,8 @@ constexpr int RN_CHUNK = 4096;   // floats of one row staged in LDS at a time (1
 
 // KernelBackend::rmsnorm (crates/ferrite-kernel/src/cpu.rs:124-143).  The reference sums the squares of a row left
 // to right in f32, so the sum is a serial chain of `dim` adds.  One wave per row: the lanes square 64 elements at a
-// time into LDS (order-independent, each rounded once), then the wave sums the staged chunk (sumsq_walk).  Second pass:
-// out = (x * inv) * w.  2047 rows of 4096: 26 us (38 us with the chain walked value by value).
+// time into LDS (order-independent, each rounded once), then the wave sums the staged chunk (sumsq_chain, sumsq_walk).  Second pass:
+// out = (x * inv) * w.  2047 rows of 4096: 20 us (28 us with the chain alone).
 __global__ __launch_bounds__(64) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w, float eps,
                                                      float* __restrict__ out, int dim) {
     __shared__ __align__(16) float sq[RN_CHUNK];
@@ -50,7 +50,8 @@ __global__ __launch_bounds__(64) void rmsnorm_kernel(const float* __restrict__ x
             }
         }
         __syncthreads();
-        ss = sumsq_walk(reinterpret_cast<const float4*>(sq), len4 / 4, ss);
+        const float4* s4 = reinterpret_cast<const float4*>(sq);
+        ss = dim <= 4 * SUMSQ_SHORT ? sumsq_chain(s4, len4 / 4, ss) : sumsq_walk(s4, len4 / 4, ss);
         __syncthreads();
     }
     ss = fdiv(ss, (float)dim);
@@ -71,12 +72,12 @@ __global__ __launch_bounds__(64) void rmsnorm_kernel(const float* __restrict__ x
 
 // The same with four waves per row, for rows of up to 8192 16-byte-aligned floats: every thread keeps its part of
 // the row and of w in registers (one pass over memory instead of two, four times the loads in flight), wave 0 walks
-// the chain over the whole row's squares, the others wait.  192 rows of 4096: 11.1 us (14.8 us with the chain walked value
-// by value, 21.5 us before that with one wave per row).
+// the chain over the whole row's squares, the others wait.  192 rows of 4096: 11 us (14.3 us with the chain alone,
+// 21.5 us before that with one wave per row).
 constexpr int RN_ROW_MAX = 8192;
 
 template <int NV>
-__global__ __launch_bounds__(256, NV == 8 ? 2 : 4) void rmsnorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(256, 4) void rmsnorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                           float eps, float* __restrict__ out, int dim) {
     extern __shared__ __align__(16) float sq[];   // the row's squares, zero padded to whole pieces of 256 values, + 1/rms
     const int tid = threadIdx.x;
@@ -103,7 +104,10 @@ __global__ __launch_bounds__(256, NV == 8 ? 2 : 4) void rmsnorm_row_kernel(const
     }
     __syncthreads();
     if (tid < 64) {
-        float ss = sumsq_walk(reinterpret_cast<const float4*>(sq), pad4, 0.0f);
+        const float4* s4 = reinterpret_cast<const float4*>(sq);
+        float ss = 0.0f;   // (a kernel of one length class has the registers of one form)
+        if (NV == 1 || (NV == 2 && pad4 <= SUMSQ_SHORT)) ss = sumsq_chain(s4, pad4, ss);
+        else ss = sumsq_walk(s4, pad4, ss);
         ss = fdiv(ss, (float)dim);
         const float inv = fdiv(1.0f, fsqrt(fadd(ss, eps)));
         if (tid == 0) sq[pad4 * 4] = inv;

@@ -115,22 +115,50 @@ __device__ __forceinline__ uint32_t quant_block32_x2(const XT* __restrict__ src,
     return s1 | (s2 << 8);
 }
 
-// The chain itself over n4 float4 of LDS: every lane reads the same addresses and holds the same running sum.
-__device__ __forceinline__ float sumsq_chain(const float4* p, int n4, float ss) {
-    int j = 0;
-#pragma unroll 1
-    for (; j + 4 <= n4; j += 4) {
-        const float4 r[4] = {p[j], p[j + 1], p[j + 2], p[j + 3]};
+// The left-to-right f32 sum (separately rounded adds, the reference's rmsnorm order: cpu.rs:124-143) of the n4 float4 at
+// s4 in LDS, continued from ss.  Every lane reads the same addresses and holds the same running sum.  For short rows.
+// Straight-line pieces of eight batches (256 values): a batch of eight 16-byte reads is in flight while the 32
+// dependent adds of the batch before it run, and nothing is in flight at the end of a piece.  With the two
+// register buffers carried around a loop instead, the compiler copied one buffer into the other every iteration and
+// waited for every outstanding read at the top of a batch: 15 us for 4096 values against 10 us this way.
+constexpr int SUMSQ_SHORT = 384;   // float4; beyond that sumsq_walk is sooner through
+__device__ __forceinline__ float sumsq_piece(const float4* p, float ss) {
+    constexpr int NB = 8;
+    float4 r[2][8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            ss = fadd(ss, r[i].x);
-            ss = fadd(ss, r[i].y);
-            ss = fadd(ss, r[i].z);
-            ss = fadd(ss, r[i].w);
+    for (int j = 0; j < 8; ++j) r[0][j] = p[j];
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+        if (g + 1 < NB) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[(g + 1) & 1][j] = p[(g + 1) * 8 + j];
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xC87F);   // lgkmcnt <= 8: everything but the batch just issued
+        } else {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xC07F);
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float4 q = r[g & 1][j];
+            ss = fadd(ss, q.x);
+            ss = fadd(ss, q.y);
+            ss = fadd(ss, q.z);
+            ss = fadd(ss, q.w);
+        }
+        // pins the batch's adds in front of the next batch's reads (the optimiser otherwise hoists all 64 reads of
+        // the piece to its top, 256 registers) and the reads behind it
+        asm volatile("" : "+v"(ss) : : "memory");
+        __builtin_amdgcn_sched_barrier(0);
     }
-    for (; j < n4; ++j) {
-        const float4 q = p[j];
+    return ss;
+}
+
+__device__ __forceinline__ float sumsq_chain(const float4* s4, int n4, float ss) {
+    const int pieces = n4 >> 6;
+    for (int i = 0; i < pieces; ++i) ss = sumsq_piece(s4 + i * 64, ss);
+    for (int j = pieces * 64; j < n4; ++j) {
+        const float4 q = s4[j];
         ss = fadd(ss, q.x);
         ss = fadd(ss, q.y);
         ss = fadd(ss, q.z);
@@ -139,77 +167,141 @@ __device__ __forceinline__ float sumsq_chain(const float4* p, int n4, float ss) 
     return ss;
 }
 
-// Inclusive sum over the wave's lanes.
+// A wave's inclusive scan: of sums, or of steps (see sumsq_walk), where a lane's step is taken behind those before it.
+// row_shr 1, 2, 4, 8 within rows of 16; lane 15 of rows 0, 2 to rows 1, 3; lane 31 to rows 2 and 3.  Lanes without a
+// source get 0, the step that changes nothing.
+#define FE_WAVE_SCAN(STEP) \
+    STEP(0x111, 0xf, true) STEP(0x112, 0xf, true) STEP(0x114, 0xf, true) STEP(0x118, 0xf, true) STEP(0x142, 0xa, false) STEP(0x143, 0xc, false)
 __device__ __forceinline__ int wave_prefix(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr 1, 2, 4, 8: within rows of 16
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // lane 15 of rows 0, 2 to rows 1, 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // lane 31 to rows 2 and 3
+#define FE_STEP(CTRL, ROWS, BOUND) v += __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, BOUND);
+    FE_WAVE_SCAN(FE_STEP)
+#undef FE_STEP
     return v;
 }
+__device__ __forceinline__ void wave_prefix_steps(int& even, int& odd) {
+#define FE_STEP(CTRL, ROWS, BOUND)                                                                                             \
+    {                                                                                                                          \
+        const int e = __builtin_amdgcn_update_dpp(0, even, CTRL, ROWS, 0xf, BOUND);                                             \
+        const int o = __builtin_amdgcn_update_dpp(0, odd, CTRL, ROWS, 0xf, BOUND);                                              \
+        const int ne = e + ((e & 1) ? odd : even), no = o + ((o & 1) ? even : odd);                                            \
+        even = ne;                                                                                                             \
+        odd = no;                                                                                                              \
+    }
+    FE_WAVE_SCAN(FE_STEP)
+#undef FE_STEP
+}
+#undef FE_WAVE_SCAN
 
-// The left-to-right f32 sum (separately rounded adds, the reference's rmsnorm order: cpu.rs:124-143) of the n4 float4 at
-// s4 in LDS, all values >= 0 or NaN, continued from ss >= 0; called by a whole wave, the result is in every lane.
-// The chain is serial, but most of it can be walked in parallel with the same bits.  While the running sum s stays
+// The same sum for long rows, all values >= +0 or NaN and ss >= 0; called by a whole wave.
+// The chain is serial, but most of it can be worked out in parallel with the same bits.  While the running sum s stays
 // within one binade it is M ulp with M in [2^23, 2^24), and adding q rounds to M + rint(q / ulp), whatever M is, unless
-// q / ulp lies halfway between two integers (round to even then asks for M's parity).  So a lane takes 16 consecutive
-// values of a chunk of 1024 and adds their integers; a prefix sum over the lanes says up to which lane s stays in its
-// binade.  What does not fit - the first 128 values and sums below 2^-100, the 16 values in which s passes a power of
-// two or a tie occurs, values above s / 8 (which keeps the integers small and exact) - is walked by the chain itself,
-// then the rest of the chunk goes on.  4096 normal values take about 4 + 12 rounds and 6 us, 10 us with the chain alone (192 rows
-// of rmsnorm 15.0 -> 11.1 us, 2047 rows 38 -> 26 us, the head of one token with its norm 40 -> 36 us).
+// q / ulp lies halfway between two integers (a tie): then the even neighbour of the exact sum is taken, which depends on
+// M's parity.  So a lane takes 16 consecutive values of a chunk of 1024 and adds their integers; a prefix sum over the
+// lanes says up to which lane s stays in its binade.  What does not fit - the first 128 values and sums below 2^-100, the
+// 16 values in which s passes a power of two - is walked value by value: every lane adds its own 16 to s, and the result
+// of the lane whose turn it is counts.  So are lanes with a tie while they are few; where they are many (rows of values
+// that were rounded to bf16 or fp8) every lane works out the step that its values make from an even M and from an odd
+// one, and the scan composes steps.  Zeros are passed over; a chunk that has been left ten times is walked to its end.
+//
+// us of rmsnorm, 192 rows           2048: normal bf16    4096: normal bf16 zeros     7168: normal bf16
+//   chain alone                           8.0    8.0           14.3   14.2   14.4          23.7   23.8
+//   without steps, zeros walked           8.5   27.9           10.7   31.4   26.0          13.5   80.2
+//   this way                              8.3    8.4           11.0   10.7    3.9          13.4   15.0
+// At 1024 values the chain takes 5.0 us, this way 6.2 to 7.3; at 8192 rows of 2048 45 and 37.  With steps from 3 / 5 / 9 / 13
+// tied lanes on (one run): 4096 bf16 10.8 / 11.5 / 12.7 / 13.4, 7168 normal 14.6 / 14.0 / 13.9 / 13.8.
+constexpr int SUMSQ_TIES = 4;
 __device__ __forceinline__ float sumsq_walk(const float4* s4, int n4, float ss) {
     const int lane = threadIdx.x & 63;
     uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)f2u(ss));
 #pragma unroll 1
     for (int base = 0; base < n4; base += 256) {
-        float4 q[4];   // values past the end are +0: adding them changes nothing
+        const float4* p = s4 + base + lane * 4;
+        float4 v[4];
+        if (base + 256 <= n4) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            q[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (base + lane * 4 + i < n4) q[i] = s4[base + lane * 4 + i];
+            for (int i = 0; i < 4; ++i) v[i] = p[i];
+        } else {   // values past the end are +0: adding them changes nothing
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (base + lane * 4 + i < n4) v[i] = p[i];
+            }
         }
-        int first = 0, ex_of = -1, prefix = 0, taken = 0;   // lanes below `first` are in s; their prefix is `taken`
-        bool bad = false;
+        const float q[16] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w,
+                             v[2].x, v[2].y, v[2].z, v[2].w, v[3].x, v[3].y, v[3].z, v[3].w};
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bits |= f2u(q[i]);
+        unsigned long long todo = __ballot(bits != 0);   // lanes that are not in s yet; zeros need not be
+        int ex_of = -1, left = 0;
+        int even = 0, odd = 0;   // the lane's step in ulp of ex_of; 2^24, past any binade's end, where it has none
+        bool ties = false;
 #pragma unroll 1
-        while (first < 64) {
+        while (todo != 0) {
+            int first = __builtin_ctzll(todo);
             const int ex = (int)(sb >> 23);
-            int lanes = 8;   // that the chain walks next
+            int walk = 8;   // lanes that are walked next
             if (ex >= 27 && ex < 255) {
                 if (ex != ex_of) {
                     const float scale = u2f((uint32_t)(277 - ex) << 23);   // 1 / ulp
-                    float total = 0.0f, top = 0.0f, off = 0.0f;
-                    bool nan = false;
+                    float total = 0.0f, off = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float tx = q[i].x * scale, ty = q[i].y * scale, tz = q[i].z * scale, tw = q[i].w * scale;
-                        const float rx = rintf(tx), ry = rintf(ty), rz = rintf(tz), rw = rintf(tw);
-                        top = fmaxf(fmaxf(top, fmaxf(tx, ty)), fmaxf(tz, tw));   // ignores NaN
-                        off = fmaxf(fmaxf(off, fmaxf(fabsf(tx - rx), fabsf(ty - ry))), fmaxf(fabsf(tz - rz), fabsf(tw - rw)));
-                        total += (rx + ry) + (rz + rw);   // at most 2^24: exact
+                    for (int i = 0; i < 16; i += 2) {
+                        const float t0 = q[i] * scale, t1 = q[i + 1] * scale, r0 = rintf(t0), r1 = rintf(t1);
+                        off = fmaxf(off, fmaxf(fabsf(t0 - r0), fabsf(t1 - r1)));
+                        total += r0 + r1;   // exact up to 2^24
                     }
-                    nan = !(total <= 16777216.0f);
-                    bad = nan || top > 1048576.0f || off == 0.5f;
-                    prefix = wave_prefix(bad ? 0 : (int)total);
-                    taken = first > 0 ? __builtin_amdgcn_readlane(prefix, first - 1) : 0;
+                    const bool none = !(total <= 16777216.0f);   // NaN too
+                    const bool tied = !none && off == 0.5f;
+                    ties = __builtin_popcountll(__ballot(tied) & todo) > SUMSQ_TIES;
+                    if (ties) {
+                        float again = scale;          // the quotients are worked out a second time: kept, they take
+                        asm("" : "+v"(again));        // 32 registers, which cost the rows' kernels a block per CU
+                        even = 0;
+                        odd = 1;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            const float t = q[i] * again, r = rintf(t), f = fabsf(t - r) == 0.5f ? t : r;
+                            const int twice = (int)(f + f), whole = twice >> 1, half = twice & 1;
+                            even += whole;
+                            even += even & half;   // a half that follows an odd number makes it even, else it is dropped
+                            odd += whole;
+                            odd += odd & half;
+                        }
+                        odd -= 1;
+                        if (none) even = odd = 1 << 24;
+                    } else {
+                        even = (none || tied) ? 1 << 24 : (int)total;
+                    }
                     ex_of = ex;
                 }
-                int m = (int)((sb & 0x7fffffu) | 0x800000u);
-                const unsigned long long stop = __ballot(lane >= first && (bad || m + (prefix - taken) > 0xffffff));
-                const int last = stop ? __builtin_ctzll(stop) : 64;
-                if (last > first) m += __builtin_amdgcn_readlane(prefix, last - 1) - taken;
-                sb = ((uint32_t)ex << 23) | ((uint32_t)m & 0x7fffffu);
-                if (last == 64) break;
-                first = last;
-                lanes = 1;
-                taken = __builtin_amdgcn_readlane(prefix, last);
+                const int m = (int)((sb & 0x7fffffu) | 0x800000u);
+                int at = lane >= first ? even : 0;
+                if (ties) {
+                    int from_odd = lane >= first ? odd : 0;
+                    wave_prefix_steps(at, from_odd);
+                    if (m & 1) at = from_odd;
+                } else {
+                    at = wave_prefix(at);
+                }
+                at += m;   // where s stands behind this lane
+                const unsigned long long stop = __ballot(at > 0xffffff);
+                if (stop == 0) {
+                    sb = ((uint32_t)ex << 23) | ((uint32_t)__builtin_amdgcn_readlane(at, 63) & 0x7fffffu);
+                    break;
+                }
+                first = __builtin_ctzll(stop);
+                if (first > 0) sb = ((uint32_t)ex << 23) | ((uint32_t)__builtin_amdgcn_readlane(at, first - 1) & 0x7fffffu);
+                walk = ++left > 10 ? 64 : 1;
             }
-            const int at = base + first * 4;
-            ss = sumsq_chain(s4 + at, min(4 * lanes, n4 - at), u2f(sb));
-            sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)f2u(ss));
-            first += lanes;
+#pragma unroll 1
+            do {
+                float t = u2f(sb);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) t = fadd(t, q[i]);
+                sb = (uint32_t)__builtin_amdgcn_readlane((int)f2u(t), first++);
+            } while (--walk > 0 && first < 64);
+            todo = first < 64 ? todo >> first << first : 0;
         }
     }
     return u2f(sb);

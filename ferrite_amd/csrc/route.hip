@@ -814,7 +814,8 @@ __device__ __forceinline__ void head_first_sync(const HeadNorm& nm) {
     const int tid = threadIdx.x;
     if (tid < 64) {
         for (int ti = 0; ti < nm.T; ++ti) {
-            float ss = sumsq_walk(nm.sq + (size_t)ti * nm.nk4, nm.nk4, 0.0f);
+            const float4* sq = nm.sq + (size_t)ti * nm.nk4;
+            float ss = nm.nk4 <= SUMSQ_SHORT ? sumsq_chain(sq, nm.nk4, 0.0f) : sumsq_walk(sq, nm.nk4, 0.0f);
             ss = fdiv(ss, (float)(nm.nk4 * 4));
             const float inv = fdiv(1.0f, fsqrt(fadd(ss, nm.eps)));
             if (tid == 0) nm.inv[ti] = inv;

@@ -1,5 +1,7 @@
 """GPU parity of the op-level entry points against the CPU oracle, through the C ABI.
 Integer/byte results and everything routing depends on are compared bit for bit."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -105,6 +107,58 @@ def test_rmsnorm_sum_of_squares_is_the_serial_chain(hip, oracle, dim):
     out = torch.empty(bad.shape, device=hip.device)
     hip.rmsnorm(dev(hip, bad), dev(hip, w), 1e-6, out)
     assert np.array_equal(host(hip, out), oracle.rmsnorm(bad, w, 1e-6), equal_nan=True)
+
+
+def _narrow(x, keep):
+    """f32 values rounded to `keep` mantissa bits (7: bf16)."""
+    drop = 23 - keep
+    u = x.view(np.uint32).astype(np.uint64)
+    u = (u + (1 << (drop - 1)) - 1 + ((u >> drop) & 1)) >> drop << drop
+    return u.astype(np.uint32).view(np.float32)
+
+
+def _value_kinds(rows, dim):
+    """What a residual stream may hold: squares of narrow values make ties of the running sum, zeros leave it as it is."""
+    x = np.random.default_rng(dim).normal(0, 1, (rows, dim)).astype(np.float32)
+    sparse = x * (np.random.default_rng(dim + 1).random((rows, dim)) < 0.1)
+    return dict(normal=x, bf16=_narrow(x, 7), bf16_small=_narrow(x * np.float32(0.037), 7), fp16=_narrow(x, 10), fp8=_narrow(x, 3),
+                zeros=np.zeros_like(x), sparse=sparse.astype(np.float32))
+
+
+@pytest.mark.parametrize("dim", [256, 1028, 4096, 7168])
+def test_rmsnorm_of_narrow_values_is_the_serial_chain(hip, oracle, dim):
+    w = np.random.default_rng(3).normal(1, 0.1, dim).astype(np.float32)
+    for kind, x in _value_kinds(40, dim).items():
+        out = torch.empty(x.shape, device=hip.device)
+        hip.rmsnorm(dev(hip, x), dev(hip, w), 1e-6, out)
+        assert np.array_equal(host(hip, out), oracle.rmsnorm(x, w, 1e-6)), kind
+
+
+@pytest.mark.parametrize("dim", [4096, 7168])
+def test_rmsnorm_takes_no_longer_for_narrow_values(hip, dim):
+    """Rows of bf16 values or of zeros go the same parallel way as any others.  (Walked value by value they took three
+    to seven times as long; 2 leaves room for the parity scan and for the clock.)"""
+    w = torch.ones(dim, device=hip.device)
+    took = {}
+    for kind, x in _value_kinds(192, dim).items():
+        x, out = dev(hip, x), torch.empty(192, dim, device=hip.device)
+        hip.rmsnorm(x, w, 1e-6, out)
+        hip.begin_capture()
+        for _ in range(50):
+            hip.rmsnorm(x, w, 1e-6, out)
+        trace = hip.end_capture()
+        hip.begin_verify(trace)
+        times = []
+        for _ in range(5):
+            hip.sync()
+            t0 = time.perf_counter()
+            hip.begin_verify(trace)
+            hip.sync()
+            times.append(time.perf_counter() - t0)
+        hip.graph_destroy(trace)
+        took[kind] = min(times) / 50 * 1e6
+    print({k: round(v, 1) for k, v in took.items()})
+    assert max(took.values()) < 2.0 * took["normal"], took
 
 
 # ---- swiglu ----
