@@ -9,8 +9,8 @@ namespace fe {
 // ------------------------------------------------------------------------------------------------
 // x . w^T with the reference's arithmetic (crates/ferrite-kernel/src/cpu.rs:106-111): for every output one
 // chain s = 0; s = fl(s + fl(x[l] * w[l])) in ascending l.  The chain cannot be re-associated, its adds stay on the
-// vector ALU.  Two kernels; both stage x and w through LDS as f32 in chunks of 64 k, with the fetches of several chunks
-// in flight in registers and one barrier per chunk.
+// vector ALU.  Three kernels; all stage x and w through LDS as f32 in chunks of 64 k, the first two with the fetches of
+// several chunks in flight in registers and one barrier per chunk.
 //
 // chain_mfma_kernel, for enough chains: the products come from the matrix cores (an f32 MFMA on a zero accumulator
 // gives the correctly rounded product; -0 comes out as +0, which a chain that starts at +0 cannot see).  A wave owns
@@ -24,6 +24,9 @@ namespace fe {
 // chain_valu_kernel, for few chains, where a chain's own length is the time: one chain per lane (8 tokens x 8 outputs per
 // wave), multiply and add on the vector ALU.  A lone wave issues one instruction per four cycles.
 //
+// chain_rows_kernel, for a few rows of x against very many outputs, where w's way through memory is the time: a wave has one
+// row, a lane one output, so that the chip is not occupied with padding rows.
+//
 // us:                                                   before    mfma    valu
 //   router 8192 tokens x 256, H 7168 (bf16 x)              735     648     -       (valu, 4 x 4 chains per lane: 620)
 //   router 4096 x 128, H 4096 (bf16 x)                     149     105     -       (2 x 2 chains per lane: 125)
@@ -31,6 +34,14 @@ namespace fe {
 //   router 509 x 128, H 4096 (bf16 x)                       47      50     42
 //   100 x 3072, k 4096 / 100 x 4096, k 1536             168 / 78   91 / 40  -      (2 x 2: 109 / 47)
 //   100 x 128, k 4096 / 27 x 32, k 2080                  70 / 37   46 / 25  35 / 20
+// The lines between them, us:                          mfma    valu    rows
+//   384 / 512 tiles (32 x 3072, 1024 x 128), k 4096      64      46
+//   560 / 672 / 768 tiles                                64      63 / 63 / 66
+//   784 / 1024 tiles                                     64 / 65 79 / 84
+//   512 / 640 / 768 tiles, k 7168                       109      76 / 106 / 109
+//   4 x 17000 / 32768 / 65536, k 4096              86 / 127 / 238  82 / 174 / 332  67 / 123 / 199
+//   4 x 32768 / 65536, k 256                          9.8 / 20  12 / 22  7.0 / 13
+//   8 x 65536, k 4096 / 256                           236 / 21  341 / 22  384 / 23 (two passes over w)
 // Also built: x through DPP broadcasts or v_readlane instead of LDS (161 and 177 us for the second line: both instructions
 // cost several plain ones); operands read from memory in MFMA order without LDS (64 requests per load to the address
 // unit: 121 us for 100 x 3072); one chunk in flight instead of three (51 against 46 us for 100 x 128).
@@ -73,7 +84,7 @@ __device__ __forceinline__ bool chain_block(const ChainArgs& a, int& t0, int& o0
 // of the block, its rows or pieces group * 4 * WN .. are fetched by the calling wave.  Piece j of row r sits at slot
 // 16 r + (j ^ r) of its tile: the sixteen neighbouring lanes of a write and of a read touch different banks.  Rows past
 // the end repeat the last one, pieces past K are zero (they add +0 to the chains).
-template <typename XT, bool kPackedW, int WN>
+template <typename XT, bool kPackedW, int WN, bool kShort>
 struct ChainFetch {
     const XT* xrow;
     const float* wrow[WN];
@@ -100,6 +111,7 @@ struct ChainFetch {
         }
     }
     __device__ __forceinline__ void load(Set& f, int c) const {   // past the end the last chunk again, never used
+        if (kShort && c >= nchunk) return;
         c = min(c, nchunk - 1);
         const int k = min(c * CH_KC + pj * 4, K - 4);
         if constexpr (sizeof(XT) == 4) {
@@ -114,6 +126,7 @@ struct ChainFetch {
             f.w[i] = *reinterpret_cast<const ch_f4*>(wrow[i] + (kPackedW ? (size_t)c * CH_PIECES * 4 * w_pitch : (size_t)k));
     }
     __device__ __forceinline__ void store(const Set& f, int c, ch_f4* xs, ch_f4* ws) const {
+        if (kShort && c >= nchunk) return;
         const bool in = min(c, nchunk - 1) * CH_KC + pj * 4 < K;   // the transposed weight comes with K % 64 == 0
         const ch_f4 zero = {0.f, 0.f, 0.f, 0.f};
         ch_f4 xv = f.x;
@@ -129,7 +142,7 @@ struct ChainFetch {
 
 // Block = 4 waves: 16 tokens x 64 outputs.  Chunks c and c + 1 are readable while chunk c is walked, chunk c + 2 is
 // written at its start; three more chunks are on their way.
-template <typename XT, bool kPackedW>
+template <typename XT, bool kPackedW, bool kShort>
 __global__ __launch_bounds__(256, 2) void chain_mfma_kernel(ChainArgs a) {
     __shared__ ch_f4 xs[3][CH_TILE];
     __shared__ ch_f4 ws[4][3][CH_TILE];
@@ -138,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void chain_mfma_kernel(ChainArgs a) {
     int t0, o0;
     if (!chain_block<4>(a, t0, o0)) return;   // the whole block
     o0 += wave * CH_T;                        // may lie past o: such a wave works on the last row
-    const ChainFetch<XT, kPackedW, 4> src(a, t0, o0, 0);
+    const ChainFetch<XT, kPackedW, 4, kShort> src(a, t0, o0, 0);
     const int nchunk = src.nchunk;
     ch_f4 xo[2], wo[2];
     auto read = [&](int at, int u, int to) {
@@ -149,7 +162,7 @@ __global__ __launch_bounds__(256, 2) void chain_mfma_kernel(ChainArgs a) {
     const ch_f16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 
-    typename ChainFetch<XT, kPackedW, 4>::Set f[3];   // f[c % 3]: chunk c
+    typename ChainFetch<XT, kPackedW, 4, kShort>::Set f[3];   // f[c % 3]: chunk c
     src.load(f[0], 0);
     src.load(f[1], 1);
     src.load(f[2], 2);
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(256, 2) void chain_mfma_kernel(ChainArgs a) {
 
 // Block = 4 waves, two by two: 16 tokens x 16 outputs.  Chunk c + 1 is written while chunk c is walked; three more are
 // on their way.
-template <typename XT, bool kPackedW>
+template <typename XT, bool kPackedW, bool kShort>
 __global__ __launch_bounds__(256, 2) void chain_valu_kernel(ChainArgs a) {
     constexpr int FD = 4;   // even: a register set's LDS slot is a constant
     __shared__ ch_f4 xs[2][CH_TILE], ws[2][CH_TILE];
@@ -210,11 +223,11 @@ __global__ __launch_bounds__(256, 2) void chain_valu_kernel(ChainArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int t0, o0;
     if (!chain_block<1>(a, t0, o0)) return;   // the whole block
-    const ChainFetch<XT, kPackedW, 1> src(a, t0, o0, wave);
+    const ChainFetch<XT, kPackedW, 1, kShort> src(a, t0, o0, wave);
     const int nchunk = src.nchunk;
     const int xr = (wave >> 1) * 8 + (lane >> 3), wr = (wave & 1) * 8 + (lane & 7);
     float acc = 0.0f;
-    typename ChainFetch<XT, kPackedW, 1>::Set f[FD];   // f[c % FD]: chunk c
+    typename ChainFetch<XT, kPackedW, 1, kShort>::Set f[FD];   // f[c % FD]: chunk c
 #pragma unroll
     for (int i = 0; i < FD; ++i) src.load(f[i], i);
     src.store(f[0], 0, xs[0], ws[0]);
@@ -249,18 +262,77 @@ __global__ __launch_bounds__(256, 2) void chain_valu_kernel(ChainArgs a) {
     if (t < a.n && col < a.o) a.out[(size_t)t * a.o + col] = a.bias ? fadd(acc, a.bias[col]) : acc;
 }
 
-// The line between the two: 512 tiles of 16 x 16 chains are two waves of the one-chain-per-lane kernel for each of the
-// chip's 1024 SIMDs; beyond that its LDS reads bound it, and below that the matrix-core kernel leaves SIMDs idle.
+// Block = 4 waves: up to 4 rows x 64 outputs, w transposed in LDS so that a lane reads four consecutive k of its row
+// at once, two buffers.
+constexpr int CR_ROWS = 4, CR_OUTS = 64;
+
+__global__ __launch_bounds__(256, 4) void chain_rows_kernel(ChainArgs a) {
+    __shared__ ch_f4 ws[2][CH_PIECES][CR_OUTS + 1];
+    __shared__ ch_f4 xs[2][CR_ROWS][CH_PIECES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int o0 = blockIdx.x * CR_OUTS, K = a.k;
+    const int nchunk = (K + CH_KC - 1) / CH_KC;
+    const int pr = tid >> 4, pj = tid & 15;   // a thread stages piece pj of w rows pr, pr + 16, .. and of x row pr
+    const float* xrow = static_cast<const float*>(a.x) + (size_t)min(pr, a.n - 1) * K;
+    const ch_f4 zero = {0.f, 0.f, 0.f, 0.f};
+    ch_f4 w[4], x = zero;
+    auto fetch = [&](int c) {   // pieces past K are zero, rows past the end repeat the last one
+        const int k = c * CH_KC + pj * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            w[i] = k < K ? *reinterpret_cast<const ch_f4*>(a.w + (size_t)min(o0 + pr + 16 * i, a.o - 1) * K + k) : zero;
+        if (pr < CR_ROWS) x = k < K ? *reinterpret_cast<const ch_f4u*>(xrow + k) : zero;
+    };
+    auto stash = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ws[buf][pj][pr + 16 * i] = w[i];
+        if (pr < CR_ROWS) xs[buf][pr][pj] = x;
+    };
+    float acc = 0.0f;
+    fetch(0);
+    stash(0);
+    __syncthreads();
+    for (int c = 0; c < nchunk; ++c) {
+        const int buf = c & 1;
+        if (c + 1 < nchunk) fetch(c + 1);
+#pragma unroll 4
+        for (int j = 0; j < CH_PIECES; ++j) {
+            const ch_f4 wv = ws[buf][j][lane], xv = xs[buf][wave][j];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = fadd(acc, fmul(xv[q], wv[q]));
+        }
+        if (c + 1 < nchunk) stash(buf ^ 1);
+        __syncthreads();
+    }
+    const int col = o0 + lane;
+    if (wave < a.n && col < a.o) a.out[(size_t)wave * a.o + col] = a.bias ? fadd(acc, a.bias[col]) : acc;
+}
+
+// Which kernel (figures at the top): 512 tiles of 16 x 16 chains are two waves of the one-chain-per-lane kernel for each of
+// the chip's 1024 SIMDs; beyond that its LDS reads bound it, and below that the matrix-core kernel leaves SIMDs idle.  Up to
+// four rows against more than 1024 tiles of outputs take the kernel that has no padding rows.
+// Up to 128 k the fetches that run ahead are not made past the end: they would be most of all fetches (24 x 65536, k 64:
+// 15 -> 11 us; 1 x 12288: 4.3 -> 3.7).  At 256 k, and with it in the loop of longer chains, the waits that the conditional loads
+// need cost more than the fetches (131072 outputs, k 256: 35 -> 38; 32768, k 4096: 127 -> 143).
+constexpr int CH_SHORT = 128, CH_ROWS_TILES = 1024;
+
 template <typename XT, bool kPackedW>
 static int launch_chain(ChainArgs a, hipStream_t st) {
     const long tg = ((long)a.n + CH_T - 1) / CH_T, ot = ((long)a.o + CH_T - 1) / CH_T;
+    if constexpr (sizeof(XT) == 4 && !kPackedW) {
+        if (a.n <= CR_ROWS && ot > CH_ROWS_TILES) {
+            chain_rows_kernel<<<(unsigned)((a.o + CR_OUTS - 1) / CR_OUTS), 256, 0, st>>>(a);
+            return check_launch("chain_rows");
+        }
+    }
     const bool mfma = tg * ot > 512;
     const long og = mfma ? (ot + 3) / 4 : ot;
     a.x_major = (size_t)a.n * sizeof(XT) >= (size_t)a.o * sizeof(float);
     const long blocks = ((a.x_major ? tg : og) + 7) / 8 * 8 * (a.x_major ? og : tg);
     if (blocks > 0x7fffffffL) return FERRITE_DECLINED;
-    if (mfma) chain_mfma_kernel<XT, kPackedW><<<(unsigned)blocks, 256, 0, st>>>(a);
-    else chain_valu_kernel<XT, kPackedW><<<(unsigned)blocks, 256, 0, st>>>(a);
+    auto go = [&](auto kernel) { kernel<<<(unsigned)blocks, 256, 0, st>>>(a); };
+    if (a.k <= CH_SHORT) mfma ? go(chain_mfma_kernel<XT, kPackedW, true>) : go(chain_valu_kernel<XT, kPackedW, true>);
+    else mfma ? go(chain_mfma_kernel<XT, kPackedW, false>) : go(chain_valu_kernel<XT, kPackedW, false>);
     return check_launch("chain");
 }
 

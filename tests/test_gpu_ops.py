@@ -21,6 +21,25 @@ def host(hip, t):
     return t.cpu().numpy()
 
 
+def replay_us(hip, call, copies=50):
+    """Time of one of `copies` calls in a captured graph, best of five replays."""
+    call()
+    hip.begin_capture()
+    for _ in range(copies):
+        call()
+    trace = hip.end_capture()
+    hip.begin_verify(trace)
+    times = []
+    for _ in range(5):
+        hip.sync()
+        t0 = time.perf_counter()
+        hip.begin_verify(trace)
+        hip.sync()
+        times.append(time.perf_counter() - t0)
+    hip.graph_destroy(trace)
+    return min(times) / copies * 1e6
+
+
 # ---- matmul: the reference's sequential-k chain, bit for bit ----
 def test_matmul_matches_manual(hip):  # golden.rs:14-27
     x, w = dev(hip, np.array([[1, 2], [3, 4]], np.float32)), dev(hip, np.array([[5, 6], [7, 8]], np.float32))
@@ -44,11 +63,28 @@ def test_matmul_bit_exact_vs_oracle(hip, oracle, n, k, o):
     assert np.array_equal(host(hip, out), oracle.matmul(x, w, b))
 
 
-# tile edges (16 rows, 16 outputs, 64 outputs a block), k remainders of the 16-wide steps and of the rounds of four,
-# both kernels (the line is 512 tiles of 16 x 16), rows that are only 4-byte aligned, values whose products are denormal or -0
-@pytest.mark.parametrize("n,k,o", [(1, 4, 1024), (15, 12, 80), (16, 16, 64), (17, 20, 65), (33, 52, 31), (64, 64, 16), (31, 68, 129),
-                                   (100, 132, 3072), (7, 736, 2080), (1030, 100, 272), (257, 260, 1041)])
-def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o):
+# tile edges (16 rows, 16 outputs, 64 outputs a block); k remainders of the 16-wide steps, of the 64-wide chunks and of the
+# rounds of three (matrix cores) and four chunks; rows that are only 4-byte aligned; values whose products are denormal or -0.
+# The kernel each row is there for is asserted: the one-chain-per-lane kernel up to 512 tiles of 16 x 16, the matrix-core one
+# beyond, and for up to four rows beyond 1024 tiles the one without padding rows.
+def _chain_kernel(n, k, o):
+    tiles = -(-n // 16) * -(-o // 16)
+    if k % 4 or n * o < 1024:
+        return "simple"
+    return "rows" if n <= 4 and tiles > 1024 else "mfma" if tiles > 512 else "valu"
+
+
+VALU_SHAPES = [(1, 4, 1024), (15, 12, 80), (16, 16, 64), (17, 20, 65), (33, 52, 32), (64, 64, 16), (31, 68, 129), (100, 132, 128),
+               (3, 128, 400), (20, 192, 90), (40, 260, 33), (9, 324, 130)]
+MFMA_SHAPES = [(n, k, o) for n, o in ((520, 272), (17, 8200), (3, 8300)) for k in (4, 8, 12, 16, 60, 64, 72, 128)] + \
+              [(1030, 100, 272), (257, 260, 1041), (100, 132, 3072), (7, 736, 9000), (513, 192, 260), (520, 204, 270), (530, 328, 272)]
+ROWS_SHAPES = [(1, 4, 16400), (2, 60, 16385), (3, 64, 16449), (4, 68, 20000), (4, 132, 16447), (1, 1000, 17000)]
+
+
+@pytest.mark.parametrize("n,k,o,kernel", [s + ("valu",) for s in VALU_SHAPES] + [s + ("mfma",) for s in MFMA_SHAPES] +
+                         [s + ("rows",) for s in ROWS_SHAPES])
+def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o, kernel):
+    assert _chain_kernel(n, k, o) == kernel
     rng = np.random.default_rng(n * 1000 + k)
     x = rng.normal(0, 1, (n, k)).astype(np.float32)
     w = rng.normal(0, 0.02, (o, k)).astype(np.float32)
@@ -61,6 +97,17 @@ def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o):
     out = torch.full((n, o), -1.0, device=hip.device)
     hip.matmul(xd, dev(hip, w), None, out)
     assert np.array_equal(host(hip, out), oracle.matmul(x, w))
+
+
+def test_matmul_of_few_rows_is_not_padded_to_sixteen(hip):
+    """Against very many outputs four rows take half the time of twelve; in tiles of 16 rows they took as long."""
+    w = torch.randn(131072, 64, device=hip.device)
+    took = {}
+    for n in (4, 12):
+        x, out = torch.randn(n, 64, device=hip.device), torch.empty(n, 131072, device=hip.device)
+        took[n] = replay_us(hip, lambda: hip.matmul(x, w, None, out))
+    print(took)
+    assert took[4] < 0.75 * took[12], took
 
 
 def test_matmul_shape_errors(hip):
@@ -142,21 +189,7 @@ def test_rmsnorm_takes_no_longer_for_narrow_values(hip, dim):
     took = {}
     for kind, x in _value_kinds(192, dim).items():
         x, out = dev(hip, x), torch.empty(192, dim, device=hip.device)
-        hip.rmsnorm(x, w, 1e-6, out)
-        hip.begin_capture()
-        for _ in range(50):
-            hip.rmsnorm(x, w, 1e-6, out)
-        trace = hip.end_capture()
-        hip.begin_verify(trace)
-        times = []
-        for _ in range(5):
-            hip.sync()
-            t0 = time.perf_counter()
-            hip.begin_verify(trace)
-            hip.sync()
-            times.append(time.perf_counter() - t0)
-        hip.graph_destroy(trace)
-        took[kind] = min(times) / 50 * 1e6
+        took[kind] = replay_us(hip, lambda: hip.rmsnorm(x, w, 1e-6, out))
     print({k: round(v, 1) for k, v in took.items()})
     assert max(took.values()) < 2.0 * took["normal"], took
 
