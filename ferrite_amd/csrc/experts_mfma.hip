@@ -259,47 +259,64 @@ struct BSource {
 };
 
 // Copies k steps [kt0, kt0 + wkt) of the unit's rows into LDS in B-operand order and builds the packed scale words.
-// row_src(r) gives the source row of unit row r (or -1: zeros).  Work is dealt in pieces of 512 bytes (four k steps of one
-// row and plane), two to a wave's load; four loads are in flight.
-// At 192 tokens (two terms, 12 rows a unit) the gate/up kernel takes 168 us, 175 us with a loop of one load and one store
-// at a time, an integer division per 16 bytes and sixteen lanes of a store on the same banks (down, half as much per block, 92.9 -> 95.5).
-template <bool kX2, int NR = 16, typename RowFn>
+// row_src(r) gives the source row of unit row r (or -1: zeros).
+// FILL 0: one 16-byte chunk per thread and round.  Else: work is dealt in pieces of 512 bytes (four k steps of one row and
+// plane), two to a wave's load, without divisions, FILL loads in flight; windows of less than a piece go the first way.
+// us of the kernels (two terms unless said), fill:                     0      1      4
+//   gate/up, 192 tokens, 8 waves, 12 rows a unit                      163.9  156.5  155.5
+//   gate/up, 2 tokens / 4 at hidden 5120 / 8, one term                24.9 / 28.7 / 59.3  24.9 / 28.6 / 58.7  27.1 / 32.1 / 62.3
+//   gate/up split, 1 token, hidden 4096 / 7168                        15.0 / 35.1  15.3 / 34.9  14.5 / 31.7
+//   down, 2 tokens / 192                                              16.0 / 87.8  17.8 / 91.3  18.0 / 89.6
+//   down split, 1 token                                               10.6   10.7   11.5
+template <int FILL, bool kX2, int NR = 16, typename RowFn>
 __device__ __forceinline__ void fill_b_window(const BSource<kX2>& s, RowFn row_src, int kt0, int wkt,
                                               const BPlanes<kX2, NR>& d) {
-    constexpr int NP = kX2 ? 2 : 1, BATCH = 4;
-    const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int chunks = wkt * 8, segs = (wkt + 3) / 4;   // 16-byte chunks of a row's window, pieces of 32 chunks
-    const int rows = s.nrows * NP;                      // (row, plane) pairs, planes of a row together
-    const int ids = (lane & 15) < s.nrows ? row_src(lane & 15) : -1;   // the unit's rows, one per lane
-    int rp = 0, seg = 2 * wave;                         // of the wave's first piece; the second is the one behind it
-    while (seg >= segs) { seg -= segs; ++rp; }
-    while (rp < rows) {
-        u4v v[BATCH];
-        int slot[BATCH];
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b) {
-            slot[b] = -1;
-            v[b] = (u4v){0u, 0u, 0u, 0u};
-            if (rp < rows) {   // wave-uniform
-                const bool wrap = seg + 1 >= segs;
-                const int rp1 = min(rp + (wrap ? 1 : 0), rows - 1), seg1 = wrap ? 0 : seg + 1;
-                const int r0 = __builtin_amdgcn_readlane(ids, rp / NP), r1 = __builtin_amdgcn_readlane(ids, rp1 / NP);
-                const bool second = lane >= 32;
-                const int rpl = second ? rp1 : rp, r = second ? r1 : r0;
-                const int c = rpl / NP, p = rpl % NP, j = (second ? seg1 : seg) * 32 + (lane & 31);
-                if (j < chunks && !(second && wrap && rp + 1 >= rows)) {
-                    const uint8_t* plane = p ? s.src.q2 : s.src.q;
-                    if (r >= 0) v[b] = *reinterpret_cast<const u4v*>(plane + (size_t)r * s.pitch + (size_t)kt0 * 128 + (size_t)j * 16);
-                    slot[b] = (p << 30) | b_slot<NR>(j >> 3, (j >> 2) & 1, j & 3, c);
-                }
-                seg += 2 * waves;
-                while (seg >= segs) { seg -= segs; ++rp; }
-            }
+    constexpr int NP = kX2 ? 2 : 1, BATCH = FILL > 0 ? FILL : 1;
+    if (FILL == 0 || wkt < 4) {
+        const int chunks = wkt * 8, plane_chunks = s.nrows * chunks;
+        for (int idx = threadIdx.x; idx < NP * plane_chunks; idx += blockDim.x) {
+            const int p = idx >= plane_chunks ? 1 : 0, rem = idx - p * plane_chunks;
+            const int c = rem / chunks, j = rem % chunks;
+            const int r = row_src(c);
+            u4v v = (u4v){0u, 0u, 0u, 0u};
+            if (r >= 0) v = *reinterpret_cast<const u4v*>((p ? s.src.q2 : s.src.q) + (size_t)r * s.pitch + (size_t)kt0 * 128 + (size_t)j * 16);
+            (p ? d.bq2 : d.bq)[b_slot<NR>(j >> 3, (j >> 2) & 1, j & 3, c)] = v;
         }
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b)
-            if (slot[b] >= 0) ((slot[b] >> 30) ? d.bq2 : d.bq)[slot[b] & 0x3fffffff] = v[b];
+    } else {
+        const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int chunks = wkt * 8, segs = (wkt + 3) / 4;   // 16-byte chunks of a row's window, pieces of 32 chunks
+        const int rows = s.nrows * NP;                      // (row, plane) pairs, planes of a row together
+        const int ids = (lane & 15) < s.nrows ? row_src(lane & 15) : -1;   // the unit's rows, one per lane
+        int rp = 0, seg = 2 * wave;                         // of the wave's first piece; the second is the one behind it
+        while (seg >= segs) { seg -= segs; ++rp; }
+        while (rp < rows) {
+            u4v v[BATCH];
+            int slot[BATCH];
+    #pragma unroll
+            for (int b = 0; b < BATCH; ++b) {
+                slot[b] = -1;
+                v[b] = (u4v){0u, 0u, 0u, 0u};
+                if (rp < rows) {   // wave-uniform
+                    const bool wrap = seg + 1 >= segs;
+                    const int rp1 = min(rp + (wrap ? 1 : 0), rows - 1), seg1 = wrap ? 0 : seg + 1;
+                    const int r0 = __builtin_amdgcn_readlane(ids, rp / NP), r1 = __builtin_amdgcn_readlane(ids, rp1 / NP);
+                    const bool second = lane >= 32;
+                    const int rpl = second ? rp1 : rp, r = second ? r1 : r0;
+                    const int c = rpl / NP, p = rpl % NP, j = (second ? seg1 : seg) * 32 + (lane & 31);
+                    if (j < chunks && !(second && wrap && rp + 1 >= rows)) {
+                        const uint8_t* plane = p ? s.src.q2 : s.src.q;
+                        if (r >= 0) v[b] = *reinterpret_cast<const u4v*>(plane + (size_t)r * s.pitch + (size_t)kt0 * 128 + (size_t)j * 16);
+                        slot[b] = (p << 30) | b_slot<NR>(j >> 3, (j >> 2) & 1, j & 3, c);
+                    }
+                    seg += 2 * waves;
+                    while (seg >= segs) { seg -= segs; ++rp; }
+                }
+            }
+    #pragma unroll
+            for (int b = 0; b < BATCH; ++b)
+                if (slot[b] >= 0) ((slot[b] >> 30) ? d.bq2 : d.bq)[slot[b] & 0x3fffffff] = v[b];
+        }
     }
     const int wg = (wkt + 3) / 4;
     const int c = threadIdx.x % NR, g = (threadIdx.x / NR) & 3;
@@ -315,7 +332,7 @@ __device__ __forceinline__ void fill_b_window(const BSource<kX2>& s, RowFn row_s
 // The reduction of `rounds` items per wave against one unit's activation rows.  item(round, wp, sp) gives the
 // round's weight stream of this wave (false: no item, the wave only keeps the barriers company); the first round's
 // group 0 must already be in flight in buffer 0.  done(round, acc) receives the finished accumulators.  Every wave of the block makes the same calls: the barriers inside are block-wide.
-template <bool kKeep, bool kX2, int WIN, typename RowFn, typename ItemFn, typename DoneFn>
+template <int FILL, bool kKeep, bool kX2, int WIN, typename RowFn, typename ItemFn, typename DoneFn>
 __device__ __forceinline__ void run_unit(const BSource<kX2>& s, RowFn row_src, int KT, int rounds, ItemFn item, DoneFn done,
                                          StreamRegs& regs, unsigned char* lds, int lane) {
     const int WKT = window_kt<WIN>(KT), nw = (KT + WKT - 1) / WKT;
@@ -335,7 +352,7 @@ __device__ __forceinline__ void run_unit(const BSource<kX2>& s, RowFn row_src, i
             const int kt0 = w * WKT, wkt = min(WKT, KT - kt0);
             if (nw > 1 || !filled) {
                 if (filled) __syncthreads();   // every wave is done with the window that is in LDS
-                fill_b_window<kX2>(s, row_src, kt0, wkt, d);
+                fill_b_window<FILL, kX2>(s, row_src, kt0, wkt, d);
                 __syncthreads();
                 filled = true;
             }
@@ -462,7 +479,7 @@ __device__ __forceinline__ void gate_up_rows(const MfmaArgs& a, int e, int row0,
         stream_load_group<kKeep>(regs, wp0, sp0, KT, lane, 0, 0);
     }
     const BSource<kX2> bsrc{xin, (size_t)H, scale_pitch(H), nrows};
-    run_unit<kKeep, kX2, WIN>(
+    run_unit<WAVES == 8 ? 4 : 1, kKeep, kX2, WIN>(
         bsrc, row_src, KT, 1,
         [&](int, const u4v*& wp, const u4v*& sp) { wp = wp0; sp = sp0; return live; },
         [&](int, v4f (&acc)[4]) { gate_up_store<kX2>(a, acc, item, row0, nrows, act, lane); },
@@ -527,7 +544,7 @@ __device__ __forceinline__ void down_unit(const MfmaArgs& a, int u, int ig, cons
     // activation rows have pitch act_ld; only the first `inter` columns are meaningful for this expert
     const BSource<kX2> bsrc{act, (size_t)a.act_ld, scale_pitch(a.act_ld), nrows};
     const int c = lane & 15, g = lane >> 4;
-    run_unit<kKeep, kX2, kX2 ? kWindowKt : 0>(
+    run_unit<0, kKeep, kX2, kX2 ? kWindowKt : 0>(
         bsrc, [&](int col) { return row0 + col; }, KT, IPW,
         [&](int r, const u4v*& wp, const u4v*& sp) {
             const int item = item0 + r;
@@ -568,7 +585,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void down_mfma_kernel(MfmaArgs a, in
 // (two tokens) 89.9 -> 90.8, 1584 (four) 110.6 -> 115.5.
 constexpr int SPLIT_WAVES = 4, SPLIT_ROWS = 4, SPLIT_ITEMS = 640;
 
-template <bool kX2, typename RowFn>
+template <int FILL, bool kX2, typename RowFn>
 __device__ __forceinline__ bool split_item(const BSource<kX2>& s, RowFn row_src, const uint8_t* cbase, const uint8_t* sbase,
                                            int item, int KT, unsigned char* lds, v4f (&acc)[4]) {
     const int KT4 = (KT + 3) / 4, lane = threadIdx.x & 63, waves = blockDim.x >> 6;
@@ -579,7 +596,7 @@ __device__ __forceinline__ bool split_item(const BSource<kX2>& s, RowFn row_src,
     StreamRegs regs;
     stream_load_group<false>(regs, wp, sp, KT, lane, g_lo, 0);   // weights fly while the activations are staged
     const BPlanes<kX2, SPLIT_ROWS> d(lds, KT);
-    fill_b_window<kX2, SPLIT_ROWS>(s, row_src, 0, KT, d);
+    fill_b_window<FILL, kX2, SPLIT_ROWS>(s, row_src, 0, KT, d);
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -620,7 +637,7 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void gate_up_split_kernel(Mfma
     const int H = a.hidden, nk = a.n * a.topk, topk = a.topk;
     const BSource<kX2> src{xin, (size_t)H, scale_pitch(H), nrows};
     v4f acc[4];
-    if (split_item<kX2>(
+    if (split_item<4, kX2>(
             src,
             [&](int c) -> int {
                 if (shared) return row0 + c - nk;
@@ -643,7 +660,7 @@ __global__ __launch_bounds__(SPLIT_WAVES * 64, 2) void down_split_kernel(MfmaArg
     const bool shared = e == a.n_experts;
     const BSource<kX2> src{act, (size_t)a.act_ld, scale_pitch(a.act_ld), nrows};
     v4f acc[4];
-    if (!split_item<kX2>(
+    if (!split_item<0, kX2>(
             src, [&](int c) { return row0 + c; }, shared ? a.sh_codes : a.codes + (size_t)e * a.codes_per_expert,
             shared ? a.sh_scales : a.scales + (size_t)e * a.scales_per_expert, item, (shared ? a.shared_inter : a.inter) / 128,
             lds_raw, acc))
