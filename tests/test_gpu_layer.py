@@ -116,13 +116,29 @@ def test_layer_small_shapes_all_modes(hip, oracle, seed, n):
     check_mfma(hip, oracle, layer, inp, MODE_MFMA_FP8_X2, ref32)
 
 
-@pytest.mark.parametrize("n,hidden,inter,shared", [(1, 32, 32, 0), (5, 544, 96, 64), (40, 1056, 736, 32), (3, 2080, 1120, 736),
-                                                   (130, 480, 160, 320)])
-def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared):
+def max_units(n, topk, n_experts, shared):
+    """Units of up to 16 rows that a call may have (what grids are sized for)."""
+    return n * topk // 16 + min(n * topk, n_experts) + (-(-n // 16) if shared else 0)
+
+
+def f32_waves_share_a_pair(cfg):
+    """(gate/up, down): whether the four waves of a block share a pair of tiles in the f32 mode."""
+    units = max_units(cfg.n, cfg.topk, cfg.n_experts, cfg.shared_inter)
+    return units * (max(cfg.inter, cfg.shared_inter) // 16) <= 1024, units * (cfg.hidden // 32) <= 1024
+
+
+@pytest.mark.parametrize("n,hidden,inter,shared,experts,topk,share", [
+    (1, 32, 32, 0, 8, 3, (True, True)), (5, 544, 96, 64, 8, 3, (True, True)), (40, 1056, 736, 32, 8, 3, (True, True)),
+    (3, 2080, 1120, 736, 8, 3, (True, True)), (130, 480, 160, 320, 8, 3, (True, True)),
+    (40, 2080, 736, 736, 32, 6, (False, False)), (24, 1056, 992, 96, 32, 4, (False, False)), (30, 160, 1504, 64, 32, 4, (False, True)),
+    (50, 4128, 224, 0, 32, 4, (True, False))])
+def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared, experts, topk, share):
     """The f32 mode on sizes that are multiples of 32 only: reductions shorter than a block of 128, longer than the
-    activation window and ragged in both, odd numbers of row tiles, units of 1..16 rows, weights shared out to one wave
-    per pair of tiles or to four; zero scales."""
-    cfg = synth.MoeConfig(n, hidden, 8, 3, inter, shared, 4, 2)
+    activation window and ragged in both, numbers of row tiles that are odd or no multiple of the four waves', a shared
+    expert so short that whole blocks drop out, units of 1..16 rows, weights shared out to one wave per pair of tiles or
+    to four; zero scales."""
+    cfg = synth.MoeConfig(n, hidden, experts, topk, inter, shared, 4, 2)
+    assert f32_waves_share_a_pair(cfg) == share
     inp = synth.make_inputs(cfg, seed=n + hidden)
     inp.gate_s.reshape(-1)[::7] = 0
     inp.down_s.reshape(-1)[::5] = 0
@@ -131,6 +147,28 @@ def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared):
     out, v = run_layer(hip, layer, inp.x, MODE_F32_CHECK)
     check_routing(v, ref, oracle, cfg)
     assert max_abs_rel(out, ref["out"]) <= TOL_F32
+
+
+@pytest.mark.parametrize("n,experts,topk,share", [(12, 8, 2, (True, True)), (40, 32, 4, (False, False))])
+def test_f32_mode_keeps_nan_where_it_belongs(hip, oracle, n, experts, topk, share):
+    """NaN scales (byte 255) in every matrix, at the ends of rows and of ragged blocks: NaN exactly where the oracle has it,
+    everything else as close as ever.  A unit's rows share weight registers and MFMAs, its blocks LDS."""
+    cfg = synth.MoeConfig(n, 1056, experts, topk, 992, 96, 4, 2)
+    assert f32_waves_share_a_pair(cfg) == share
+    inp = synth.make_inputs(cfg, seed=n)
+    inp.down_s.reshape(experts, cfg.hidden, -1)[1, 5, 2] = 255
+    inp.down_s.reshape(experts, cfg.hidden, -1)[3, 1055, 30] = 255
+    inp.gate_s.reshape(experts, cfg.inter, -1)[2, 991, 32] = 255
+    inp.up_s.reshape(experts, cfg.inter, -1)[4, 0, 0] = 255
+    inp.sh_down_s.reshape(cfg.hidden, -1)[17, 2] = 255
+    layer = hip.load_moe_layer(inp, pack=False)
+    ref = oracle.moe_ffn_mxfp4(inp, n_threads=8)
+    out, v = run_layer(hip, layer, inp.x, MODE_F32_CHECK)
+    assert np.array_equal(v["ids"], ref["ids"].astype(np.int32))
+    assert np.array_equal(np.isnan(out), np.isnan(ref["out"]))
+    fine = np.isfinite(ref["out"])
+    assert 0.05 < fine.mean() < 0.999 and np.isnan(ref["out"][:, 17]).all() and np.isnan(ref["out"][~fine]).all()
+    assert max_abs_rel(out[fine], ref["out"][fine]) <= TOL_F32
 
 
 @pytest.mark.parametrize("n,hidden,inter,shared", [(24, 2304, 2304, 2304), (19, 2176, 128, 2432), (5, 4096, 256, 0)])
@@ -743,14 +781,28 @@ def test_layer_c3_skewed_scale(hip, oracle):
     assert 0.35 <= top <= 0.65, top
 
 
+def split_waves(cfg):
+    """Waves that share an item of gate/up and of down in the MFMA modes, 0 where the item is one wave's: up to four tokens,
+    up to 640 items, and every wave needs a group of four k steps of the routed and of the shared reduction."""
+    units = max_units(cfg.n, cfg.topk, cfg.n_experts, cfg.shared_inter)
+    groups = lambda k: -(-k // 512)
+    gate_up = min(4, groups(cfg.hidden)) if units * (max(cfg.inter, cfg.shared_inter) // 32) <= 640 else 0
+    down = min(4, groups(cfg.inter), groups(cfg.shared_inter or cfg.inter)) if units * (cfg.hidden // 64) <= 640 else 0
+    return tuple(w if cfg.n <= 4 and w > 1 else 0 for w in (gate_up, down))
+
+
 @pytest.mark.parametrize("mode", [MODE_MFMA_FP8, MODE_MFMA_FP8_X2])
-@pytest.mark.parametrize("n,hidden,inter,shared", [(1, 4096, 1536, 1536), (4, 640, 1152, 512), (3, 2176, 512, 2432), (2, 1024, 2048, 0),
-                                                   (5, 1024, 1024, 512)])
-def test_few_tokens_share_items_among_waves(hip, oracle, n, hidden, inter, shared, mode):
+@pytest.mark.parametrize("n,hidden,inter,shared,waves", [
+    (1, 4096, 1536, 1536, (4, 3)), (4, 640, 1152, 512, (2, 0)), (3, 2176, 512, 2432, (0, 0)), (2, 1024, 2048, 0, (2, 4)),
+    (5, 1024, 1024, 512, (0, 0)),
+    (1, 2176, 512, 512, (4, 0)), (4, 2560, 512, 512, (4, 0)), (1, 3328, 512, 0, (4, 0)),      # 5, 5 and 7 groups on four waves
+    (1, 1024, 2432, 1152, (2, 3)), (1, 1024, 1152, 2432, (2, 3)), (3, 1024, 1664, 640, (2, 2))])   # 5 | 3, 3 | 5, 4 | 2 groups
+def test_few_tokens_share_items_among_waves(hip, oracle, n, hidden, inter, shared, waves, mode):
     """A few tokens with a few hundred items: the waves of a block split an item's reduction.  Groups that do not divide
     among the waves, last groups of less than four k steps, routed and shared reductions of different lengths; five
-    tokens do not split."""
+    tokens do not split, nor do more than 640 items or reductions of a single group."""
     cfg = synth.MoeConfig(n, hidden, 8, 4, inter, shared, 4, 2)
+    assert split_waves(cfg) == waves
     inp = synth.make_inputs(cfg, seed=n)
     layer = hip.load_moe_layer(inp)
     check_mfma(hip, oracle, layer, inp, mode)

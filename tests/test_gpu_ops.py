@@ -82,7 +82,7 @@ ROWS_SHAPES = [(1, 4, 16400), (2, 60, 16385), (3, 64, 16449), (4, 68, 20000), (4
 
 
 @pytest.mark.parametrize("n,k,o,kernel", [s + ("valu",) for s in VALU_SHAPES] + [s + ("mfma",) for s in MFMA_SHAPES] +
-                         [s + ("rows",) for s in ROWS_SHAPES])
+                         [s + ("rows",) for s in ROWS_SHAPES] + [(33, 52, 31, "simple"), (17, 50, 70, "simple")])
 def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o, kernel):
     assert _chain_kernel(n, k, o) == kernel
     rng = np.random.default_rng(n * 1000 + k)
@@ -97,6 +97,24 @@ def test_matmul_tiles_bit_exact_vs_oracle(hip, oracle, n, k, o, kernel):
     out = torch.full((n, o), -1.0, device=hip.device)
     hip.matmul(xd, dev(hip, w), None, out)
     assert np.array_equal(host(hip, out), oracle.matmul(x, w))
+
+
+@pytest.mark.parametrize("n,k,o,kernel", [(40, 100, 48, "valu"), (40, 324, 48, "valu"), (530, 100, 272, "mfma"), (530, 328, 272, "mfma"),
+                                          (4, 100, 16400, "rows"), (33, 52, 31, "simple")])
+def test_matmul_nan_and_infinity_vs_oracle(hip, oracle, n, k, o, kernel):
+    """Infinities (also against zero weights and against each other), NaN and products that overflow stay in their row or
+    output and come out as the chain has them."""
+    assert _chain_kernel(n, k, o) == kernel
+    rng = np.random.default_rng(n + k)
+    x = rng.normal(0, 1, (n, k)).astype(np.float32)
+    w = rng.normal(0, 1, (o, k)).astype(np.float32)
+    x[0, k - 1], x[1, 3], x[n - 1, 0], x[2, 5], x[2, 6] = np.inf, np.nan, -np.inf, 3e38, -3e38
+    w[3, 0], w[5, 7], w[o - 1, k - 1], w[7] = 0.0, np.nan, np.inf, 1e30
+    out = torch.empty(n, o, device=hip.device)
+    hip.matmul(dev(hip, x), dev(hip, w), None, out)
+    ref = oracle.matmul(x, w)
+    assert np.isnan(ref).any() and np.isinf(ref).any() and np.isfinite(ref).any()
+    assert np.array_equal(host(hip, out), ref, equal_nan=True)
 
 
 def test_matmul_of_few_rows_is_not_padded_to_sixteen(hip):
@@ -127,6 +145,8 @@ def _sumsq_rows(dim, rng):
     rows += [np.exp(np.linspace(-20, 20, dim)), np.exp(np.linspace(20, -20, dim))]       # a binade every few values / one
     spike = rng.normal(0, 1, dim)
     spike[dim // 2], spike[dim // 3] = 4096.0, 64.0
+    rows += [np.exp(np.linspace(np.log(1e-18), np.log(1e-14), dim)), np.exp(np.linspace(np.log(1e-14), np.log(1e-18), dim)),
+             rng.normal(0, 2.0 ** -53, dim), rng.normal(0, 2.0 ** -75, dim)]   # sums around 2^-100, where walking begins; denormals
     late = np.zeros(dim)
     late[-3:] = [1e-30, 1e-12, 3.0]
     rng_ties = 2.0 ** rng.integers(-13, 1, dim)                                           # halves of the running sum's ulp
@@ -144,11 +164,15 @@ def test_rmsnorm_sum_of_squares_is_the_serial_chain(hip, oracle, dim):
     out = torch.empty(x.shape, device=hip.device)
     hip.rmsnorm(dev(hip, x), dev(hip, w), 1e-6, out)
     assert np.array_equal(host(hip, out), oracle.rmsnorm(x, w, 1e-6))
+    # without eps the smallest sums show as well
+    hip.rmsnorm(dev(hip, x), dev(hip, w), 0.0, out)
+    assert np.array_equal(host(hip, out), oracle.rmsnorm(x, w, 0.0), equal_nan=True)
     # more rows than the four-waves-per-row kernel takes
     many = np.tile(x, (1100 // len(x) + 1, 1))
     out = torch.empty(many.shape, device=hip.device)
-    hip.rmsnorm(dev(hip, many), dev(hip, w), 1e-6, out)
-    assert np.array_equal(host(hip, out)[:len(x)], oracle.rmsnorm(x, w, 1e-6))
+    for eps in (1e-6, 0.0):
+        hip.rmsnorm(dev(hip, many), dev(hip, w), eps, out)
+        assert np.array_equal(host(hip, out)[:len(x)], oracle.rmsnorm(x, w, eps), equal_nan=True)
     bad = x[:3].copy()
     bad[0, dim // 2], bad[1, dim - 1], bad[2, 0] = np.inf, np.nan, 3e38
     out = torch.empty(bad.shape, device=hip.device)
