@@ -163,7 +163,10 @@ int launch_rmsnorm(const float* x, const float* w, float eps, float* out, int n,
     if (n == 0) return FERRITE_OK;
     const bool vec4 = (dim & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
                                            reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    // beyond ~1000 rows the chip is full either way and one wave per row wastes no idle waves (4096 rows: 62 against 66 us)
+    // Beyond about 1000 rows the chip is full either way and it depends on the length.  Four waves against one per row, us:
+    //   1024 rows of 2048 / 4096 / 7168    9.9 10.5   13.7 14.0   19.4 21.4
+    //   2047                              16.6 12.4   18.7 20.0   34.8 31.8
+    //   4096                              27.7 23.2   30.9 38.8   58.4 59.1
     if (vec4 && dim <= RN_ROW_MAX && n <= 1024) {
         const size_t lds = ((size_t)((dim + 255) & ~255) + 4) * sizeof(float);
         if (dim <= 1024) rmsnorm_row_kernel<1><<<n, 256, lds, st>>>(x, w, eps, out, dim);

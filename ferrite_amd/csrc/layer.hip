@@ -305,21 +305,14 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
     if (fused_head) {
         // 1-3 (+ activation quantisation) as one launch
         PackedLayout L = packed_layout(s);
-        const int fuse_perm = 1;   // the block that routes the last token builds the tables
         if ((rc = launch_moe_head(x, x_dtype, reinterpret_cast<const float*>(packed + L.router_t), wts->router_bias, s,
                                   n, logits, probs, ids_f32, ids, xq, reinterpret_cast<int32_t*>(b + w.counters),
                                   reinterpret_cast<int32_t*>(b + w.counts), reinterpret_cast<int32_t*>(b + w.starts),
                                   perm_map, gather_src, reinterpret_cast<int32_t*>(b + w.active),
-                                  reinterpret_cast<int32_t*>(b + w.n_active), &units, fuse_perm, norm_w, norm_eps, st)))
+                                  reinterpret_cast<int32_t*>(b + w.n_active), units, norm_w, norm_eps, st)))
             return rc;
         if ((rc = mark(ev, 1, st))) return rc;
         if ((rc = mark(ev, 2, st))) return rc;
-        if (!fuse_perm &&
-            (rc = launch_permute(ids, n, s.topk, s.n_experts, reinterpret_cast<int32_t*>(b + w.counts),
-                                 reinterpret_cast<int32_t*>(b + w.starts), perm_map, gather_src,
-                                 reinterpret_cast<int32_t*>(b + w.active), reinterpret_cast<int32_t*>(b + w.n_active),
-                                 b + w.perm_scratch, w.perm_scratch_bytes, &units, has_shared, st)))
-            return rc;
         if ((rc = mark(ev, 3, st))) return rc;
         if ((rc = mark(ev, 4, st))) return rc;
     } else {
@@ -328,10 +321,6 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
         PackedLayout L = packed_layout(s);
         rc = launch_router_chain(x, x_dtype, reinterpret_cast<const float*>(packed + L.router_t), n, s.hidden,
                                  s.n_experts, logits, st);
-        if (rc == FERRITE_DECLINED) {
-            if (!wts->router_w) return FERRITE_ERR_INVALID_ARG;   // this shape needs the checkpoint-layout router
-            rc = launch_matmul_exact(x, x_dtype, wts->router_w, nullptr, logits, n, s.hidden, s.n_experts, st);
-        }
     } else {
         rc = launch_matmul_exact(x, x_dtype, wts->router_w, nullptr, logits, n, s.hidden, s.n_experts, st);
     }

@@ -28,7 +28,8 @@ namespace fe {
 // row, a lane one output, so that the chip is not occupied with padding rows.
 //
 // us:                                                   before    mfma    valu
-//   router 8192 tokens x 256, H 7168 (bf16 x)              735     648     -       (valu, 4 x 4 chains per lane: 620)
+//   router 8192 tokens x 256, H 7168 (bf16 x)              735     648     -       (valu, 4 x 4 chains per lane: 620;
+//                                                                                   nowhere else faster, not kept)
 //   router 4096 x 128, H 4096 (bf16 x)                     149     105     -       (2 x 2 chains per lane: 125)
 //   router 2047 x 128, H 4096 (f32 x)                      146      76     -       (2 x 2: 101)
 //   router 509 x 128, H 4096 (bf16 x)                       47      50     42
@@ -812,7 +813,6 @@ struct HeadArgs {
     int32_t* ids;
     ActPlanes xq;         // q may be NULL: no quantisation blocks are launched then; q2 set: two-term
     int32_t* counters;    // [1 + n]
-    int fuse_perm;        // the block that routes the last token also builds the permutation; else a separate launch does
     const float* norm_w;  // not NULL: x is the un-normalised f32 stream and every block applies rmsnorm(x, norm_w, eps)
     float eps;            // to its token(s) first (cpu.rs:124-143), so the normalised activations never go through HBM
     PermArgs perm;
@@ -866,18 +866,18 @@ __device__ __forceinline__ void head_pmul(const HeadSet<T, W>& st, const float4*
     }
 }
 
-// rmsnorm of the block's token(s) in place of the first barrier ("x is in LDS") of every wave's role.  On entry
-// every thread has staged its share of the raw rows in xl and of their squares (each rounded once) in sq.  The
-// reference sums the squares of a row left to right in f32 (cpu.rs:124-143): a serial chain, which wave 0 works out
-// (sumsq_walk) while the producer waves' first weight loads are already in flight.
+// rmsnorm of the block's token in place of the first barrier ("x is in LDS") of every wave's role.  On entry every
+// thread has staged its share of the raw row in xl and of its squares (each rounded once) in sq.  The reference sums
+// the squares of a row left to right in f32 (cpu.rs:124-143): a serial chain, which wave 0 works out (sumsq_chain,
+// sumsq_walk) while the producer waves' first weight loads are already in flight.
 // Then all waves scale xl to (x * inv) * w, which is what the router chain and the quantisation see.
 struct HeadNorm {
     const float* w;
     float eps;
     float4* xl;
     const float4* sq;
-    float* inv;   // [T] in LDS
-    int nk4, T;
+    float* inv;   // in LDS
+    int nk4;
 };
 
 __device__ __forceinline__ void head_first_sync(const HeadNorm& nm) {
@@ -885,23 +885,19 @@ __device__ __forceinline__ void head_first_sync(const HeadNorm& nm) {
     if (nm.w == nullptr) return;
     const int tid = threadIdx.x;
     if (tid < 64) {
-        for (int ti = 0; ti < nm.T; ++ti) {
-            const float4* sq = nm.sq + (size_t)ti * nm.nk4;
-            float ss = nm.nk4 <= SUMSQ_SHORT ? sumsq_chain(sq, nm.nk4, 0.0f) : sumsq_walk(sq, nm.nk4, 0.0f);
-            ss = fdiv(ss, (float)(nm.nk4 * 4));
-            const float inv = fdiv(1.0f, fsqrt(fadd(ss, nm.eps)));
-            if (tid == 0) nm.inv[ti] = inv;
-        }
+        float ss = nm.nk4 <= SUMSQ_SHORT ? sumsq_chain(nm.sq, nm.nk4, 0.0f) : sumsq_walk(nm.sq, nm.nk4, 0.0f);
+        ss = fdiv(ss, (float)(nm.nk4 * 4));
+        const float inv = fdiv(1.0f, fsqrt(fadd(ss, nm.eps)));
+        if (tid == 0) *nm.inv = inv;
     }
     __syncthreads();
-    for (int i = tid; i < nm.T * nm.nk4; i += blockDim.x) {
-        const int ti = i / nm.nk4, k4 = i - ti * nm.nk4;
-        const float iv = nm.inv[ti];
-        const float4 v = nm.xl[i], g = reinterpret_cast<const float4*>(nm.w)[k4];
+    const float iv = *nm.inv;
+    for (int i = tid; i < nm.nk4; i += blockDim.x) {
+        const float4 v = nm.xl[i], g = reinterpret_cast<const float4*>(nm.w)[i];
         nm.xl[i] = make_float4(fmul(fmul(v.x, iv), g.x), fmul(fmul(v.y, iv), g.y), fmul(fmul(v.z, iv), g.z),
                                fmul(fmul(v.w, iv), g.w));
     }
-    __syncthreads();   // the normalised rows are in place and the squares' space is free for the products
+    __syncthreads();   // the normalised row is in place and the squares' space is free for the products
 }
 
 // Products of chunk c+1 are made while the chain consumes chunk c; register set c%4 holds the weights of chunk c
@@ -1035,7 +1031,7 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
                         row[i] = v;
                         sq[i] = make_float4(fmul(v.x, v.x), fmul(v.y, v.y), fmul(v.z, v.z), fmul(v.w, v.w));
                     }
-                    head_first_sync(HeadNorm{a.norm_w, a.eps, row, sq, inv, H / 4, 1});
+                    head_first_sync(HeadNorm{a.norm_w, a.eps, row, sq, inv, H / 4});
                     xrow = reinterpret_cast<const XT*>(row);
                 }
             }
@@ -1072,7 +1068,7 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
         }
     }
     const HeadNorm nm{kNorm ? a.norm_w : nullptr, a.eps, xl, ring,
-                      reinterpret_cast<float*>(head_lds + HeadCfg<T, W>::RING_BYTES + (size_t)T * H * 4), nk4, T};
+                      reinterpret_cast<float*>(head_lds + HeadCfg<T, W>::RING_BYTES + (size_t)T * H * 4), nk4};
     // wave 0 chains; wave 4 would share its SIMD (and its VALU issue slots) and only keeps the barriers company; the
     // others produce
     float s[T];
@@ -1088,10 +1084,8 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
         case 7: head_producer<T, W, 5>(wp, a.Epad, nk4, xl, ring, lane, nm); break;
         default: head_bystander<T, W>(nk4, nm); break;
     }
-    // From here on wave 0 works alone (LDS is free for its scratch); with a fused permutation the other waves wait
-    // at the barrier below and join in if this block turns out to be the one that routed the last token.
-    const bool block_perm = a.fuse_perm;
-    if (wave != 0 && !block_perm) return;
+    // From here on wave 0 works alone (LDS is free for its scratch); the other waves wait at the barrier below and join
+    // in if this block turns out to be the one that routed the last token.
     __shared__ int perm_here;
     int do_perm = 0;
     if (wave == 0) {
@@ -1125,7 +1119,6 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
         }
         if (lane == 0) perm_here = do_perm;
     }
-    if (!block_perm) return;
     __syncthreads();
     if (perm_here) permute_in_block<true, false>(a.perm, reinterpret_cast<unsigned long long*>(head_lds));
 }
@@ -1151,10 +1144,11 @@ static size_t head_lds_bytes(int n, int H, int E) {
     return b;
 }
 
-// The fused rmsnorm keeps the squares of the block's rows where the product ring will be.  Every block of a token
-// walks that token's sum-of-squares chain again, which pays while each block has a CU to itself (32 tokens, H 4096:
-// the block call 4 us shorter than with rmsnorm as a launch of its own) and no longer when two blocks share one
-// (192 tokens: 6 us longer): offered for the one-block-per-CU shape only.
+// The fused rmsnorm keeps the squares of the block's row where the product ring will be.  Every block of a token
+// works out that token's sum of squares again, which pays while each block has a CU to itself (32 tokens, H 4096: the
+// block call 4 us shorter than with rmsnorm as a launch of its own).  With two blocks on a CU it gains and loses (H 4096,
+// 128 experts: 128 tokens 99 against 103 us, 192 tokens 109 and 111 against 110 and 111, 250 tokens 131 against 128):
+// offered for the one-block-per-CU shape only.
 bool head_norm_supported(int n, int H, int E) {
     if (!head_supported(n, H, E)) return false;
     const HeadShape hs = head_shape(n, (E + 63) / 64);
@@ -1185,7 +1179,7 @@ static int launch_head_t(const HeadArgs& a, int quant, size_t lds, hipStream_t s
 int launch_moe_head(const void* x, int x_dtype, const float* router_t, const float* bias, const ferrite_moe_shape& s,
                     int n, float* logits, float* probs, float* ids_f32, int32_t* ids, const ActPlanes& xq,
                     int32_t* counters, int32_t* counts, int32_t* starts, int32_t* perm_map, int32_t* gather_src,
-                    int32_t* active, int32_t* n_active, const UnitTables* units, int fuse_perm, const float* norm_w,
+                    int32_t* active, int32_t* n_active, const UnitTables& units, const float* norm_w,
                     float eps, hipStream_t st) {
     if (!head_supported(n, s.hidden, s.n_experts)) return FERRITE_DECLINED;
     if (norm_w && (x_dtype != FERRITE_DT_F32 || !head_norm_supported(n, s.hidden, s.n_experts))) return FERRITE_DECLINED;
@@ -1195,17 +1189,14 @@ int launch_moe_head(const void* x, int x_dtype, const float* router_t, const flo
     a.n_group = (s.n_group > 1 && s.topk_group < s.n_group) ? s.n_group : 1;
     a.topk_group = s.topk_group; a.scaling = s.routed_scaling;
     a.logits = logits; a.probs = probs; a.ids_f32 = ids_f32; a.ids = ids; a.xq = xq; a.counters = counters;
-    a.fuse_perm = fuse_perm;
     a.norm_w = norm_w; a.eps = eps;
     PermArgs& p = a.perm;
     p.ids = ids; p.n = n; p.topk = s.topk; p.n_experts = s.n_experts;
     p.counts = counts; p.starts = starts; p.perm_map = perm_map; p.gather_src = gather_src;
     p.active = active; p.n_active = n_active; p.has_shared = s.shared_inter > 0;
-    if (units) {
-        p.unit_expert = units->unit_expert; p.unit_row0 = units->unit_row0; p.unit_rows = units->unit_rows;
-        p.unit_first = units->unit_first; p.unit_count = units->unit_count;
-        p.n_units = units->n_units; p.unit_cap = units->unit_rows_cap; p.max_units = units->max_units;
-    }
+    p.unit_expert = units.unit_expert; p.unit_row0 = units.unit_row0; p.unit_rows = units.unit_rows;
+    p.unit_first = units.unit_first; p.unit_count = units.unit_count;
+    p.n_units = units.n_units; p.unit_cap = units.unit_rows_cap; p.max_units = units.max_units;
     const size_t lds = head_lds_bytes(n, s.hidden, s.n_experts);
     if (x_dtype == FERRITE_DT_F32) return launch_head_t<float>(a, xq.q ? 1 : 0, lds, st);
     if (x_dtype == FERRITE_DT_BF16) return launch_head_t<uint16_t>(a, xq.q ? 1 : 0, lds, st);
