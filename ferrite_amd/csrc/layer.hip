@@ -248,8 +248,10 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
                           bool clear_counters = false) {
     int rc = check_shape(shape, n, mode);
     if (rc) return rc;
-    // the packed buffer carries the router weight (transposed); the checkpoint-layout one is read only without it
-    if (!wts || (!packed && !wts->router_w) || !x || !out || !workspace) return FERRITE_ERR_INVALID_ARG;
+    // the packed buffer of a shape that has one carries the router weight (transposed); otherwise the checkpoint-layout one
+    // is read
+    const bool router_packed = packed != nullptr && shape->hidden % 128 == 0;
+    if (!wts || (!router_packed && !wts->router_w) || !x || !out || !workspace) return FERRITE_ERR_INVALID_ARG;
     if ((reinterpret_cast<uintptr_t>(workspace) & 255) || (reinterpret_cast<uintptr_t>(x) & 15) ||
         (reinterpret_cast<uintptr_t>(out) & 15))
         return FERRITE_ERR_INVALID_ARG;
@@ -317,7 +319,7 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
         if ((rc = mark(ev, 4, st))) return rc;
     } else {
     // 1. router logits: the reference's sequential-k f32 chain (exec/lib.rs:1107)
-    if (packed != nullptr && s.hidden % 128 == 0) {
+    if (router_packed) {
         PackedLayout L = packed_layout(s);
         rc = launch_router_chain(x, x_dtype, reinterpret_cast<const float*>(packed + L.router_t), n, s.hidden,
                                  s.n_experts, logits, st);

@@ -67,6 +67,19 @@ def test_layer_refuses_routing_parameters_outside_the_kernels_limits():
     assert _layer_rc(lib, backend, 0) == backend.ERR_INVALID_ARG
 
 
+def test_layer_refuses_a_missing_router_weight_whatever_else_is_given():
+    """A hidden size that the packed layout does not take is routed with the checkpoint-layout weight: without one the call
+    is refused, also where a packed buffer is passed along."""
+    from ferrite_amd import backend
+    lib = backend.load_library()
+    shape = backend.MoeShape(160, 8, 2, 128, 0, 1, 1, 2.5, 10.0)
+    d = C.c_void_p(4096)
+    w = backend.MoeWeights(**{k: 4096 for k, _ in backend.MoeWeights._fields_ if k not in ("router_w", "router_bias")})
+    for packed in (None, d):
+        assert lib.ferrite_moe_layer_mxfp4(C.byref(shape), C.byref(w), packed, d, backend.DT_F32, 4, d, backend.DT_F32,
+                                           backend.MODE_F32_CHECK, d, 1 << 30, None) == backend.ERR_INVALID_ARG
+
+
 def test_static_workspace_entry_refuses_oversize_before_touching_a_gpu():
     """The size check of ferrite_moe_layer_mxfp4_static is host arithmetic: it answers without a GPU."""
     from ferrite_amd import backend
