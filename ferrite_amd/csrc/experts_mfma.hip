@@ -580,9 +580,10 @@ __global__ __launch_bounds__(WAVES * 64, 2) void down_mfma_kernel(MfmaArgs a, in
 // waves that stream 128 KiB each, down 72 blocks.  Here the waves of a block share one item: wave w takes the w-th part of its
 // groups of four k steps, the partial sums meet in LDS and wave 0 finishes the item.  The activations' operand image
 // is sized for four rows.  Bound by the launch and the dependent reads at its start (tables, rows, weights) rather than
-// by 60 / 30 MB.  One token, two-term activations, per layer: gate/up 22.9 -> 16.2 us, down 14.3 -> 11.2 us.
-// Taken while there are at most SPLIT_ITEMS items: 432 items 84.0 -> 73.6 us a layer, 576 (hidden 7168) 133 -> 131, 816
-// (two tokens) 89.9 -> 90.8, 1584 (four) 110.6 -> 115.5.
+// by 60 / 30 MB.  One token, two-term activations: gate/up 22.1 -> 14.5 us, down 14.6 -> 10.7 us.
+// Taken while there are at most SPLIT_ITEMS items.  Layer without / with, us: 432 items (one token) 68.9 / 56.6, 576 (hidden
+// 7168) 106 / 101, 600 (four tokens, hidden 2048) 45.0 / 41.3; beyond the line 816 and 1088 (gate/up and down of two tokens)
+// 71.9 / 69.8, 1584 and 2112 (four) 90 / 96, 2112 and 3696 (four, hidden 7168) 168 / 180.
 constexpr int SPLIT_WAVES = 4, SPLIT_ROWS = 4, SPLIT_ITEMS = 640;
 
 template <int FILL, bool kX2, typename RowFn>

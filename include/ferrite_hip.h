@@ -39,7 +39,8 @@ extern "C" {
 #define FERRITE_DT_BF16 1
 
 /* layer arithmetic modes */
-#define FERRITE_MODE_F32_CHECK 0   /* f32 activations, weights dequantised exactly, f32 FMA dot products */
+#define FERRITE_MODE_F32_CHECK 0   /* f32 activations, weights dequantised exactly, f32 products on the matrix cores: blocks of
+                                    * 128 k summed in f32, the blocks in f64.  Serves the shapes the other modes decline. */
 #define FERRITE_MODE_MFMA_FP8 1    /* activations quantised e4m3 per 32 (e8m0 scale), block-scaled MFMA */
 #define FERRITE_MODE_MFMA_FP8_X2 2 /* the same with two-term activations: x ~ q1*s1 + q2*s2, the second term being the
                                     * e4m3-per-32 quantisation of what the first leaves over (about 8 significant
