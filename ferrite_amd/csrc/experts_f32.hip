@@ -23,8 +23,8 @@ typedef unsigned int fx_u4 __attribute__((ext_vector_type(4), aligned(4)));   //
 // to a sum in f64: 4.6e-7 from the 64-bit layer with f32 accumulators over the whole of K (27 tokens, hidden 2080), 2.5e-7
 // this way, 2.6e-7 with the lane-wise sums that this kernel replaced (one wave per output row and token, the weights
 // read again for every token: 283 + 157 us there, 58 + 32 us this way).
-// Bound by the matrix pipe: 32 cycles per MFMA, padding of the units to 16 rows included, next to 1.5 vector
-// instructions per weight for the decoding.
+// Most of the time goes to the matrix pipe, padding of the units to 16 rows included: it is busy in 50 % of the cycles that
+// a CU is busy at that shape (32 cycles per MFMA), vector instructions (1.5 per weight for the decoding) in 25 %.
 constexpr int FX_WIN = 512, FX_PITCH = FX_WIN + 4, FX_SETS = 4;
 
 struct FxArgs {

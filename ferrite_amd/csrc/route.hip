@@ -18,8 +18,9 @@ namespace fe {
 // tokens and outputs at four different k: lane l = (q = l / 16, r = l % 16) holds x[t0 + r] and w[o0 + r] at
 // k = 16 s + 4 q .. + 3, the MFMA of component c leaves in register 4 b + v the product of token 4 q + v, output r at
 // k = 16 s + 4 b + c.  A step of 16 k is two 16-byte LDS reads per lane, four MFMAs and 64 adds (four chains per lane);
-// the products of step s + 1 are made while the adds of step s run.  Bound by the matrix pipe (66 cycles per MFMA) and
-// the adds, which overlap between the waves of a SIMD only.
+// the products of step s + 1 are made while the adds of step s run.  Bound by the adds: of the cycles that a CU is busy
+// (4096 x 128, counters) vector instructions issue in 78 %, nine tenths of them adds; the matrix pipe is busy in 34 % (32
+// cycles per MFMA), nothing waits for LDS banks.
 //
 // chain_valu_kernel, for few chains, where a chain's own length is the time: one chain per lane (8 tokens x 8 outputs per
 // wave), multiply and add on the vector ALU.  A lone wave issues one instruction per four cycles.
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(256, 4) void chain_rows_kernel(ChainArgs a) {
 }
 
 // Which kernel (figures at the top): 512 tiles of 16 x 16 chains are two waves of the one-chain-per-lane kernel for each of
-// the chip's 1024 SIMDs; beyond that its LDS reads bound it, and below that the matrix-core kernel leaves SIMDs idle.  Up to
+// the chip's 1024 SIMDs; beyond that its multiplies and LDS reads bound it, and below that the matrix-core kernel leaves SIMDs idle.  Up to
 // four rows against more than 1024 tiles of outputs take the kernel that has no padding rows.
 // Up to 128 k the fetches that run ahead are not made past the end: they would be most of all fetches (24 x 65536, k 64:
 // 15 -> 11 us; 1 x 12288: 4.3 -> 3.7).  At 256 k, and with it in the loop of longer chains, the waits that the conditional loads
