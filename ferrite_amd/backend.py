@@ -238,10 +238,10 @@ class MoeLayer:
 
 class _Launch:
     """`with backend._launch() as st:` - st is the stream that the call's launches go to (HipBackend._begin_call)."""
-    __slots__ = ("be", "stream", "device")
+    __slots__ = ("be", "shared", "stream", "queued", "device")
 
-    def __init__(self, be: "HipBackend"):
-        self.be = be
+    def __init__(self, be: "HipBackend", shared: bool):
+        self.be, self.shared = be, shared
 
     def __enter__(self):
         be = self.be
@@ -250,7 +250,7 @@ class _Launch:
         try:
             if self.device != be.device.index:   # a handle of 0 means the current device's default stream
                 torch.cuda.set_device(be.device)
-            self.stream = be._begin_call()
+            self.stream, self.queued = be._begin_call(self.shared)
         except BaseException:
             self._restore()
             raise
@@ -258,7 +258,8 @@ class _Launch:
 
     def __exit__(self, *exc):
         try:
-            self.be._end_call(self.stream)
+            if self.queued:
+                self.be._end_call(self.stream)
         finally:
             self._restore()
 
@@ -312,23 +313,25 @@ class HipBackend:
             raise InvalidArg(f"{what} must be contiguous")
         return t
 
-    def _launch(self) -> _Launch:
-        return _Launch(self)
+    def _launch(self, shared: bool = False) -> _Launch:
+        """shared: the call uses memory that calls have in common (workspaces, buffers of a captured graph)."""
+        return _Launch(self, shared)
 
-    def _begin_call(self):
+    def _begin_call(self, shared: bool):
         """The stream a call runs on: torch's current one, behind the backend's earlier calls; the backend's own while its
-        capture is open (a capture stays on one stream)."""
+        capture is open (a capture stays on one stream).  And whether later calls have to wait for it."""
         if self._capturing:
-            return self._own
+            return self._own, True
         cur = torch.cuda.current_stream(self.device)
-        if torch.cuda.is_current_stream_capturing():
-            # another capture orders nothing against this backend's other calls, and a workspace made inside it would
-            # belong to its graph
-            if cur.cuda_stream != self._own.cuda_stream:
-                raise FerriteError("a capture that this backend has not begun is open on torch's current stream")
-        else:
+        if not torch.cuda.is_current_stream_capturing():
             self._follow(cur)
-        return cur
+        elif cur.cuda_stream != self._own.cuda_stream:
+            # a capture that the program opened orders nothing against the backend's other calls (and a workspace made
+            # inside it would belong to its graph), so it takes the calls that need no such order
+            if shared:
+                raise FerriteError("a capture that this backend has not begun is open on torch's current stream")
+            return cur, False
+        return cur, True
 
     def _outlives_calls(self, stream):
         return stream.cuda_stream in (0, self._own.cuda_stream)
@@ -617,7 +620,7 @@ class HipBackend:
             if nbytes == 0:
                 raise InvalidArg("unsupported shape / mode")
             ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            with self._launch() as st:
+            with self._launch(shared=True) as st:
                 self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
                                                                    st), "workspace_init")
             layer._ws[key] = ws
@@ -626,7 +629,7 @@ class HipBackend:
     def _on_this_stream(self, ws: torch.Tensor) -> torch.Tensor:
         """A cached workspace may be dropped with its layer while a call on another stream than the one it was allocated
         on still uses it."""
-        if not self._capturing:
+        if not (self._capturing or torch.cuda.is_current_stream_capturing()):
             ws.record_stream(torch.cuda.current_stream(self.device))
         return ws
 
@@ -655,7 +658,7 @@ class HipBackend:
         ws = workspace if workspace is not None else self.workspace(layer, n, mode)
         if stage_events is not None and len(stage_events) != STAGE_EVENTS:
             raise InvalidArg(f"stage_events must hold {STAGE_EVENTS} event handles")
-        with self._launch() as st:
+        with self._launch(shared=True) as st:
             args = (C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
                     x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, ws.data_ptr(), ws.numel(), st)
             if stage_events is None:
@@ -675,7 +678,7 @@ class HipBackend:
         dts = {torch.float32: DT_F32, torch.bfloat16: DT_BF16}
         if x.dtype not in dts or out.dtype not in dts or not x.is_contiguous() or not out.is_contiguous():
             raise InvalidArg("x/out must be contiguous f32 or bf16 device tensors")
-        with self._launch() as st:
+        with self._launch(shared=True) as st:
             rc = self.lib.ferrite_moe_layer_mxfp4_static(
                 C.byref(layer.shape), C.byref(layer.weights), None if layer.packed is None else layer.packed.data_ptr(),
                 x.data_ptr(), dts[x.dtype], n, out.data_ptr(), dts[out.dtype], mode, st)
@@ -691,7 +694,7 @@ class HipBackend:
             if nbytes == 0:
                 raise InvalidArg("unsupported shape / mode")
             ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            with self._launch() as st:
+            with self._launch(shared=True) as st:
                 self._ck(self.lib.ferrite_moe_layer_workspace_init(C.byref(layer.shape), n, mode, ws.data_ptr(), nbytes,
                                                                    st), "workspace_init")
             layer._ws[key] = ws
@@ -727,7 +730,7 @@ class HipBackend:
         ws = workspace if workspace is not None else self.block_workspace(layer, n, mode)
         ptr = lambda t: None if t is None else t.data_ptr()
         blk = MoeBlockArgs(norm_w.data_ptr(), eps, ptr(residual), ptr(post), ptr(comb), nh)
-        with self._launch() as st:
+        with self._launch(shared=True) as st:
             self._ck(self.lib.ferrite_moe_block_mxfp4(C.byref(layer.shape), C.byref(layer.weights),
                                                       None if layer.packed is None else layer.packed.data_ptr(),
                                                       li.data_ptr(), C.byref(blk), n, out.data_ptr(), mode, ws.data_ptr(),
@@ -787,7 +790,7 @@ class HipBackend:
         """Replay launch of the captured graph into the same static buffers."""
         if trace.graph_exec is None:
             raise InvalidArg("trace holds no graph")
-        with self._launch() as st:
+        with self._launch(shared=True) as st:
             rc = self.lib.ferrite_graph_launch(C.c_void_p(trace.graph_exec), st)
         self._verify_ok = rc == OK
 

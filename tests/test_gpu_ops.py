@@ -518,6 +518,33 @@ def test_hc_post_bit_exact_vs_oracle(hip, oracle, s, nh, h):  # gpu_smoke.rs:308
     assert np.array_equal(out.cpu().numpy(), oracle.hc_post(x, res, post, comb))
 
 
+def test_ops_in_a_capture_of_the_programs_own(hip):
+    """torch.cuda.graph around calls that need no workspace: every replay gives what the eager calls give."""
+    g = torch.Generator().manual_seed(5)
+    x, w = (torch.randn(r, 256, generator=g).cuda() for r in (8, 48))
+    norm, logits = torch.empty_like(x), torch.empty(8, 48, device="cuda")
+
+    def calls():
+        hip.rmsnorm(x, w[0], 1e-6, norm)
+        hip.matmul(norm, w, None, logits)
+        codes, scales = hip.mxfp4_quant(norm)
+        return [norm, logits, codes, scales, hip.mxfp4_dequant(codes, scales), *hip.act_quant_fp8(norm),
+                *hip.act_quant_fp8_x2(norm)]
+
+    calls()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = calls()
+    for _ in range(3):
+        x.copy_(torch.randn(8, 256, generator=g))
+        graph.replay()
+        got = [t.clone() for t in captured]
+        for a, b in zip(got, calls()):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        torch.cuda.synchronize()
+
+
 def test_hc_post_shape_errors(hip):
     from ferrite_amd.backend import Declined, ShapeMismatch
     z = lambda *sh: torch.zeros(*sh, device=hip.device)

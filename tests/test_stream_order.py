@@ -180,12 +180,30 @@ def test_a_capture_records_on_one_stream(hip):
     assert f"launch {len(Sim.launches) - 1}" in Sim.current.op("output")
 
 
-def test_another_capture_is_refused_except_on_the_backends_own_stream(hip):
+SHARED = ("layer", "layer_static", "block", "replay")   # calls that use memory other calls use too
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_a_capture_that_the_program_opened(hip, call):
+    """Calls that share nothing are recorded on its stream, and nothing eager waits for them; the others are refused there."""
+    Sim.current = side = Stream()
+    CALLS["rmsnorm"](hip)
+    side.capturing = True
+    if call in SHARED:
+        with pytest.raises(backend.FerriteError, match="capture"):
+            CALLS[call](hip)
+        assert len(Sim.launches) == 1
+    else:
+        CALLS[call](hip)
+        assert Sim.launches[-1][1] is side and len(Sim.launches) == 2
     Sim.current = Stream()
-    Sim.current.capturing = True
-    with pytest.raises(backend.FerriteError, match="capture"):
-        _layer_call(hip)
+    _layer_call(hip)
+    assert Sim.launches[-1][2] == {"launch 0"}
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_a_capture_that_the_program_opened_on_the_backends_own_stream(hip, call):
     Sim.current = hip.stream
     Sim.current.capturing = True
-    _layer_call(hip)
+    CALLS[call](hip)
     assert Sim.launches[-1][1] is Sim.current
