@@ -32,6 +32,32 @@ __device__ __forceinline__ uint32_t e4m3_encode4_hw(float a, float b, float c, f
     return (uint32_t)w;
 }
 
+// The same for finite values of magnitude <= 448 (a block divided by its own scale): below 2^-6 the step is 2^-9, and
+// a value held to +-7 * 2^-9 rounds to the code that the rule asks for.
+__device__ __forceinline__ float e4m3_prepare_finite(float x) {
+    const float small = __builtin_amdgcn_fmed3f(x, -0x1.cp-7f, 0x1.cp-7f);
+    return fabsf(x) < 0x1p-6f ? small : x;
+}
+__device__ __forceinline__ uint32_t e4m3_encode4_finite(float a, float b, float c, float d) {
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(e4m3_prepare_finite(a), e4m3_prepare_finite(b), 0, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(e4m3_prepare_finite(c), e4m3_prepare_finite(d), w, true);
+    return (uint32_t)w;
+}
+
+// What four codes leave over of the values they were made from: v - decode(code) * scale.  The product is exact (four
+// significant bits times a power of two), so one fused operation rounds as the subtraction alone does.
+__device__ __forceinline__ void e4m3_residual4(uint32_t codes, float scale, float* v) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    const f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, true);
+    v[0] = fmaf(-lo[0], scale, v[0]);
+    v[1] = fmaf(-lo[1], scale, v[1]);
+    v[2] = fmaf(-hi[0], scale, v[2]);
+    v[3] = fmaf(-hi[1], scale, v[3]);
+}
+
+// Larger magnitude, NaN if either is (fmaxf would drop it).
+__device__ __forceinline__ float amax_nan(float amax, float x) { return __builtin_elementwise_maximum(amax, fabsf(x)); }
+
 // Clamped SwiGLU (cpu.rs:192-201) for the MFMA mode, whose results are rounded to e4m3 right afterwards: the
 // hardware exponential and reciprocal (a few ulp) instead of the bit-exact expf and division of swiglu_ref().
 __device__ __forceinline__ float swiglu_fast(float g, float u, float limit) {
@@ -39,6 +65,13 @@ __device__ __forceinline__ float swiglu_fast(float g, float u, float limit) {
     // would turn a NaN accumulator into +-limit
     const float gi = g > limit ? limit : g;
     const float ui = u < -limit ? -limit : (u > limit ? limit : u);
+    return gi * __builtin_amdgcn_rcpf(1.0f + __expf(-gi)) * ui;
+}
+
+// The same for limit >= 0: NaN-propagating minimum and maximum are the two selects.
+__device__ __forceinline__ float swiglu_fast_min(float g, float u, float limit) {
+    const float gi = __builtin_elementwise_minimum(g, limit);
+    const float ui = __builtin_elementwise_maximum(__builtin_elementwise_minimum(u, limit), -limit);
     return gi * __builtin_amdgcn_rcpf(1.0f + __expf(-gi)) * ui;
 }
 
@@ -75,18 +108,31 @@ template <bool kResidual>
 __device__ __forceinline__ uint32_t encode_block32(float (&v)[32], uint8_t* __restrict__ q) {
     float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
-    const uint32_t sb = block_scale_e8m0(amax);
-    const float inv = u2f((254u - sb) << 23);   // 2^(127 - sb): exact reciprocal of the power-of-two scale
-    const float sc = u2f(sb << 23);
-    uint32_t out[8];
+    for (int i = 0; i < 32; ++i) amax = amax_nan(amax, v[i]);
+    uint32_t out[8], sb;
+    if (amax < __builtin_inff()) {
+        sb = block_scale_e8m0(amax);
+        const float inv = u2f((254u - sb) << 23);   // 2^(127 - sb): exact reciprocal of the power-of-two scale
+        const float sc = u2f(sb << 23);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        out[i] = e4m3_encode4_hw(v[4 * i] * inv, v[4 * i + 1] * inv, v[4 * i + 2] * inv, v[4 * i + 3] * inv);
-        if constexpr (kResidual) {
+        for (int i = 0; i < 8; ++i) {
+            out[i] = e4m3_encode4_finite(v[4 * i] * inv, v[4 * i + 1] * inv, v[4 * i + 2] * inv, v[4 * i + 3] * inv);
+            if constexpr (kResidual) e4m3_residual4(out[i], sc, &v[4 * i]);
+        }
+    } else {   // infinities or NaN in the block
+        amax = 0.0f;
+        for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        sb = block_scale_e8m0(amax);
+        const float inv = u2f((254u - sb) << 23);
+        const float sc = u2f(sb << 23);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[4 * i + j] = fadd(v[4 * i + j], -fmul(e4m3_decode((out[i] >> (8 * j)) & 0xffu), sc));
+        for (int i = 0; i < 8; ++i) {
+            out[i] = e4m3_encode4_hw(v[4 * i] * inv, v[4 * i + 1] * inv, v[4 * i + 2] * inv, v[4 * i + 3] * inv);
+            if constexpr (kResidual) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    v[4 * i + j] = fadd(v[4 * i + j], -fmul(e4m3_decode((out[i] >> (8 * j)) & 0xffu), sc));
+            }
         }
     }
     uint4* o = reinterpret_cast<uint4*>(q);

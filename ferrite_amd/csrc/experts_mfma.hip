@@ -404,7 +404,57 @@ __device__ __forceinline__ bool unit_block_work(const MfmaArgs& a, int groups, i
     return true;
 }
 
-// Clamped SwiGLU of one item's 32 gate and up rows for the unit's tokens, quantised to e4m3 (one or two terms).
+// The codes and scale bytes of 4 + 4 values per lane, whose block of 32 is spread over four lanes (lane, lane ^ 16, ...).
+struct QuantPair {
+    uint32_t p0, p1, sb;
+};
+
+// Lanes that share a block: the larger of their magnitudes, NaN if any is.
+__device__ __forceinline__ float block_amax(float amax) {
+    amax = amax_nan(amax, __shfl_xor(amax, 16, 64));
+    return amax_nan(amax, __shfl_xor(amax, 32, 64));
+}
+
+// One term of finite values; kResidual: they are replaced by what the term leaves over.
+template <bool kResidual>
+__device__ __forceinline__ QuantPair quant_pair_finite(float (&r0)[4], float (&r1)[4], float amax) {
+    const uint32_t sb = block_scale_e8m0(amax);
+    const float inv = u2f((254u - sb) << 23);
+    const uint32_t p0 = e4m3_encode4_finite(r0[0] * inv, r0[1] * inv, r0[2] * inv, r0[3] * inv);
+    const uint32_t p1 = e4m3_encode4_finite(r1[0] * inv, r1[1] * inv, r1[2] * inv, r1[3] * inv);
+    if constexpr (kResidual) {
+        const float sc = u2f(sb << 23);
+        e4m3_residual4(p0, sc, r0);
+        e4m3_residual4(p1, sc, r1);
+    }
+    return QuantPair{p0, p1, sb};
+}
+
+// One term of any values (the reference's encoder: NaN and infinities become +-448).
+__device__ __forceinline__ QuantPair quant_pair_any(float (&r0)[4], float (&r1)[4]) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) amax = fmaxf(amax, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    const uint32_t sb = block_scale_e8m0(amax);
+    const float inv = u2f((254u - sb) << 23), sc = u2f(sb << 23);
+    const uint32_t p0 = e4m3_encode4_hw(r0[0] * inv, r0[1] * inv, r0[2] * inv, r0[3] * inv);
+    const uint32_t p1 = e4m3_encode4_hw(r1[0] * inv, r1[1] * inv, r1[2] * inv, r1[3] * inv);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        r0[v] = fadd(r0[v], -fmul(e4m3_decode((p0 >> (8 * v)) & 0xffu), sc));
+        r1[v] = fadd(r1[v], -fmul(e4m3_decode((p1 >> (8 * v)) & 0xffu), sc));
+    }
+    return QuantPair{p0, p1, sb};
+}
+
+// Clamped SwiGLU of one item's 32 gate and up rows for the unit's tokens, quantised to e4m3 (one or two terms; the second
+// is the same quantiser on what the first leaves over).  Every lane of the wave must call this.
+// Vector instructions bound it: a wave of the tiled kernels has 32-64 values a lane to finish while nothing else runs on its
+// SIMD.  Finite values (any others in the wave take the general encoder) need no clamp to +-448, and the hardware
+// decodes the first term.  Layer before -> after, us: 4096 tokens of the decode shape two terms 1472 -> 1443, one term 895 -> 886;
+// 509 tokens two terms 400 -> 395.
 template <bool kX2>
 __device__ __forceinline__ void gate_up_store(const MfmaArgs& a, const v4f (&acc)[4], int item, int row0, int nrows,
                                               const ActPlanes& act, int lane) {
@@ -413,45 +463,40 @@ __device__ __forceinline__ void gate_up_store(const MfmaArgs& a, const v4f (&acc
     float amax = 0.0f;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        r0[v] = swiglu_fast(acc[0][v], acc[2][v], a.limit);
-        r1[v] = swiglu_fast(acc[1][v], acc[3][v], a.limit);
-        amax = fmaxf(amax, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
+        r0[v] = swiglu_fast_min(acc[0][v], acc[2][v], a.limit);
+        r1[v] = swiglu_fast_min(acc[1][v], acc[3][v], a.limit);
+        amax = amax_nan(amax_nan(amax, r0[v]), r1[v]);
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    const int c = lane & 15, g = lane >> 4;
-    const uint32_t sb = block_scale_e8m0(amax);
-    const float inv = u2f((254u - sb) << 23);
-    const uint32_t p0 = e4m3_encode4_hw(r0[0] * inv, r0[1] * inv, r0[2] * inv, r0[3] * inv);
-    const uint32_t p1 = e4m3_encode4_hw(r1[0] * inv, r1[1] * inv, r1[2] * inv, r1[3] * inv);
-    const size_t qoff = (size_t)(row0 + c) * a.act_ld + (size_t)item * 32 + g * 4;
-    const size_t soff = (size_t)(row0 + c) * scale_pitch(a.act_ld) + scale_pos(item);
-    if (c < nrows) {
-        *reinterpret_cast<uint32_t*>(act.q + qoff) = p0;
-        *reinterpret_cast<uint32_t*>(act.q + qoff + 16) = p1;
-        if (g == 0) act.s[soff] = (uint8_t)sb;
-    }
-    if constexpr (kX2) {
-        // second term: the same quantiser on what the first leaves over
-        const float sc = u2f(sb << 23);
-        float amax2 = 0.0f;
+    amax = block_amax(amax);
+    QuantPair q, q2{};
+    if (a.limit >= 0.0f && !__any(!(amax < __builtin_inff()))) {   // wave-uniform
+        q = quant_pair_finite<kX2>(r0, r1, amax);
+        if constexpr (kX2) {
+            float amax2 = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) amax2 = amax_nan(amax_nan(amax2, r0[v]), r1[v]);
+            q2 = quant_pair_finite<false>(r0, r1, block_amax(amax2));
+        }
+    } else {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            r0[v] = fadd(r0[v], -fmul(e4m3_decode((p0 >> (8 * v)) & 0xffu), sc));
-            r1[v] = fadd(r1[v], -fmul(e4m3_decode((p1 >> (8 * v)) & 0xffu), sc));
-            amax2 = fmaxf(amax2, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
+            r0[v] = swiglu_fast(acc[0][v], acc[2][v], a.limit);
+            r1[v] = swiglu_fast(acc[1][v], acc[3][v], a.limit);
         }
-        amax2 = fmaxf(amax2, __shfl_xor(amax2, 16, 64));
-        amax2 = fmaxf(amax2, __shfl_xor(amax2, 32, 64));
-        const uint32_t sb2 = block_scale_e8m0(amax2);
-        const float inv2 = u2f((254u - sb2) << 23);
-        const uint32_t t0 = e4m3_encode4_hw(r0[0] * inv2, r0[1] * inv2, r0[2] * inv2, r0[3] * inv2);
-        const uint32_t t1 = e4m3_encode4_hw(r1[0] * inv2, r1[1] * inv2, r1[2] * inv2, r1[3] * inv2);
-        if (c < nrows) {
-            *reinterpret_cast<uint32_t*>(act.q2 + qoff) = t0;
-            *reinterpret_cast<uint32_t*>(act.q2 + qoff + 16) = t1;
-            if (g == 0) act.s2[soff] = (uint8_t)sb2;
-        }
+        q = quant_pair_any(r0, r1);
+        if constexpr (kX2) q2 = quant_pair_any(r0, r1);
+    }
+    const int c = lane & 15, g = lane >> 4;
+    if (c >= nrows) return;
+    const size_t qoff = (size_t)(row0 + c) * a.act_ld + (size_t)item * 32 + g * 4;
+    const size_t soff = (size_t)(row0 + c) * scale_pitch(a.act_ld) + scale_pos(item);
+    *reinterpret_cast<uint32_t*>(act.q + qoff) = q.p0;
+    *reinterpret_cast<uint32_t*>(act.q + qoff + 16) = q.p1;
+    if (g == 0) act.s[soff] = (uint8_t)q.sb;
+    if constexpr (kX2) {
+        *reinterpret_cast<uint32_t*>(act.q2 + qoff) = q2.p0;
+        *reinterpret_cast<uint32_t*>(act.q2 + qoff + 16) = q2.p1;
+        if (g == 0) act.s2[soff] = (uint8_t)q2.sb;
     }
 }
 
@@ -874,35 +919,15 @@ __global__ __launch_bounds__(PF_WAVES * 64, PF_WAVES == 4 ? 2 : 1) void gate_up_
     v4f acc[2][4][4];
     pf_mainloop(c, reinterpret_cast<u4v*>(lds_raw), acc);
 
-    const int cc = c.lane & 15, g = c.lane >> 4;
-    const int apitch = scale_pitch(a.act_ld);
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii) {
         const int item = item0 + c.wi * 2 + ii;
         if (item >= items) break;
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
-            const int col = (c.wt * 4 + tt) * 16 + cc;
-            float r0[4], r1[4];
-            float amax = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                r0[v] = swiglu_fast(acc[ii][0][tt][v], acc[ii][2][tt][v], a.limit);
-                r1[v] = swiglu_fast(acc[ii][1][tt][v], acc[ii][3][tt][v], a.limit);
-                amax = fmaxf(amax, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
-            }
-            amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-            if (col < nrows) {
-                const uint32_t sb = block_scale_e8m0(amax);
-                const float inv = u2f((254u - sb) << 23);
-                const uint32_t p0 = e4m3_encode4_hw(r0[0] * inv, r0[1] * inv, r0[2] * inv, r0[3] * inv);
-                const uint32_t p1 = e4m3_encode4_hw(r1[0] * inv, r1[1] * inv, r1[2] * inv, r1[3] * inv);
-                uint8_t* dst = act_q + (size_t)(row0 + col) * a.act_ld + (size_t)item * 32 + g * 4;
-                *reinterpret_cast<uint32_t*>(dst) = p0;
-                *reinterpret_cast<uint32_t*>(dst + 16) = p1;
-                if (g == 0) act_s[(size_t)(row0 + col) * apitch + scale_pos(item)] = (uint8_t)sb;
-            }
+            const v4f t4[4] = {acc[ii][0][tt], acc[ii][1][tt], acc[ii][2][tt], acc[ii][3][tt]};
+            const int tile0 = (c.wt * 4 + tt) * 16;
+            gate_up_store<false>(a, t4, item, row0 + tile0, nrows - tile0, ActPlanes{act_q, act_s, nullptr, nullptr}, c.lane);
         }
     }
 }
@@ -1262,56 +1287,11 @@ __global__ __launch_bounds__(W * 64, W * NT <= 32 ? 2 : 1) void gate_up_stream_k
     st_mainloop<P>(c, reinterpret_cast<u4v*>(lds_raw), acc);
     if (item >= items) return;
 
-    // tiles 0,1 = gate rows [0,16),[16,32) of the item; tiles 2,3 = the same up rows
-    const int cc = c.lane & 15, g = c.lane >> 4;
-    const int apitch = scale_pitch(a.act_ld);
 #pragma unroll
     for (int tt = 0; tt < RT; ++tt) {
         if (tt >= c.ntile) continue;
-        const int col = tt * 16 + cc;
-        float r0[4], r1[4];
-        float amax = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            r0[v] = swiglu_fast(acc[0][tt][v], acc[2][tt][v], a.limit);
-            r1[v] = swiglu_fast(acc[1][tt][v], acc[3][tt][v], a.limit);
-            amax = fmaxf(amax, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
-        }
-        amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-        amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-        const uint32_t sb = block_scale_e8m0(amax);
-        const float inv = u2f((254u - sb) << 23);
-        const uint32_t p0 = e4m3_encode4_hw(r0[0] * inv, r0[1] * inv, r0[2] * inv, r0[3] * inv);
-        const uint32_t p1 = e4m3_encode4_hw(r1[0] * inv, r1[1] * inv, r1[2] * inv, r1[3] * inv);
-        const size_t qoff = (size_t)(row0 + col) * a.act_ld + (size_t)item * 32 + g * 4;
-        const size_t soff = (size_t)(row0 + col) * apitch + scale_pos(item);
-        if (col < nrows) {
-            *reinterpret_cast<uint32_t*>(act.q + qoff) = p0;
-            *reinterpret_cast<uint32_t*>(act.q + qoff + 16) = p1;
-            if (g == 0) act.s[soff] = (uint8_t)sb;
-        }
-        if constexpr (P == 2) {
-            // second term: the same quantiser on what the first leaves over (as in the 16-row kernel)
-            const float sc = u2f(sb << 23);
-            float amax2 = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                r0[v] = fadd(r0[v], -fmul(e4m3_decode((p0 >> (8 * v)) & 0xffu), sc));
-                r1[v] = fadd(r1[v], -fmul(e4m3_decode((p1 >> (8 * v)) & 0xffu), sc));
-                amax2 = fmaxf(amax2, fmaxf(fabsf(r0[v]), fabsf(r1[v])));
-            }
-            amax2 = fmaxf(amax2, __shfl_xor(amax2, 16, 64));
-            amax2 = fmaxf(amax2, __shfl_xor(amax2, 32, 64));
-            const uint32_t sb2 = block_scale_e8m0(amax2);
-            const float inv2 = u2f((254u - sb2) << 23);
-            const uint32_t t0 = e4m3_encode4_hw(r0[0] * inv2, r0[1] * inv2, r0[2] * inv2, r0[3] * inv2);
-            const uint32_t t1 = e4m3_encode4_hw(r1[0] * inv2, r1[1] * inv2, r1[2] * inv2, r1[3] * inv2);
-            if (col < nrows) {
-                *reinterpret_cast<uint32_t*>(act.q2 + qoff) = t0;
-                *reinterpret_cast<uint32_t*>(act.q2 + qoff + 16) = t1;
-                if (g == 0) act.s2[soff] = (uint8_t)sb2;
-            }
-        }
+        const v4f t4[4] = {acc[0][tt], acc[1][tt], acc[2][tt], acc[3][tt]};
+        gate_up_store<P == 2>(a, t4, item, row0 + tt * 16, nrows - tt * 16, act, c.lane);
     }
 }
 

@@ -139,13 +139,14 @@ FE_HD float e4m3_decode(uint32_t b) {
 }
 
 // quant.rs:155-165,190-198: 2^ceil(log2(amax/448)) floored at the smallest normal; returns the e8m0 byte
+// Worked out on the bits of amax instead of by a division: 448 = 1.75 * 2^8, so ceil(log2(amax / 448)) is amax's exponent
+// - 8, and one more if its mantissa is beyond 1.75 (the rounded quotient of such a value never falls back to a power of
+// two: the first one is 1 + 0.57 ulp, and the last one below 1.75 stays 1.14 ulp under 2).
 FE_HD uint32_t block_scale_e8m0(float amax) {
-    float q = fdiv(amax, 448.0f);
-    uint32_t bits = f2u(q);
-    int ex = (int)((bits >> 23) & 0xFFu);
-    int e = ex - 127 + ((bits & 0x7FFFFFu) ? 1 : 0);
-    int biased = e + 127;           // fast_pow2 bit pattern (biased << 23); 0 -> 0.0 -> floored to 2^-126
-    return (uint32_t)(biased < 1 ? 1 : biased);
+    const uint32_t bits = f2u(amax);                          // amax >= 0
+    if (bits >= 0x7f800000u) return bits > 0x7f800000u ? 256u : 255u;   // what the quotient's bits give for NaN and infinity
+    const uint32_t e = (bits + 0x1fffffu) >> 23;
+    return e < 9u ? 1u : e - 8u;
 }
 
 // quant.rs:98-124, including its subnormal rule: round(a*512) clamped to 7 (so [7.5/512, 8/512) encodes as 7)

@@ -459,6 +459,24 @@ def test_act_quant_two_terms_bit_exact_vs_oracle(hip, oracle, dtype):
     assert np.array_equal(host(hip, q).ravel(), q1) and np.array_equal(host(hip, s).ravel(), s1)
 
 
+def test_act_quant_blocks_with_nan_and_scale_edges(hip, oracle):
+    """NaN (either sign) in a block takes the general encoder, its neighbours the finite one; magnitudes on either side of
+    every step of the power-of-two scale (448 * 2^e)."""
+    rng = np.random.default_rng(9)
+    x = rng.normal(0, 1, (40, 64)).astype(np.float32)
+    x[:40, 32] = (448.0 * 2.0 ** np.arange(-20, 20)).astype(np.float32)
+    x[1::3, 32] = np.nextafter(x[1::3, 32], np.float32(np.inf))
+    x[2::3, 32] = np.nextafter(x[2::3, 32], np.float32(0))
+    x[4, 3], x[7, 31], x[9, 0:32:5] = np.nan, -np.nan, np.nan
+    q1, s1, q2, s2 = (host(hip, t).ravel() for t in hip.act_quant_fp8_x2(torch.from_numpy(x).to(hip.device)))
+    o1, t1, o2, t2 = oracle.act_quant_fp8_x2(x)
+    nan_blocks = np.isnan(x.reshape(-1, 32)).any(1)
+    assert nan_blocks.sum() == 3
+    assert np.array_equal(q1, o1) and np.array_equal(np.exp2(s1.astype(np.float64) - 127), t1.astype(np.float64))
+    assert np.array_equal(q2.reshape(-1, 32)[~nan_blocks], o2.reshape(-1, 32)[~nan_blocks])
+    assert np.array_equal(np.exp2(s2.astype(np.float64) - 127)[~nan_blocks], t2.astype(np.float64)[~nan_blocks])
+
+
 def test_pack_is_a_pure_permutation(hip, oracle):
     """dequant(packed) == dequant(checkpoint layout) for every matrix of several experts, bit for bit."""
     cfg = synth.MoeConfig(4, 256, 3, 2, 128, 256, 1, 1)

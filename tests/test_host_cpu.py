@@ -271,3 +271,13 @@ def test_format_primitives_match_the_oracle(shim, oracle):
         byte = shim.shim_block_scale_e8m0(a)
         _, s = oracle.act_quant_fp8(np.array([a] + [0.0] * 31, np.float32), 32, True)
         assert 2.0 ** (byte - 127) == float(s[0]), a
+
+
+def test_block_scale_is_the_rounded_quotient_s_exponent(shim):
+    """The scale from the bits of amax against the division it stands for: every exponent, mantissas around 1.75 and the ends."""
+    man = np.array([0, 1, 2, 0x400000, 0x5ffffe, 0x5fffff, 0x600000, 0x600001, 0x600002, 0x7ffffe, 0x7fffff], np.uint32)
+    amax = ((np.arange(256, dtype=np.uint32)[:, None] << 23) | man).ravel().view(np.float32)
+    with np.errstate(invalid="ignore"):
+        bits = (amax / np.float32(448.0)).view(np.uint32)
+    want = np.maximum(((bits >> 23) & 0xff).astype(int) + ((bits & 0x7fffff) != 0), 1)
+    assert [shim.shim_block_scale_e8m0(float(a)) for a in amax] == want.tolist()
