@@ -26,9 +26,9 @@ typedef unsigned int u4v __attribute__((ext_vector_type(4)));  // 128-bit vector
 
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// Which main loop the 128-row units run on (a test hook, ferrite_hip_set_override): 0 = the faster one for each GEMM
-// (gate/up: weights streamed into registers by blocks of 8 waves; down, whose reduction is a third as long: both
-// operands staged through LDS), 1 = staged for both, 2 / 3 = streamed by blocks of 8 / 4 waves for both.
+// Which main loop the tiled units run on (a test hook, ferrite_hip_set_override): 0 = the faster one for each GEMM and size
+// (gate/up: weights streamed into registers; down: streamed or both operands staged through LDS), 1 = staged for both
+// (one-term activations), 2 / 3 = streamed for both, several passes per block / a block per pass.
 static std::atomic<int> g_prefill_variant{0};
 void set_prefill_variant(int v) { g_prefill_variant.store(v, std::memory_order_relaxed); }
 
@@ -370,6 +370,7 @@ struct MfmaArgs {
     size_t codes_per_expert, scales_per_expert;
     const int32_t *unit_expert, *unit_row0, *unit_rows, *unit_first, *unit_count, *n_units;
     int n, topk, n_experts, hidden, inter, shared_inter, act_ld, unit_cap, max_units;
+    int cached;                   // the layer's weights fit the memory-side cache (256 MB): plain loads in the streamed passes
     float limit;
 };
 
@@ -1028,18 +1029,25 @@ __global__ __launch_bounds__(PF_WAVES * 64, PF_WAVES == 4 ? 2 : 1) void down_pre
 }
 
 // ---- prefill kernels, weight-streaming form --------------------------------------------------------------
-// One block (W waves) computes W items x NT*16 grouped rows of one unit.  Wave w owns item w for all of the rows:
-// its weights go from global memory straight into registers, 16 bytes per lane and tile as in the 16-row kernels,
-// through a ring of three k steps, so that a k step's tiles were asked for two to three steps before they are
-// used: far enough ahead for HBM.  Only the activations are shared by the block's waves and go through LDS: a ring
-// of three stages of one k step each ([tile][half][64 lanes] 16-byte slots in the operand order and slot swizzle
-// of the LDS-staged kernels, then [tile][64 lanes] scale words), filled through registers (ordinary loads keep the
-// compiler's wait counts exact, which loads that write LDS directly do not): the loads of step k+2 are issued at
-// the top of step k, written to their stage at the top of step k+1 and read during step k+2, one barrier per step.
+// A pass of a block (W waves) computes up to W items x NT*16 grouped rows of one unit.  Wave w owns one item for all of the
+// rows: its weights go from global memory straight into registers, 16 bytes per lane and tile as in the 16-row kernels,
+// D k steps ahead.  Only the activations are shared by the block's waves and go through LDS: a ring of four stages of
+// one k step each ([tile][half][64 lanes] 16-byte slots in the operand order and slot swizzle of the LDS-staged kernels;
+// behind all stages their scale words, [tile][64 lanes]), filled through registers (ordinary loads keep the compiler's
+// wait counts exact, which loads that write LDS directly do not): the loads of step k+3 are issued in step k, written to
+// their stage in step k+1 and first read in step k+2, one barrier per step.
+// A block goes through several passes with its loads running on from one into the next (stream_persistent has the line).
+// What bounds it, 509 tokens of the decode shape, two terms (gate/up 235 us with one block per pass, a ring of three k
+// steps and the fill and first operand reads between the barrier and the MFMAs; 188 us now): the weights' way from HBM (150 us
+// without MFMAs, epilogue and fills) and the steps themselves (146 us without any load), which overlap in part.  Each
+// pass began and ended with about 16 us in which nothing was in flight, and 3.2 rounds of blocks took as long as 4.
+// Prefetching deeper (three, four or six k steps; two or three sets of the fill's loads) and blocks of four waves, two per CU,
+// gained nothing: it is not latency.  With full units (4096 tokens, one term) the MFMAs, their operand reads and the
+// epilogue alone take 385 of 430 us.
 // Accumulation order over k is that of the other kernels: the same bits.
 template <int W, int NT>
 struct StCfg {
-    static constexpr int STAGES = 3;
+    static constexpr int STAGES = 4;
     static constexpr int CODE_SLOTS = NT * 128;            // 16-byte slots of e4m3 codes per stage
     static constexpr int STAGE_SLOTS = CODE_SLOTS + NT * 16;   // + NT * 64 scale words
     static constexpr size_t LDS_BYTES = (size_t)STAGES * STAGE_SLOTS * 16;
@@ -1051,6 +1059,7 @@ struct StCfg {
 // All four streams of a block are read through buffer resources (a wave-uniform base in scalar registers, a 32-bit
 // byte offset per lane that does not change over k, and the k step as a scalar offset): no 64-bit address
 // arithmetic in vector registers, of which this kernel has none to spare, and reads past a stream's end return 0.
+constexpr uint32_t ST_OUT = 0xfffff000u;   // a lane's offset past the end of any stream: reads as zeros, without traffic
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, size_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(bytes > 0xffffffffull ? 0xffffffffull : bytes),
@@ -1059,52 +1068,31 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, size_t bytes) {
 __device__ __forceinline__ u4v rsrc_ld16(rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
 }
+__device__ __forceinline__ u4v rsrc_ld16_nt(rsrc_t r, uint32_t voff, uint32_t soff) {   // non-temporal
+    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 2);
+}
 __device__ __forceinline__ uint32_t rsrc_ld4(rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0);
 }
 
+// What a pass reads: one wave's item against one unit's rows.  The streams' resources are wave-uniform (scalar registers).
 template <int W, int NT>
 struct StCtx {
     rsrc_t ra, ras;          // this wave's item: codes [KT][4 tiles][64 lanes][16 B], scale words [KT4][64 lanes][16 B]
     rsrc_t rb, rbs;          // activation codes and scale rows (operand order)
-    uint32_t aoff;           // 16 * lane
     uint32_t coff[StCfg<W, NT>::CF];   // byte offset of the lane's chunk of piece i at k step 0
     uint32_t soff[StCfg<W, NT>::SF];   // byte offset of the lane's scale word of piece i, group 0
-    int KT, lane, wave, ntile, bslot;
+    uint32_t aoff;           // 16 * lane, ST_OUT for a wave without an item
+    int KT, ntile;
+    // Plain loads where the weights are wanted again: by the expert's other units, or by the next call if the whole layer
+    // stays in the memory-side cache.  Otherwise non-temporal ones (us, plain / non-temporal: 300 tokens at 1.3 GB of weights
+    // 343 / 332, 509 366 / 357; 500 tokens at 200 MB 100 / 111; units that share an expert, 2047 tokens 749 / 797).
+    int keep;
 };
 
-// A stage holds NT operand tiles of 16 rows each.  With one-term activations tile v is rows 16 v .. 16 v + 15 of the
-// unit; with two-term activations (P = 2 planes) the unit has NT / 2 tiles of rows and tile v is plane v % 2 of row
-// tile v / 2: both planes of a row tile accumulate into the same registers, and the tiles that hold rows of the unit
-// are the first ones of the stage in either case.
-// row_q(v, r) / row_s(v, r): byte offsets of row r of tile v's code row / scale row from bq / bs.
-template <int P, int W, int NT, typename RowQ, typename RowS>
-__device__ __forceinline__ void st_context(StCtx<W, NT>& c, const uint8_t* cbase, const uint8_t* sbase, int item, int KT,
-                                           int nrows, const uint8_t* bq, size_t bq_bytes, const uint8_t* bs,
-                                           size_t bs_bytes, RowQ row_q, RowS row_s) {
-    using Cfg = StCfg<W, NT>;
-    const int KT4 = (KT + 3) >> 2;
-    c.KT = KT;
-    c.lane = threadIdx.x & 63;
-    c.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    c.ntile = min(NT / P, (nrows + 15) >> 4);
-    c.ra = make_rsrc(cbase + (size_t)item * KT * 4096, (size_t)KT * 4096);
-    c.ras = make_rsrc(sbase + (size_t)item * KT4 * 1024, (size_t)KT4 * 1024);
-    c.rb = make_rsrc(bq, bq_bytes);
-    c.rbs = make_rsrc(bs, bs_bytes);
-    c.aoff = (uint32_t)c.lane * 16;
-    const int cc = c.lane & 15, g = c.lane >> 4;
-    // piece j of a stage = (tile j/2, half j%2): the four lanes of a quad fetch 64 consecutive bytes of row lane/4 of
-    // the tile, the chunk a lane fetches XORed with (row/2)%4 (see pf_context)
-#pragma unroll
-    for (int i = 0; i < Cfg::CF; ++i) {
-        const int j = c.wave * Cfg::CF + i;
-        c.coff[i] = row_q(j >> 1, c.lane >> 2) + (uint32_t)((j & 1) * 64 + ((c.lane & 3) ^ ((c.lane >> 3) & 3)) * 16);
-    }
-#pragma unroll
-    for (int i = 0; i < Cfg::SF; ++i) c.soff[i] = row_s(min(c.wave * Cfg::SF + i, NT - 1), cc) + (uint32_t)(g * 4);
-    c.bslot = 4 * cc + (g ^ ((cc >> 1) & 3));
-}
+struct StLane {
+    int lane, wave, bslot;
+};
 
 template <int W, int NT>
 struct StFill {
@@ -1121,116 +1109,192 @@ __device__ __forceinline__ void st_load(const StCtx<W, NT>& c, int kt, StFill<W,
 }
 
 template <int W, int NT>
-__device__ __forceinline__ void st_store(const StCtx<W, NT>& c, u4v* stage, const StFill<W, NT>& f) {
+__device__ __forceinline__ void st_store(const StLane& l, u4v* lds, int st, const StFill<W, NT>& f) {
     using Cfg = StCfg<W, NT>;
+    u4v* stage = lds + st * Cfg::CODE_SLOTS;
 #pragma unroll
-    for (int i = 0; i < Cfg::CF; ++i) stage[(c.wave * Cfg::CF + i) * 64 + c.lane] = f.cr[i];
-    uint32_t* sw = reinterpret_cast<uint32_t*>(stage + Cfg::CODE_SLOTS);
+    for (int i = 0; i < Cfg::CF; ++i) stage[(l.wave * Cfg::CF + i) * 64 + l.lane] = f.cr[i];
+    uint32_t* sw = reinterpret_cast<uint32_t*>(lds + Cfg::STAGES * Cfg::CODE_SLOTS) + st * NT * 64;
 #pragma unroll
     for (int i = 0; i < Cfg::SF; ++i)
-        if (c.wave * Cfg::SF + i < NT) sw[(c.wave * Cfg::SF + i) * 64 + c.lane] = f.sr[i];
+        if (W * Cfg::SF == NT || l.wave * Cfg::SF + i < NT) sw[(l.wave * Cfg::SF + i) * 64 + l.lane] = f.sr[i];
 }
-
-// The weights of k step kt (4 tiles) and the scale words of its group of four k steps.
-struct StWeights {
-    u4v a[4];
-    u4v sc;
-};
 
 template <int W, int NT>
-__device__ __forceinline__ void st_load_a(const StCtx<W, NT>& c, int kt, StWeights& w) {
+__device__ __forceinline__ void st_load_a(const StCtx<W, NT>& c, int kt, u4v (&a)[4]) {
+    if (c.keep) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) w.a[t] = rsrc_ld16(c.ra, c.aoff + t * 1024, (uint32_t)kt * 4096);
-    w.sc = rsrc_ld16(c.ras, c.aoff, (uint32_t)(kt >> 2) * 1024);
+        for (int t = 0; t < 4; ++t) a[t] = rsrc_ld16(c.ra, c.aoff, (uint32_t)(kt * 4096 + t * 1024));
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) a[t] = rsrc_ld16_nt(c.ra, c.aoff, (uint32_t)(kt * 4096 + t * 1024));
+    }
 }
 
-// k step kt against stage R = kt % 3 of the ring, with the weights in ring slot R.  The scale operands select their
-// byte with op_sel 0: the words are shifted by the k step's byte (kt % 4) first, which leaves the unrolling free
-// to follow the rings.  Every load is issued whatever kt is (past the end the last k step is fetched again and never
-// used): a load behind a branch makes the compiler wait for all loads at the next use of any.
-// kFull: all NT tiles of rows are live; otherwise tiles beyond ntile get no MFMAs (a unit's last block of rows is
-// usually far from full).
-template <int R, bool kFull, int P, int W, int NT>
-__device__ __forceinline__ void st_step(const StCtx<W, NT>& c, u4v* lds, int kt, StWeights (&w)[3], StFill<W, NT>& f,
-                                        v4f (&acc)[4][NT / P]) {
-    using Cfg = StCfg<W, NT>;
-    __syncthreads();   // stage R is complete; nobody reads the stage that is written next any more
-    st_store(c, lds + ((R + 1) % 3) * Cfg::STAGE_SLOTS, f);
-    __builtin_amdgcn_sched_barrier(0);
-    st_load(c, min(kt + 2, c.KT - 1), f);
-    __builtin_amdgcn_sched_barrier(0);
-    const u4v* stage = lds + R * Cfg::STAGE_SLOTS;
-    const uint32_t* sw = reinterpret_cast<const uint32_t*>(stage + Cfg::CODE_SLOTS);
-    const int sh = (kt & 3) * 8;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) w[R].sc[t] >>= sh;   // in place: a slot's scale words are used by this step only
-    // operand registers of the row tiles: two sets used in turn (a tile is read while the MFMAs of the tile before
-    // it run), or one where registers are short (the other wave of the SIMD then covers the read)
-    constexpr int NB = W * NT <= 32 ? 1 : 2;
-    u4v b[NB][2];
-    uint32_t bs[NB];
-    auto read_tile = [&](int tt) {
-        const u4v* bt = stage + tt * 128 + c.bslot;
-        b[tt % NB][0] = bt[0];
-        b[tt % NB][1] = bt[64];
-        bs[tt % NB] = sw[tt * 64 + c.lane];
+// Registers of the main loop: a ring of D k steps of weights, the scale words of the group of four k steps in use and of
+// the next one, the fill's loads, and two operand tiles.
+template <int W, int NT, int D>
+struct StRegs {
+    u4v a[D][4];
+    u4v sc, scn;
+    StFill<W, NT> f;
+    u4v b[2][2];
+    uint32_t bs[2];
+};
+
+template <int W, int NT, int D>
+__device__ __forceinline__ void st_read_tile(const StLane& l, const u4v* lds, int tile, int set, StRegs<W, NT, D>& r) {
+    const u4v* bt = lds + tile * 128 + l.bslot;
+    r.b[set][0] = bt[0];
+    r.b[set][1] = bt[64];
+    r.bs[set] = reinterpret_cast<const uint32_t*>(lds + StCfg<W, NT>::STAGES * StCfg<W, NT>::CODE_SLOTS)[tile * 64 + l.lane];
+}
+
+// K step kt = J modulo 4 of pass c; kLast: the pass's last group of four k steps, whose loads run on into pass n.
+// Order of a step: barrier (stage J + 1 is complete, nobody reads stage J + 2 any more), the first tile's MFMAs, whose
+// operands were read under the last tile of the step before, then the fill of stage J + 2 and its next loads, the other
+// tiles, each with the operands of the next one on their way, and the weights D steps ahead.
+// Every load is issued whatever kt is (past the end the last k step is fetched again and never used): a load behind a
+// branch makes the compiler wait for more than it has to.
+template <int J, bool kLast, int P, int D, int W, int NT>
+__device__ __forceinline__ void st_step(const StCtx<W, NT>& c, const StCtx<W, NT>& n, const StLane& l, u4v* lds, int kt,
+                                        StRegs<W, NT, D>& r, v4f (&acc)[4][NT / P]) {
+    constexpr int cur = J * NT, next = (J + 1) % 4 * NT;   // tiles of the ring
+    int ntile = kt < c.KT ? c.ntile : 0;
+    asm volatile("" : "+s"(ntile));   // or the addresses below are all worked out in front of the loop and kept
+    __syncthreads();
+    auto fill = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        st_store(l, lds, (J + 2) % 4, r.f);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kLast && J >= 1) st_load(n, min(J - 1, n.KT - 1), r.f);
+        else st_load(c, min(kt + 3, c.KT - 1), r.f);
+        __builtin_amdgcn_sched_barrier(0);
     };
-    read_tile(0);
+    if (ntile == 0) st_read_tile(l, lds, next, 0, r);
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
         const int rt = tt / P;
-        if (kFull || rt < c.ntile) {   // block-uniform; the live tiles are the first ones
-            if (NB == 2 && tt + 1 < NT) read_tile(tt + 1);
-            const u4v b0 = b[tt % NB][0], b1 = b[tt % NB][1];
-            bs[tt % NB] >>= sh;
+        if (rt < ntile) {   // block-uniform; the live tiles are the first ones
+            if (tt + 1 == NT) st_read_tile(l, lds, next, 0, r);
+            else if ((tt + 1) % P) st_read_tile(l, lds, cur + tt + 1, (tt + 1) % 2, r);
+            else st_read_tile(l, lds, (tt + 1) / P < ntile ? cur + tt + 1 : next, (tt + 1) % 2, r);
+            const u4v b0 = r.b[tt % 2][0], b1 = r.b[tt % 2][1];
             const v8i bv = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const v8i a8 = {(int)w[R].a[t][0], (int)w[R].a[t][1], (int)w[R].a[t][2], (int)w[R].a[t][3], 0, 0, 0, 0};
+                const u4v av = r.a[J % D][t];
+                const v8i a8 = {(int)av[0], (int)av[1], (int)av[2], (int)av[3], 0, 0, 0, 0};
                 acc[t][rt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a8, bv, acc[t][rt], 4 /*A e2m1*/, 0 /*B e4m3*/,
-                                                                              0, (int)w[R].sc[t], 0, (int)bs[tt % NB]);
+                                                                              J, (int)r.sc[t], J, (int)r.bs[tt % 2]);
             }
-            if (NB == 1 && tt + 1 < NT) read_tile(tt + 1);
             // Pins the tile: its MFMAs stay in front of this point and the operand reads of the tiles after the next
             // behind it.  Without it the compiler reads all tiles of the step first (64 more registers than there are).
             asm volatile("" : "+v"(acc[0][rt]), "+v"(acc[1][rt]), "+v"(acc[2][rt]), "+v"(acc[3][rt]) : : "memory");
         }
+        if (tt == 0) fill();
     }
-    st_load_a(c, min(kt + 3, c.KT - 1), w[R]);
+    if (P == 1 && (ntile & 1)) {   // the last live tile read the next step's first operands into the other set
+        r.b[0][0] = r.b[1][0]; r.b[0][1] = r.b[1][1]; r.bs[0] = r.bs[1];
+    }
+    if constexpr (J == 0) {
+        if constexpr (kLast) r.scn = rsrc_ld16(n.ras, n.aoff, 0);
+        else r.scn = rsrc_ld16(c.ras, c.aoff, (uint32_t)((kt >> 2) + 1) * 1024);
+    }
+    if constexpr (J == 3) r.sc = r.scn;
+    if constexpr (kLast && J + D >= 4) st_load_a(n, min(J + D - 4, n.KT - 1), r.a[J % D]);
+    else st_load_a(c, min(kt + D, c.KT - 1), r.a[J % D]);
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <bool kFull, int P, int W, int NT>
-__device__ __forceinline__ void st_steps(const StCtx<W, NT>& c, u4v* lds, StWeights (&w)[3], StFill<W, NT>& f,
-                                         v4f (&acc)[4][NT / P]) {
-    const int KT = c.KT;
-    int kt = 0;
-#pragma unroll 1
-    for (; kt + 3 <= KT; kt += 3) {
-        st_step<0, kFull, P>(c, lds, kt, w, f, acc);
-        st_step<1, kFull, P>(c, lds, kt + 1, w, f, acc);
-        st_step<2, kFull, P>(c, lds, kt + 2, w, f, acc);
-    }
-    const int rem = KT - kt;   // block-uniform
-    if (rem > 0) st_step<0, kFull, P>(c, lds, kt, w, f, acc);
-    if (rem > 1) st_step<1, kFull, P>(c, lds, kt + 1, w, f, acc);
+// Fills the pipeline for the first pass of a block.
+template <int D, int W, int NT>
+__device__ __forceinline__ void st_start(const StCtx<W, NT>& c, const StLane& l, u4v* lds, StRegs<W, NT, D>& r) {
+    StFill<W, NT> f0, f1;
+    st_load(c, 0, f0);
+    st_load(c, min(1, c.KT - 1), f1);
+    r.sc = rsrc_ld16(c.ras, c.aoff, 0);
+#pragma unroll
+    for (int q = 0; q < D; ++q) st_load_a(c, min(q, c.KT - 1), r.a[q]);
+    st_store(l, lds, 0, f0);
+    st_store(l, lds, 1, f1);
+    st_load(c, min(2, c.KT - 1), r.f);
+    __syncthreads();
+    st_read_tile(l, lds, 0, 0, r);
 }
 
-template <int P, int W, int NT>
-__device__ __forceinline__ void st_mainloop(const StCtx<W, NT>& c, u4v* lds, v4f (&acc)[4][NT / P]) {
-    const int KT = c.KT;
-    StWeights w[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) st_load_a(c, min(q, KT - 1), w[q]);
-    StFill<W, NT> f;
-    st_load(c, 0, f);
+// One pass: all k steps of c, after which the first ones of n are on their way.
+template <int P, int D, int W, int NT>
+__device__ __forceinline__ void st_pass(const StCtx<W, NT>& c, const StCtx<W, NT>& n, const StLane& l, u4v* lds,
+                                        StRegs<W, NT, D>& r, v4f (&acc)[4][NT / P]) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int tt = 0; tt < NT / P; ++tt) acc[t][tt] = (v4f){0.f, 0.f, 0.f, 0.f};
-    st_store(c, lds, f);
-    st_load(c, min(1, KT - 1), f);
-    st_steps<false, P>(c, lds, w, f, acc);
+    int kt = 0;
+#pragma unroll 1
+    for (; kt + 4 < c.KT; kt += 4) {
+        st_step<0, false, P>(c, n, l, lds, kt, r, acc);
+        st_step<1, false, P>(c, n, l, lds, kt + 1, r, acc);
+        st_step<2, false, P>(c, n, l, lds, kt + 2, r, acc);
+        st_step<3, false, P>(c, n, l, lds, kt + 3, r, acc);
+    }
+    st_step<0, true, P>(c, n, l, lds, kt, r, acc);
+    st_step<1, true, P>(c, n, l, lds, kt + 1, r, acc);
+    st_step<2, true, P>(c, n, l, lds, kt + 2, r, acc);
+    st_step<3, true, P>(c, n, l, lds, kt + 3, r, acc);
+}
+
+// A pass of a block: expert, first row, rows (0: the tables were not well formed, nothing is stored), item group and
+// units of the expert.
+constexpr int ST_CUS = 256, ST_MAX_PASSES = 128;
+struct StPass {
+    int e, row0, nrows, ig, ne;
+};
+
+// Pass v of the launch, in the order of unit_block_work.
+__device__ __forceinline__ StPass st_lookup(const MfmaArgs& a, int n_units, int groups, int v) {
+    StPass p{0, 0, 0, 0, 0};
+    const int up = v / groups, first = a.unit_first[up], ne = a.unit_count[up];
+    if (first < 0 || ne < 1 || up < first || up >= first + ne || first + ne > n_units) return p;
+    const int vl = v - first * groups;
+    p.ig = vl / ne;
+    const int u = first + (vl - p.ig * ne), e = a.unit_expert[u], row0 = a.unit_row0[u], nrows = a.unit_rows[u];
+    if (unit_ok(a, e, row0, nrows)) { p.e = e; p.row0 = row0; p.nrows = nrows; p.ne = ne; }
+    return p;
+}
+
+// The passes of this block: block b works through passes xcd * per_xcd + slot, + slots, ... of its XCD's share, slot = b / 8.
+// kOne: the only one, into `one`; otherwise all of them, looked up at once, into `table`.  Returns their number.
+// groups comes in as a wave per item; several passes raise it as far as that leaves the rounds of passes the same, so
+// that the last round is not nearly empty (at 509 tokens of the decode shape 136 units x 6 groups are 3.2 rounds, x 7 are 3.7).
+template <bool kOne>
+__device__ __forceinline__ int st_passes(const MfmaArgs& a, int items, int& groups, StPass* table, StPass& one) {
+    const int n_units = min(*a.n_units, a.max_units);
+    if (n_units <= 0) return 0;
+    const int slots = gridDim.x >> 3, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    if constexpr (!kOne) {
+        const int rounds = (n_units * groups + ST_CUS - 1) / ST_CUS;
+        groups = max(groups, min(rounds * ST_CUS / n_units, min(2 * groups, items)));
+    }
+    const int total = n_units * groups, per_xcd = (total + 7) >> 3;
+    const int hi = min(per_xcd, total - xcd * per_xcd);   // passes of this XCD
+    if (slot >= hi) return 0;
+    if constexpr (kOne) {
+        one = st_lookup(a, n_units, groups, xcd * per_xcd + slot);
+        return one.nrows > 0 ? 1 : 0;
+    } else {
+        const int count = min((hi - slot + slots - 1) / slots, ST_MAX_PASSES);
+        for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup(a, n_units, groups, xcd * per_xcd + slot + i * slots);
+        __syncthreads();
+        return count;
+    }
+}
+
+__device__ __forceinline__ StPass st_pass_at(const StPass* table, int i) {
+    const StPass p = table[i];
+    return StPass{__builtin_amdgcn_readfirstlane(p.e), __builtin_amdgcn_readfirstlane(p.row0),
+                  __builtin_amdgcn_readfirstlane(p.nrows), __builtin_amdgcn_readfirstlane(p.ig), __builtin_amdgcn_readfirstlane(p.ne)};
 }
 
 // The span of two planes that one buffer resource covers: plane p starts d[p] bytes after lo.
@@ -1249,102 +1313,216 @@ __device__ __forceinline__ PlaneSpan plane_span(const uint8_t* p0, const uint8_t
 
 // P = 1: one-term activations, units of up to NT * 16 rows.  P = 2: two-term activations (both planes of x in, both
 // planes of the SwiGLU output out), units of up to NT * 8 rows: per k step and tile of rows a second MFMA against
-// the second plane with the same weight registers, so the stage, the fills and the MFMAs per block are those of
-// P = 1 and a launch has twice the blocks.
-template <int W, int NT, int P>
-__global__ __launch_bounds__(W * 64, W * NT <= 32 ? 2 : 1) void gate_up_stream_kernel(
-    MfmaArgs a, int groups, ActPlanes xin, const int32_t* __restrict__ gather_src, ActPlanes act) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int RT = NT / P;
-    int u, ig, ne;
-    if (!unit_block_work(a, groups, u, ig, ne)) return;
-    const int e = a.unit_expert[u], row0 = a.unit_row0[u], nrows = a.unit_rows[u];
-    if (!unit_ok(a, e, row0, nrows)) return;
-    const bool shared = e == a.n_experts;
-    const int inter = shared ? a.shared_inter : a.inter;
-    const int items = inter / 32, item0 = ig * W;
-    if (item0 >= items) return;
-    const int H = a.hidden, nk = a.n * a.topk, topk = a.topk, n = a.n;
-    const int spitch = scale_pitch(H);
-    auto token = [&](int col) -> int {
-        const int gr = row0 + (col < nrows ? col : 0);
-        if (shared) return gr - nk;
-        const int i = gather_src[gr];
-        const int tk = (i < 0 || i >= nk) ? 0 : i / topk;
-        return tk < n ? tk : 0;
-    };
-    const PlaneSpan xq = plane_span(xin.q, P == 2 ? xin.q2 : nullptr, (size_t)n * H);
-    const PlaneSpan xs = plane_span(xin.s, P == 2 ? xin.s2 : nullptr, (size_t)n * spitch);
-    StCtx<W, NT> c;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = item0 + wave;
-    st_context<P>(c, shared ? a.sh_codes : a.codes + (size_t)e * a.codes_per_expert,
-                  shared ? a.sh_scales : a.scales + (size_t)e * a.scales_per_expert, min(item, items - 1), H / 128, nrows,
-                  xq.lo, xq.bytes, xs.lo, xs.bytes,
-                  [&](int v, int r) { return xq.at(v % P) + (uint32_t)token((v / P) * 16 + r) * (uint32_t)H; },
-                  [&](int v, int r) { return xs.at(v % P) + (uint32_t)token((v / P) * 16 + r) * (uint32_t)spitch; });
-    v4f acc[4][RT];
-    st_mainloop<P>(c, reinterpret_cast<u4v*>(lds_raw), acc);
-    if (item >= items) return;
+// the second plane with the same weight registers, so the stage, the fills and the MFMAs per pass are those of
+// P = 1 and a launch has twice the passes.
+// A stage holds NT operand tiles of 16 rows each.  With one-term activations tile v is rows 16 v .. 16 v + 15 of the
+// unit; with two-term activations (P = 2 planes) the unit has NT / 2 tiles of rows and tile v is plane v % 2 of row
+// tile v / 2: both planes of a row tile accumulate into the same registers, and the tiles that hold rows of the unit
+// are the first ones of the stage in either case.
+// Piece j of a stage = (tile j/2, half j%2): the four lanes of a quad fetch 64 consecutive bytes of row lane/4 of
+// the tile, the chunk a lane fetches XORed with (row/2)%4 (see pf_context).
+template <int W, int NT>
+__device__ __forceinline__ uint32_t st_chunk(const StLane& l, int j) {
+    return (uint32_t)((j & 1) * 64 + ((l.lane & 3) ^ ((l.lane >> 3) & 3)) * 16);
+}
 
+template <int W>
+__device__ __forceinline__ StLane st_lane() {
+    StLane l;
+    l.lane = threadIdx.x & 63;
+    l.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cc = l.lane & 15, g = l.lane >> 4;
+    l.bslot = 4 * cc + (g ^ ((cc >> 1) & 3));
+    return l;
+}
+
+// The weights' side of a pass, an item of the unit's expert per wave: items ig * W .. of a block's only pass, the ig-th of
+// `groups` even parts otherwise.  Returns the wave's item, -1 for a wave without one (its loads return zeros).
+template <bool kDown, bool kOne, int P, int W, int NT>
+__device__ __forceinline__ int st_weights(StCtx<W, NT>& c, const MfmaArgs& a, const StPass& p, int groups, const StLane& l) {
+    const bool shared = p.e == a.n_experts;
+    const int inter = shared ? a.shared_inter : a.inter;
+    const int items = kDown ? a.hidden / 64 : inter / 32;
+    const int item = (kOne ? p.ig * W : p.ig * items / groups) + l.wave;
+    const bool live = item < (kOne ? items : (p.ig + 1) * items / groups) && p.nrows > 0;
+    c.KT = (kDown ? inter : a.hidden) / 128;
+    c.ntile = min(NT / P, (p.nrows + 15) >> 4);
+    c.keep = a.cached || p.ne > 1;
+    const int KT4 = (c.KT + 3) >> 2;
+    const uint8_t* cb = shared ? a.sh_codes : a.codes + (size_t)p.e * a.codes_per_expert;
+    const uint8_t* sb = shared ? a.sh_scales : a.scales + (size_t)p.e * a.scales_per_expert;
+    c.ra = make_rsrc(cb + (size_t)(live ? item : 0) * c.KT * 4096, (size_t)c.KT * 4096);
+    c.ras = make_rsrc(sb + (size_t)(live ? item : 0) * KT4 * 1024, (size_t)KT4 * 1024);
+    c.aoff = live ? (uint32_t)l.lane * 16 : ST_OUT;
+    return live ? item : -1;
+}
+
+// A pass of the same length whose loads all return zeros: what follows a block's only pass.
+template <int W, int NT>
+__device__ __forceinline__ void st_nothing(StCtx<W, NT>& n, const StCtx<W, NT>& c) {
+    n = c;
+    n.aoff = ST_OUT;
 #pragma unroll
-    for (int tt = 0; tt < RT; ++tt) {
-        if (tt >= c.ntile) continue;
-        const v4f t4[4] = {acc[0][tt], acc[1][tt], acc[2][tt], acc[3][tt]};
-        gate_up_store<P == 2>(a, t4, item, row0 + tt * 16, nrows - tt * 16, act, c.lane);
+    for (int i = 0; i < StCfg<W, NT>::CF; ++i) n.coff[i] = ST_OUT;
+#pragma unroll
+    for (int i = 0; i < StCfg<W, NT>::SF; ++i) n.soff[i] = ST_OUT;
+}
+
+template <int W, int NT, int P, int D, bool kOne>
+__global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, int groups, ActPlanes xin,
+                                                                   const int32_t* __restrict__ gather_src, ActPlanes act) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    using Cfg = StCfg<W, NT>;
+    constexpr int RT = NT / P;
+    u4v* lds = reinterpret_cast<u4v*>(lds_raw);
+    StPass* table = reinterpret_cast<StPass*>(lds_raw + Cfg::LDS_BYTES);
+    StPass p;
+    const int count = st_passes<kOne>(a, a.act_ld / 32, groups, table, p);
+    if (count == 0) return;
+    if constexpr (!kOne) p = st_pass_at(table, 0);
+    const int H = a.hidden, nk = a.n * a.topk, topk = a.topk, tokens = a.n;
+    const int spitch = scale_pitch(H);
+    const StLane l = st_lane<W>();
+    const PlaneSpan xq = plane_span(xin.q, P == 2 ? xin.q2 : nullptr, (size_t)tokens * H);
+    const PlaneSpan xs = plane_span(xin.s, P == 2 ? xin.s2 : nullptr, (size_t)tokens * spitch);
+    const rsrc_t rb = make_rsrc(xq.lo, xq.bytes), rbs = make_rsrc(xs.lo, xs.bytes);
+    // the grouped row of the lane's part of piece i / scale piece i, -1 beyond the unit's rows
+    auto row_of = [&](const StPass& p, int tile, int r) { const int col = tile / P * 16 + r; return col < p.nrows ? p.row0 + col : -1; };
+    auto code_row = [&](const StPass& p, int i) { return row_of(p, (l.wave * Cfg::CF + i) >> 1, l.lane >> 2); };
+    auto scale_row = [&](const StPass& p, int i) { return row_of(p, min(l.wave * Cfg::SF + i, NT - 1), l.lane & 15); };
+    // what gather_src holds for it (the shared expert's rows and rows beyond the unit read entry 0 and drop it)
+    auto gather = [&](const StPass& p, int row) { return gather_src[row >= 0 && p.e != a.n_experts ? row : 0]; };
+    auto token = [&](const StPass& p, int row, int gathered) {
+        if (p.e == a.n_experts) return row - nk;
+        const int tk = gathered < 0 || gathered >= nk ? 0 : gathered / topk;
+        return tk < tokens ? tk : 0;
+    };
+    auto offsets = [&](StCtx<W, NT>& c, const StPass& p, const int (&gc)[Cfg::CF], const int (&gs)[Cfg::SF]) {
+#pragma unroll
+        for (int i = 0; i < Cfg::CF; ++i) {
+            const int j = l.wave * Cfg::CF + i, row = code_row(p, i);
+            c.coff[i] = row < 0 ? ST_OUT : xq.at((j >> 1) % P) + (uint32_t)token(p, row, gc[i]) * (uint32_t)H + st_chunk<W, NT>(l, j);
+        }
+#pragma unroll
+        for (int i = 0; i < Cfg::SF; ++i) {
+            const int v = min(l.wave * Cfg::SF + i, NT - 1), row = scale_row(p, i);
+            c.soff[i] = row < 0 ? ST_OUT : xs.at(v % P) + (uint32_t)token(p, row, gs[i]) * (uint32_t)spitch + (uint32_t)((l.lane >> 4) * 4);
+        }
+    };
+    StCtx<W, NT> c, n;
+    c.rb = n.rb = rb; c.rbs = n.rbs = rbs;
+    int gc[Cfg::CF], gs[Cfg::SF];
+#pragma unroll
+    for (int i = 0; i < Cfg::CF; ++i) gc[i] = gather(p, code_row(p, i));
+#pragma unroll
+    for (int i = 0; i < Cfg::SF; ++i) gs[i] = gather(p, scale_row(p, i));
+    int item = st_weights<false, kOne, P>(c, a, p, groups, l);
+    offsets(c, p, gc, gs);
+    StRegs<W, NT, D> r;
+    st_start(c, l, lds, r);
+    const int apitch = scale_pitch(a.act_ld);
+#pragma unroll 1
+    for (int i = 0; i < count; ++i) {
+        StPass pn = p;
+        int item_n = item;
+        if constexpr (kOne) {
+            st_nothing(n, c);
+        } else {
+            pn = st_pass_at(table, min(i + 1, count - 1));
+            if (i + 1 == count) pn.nrows = 0;   // nothing follows: no traffic
+#pragma unroll
+            for (int q = 0; q < Cfg::CF; ++q) gc[q] = gather(pn, code_row(pn, q));
+#pragma unroll
+            for (int q = 0; q < Cfg::SF; ++q) gs[q] = gather(pn, scale_row(pn, q));
+            item_n = st_weights<false, kOne, P>(n, a, pn, groups, l);
+            offsets(n, pn, gc, gs);
+        }
+        v4f acc[4][RT];
+        st_pass<P>(c, n, l, lds, r, acc);
+        if (item >= 0) {
+#pragma unroll
+            for (int tt = 0; tt < RT; ++tt) {
+                if (tt >= c.ntile) continue;
+                const v4f t4[4] = {acc[0][tt], acc[1][tt], acc[2][tt], acc[3][tt]};
+                gate_up_store<P == 2>(a, t4, item, p.row0 + tt * 16, p.nrows - tt * 16, act, l.lane);
+            }
+        }
+        c = n; p = pn; item = item_n;
     }
 }
 
-template <int W, int NT, int P, typename YT>
-__global__ __launch_bounds__(W * 64, W * NT <= 32 ? 2 : 1) void down_stream_kernel(MfmaArgs a, int groups, ActPlanes act,
-                                                                                   YT* __restrict__ y) {
+template <int W, int NT, int P, int D, bool kOne, typename YT>
+__global__ __launch_bounds__(W * 64, 1) void down_stream_kernel(MfmaArgs a, int groups, ActPlanes act, YT* __restrict__ y) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    using Cfg = StCfg<W, NT>;
     constexpr int RT = NT / P;
-    int u, ig, ne;
-    if (!unit_block_work(a, groups, u, ig, ne)) return;
-    const int e = a.unit_expert[u], row0 = a.unit_row0[u], nrows = a.unit_rows[u];
-    if (!unit_ok(a, e, row0, nrows)) return;
-    const bool shared = e == a.n_experts;
-    const int inter = shared ? a.shared_inter : a.inter;
-    const int H = a.hidden, items = H / 64, item0 = ig * W;
-    if (item0 >= items) return;
-    const int apitch = scale_pitch(a.act_ld), act_ld = a.act_ld;
-    // both planes from the unit's first row on: the resources end with the unit's last row
-    const PlaneSpan aq = plane_span(act.q + (size_t)row0 * act_ld, P == 2 ? act.q2 + (size_t)row0 * act_ld : nullptr,
-                                    (size_t)nrows * act_ld);
-    const PlaneSpan as = plane_span(act.s + (size_t)row0 * apitch, P == 2 ? act.s2 + (size_t)row0 * apitch : nullptr,
-                                    (size_t)nrows * apitch);
-    StCtx<W, NT> c;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = item0 + wave;
-    auto rowc = [&](int v, int r) { const int col = (v / P) * 16 + r; return (uint32_t)(col < nrows ? col : 0); };
-    st_context<P>(c, shared ? a.sh_codes : a.codes + (size_t)e * a.codes_per_expert,
-                  shared ? a.sh_scales : a.scales + (size_t)e * a.scales_per_expert, min(item, items - 1), inter / 128, nrows,
-                  aq.lo, aq.bytes, as.lo, as.bytes,
-                  [&](int v, int r) { return aq.at(v % P) + rowc(v, r) * (uint32_t)act_ld; },
-                  [&](int v, int r) { return as.at(v % P) + rowc(v, r) * (uint32_t)apitch; });
-    v4f acc[4][RT];
-    st_mainloop<P>(c, reinterpret_cast<u4v*>(lds_raw), acc);
-    if (item >= items) return;
-
-    const int cc = c.lane & 15, g = c.lane >> 4;
+    u4v* lds = reinterpret_cast<u4v*>(lds_raw);
+    StPass* table = reinterpret_cast<StPass*>(lds_raw + Cfg::LDS_BYTES);
+    StPass p;
+    const int count = st_passes<kOne>(a, a.hidden / 64, groups, table, p);
+    if (count == 0) return;
+    if constexpr (!kOne) p = st_pass_at(table, 0);
+    const int H = a.hidden, apitch = scale_pitch(a.act_ld), act_ld = a.act_ld;
+    const StLane l = st_lane<W>();
+    auto context = [&](StCtx<W, NT>& c, const StPass& p) {
+        // both planes from the unit's first row on: the resources end with the unit's last row
+        const PlaneSpan aq = plane_span(act.q + (size_t)p.row0 * act_ld, P == 2 ? act.q2 + (size_t)p.row0 * act_ld : nullptr,
+                                        (size_t)max(p.nrows, 1) * act_ld);
+        const PlaneSpan as = plane_span(act.s + (size_t)p.row0 * apitch, P == 2 ? act.s2 + (size_t)p.row0 * apitch : nullptr,
+                                        (size_t)max(p.nrows, 1) * apitch);
+        c.rb = make_rsrc(aq.lo, aq.bytes);
+        c.rbs = make_rsrc(as.lo, as.bytes);
 #pragma unroll
-    for (int tt = 0; tt < RT; ++tt) {
-        if (tt >= c.ntile) continue;
-        if constexpr (sizeof(YT) == 4) {
-            const int col = tt * 16 + cc;
-            if (col < nrows) {
-                YT* dst = y + (size_t)(row0 + col) * H + (size_t)item * 64 + g * 4;
+        for (int i = 0; i < Cfg::CF; ++i) {
+            const int j = l.wave * Cfg::CF + i, v = j >> 1, col = v / P * 16 + (l.lane >> 2);
+            c.coff[i] = col < p.nrows ? aq.at(v % P) + (uint32_t)col * (uint32_t)act_ld + st_chunk<W, NT>(l, j) : ST_OUT;
+        }
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const v4f r = acc[t][tt];
-                    *reinterpret_cast<float4*>(dst + t * 16) = make_float4(r[0], r[1], r[2], r[3]);
+        for (int i = 0; i < Cfg::SF; ++i) {
+            const int v = min(l.wave * Cfg::SF + i, NT - 1), col = v / P * 16 + (l.lane & 15);
+            c.soff[i] = col < p.nrows ? as.at(v % P) + (uint32_t)col * (uint32_t)apitch + (uint32_t)((l.lane >> 4) * 4) : ST_OUT;
+        }
+        return st_weights<true, kOne, P>(c, a, p, groups, l);
+    };
+    StCtx<W, NT> c, n;
+    int item = context(c, p);
+    StRegs<W, NT, D> r;
+    st_start(c, l, lds, r);
+    const int cc = l.lane & 15, g = l.lane >> 4;
+#pragma unroll 1
+    for (int i = 0; i < count; ++i) {
+        StPass pn = p;
+        int item_n = item;
+        if constexpr (kOne) {
+            st_nothing(n, c);
+        } else {
+            pn = st_pass_at(table, min(i + 1, count - 1));
+            if (i + 1 == count) pn.nrows = 0;   // nothing follows: no traffic
+            item_n = context(n, pn);
+        }
+        v4f acc[4][RT];
+        st_pass<P>(c, n, l, lds, r, acc);
+        if (item >= 0) {
+#pragma unroll
+            for (int tt = 0; tt < RT; ++tt) {
+                if (tt >= c.ntile) continue;
+                if constexpr (sizeof(YT) == 4) {
+                    const int col = tt * 16 + cc;
+                    if (col < p.nrows) {
+                        YT* dst = y + (size_t)(p.row0 + col) * H + (size_t)item * 64 + g * 4;
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            const v4f q = acc[t][tt];
+                            *reinterpret_cast<float4*>(dst + t * 16) = make_float4(q[0], q[1], q[2], q[3]);
+                        }
+                    }
+                } else {
+                    store_y_tile_bf16(y + (size_t)(p.row0 + tt * 16) * H + (size_t)item * 64, (size_t)H, p.nrows - tt * 16,
+                                      acc[0][tt], acc[1][tt], acc[2][tt], acc[3][tt], l.lane);
                 }
             }
-        } else {
-            store_y_tile_bf16(y + (size_t)(row0 + tt * 16) * H + (size_t)item * 64, (size_t)H, nrows - tt * 16, acc[0][tt],
-                              acc[1][tt], acc[2][tt], acc[3][tt], c.lane);
         }
+        c = n; p = pn; item = item_n;
     }
 }
 
@@ -1355,6 +1533,26 @@ static bool planes_within_4g(const uint8_t* p0, const uint8_t* p1, size_t bytes)
     return (a > b ? a - b : b - a) + bytes < 0xffffffffull;
 }
 
+constexpr int ST_W = 8, ST_NT = 8, ST_D = 2;
+constexpr size_t ST_LDS = StCfg<ST_W, ST_NT>::LDS_BYTES + ST_MAX_PASSES * sizeof(StPass);
+// One block per CU that goes through several passes, whose loads run on from one into the next, where there are about
+// two and a half passes per CU; otherwise a block per pass, which the hardware hands to the CU that is free first.
+// A batch's units are estimated (the tables are on the device): an expert's last one is half full on average.
+// Layer, us, a block per pass / several (two terms unless said): hidden 5120, 32 experts, 300 tokens (0.9 passes per CU)
+// 171 / 178, 500 (1.7) 232 / 240, 1000 (2.1) 332 / 332, one term (1.3) 258 / 267; hidden 4096, 128 experts, 300 (3.1) 333 / 321,
+// 2047 (7.8) 783 / 744, 4096 1375 / 1310.
+static bool stream_persistent(const ferrite_moe_shape& s, int n, int cap, int groups) {
+    const int variant = g_prefill_variant.load(std::memory_order_relaxed);
+    if (variant >= 2) return variant == 2;
+    const double rows = (double)n * s.topk / s.n_experts, units = rows / cap + 0.5;
+    const double hit = rows < 1.0 ? (double)n * s.topk : (double)s.n_experts;
+    return (hit * (units > 1.0 ? units : 1.0) + (s.shared_inter > 0 ? (double)n / cap : 0.0)) * groups >= 2.5 * ST_CUS;
+}
+static unsigned stream_blocks(bool persistent, int max_units, int groups) {
+    if (!persistent) return (unsigned)(((size_t)max_units * groups + 7) / 8 * 8);
+    const size_t table = (size_t)ST_CUS * (ST_MAX_PASSES / 2);   // the kernel may double the groups
+    return (unsigned)(ST_CUS * (((size_t)max_units * groups + table - 1) / table));
+}
 constexpr int GU_WAVES = 4;
 constexpr int GU_WAVES_RESIDENT_X2 = 8;
 constexpr int DN_WAVES = 4;
@@ -1388,6 +1586,7 @@ static MfmaArgs make_args(const ferrite_moe_shape& s, const uint8_t* packed, int
     a.limit = s.swiglu_limit;
     a.unit_cap = units.unit_rows_cap;
     a.max_units = units.max_units;
+    a.cached = L.total <= (size_t)256 << 20;
     return a;
 }
 
@@ -1403,34 +1602,33 @@ int launch_gate_up_mfma(const ferrite_moe_shape& s, const uint8_t* packed, const
         // the tiled kernels: 128-row units of one-term activations, 64-row units of two-term activations
         if (units.unit_rows_cap != (x2 ? PF_ROWS_X2 : PF_ROWS)) return FERRITE_ERR_INVALID_ARG;
         const int variant = g_prefill_variant.load(std::memory_order_relaxed);
-        auto go = [&](auto kernel, int W, size_t lds) -> int {
-            const int groups = (imax / 32 + W - 1) / W;
-            const unsigned blocks = (unsigned)(((size_t)units.max_units * groups + 7) / 8 * 8);
-            hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(W * 64), (uint32_t)lds, st, k_start, k_stop, 0, a, groups,
-                                  xin, gather_src, act);
+        int rc;
+        const int groups = (imax / 32 + ST_W - 1) / ST_W;
+        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups);
+        auto go = [&](auto limit, auto kernel) -> int {
+            if ((rc = limit.ensure(ST_LDS))) return rc;
+            hipExtLaunchKernelGGL(kernel, dim3(stream_blocks(persistent, units.max_units, groups)), dim3(ST_W * 64), (uint32_t)ST_LDS, st,
+                                  k_start, k_stop, 0, a, groups, xin, gather_src, act);
             return check_launch("gate_up_stream");
         };
-        int rc;
+        auto stream = [&](auto planes, auto one) -> int {
+            constexpr int P = decltype(planes)::value;
+            constexpr bool kOne = decltype(one)::value;
+            return go(LdsLimit<&gate_up_stream_kernel<ST_W, ST_NT, P, ST_D, kOne>>{}, gate_up_stream_kernel<ST_W, ST_NT, P, ST_D, kOne>);
+        };
         if (x2) {
             // both planes through one buffer resource each: 32-bit offsets
             if (!planes_within_4g(xin.q, xin.q2, (size_t)n * s.hidden) || !planes_within_4g(xin.s, xin.s2, (size_t)n * scale_pitch(s.hidden)))
                 return FERRITE_ERR_INVALID_ARG;
-            if ((rc = LdsLimit<&gate_up_stream_kernel<8, 8, 2>>::ensure(StCfg<8, 8>::LDS_BYTES))) return rc;
-            return go(gate_up_stream_kernel<8, 8, 2>, 8, StCfg<8, 8>::LDS_BYTES);
+            return persistent ? stream(std::integral_constant<int, 2>{}, std::false_type{}) : stream(std::integral_constant<int, 2>{}, std::true_type{});
         }
-        if (variant == 3) {
-            if ((rc = LdsLimit<&gate_up_stream_kernel<4, 8, 1>>::ensure(StCfg<4, 8>::LDS_BYTES))) return rc;
-            return go(gate_up_stream_kernel<4, 8, 1>, 4, StCfg<4, 8>::LDS_BYTES);
-        }
-        if (variant != 1) {
-            if ((rc = LdsLimit<&gate_up_stream_kernel<8, 8, 1>>::ensure(StCfg<8, 8>::LDS_BYTES))) return rc;
-            return go(gate_up_stream_kernel<8, 8, 1>, 8, StCfg<8, 8>::LDS_BYTES);
-        }
-        const int groups = (imax / 32 + PF_ITEMS - 1) / PF_ITEMS;
-        const unsigned blocks = (unsigned)(((size_t)units.max_units * groups + 7) / 8 * 8);
+        if (variant != 1)
+            return persistent ? stream(std::integral_constant<int, 1>{}, std::false_type{}) : stream(std::integral_constant<int, 1>{}, std::true_type{});
+        const int pf_groups = (imax / 32 + PF_ITEMS - 1) / PF_ITEMS;
+        const unsigned blocks = (unsigned)(((size_t)units.max_units * pf_groups + 7) / 8 * 8);
         if ((rc = LdsLimit<&gate_up_prefill_kernel>::ensure(PF_LDS_BYTES))) return rc;
         hipExtLaunchKernelGGL(gate_up_prefill_kernel, dim3(blocks), dim3(PF_WAVES * 64), (uint32_t)PF_LDS_BYTES, st, k_start,
-                              k_stop, 0, a, groups, xin.q, xin.s, gather_src, act.q, act.s);
+                              k_stop, 0, a, pf_groups, xin.q, xin.s, gather_src, act.q, act.s);
         return check_launch("gate_up_prefill");
     }
     if (units.unit_rows_cap != 16) return FERRITE_ERR_INVALID_ARG;
@@ -1493,36 +1691,41 @@ int launch_down_mfma(const ferrite_moe_shape& s, const uint8_t* packed, const Ac
         const bool bf = y_dtype == FERRITE_DT_BF16;
         uint16_t* yh = static_cast<uint16_t*>(y);
         float* yf = static_cast<float*>(y);
-        auto go = [&](auto kernel, int W, size_t lds, auto* yp) -> int {
-            const int groups = (s.hidden / 64 + W - 1) / W;
-            const unsigned blocks = (unsigned)(((size_t)units.max_units * groups + 7) / 8 * 8);
-            kernel<<<blocks, W * 64, lds, st>>>(a, groups, act, yp);
+        int rc;
+        const int groups = (s.hidden / 64 + ST_W - 1) / ST_W;
+        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups);
+        auto go = [&](auto limit, auto kernel, auto* yp) -> int {
+            if ((rc = limit.ensure(ST_LDS))) return rc;
+            kernel<<<stream_blocks(persistent, units.max_units, groups), ST_W * 64, ST_LDS, st>>>(a, groups, act, yp);
             return check_launch("down_stream");
         };
+        auto stream_y = [&](auto planes, auto one, auto* yp) -> int {
+            using YT = std::remove_pointer_t<decltype(yp)>;
+            constexpr int P = decltype(planes)::value;
+            constexpr bool kOne = decltype(one)::value;
+            return go(LdsLimit<&down_stream_kernel<ST_W, ST_NT, P, ST_D, kOne, YT>>{}, down_stream_kernel<ST_W, ST_NT, P, ST_D, kOne, YT>, yp);
+        };
+        auto stream = [&](auto planes, auto one) -> int { return bf ? stream_y(planes, one, yh) : stream_y(planes, one, yf); };
         if (x2) {
             const size_t rows = (size_t)n * s.topk + (s.shared_inter > 0 ? n : 0);
             if (!planes_within_4g(act.q, act.q2, rows * a.act_ld) || !planes_within_4g(act.s, act.s2, rows * scale_pitch(a.act_ld)))
                 return FERRITE_ERR_INVALID_ARG;
-            constexpr size_t lds = StCfg<8, 8>::LDS_BYTES;
-            return bf ? go(down_stream_kernel<8, 8, 2, uint16_t>, 8, lds, yh) : go(down_stream_kernel<8, 8, 2, float>, 8, lds, yf);
+            return persistent ? stream(std::integral_constant<int, 2>{}, std::false_type{}) : stream(std::integral_constant<int, 2>{}, std::true_type{});
         }
-        if (variant == 3) {
-            constexpr size_t lds = StCfg<4, 8>::LDS_BYTES;
-            return bf ? go(down_stream_kernel<4, 8, 1, uint16_t>, 4, lds, yh) : go(down_stream_kernel<4, 8, 1, float>, 4, lds, yf);
-        }
-        if (variant == 2) {
-            constexpr size_t lds = StCfg<8, 8>::LDS_BYTES;
-            return bf ? go(down_stream_kernel<8, 8, 1, uint16_t>, 8, lds, yh) : go(down_stream_kernel<8, 8, 1, float>, 8, lds, yf);
-        }
-        const int groups = (s.hidden / 64 + PF_ITEMS - 1) / PF_ITEMS;
-        const unsigned blocks = (unsigned)(((size_t)units.max_units * groups + 7) / 8 * 8);
-        int rc;
+        // One term: the streaming form where it runs on from pass to pass and no k step is padding (a pass is a multiple of
+        // four), otherwise both operands through LDS.  Layer, us, through LDS / streamed: hidden 4096, inter 1536, 300 tokens
+        // 331 / 307, 1024 411 / 384, 4096 887 / 860; 160 experts, hidden 7168, inter 1024, 1000 535 / 511; inter 1408 (11 k steps),
+        // 500 161 / 172; hidden 2048, inter 768 (6), 1000 102 / 110.
+        if (variant >= 2 || (variant == 0 && persistent && s.inter % 512 == 0 && s.shared_inter % 512 == 0))
+            return persistent ? stream(std::integral_constant<int, 1>{}, std::false_type{}) : stream(std::integral_constant<int, 1>{}, std::true_type{});
+        const int pf_groups = (s.hidden / 64 + PF_ITEMS - 1) / PF_ITEMS;
+        const unsigned blocks = (unsigned)(((size_t)units.max_units * pf_groups + 7) / 8 * 8);
         if (bf) {
             if ((rc = LdsLimit<&down_prefill_kernel<uint16_t>>::ensure(PF_LDS_BYTES))) return rc;
-            down_prefill_kernel<uint16_t><<<blocks, PF_WAVES * 64, PF_LDS_BYTES, st>>>(a, groups, act.q, act.s, yh);
+            down_prefill_kernel<uint16_t><<<blocks, PF_WAVES * 64, PF_LDS_BYTES, st>>>(a, pf_groups, act.q, act.s, yh);
         } else {
             if ((rc = LdsLimit<&down_prefill_kernel<float>>::ensure(PF_LDS_BYTES))) return rc;
-            down_prefill_kernel<float><<<blocks, PF_WAVES * 64, PF_LDS_BYTES, st>>>(a, groups, act.q, act.s, yf);
+            down_prefill_kernel<float><<<blocks, PF_WAVES * 64, PF_LDS_BYTES, st>>>(a, pf_groups, act.q, act.s, yf);
         }
         return check_launch("down_prefill");
     }
@@ -1557,6 +1760,14 @@ int launch_down_mfma(const ferrite_moe_shape& s, const uint8_t* packed, const Ac
     return check_launch("down_mfma");
 }
 
+template <int P, bool kOne>
+static int warmup_stream() {
+    int rc;
+    if ((rc = LdsLimit<&gate_up_stream_kernel<ST_W, ST_NT, P, ST_D, kOne>>::ensure(ST_LDS))) return rc;
+    if ((rc = LdsLimit<&down_stream_kernel<ST_W, ST_NT, P, ST_D, kOne, uint16_t>>::ensure(ST_LDS))) return rc;
+    return LdsLimit<&down_stream_kernel<ST_W, ST_NT, P, ST_D, kOne, float>>::ensure(ST_LDS);
+}
+
 int warmup_experts_mfma() {
     int rc;
     if ((rc = LdsLimit<&gate_up_mfma_kernel<GU_WAVES, false, 0>>::ensure(kLdsCap))) return rc;
@@ -1568,8 +1779,8 @@ int warmup_experts_mfma() {
     if ((rc = LdsLimit<&gate_up_split_kernel<true>>::ensure(kLdsCap))) return rc;
     if ((rc = LdsLimit<&down_split_kernel<false>>::ensure(kLdsCap))) return rc;
     if ((rc = LdsLimit<&down_split_kernel<true>>::ensure(kLdsCap))) return rc;
-    if ((rc = LdsLimit<&gate_up_stream_kernel<8, 8, 1>>::ensure(StCfg<8, 8>::LDS_BYTES))) return rc;
-    if ((rc = LdsLimit<&gate_up_stream_kernel<8, 8, 2>>::ensure(StCfg<8, 8>::LDS_BYTES))) return rc;
+    if ((rc = warmup_stream<1, false>()) || (rc = warmup_stream<1, true>()) || (rc = warmup_stream<2, false>()) || (rc = warmup_stream<2, true>()))
+        return rc;
     if ((rc = LdsLimit<&gate_up_prefill_kernel>::ensure(PF_LDS_BYTES))) return rc;
     if ((rc = LdsLimit<&down_prefill_kernel<uint16_t>>::ensure(PF_LDS_BYTES))) return rc;
     return LdsLimit<&down_prefill_kernel<float>>::ensure(PF_LDS_BYTES);

@@ -68,9 +68,10 @@ int ferrite_hip_warmup(void);
  *   FERRITE_OVERRIDE_UNIT_ROWS  0 = automatic (default), 16 = force the 16-row streaming kernels, 128 = force the
  *                               tiled kernels (units of 128 rows, or of 64 rows with two-term activations)
  *   FERRITE_OVERRIDE_Y_F32      1 = keep the expert outputs `y` in f32 on the tiled path (default 0: bf16)
- *   FERRITE_OVERRIDE_PREFILL_TILE  main loop of the 128-row units: 0 = default (gate/up: weights streamed into
- *                               registers by blocks of 8 waves; down: both operands staged through LDS), 1 = staged
- *                               for both GEMMs, 2 / 3 = streamed by blocks of 8 / 4 waves for both (same bits)
+ *   FERRITE_OVERRIDE_PREFILL_TILE  main loop of the tiled units: 0 = default (gate/up: weights streamed into registers;
+ *                               down: the same or both operands staged through LDS, by size), 1 = staged for both GEMMs
+ *                               (one-term activations), 2 / 3 = streamed for both, several passes per block / a block per
+ *                               pass (same bits)
  *   FERRITE_OVERRIDE_HEAD       1 = router GEMM, routing, permutation and quantisation as separate launches whatever
  *                               the batch size (default 0: one fused launch for up to 256 tokens)  */
 #define FERRITE_OVERRIDE_UNIT_ROWS 0

@@ -265,7 +265,7 @@ def test_unit_rows_128_equals_16(hip, oracle, overrides, seed, n, hidden, inter,
                                                            (520, 7168, 2048, 2048, 8)])
 def test_prefill_main_loops_are_bit_identical(hip, overrides, n, hidden, inter, shared, experts):
     """The 128-row units have two main loops: both operands staged through LDS, or the weights streamed into
-    registers (blocks of 8 or 4 waves) and only the activations staged.  All accumulate over k in the order of the
+    registers (several passes per block, or one) and only the activations staged.  All accumulate over k in the order of the
     16-row kernels: the same bits at the benchmark's hidden and intermediate sizes (H 4096 / I 1536, H 7168 / I 2048),
     on full and ragged units, with f32 and with bf16 expert outputs."""
     from ferrite_amd.backend import OVERRIDE_PREFILL_TILE
@@ -289,6 +289,41 @@ def test_prefill_main_loops_are_bit_identical(hip, overrides, n, hidden, inter, 
     finally:
         hip.set_override(OVERRIDE_PREFILL_TILE, 0)
         layer._ws.clear()
+
+
+@pytest.mark.parametrize("mode", [MODE_MFMA_FP8, MODE_MFMA_FP8_X2])
+@pytest.mark.parametrize("n,hidden,inter,shared,experts,topk", [
+    (300, 384, 128, 640, 8, 3),      # reductions of 3 and 1 k steps, the shared expert's of 5
+    (700, 1152, 1408, 256, 8, 3),    # 9 and 11 k steps, item groups of uneven size, shared expert of one group
+    (40, 128, 128, 0, 16, 2),        # fewer passes than XCDs have blocks, one item
+    (200, 256, 1536, 0, 109, 8),     # 109 units x 6 item groups: the last round is filled by a seventh group
+    (2500, 1536, 768, 768, 4, 4),    # several passes per block by themselves, every token in every expert
+])
+def test_streamed_passes_do_not_depend_on_their_split(hip, overrides, mode, n, hidden, inter, shared, experts, topk):
+    """The streamed tiled kernels with a block per pass and with blocks whose loads run on from pass to pass: the same bits
+    as each other, as the 16-row kernels with one term, and to rounding with two (the planes are added in another order)."""
+    from ferrite_amd.backend import OVERRIDE_PREFILL_TILE
+    cfg = synth.MoeConfig(n, hidden, experts, topk, inter, shared, 4 if experts % 4 == 0 else 1, 4 if experts == 4 else 2 if experts % 4 == 0 else 1)
+    inp = synth.make_inputs(cfg, seed=n)
+    layer = hip.load_moe_layer(inp, keep_checkpoint_layout=False)
+    outs = {}
+    try:
+        for rows, variant in ((16, 0), (128, 0), (128, 2), (128, 3)):
+            overrides(unit_rows=rows, y_f32=1)
+            hip.set_override(OVERRIDE_PREFILL_TILE, variant)
+            layer._ws.clear()
+            outs[(rows, variant)], _ = run_layer(hip, layer, inp.x, mode)
+    finally:
+        hip.set_override(OVERRIDE_PREFILL_TILE, 0)
+        layer._ws.clear()
+    first = outs[(16, 0)]
+    assert np.isfinite(first).all() and float(np.abs(first).max()) > 0
+    for k in ((128, 0), (128, 2)):
+        assert np.array_equal(outs[k], outs[(128, 3)]), k
+    if mode == MODE_MFMA_FP8:
+        assert np.array_equal(outs[(128, 3)], first)
+    else:
+        assert max_abs_rel(outs[(128, 3)], first) <= 1e-4
 
 
 @pytest.mark.parametrize("seed,n,hidden,inter,shared", [(6, 150, 256, 256, 128), (7, 700, 384, 256, 384),
