@@ -121,6 +121,7 @@ __device__ __forceinline__ uint32_t encode_block32(float (&v)[32], uint8_t* __re
         }
     } else {   // infinities or NaN in the block
         amax = 0.0f;
+#pragma unroll
         for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
         sb = block_scale_e8m0(amax);
         const float inv = u2f((254u - sb) << 23);

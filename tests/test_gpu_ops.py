@@ -282,6 +282,49 @@ def test_moe_route_ties_lower_index_first(hip, oracle):  # cpu.rs:560
     assert route(hip, logits, bias, 8, 1.0)[1][0].tolist() == [5, 9, 70, 0, 1, 2, 3, 4]
 
 
+@pytest.mark.parametrize("e,k,ng,tg", [(512, 32, 8, 4), (160, 8, 8, 4), (96, 6, 8, 3), (64, 8, 64, 16), (128, 8, 2, 1), (256, 8, 2, 1),
+                                       (32, 8, 8, 4), (16, 16, 1, 1), (300, 7, 1, 1), (48, 4, 16, 2)])
+def test_moe_route_groups_and_thresholds_vs_oracle(hip, oracle, e, k, ng, tg):
+    """Groups that are aligned runs of 1 to 64 lanes, groups that are not, more than 64 experts a group; scores on a coarse grid,
+    so that many tie at the selection's threshold, in and across the 64-expert slots; infinite biases."""
+    rng = np.random.default_rng(e * 37 + ng)
+    logits = (np.round(rng.normal(0, 1.5, (24, e)) * 2) / 2).astype(np.float32)
+    logits[3] = 0.25
+    logits[5, : e // 2] = -300.0
+    bias = (rng.integers(0, 3, e) * 0.125).astype(np.float32)
+    bias[[1, e // 2]] = -np.inf
+    bias[e - 1] = np.inf
+    p, i = route(hip, logits, bias, k, 2.5, ng, tg)
+    po, io = oracle.moe_route(logits, bias, k, 2.5, ng, tg)
+    assert np.array_equal(i, io) and np.array_equal(p, po)
+
+
+@pytest.mark.parametrize("experts,topk,shared", [(16, 4, 128), (64, 32, 0), (100, 6, 128), (288, 8, 128)])
+def test_layer_tables_of_a_single_token(hip, oracle, experts, topk, shared):
+    """One token's tables come from the wave that routed it (one or several blocks of 64 experts): equal to the permutation's,
+    also where NaN scores leave slots empty, and the units are one row each."""
+    from ferrite_amd import synth
+    from ferrite_amd.backend import MODE_MFMA_FP8
+    cfg = synth.MoeConfig(1, 256, experts, topk, 128, shared, 1, 1)
+    inp = synth.make_inputs(cfg, seed=experts)
+    for nan_from in (experts, topk // 2):
+        inp.router_bias[nan_from:] = np.nan
+        layer = hip.load_moe_layer(inp)
+        x = torch.from_numpy(inp.x).to(hip.device)
+        out = torch.empty_like(x)
+        for _ in range(2):   # the second call finds the counters as the first left them
+            hip.moe_layer_dev_mxfp4(layer, x, out, MODE_MFMA_FP8)
+        hip.sync()
+        v = {k: t.cpu().numpy() for k, t in hip.workspace_view(layer, 1, MODE_MFMA_FP8).items()}
+        po, io = oracle.moe_route(v["logits"], inp.router_bias, topk, cfg.routed_scaling, 1, 1, nan_policy=1)
+        assert np.array_equal(v["ids"], io.astype(np.int32)) and np.array_equal(v["probs"], po)
+        t = oracle.moe_permute(v["ids"], experts)
+        for key in ("counts", "starts", "perm_map", "gather_src", "active"):
+            assert np.array_equal(v[key], t[key]), key
+        assert int(v["n_active"][0]) == t["n_active"] == min(topk, nan_from)
+        assert np.isfinite(out.cpu().numpy()).all()
+
+
 def test_moe_route_extreme_logits(hip, oracle):
     logits = np.array([[-200, -100, -88.5, -30, 0, 30, 88.5, 100, 200, 1e-30, -1e-30, 17.3, -17.3, 5, -5, 0.1]], np.float32)
     p, i = route(hip, logits, np.zeros(16, np.float32), 8, 2.5)
