@@ -520,6 +520,46 @@ def test_act_quant_blocks_with_nan_and_scale_edges(hip, oracle):
     assert np.array_equal(np.exp2(s2.astype(np.float64) - 127)[~nan_blocks], t2.astype(np.float64)[~nan_blocks])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_mxfp4_quant_ties_and_special_values_vs_oracle(hip, oracle, dtype):
+    """Values one ulp around every tie and code of the e2m1 grid at several block scales, signed zeros, quotients that
+    underflow, and blocks with NaN or infinities (which take the general encoder): codes and scales as the oracle's."""
+    rng = np.random.default_rng(12)
+    grid = np.array([0, .25, .5, .75, 1, 1.25, 1.5, 1.75, 2, 2.5, 3, 3.5, 4, 5, 6], np.float32)
+    near = np.concatenate([grid, np.nextafter(grid, np.float32(9)), np.nextafter(grid, np.float32(0))])
+    near = np.concatenate([near, -near, np.array([-0.0, 1e-45, -1e-45], np.float32)])
+    x = rng.choice(near, (96, 256)).astype(np.float32)
+    x[:, ::32] = 6.0
+    x *= np.repeat(2.0 ** rng.choice([-100.0, -20.0, 0.0, 3.0, 90.0], (96, 8)), 32, axis=1).astype(np.float32)
+    x[90, :32] = 0.0
+    x[91, 32:64], x[91, 32] = -1e-30, 3e38
+    x[92, 5], x[93, 40], x[94, 64:96] = np.inf, -np.inf, np.inf
+    xt = torch.from_numpy(x).to(dtype)
+    codes, scales = hip.mxfp4_quant(xt.to(hip.device))
+    want, s = oracle.act_quant_fp4(xt.float().numpy())
+    assert np.array_equal(host(hip, codes).ravel(), want)
+    finite = np.isfinite(s)
+    assert (~finite).sum() == 3
+    assert np.array_equal(np.exp2(host(hip, scales).ravel().astype(np.float64)[finite] - 127), s.astype(np.float64)[finite])
+    assert (host(hip, scales).ravel()[~finite] == 255).all()
+
+
+@pytest.mark.parametrize("hidden,inter,shared,experts", [(1152, 1408, 256, 3), (2048, 640, 0, 2)])
+def test_pack_of_uneven_reductions_is_a_pure_permutation(hip, oracle, hidden, inter, shared, experts):
+    """9, 11, 16 and 5 k steps: whole and cut chunks of a block, padded scale groups, whole-layer and per-expert packing."""
+    inp = synth.make_inputs(synth.MoeConfig(4, hidden, experts, 2, inter, shared, 1, 1), seed=hidden)
+    layer = hip.load_moe_layer(inp)
+    whole = layer.packed.clone()
+    for e in range(experts):
+        pair = lambda m: (hip.upload(getattr(inp, m + "_w")[e]), hip.upload(getattr(inp, m + "_s")[e]))
+        hip.pack_expert(layer, e, pair("gate"), pair("up"), pair("down"))
+        for which, m in enumerate(("gate", "up", "down")):
+            got = host(hip, hip.packed_dequant(layer, e, which))
+            assert np.array_equal(got, oracle.dequant_fp4_row32(getattr(inp, m + "_w")[e], getattr(inp, m + "_s")[e])), (e, which)
+    hip.sync()
+    assert torch.equal(layer.packed, whole)
+
+
 def test_pack_is_a_pure_permutation(hip, oracle):
     """dequant(packed) == dequant(checkpoint layout) for every matrix of several experts, bit for bit."""
     cfg = synth.MoeConfig(4, 256, 3, 2, 128, 256, 1, 1)
