@@ -162,6 +162,21 @@ __device__ __forceinline__ uint32_t quant_block32_x2(const XT* __restrict__ src,
     return s1 | (s2 << 8);
 }
 
+// Block b (of bpr per row) of the layer's input, codes row-major, scales in operand order.
+template <typename XT>
+__device__ __forceinline__ void quant_block_operand_order(const XT* __restrict__ x, long b, int bpr, uint8_t* __restrict__ q,
+                                                          uint8_t* __restrict__ scale, uint8_t* __restrict__ q2,
+                                                          uint8_t* __restrict__ scale2) {
+    const size_t at = (size_t)(b / bpr) * scale_pitch(bpr * 32) + scale_pos((int)(b % bpr));
+    if (q2) {
+        const uint32_t sb = quant_block32_x2(x + b * 32, q + b * 32, q2 + b * 32);
+        scale[at] = (uint8_t)(sb & 0xffu);
+        scale2[at] = (uint8_t)(sb >> 8);
+    } else {
+        scale[at] = (uint8_t)quant_block32(x + b * 32, q + b * 32);
+    }
+}
+
 // The left-to-right f32 sum (separately rounded adds, the reference's rmsnorm order: cpu.rs:124-143) of the n4 float4 at
 // s4 in LDS, continued from ss.  Every lane reads the same addresses and holds the same running sum.  For short rows.
 // Straight-line pieces of eight batches (256 values): a batch of eight 16-byte reads is in flight while the 32

@@ -136,7 +136,9 @@ int launch_hc_post(const float* x, const float* residual, const float* post, con
 
 // formats.hip
 // q2 / scale2 (both or neither): the second term of a two-term quantisation, from the residual of the first.
+int launch_route(const float* logits, const float* bias, int n, int e, int topk, int n_group, int topk_group, float scaling,
+                 float* probs, float* ids_f32, int32_t* ids_i32, const void* x, int x_dtype, int H, const ActPlanes& xq, hipStream_t st);
 int launch_act_quant(const void* x, int x_dtype, int64_t rows, int cols, uint8_t* q, uint8_t* scale, uint8_t* q2,
-                     uint8_t* scale2, int operand_order, hipStream_t st);
+                     uint8_t* scale2, hipStream_t st);
 
 }  // namespace fe

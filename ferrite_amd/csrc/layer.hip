@@ -328,9 +328,9 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
     }
     if (rc) return rc;
     if ((rc = mark(ev, 1, st))) return rc;
-    // 2. routing (exec/lib.rs:1109-1116); a NULL bias is the reference's zero bias
-    if ((rc = ferrite_moe_route(logits, wts->router_bias, n, s.n_experts, s.topk, s.n_group, s.topk_group,
-                                s.routed_scaling, probs, ids_f32, ids, stream)))
+    // 2. routing (exec/lib.rs:1109-1116); a NULL bias is the reference's zero bias.  The same launch quantises x.
+    if ((rc = launch_route(logits, wts->router_bias, n, s.n_experts, s.topk, s.n_group, s.topk_group, s.routed_scaling, probs, ids_f32,
+                           ids, x, x_dtype, s.hidden, xq, st)))
         return rc;
     if ((rc = mark(ev, 2, st))) return rc;
     // 3. permutation by expert + unit tables
@@ -340,9 +340,6 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
                              b + w.perm_scratch, w.perm_scratch_bytes, &units, has_shared, st)))
         return rc;
     if ((rc = mark(ev, 3, st))) return rc;
-    if (xq.q) {
-        if ((rc = launch_act_quant(x, x_dtype, n, s.hidden, xq.q, xq.s, xq.q2, xq.s2, 1, st))) return rc;
-    }
     if ((rc = mark(ev, 4, st))) return rc;
     }
     // 4-5. expert FFNs in grouped order, shared expert as the trailing rows

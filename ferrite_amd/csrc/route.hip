@@ -585,12 +585,31 @@ __device__ __forceinline__ void route_wave(const float* __restrict__ lg, const f
     else route_wave_ni<kCoherent, false, 8>(lg, 0.0f, bias, live, e, topk, n_group, topk_group, scaling, sc, probs, ids_f32, ids_i32);
 }
 
+// Blocks below route_blocks route four tokens each, a wave per token; the others quantise x (as act_quant_kernel in operand
+// order), which needs nothing of the routing: latency bounds the former, HBM the latter, so side by side they take little
+// more than the longer of the two.  Layer with two launches / one, us: hidden 2048, 64 experts, 300 tokens 86.5 / 84.4, 1000 tokens two
+// terms 135.9 / 132.6; hidden 4096, 128 experts, 300 303.8 / 301.6, 509 two terms 351.0 / 346.6, 2047 723 / 718, 4096 830 / 827.
+struct RouteQuant {
+    const void* x;
+    ActPlanes xq;
+    long nblocks;    // of 32 values, 0: none
+    int bpr;         // per row
+    int route_blocks;
+};
+
+template <typename XT>
 __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits,
                                                         const float* __restrict__ bias, int n, int e, int topk,
                                                         int n_group, int topk_group, float scaling,
                                                         float* __restrict__ probs, float* __restrict__ ids_f32,
-                                                        int32_t* __restrict__ ids_i32) {
+                                                        int32_t* __restrict__ ids_i32, RouteQuant rq) {
     __shared__ RouteScratch scratch[4];
+    if ((int)blockIdx.x >= rq.route_blocks) {
+        const long b = (long)((int)blockIdx.x - rq.route_blocks) * 256 + threadIdx.x;
+        if (b < rq.nblocks)
+            quant_block_operand_order(static_cast<const XT*>(rq.x), b, rq.bpr, rq.xq.q, rq.xq.s, rq.xq.q2, rq.xq.s2);
+        return;
+    }
     const int wave = threadIdx.x >> 6;
     const int t = blockIdx.x * 4 + wave;
     const bool live = t < n;
@@ -598,6 +617,18 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
     route_wave<false>(logits + tt * e, bias, live, e, topk, n_group, topk_group, scaling, scratch[wave],
                       probs + tt * topk, ids_f32 ? ids_f32 + tt * topk : nullptr,
                       ids_i32 ? ids_i32 + tt * topk : nullptr);
+}
+
+// Routing of n tokens and, with xq.q set, the quantisation of their rows of H values.  Parameters as checked by the callers.
+int launch_route(const float* logits, const float* bias, int n, int e, int topk, int n_group, int topk_group, float scaling,
+                 float* probs, float* ids_f32, int32_t* ids_i32, const void* x, int x_dtype, int H, const ActPlanes& xq, hipStream_t st) {
+    const int g = (n_group < 1 || topk_group == n_group) ? 1 : n_group;   // every group kept: the ungrouped router
+    RouteQuant rq{x, xq, xq.q ? (long)n * (H / 32) : 0, H / 32, (n + 3) / 4};
+    const unsigned grid = (unsigned)(rq.route_blocks + (rq.nblocks + 255) / 256);
+    auto go = [&](auto kernel) { kernel<<<grid, 256, 0, st>>>(logits, bias, n, e, topk, g, topk_group, scaling, probs, ids_f32, ids_i32, rq); };
+    if (x_dtype == FERRITE_DT_BF16) go(moe_route_kernel<uint16_t>);
+    else go(moe_route_kernel<float>);
+    return check_launch("moe_route");
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -647,17 +678,6 @@ struct UnitCut {
     }
 };
 
-// Inclusive sum over the lanes of a wave (row shifts, then the row totals passed on), without a trip through LDS.
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
 // wave 0 of a block: exclusive scan over experts + active list. cnt[] readable by the wave; starts_lds [E + 1] and
 // first_lds [E + 1] (an expert's first unit) are left for the rest of the block.
 __device__ __forceinline__ void perm_expert_scan(const PermArgs& a, const int32_t* cnt, int32_t* starts_lds, int32_t* first_lds) {
@@ -676,7 +696,7 @@ __device__ __forceinline__ void perm_expert_scan(const PermArgs& a, const int32_
             if (a.unit_cap > 0) ntile += (c + a.unit_cap - 1) >> cap_log;
         }
     }
-    const int s_tot = wave_scan(tot), s_act = wave_scan(nact), s_tile = wave_scan(ntile);
+    const int s_tot = wave_prefix(tot), s_act = wave_prefix(nact), s_tile = wave_prefix(ntile);
     int run = s_tot - tot, ract = s_act - nact, rtile = s_tile - ntile;
     const int total = __builtin_amdgcn_readlane(s_tot, 63), total_act = __builtin_amdgcn_readlane(s_act, 63),
               total_tile = __builtin_amdgcn_readlane(s_tile, 63);
@@ -1480,11 +1500,9 @@ extern "C" int ferrite_moe_route(const float* logits, const float* bias, int n, 
                                  int32_t* ids_i32, ferrite_stream_t stream) {
     if (n < 0 || !logits || !probs) return FERRITE_ERR_INVALID_ARG;
     if (int rc = check_routing_params(e, topk, n_group, topk_group)) return rc;
-    if (n_group < 1 || topk_group == n_group) n_group = 1;  // keeps every expert: the ungrouped router
     if (n == 0) return FERRITE_OK;
-    moe_route_kernel<<<(n + 3) / 4, 256, 0, as_stream(stream)>>>(logits, bias, n, e, topk, n_group, topk_group,
-                                                                 routed_scaling, probs, ids_f32, ids_i32);
-    return check_launch("moe_route");
+    return launch_route(logits, bias, n, e, topk, n_group, topk_group, routed_scaling, probs, ids_f32, ids_i32, nullptr, FERRITE_DT_F32, 0,
+                        ActPlanes{nullptr, nullptr, nullptr, nullptr}, as_stream(stream));
 }
 
 extern "C" size_t ferrite_moe_permute_scratch_bytes(int n, int topk, int n_experts) {
