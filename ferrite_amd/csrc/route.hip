@@ -597,14 +597,14 @@ struct RouteQuant {
     int route_blocks;
 };
 
-template <typename XT>
+template <typename XT, bool kQuant>
 __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits,
                                                         const float* __restrict__ bias, int n, int e, int topk,
                                                         int n_group, int topk_group, float scaling,
                                                         float* __restrict__ probs, float* __restrict__ ids_f32,
                                                         int32_t* __restrict__ ids_i32, RouteQuant rq) {
     __shared__ RouteScratch scratch[4];
-    if ((int)blockIdx.x >= rq.route_blocks) {
+    if (kQuant && (int)blockIdx.x >= rq.route_blocks) {
         const long b = (long)((int)blockIdx.x - rq.route_blocks) * 256 + threadIdx.x;
         if (b < rq.nblocks)
             quant_block_operand_order(static_cast<const XT*>(rq.x), b, rq.bpr, rq.xq.q, rq.xq.s, rq.xq.q2, rq.xq.s2);
@@ -626,8 +626,9 @@ int launch_route(const float* logits, const float* bias, int n, int e, int topk,
     RouteQuant rq{x, xq, xq.q ? (long)n * (H / 32) : 0, H / 32, (n + 3) / 4};
     const unsigned grid = (unsigned)(rq.route_blocks + (rq.nblocks + 255) / 256);
     auto go = [&](auto kernel) { kernel<<<grid, 256, 0, st>>>(logits, bias, n, e, topk, g, topk_group, scaling, probs, ids_f32, ids_i32, rq); };
-    if (x_dtype == FERRITE_DT_BF16) go(moe_route_kernel<uint16_t>);
-    else go(moe_route_kernel<float>);
+    if (!xq.q) go(moe_route_kernel<float, false>);   // half the registers: 1 us less for a few tokens
+    else if (x_dtype == FERRITE_DT_BF16) go(moe_route_kernel<uint16_t, true>);
+    else go(moe_route_kernel<float, true>);
     return check_launch("moe_route");
 }
 
