@@ -149,6 +149,30 @@ def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared, experts, topk, sh
     assert max_abs_rel(out, ref["out"]) <= TOL_F32
 
 
+def f32_splits_a_half_empty_round(n, topk, experts, kblocks, waves_per_unit, shared_waves):
+    """The second reason for four waves to share a pair: rounds of waves x blocks of 128 k, split against not, a tenth fewer."""
+    hit = experts * (1 - (1 - topk / experts) ** n)
+    waves = hit * max(1, n * topk / hit / 16 + 0.5) * waves_per_unit + -(-n // 16) * shared_waves
+    return waves <= 4096 and (4 * waves / 1024 + 0.5) * -(-kblocks // 4) <= 0.9 * np.ceil(0.97 * waves / 1024) * kblocks
+
+
+@pytest.mark.parametrize("n,hidden,inter,shared,experts,topk,splits", [
+    (9, 2080, 736, 736, 32, 6, (True, False)), (24, 2880, 736, 0, 32, 6, (True, False)), (5, 2080, 1504, 0, 32, 6, (False, True))])
+def test_f32_mode_split_of_a_half_empty_round(hip, oracle, n, hidden, inter, shared, experts, topk, splits):
+    """More waves than SIMDs, but so few more that the waves of a block share a pair all the same: within the f32 bar."""
+    kb = lambda k: -(-k // 128)
+    assert splits == (f32_splits_a_half_empty_round(n, topk, experts, kb(hidden), inter // 16, shared // 16),
+                      f32_splits_a_half_empty_round(n, topk, experts, kb(inter), hidden // 32, hidden // 32 if shared else 0))
+    cfg = synth.MoeConfig(n, hidden, experts, topk, inter, shared, 4, 2)
+    assert f32_waves_share_a_pair(cfg) != (True, True)
+    inp = synth.make_inputs(cfg, seed=n + hidden)
+    layer = hip.load_moe_layer(inp, pack=False)
+    ref = oracle.moe_ffn_mxfp4(inp, n_threads=8)
+    out, v = run_layer(hip, layer, inp.x, MODE_F32_CHECK)
+    check_routing(v, ref, oracle, cfg)
+    assert max_abs_rel(out, ref["out"]) <= TOL_F32
+
+
 @pytest.mark.parametrize("n,experts,topk,share", [(12, 8, 2, (True, True)), (40, 32, 4, (False, False))])
 def test_f32_mode_keeps_nan_where_it_belongs(hip, oracle, n, experts, topk, share):
     """NaN scales (byte 255) in every matrix, at the ends of rows and of ragged blocks: NaN exactly where the oracle has it,
