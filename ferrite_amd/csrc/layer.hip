@@ -43,10 +43,11 @@ static std::atomic<int> g_override_unit_rows{0};   // 0 = automatic, else 16 or 
 static std::atomic<int> g_override_y_f32{0};       // 1 = expert outputs stay f32 on the 128-row path
 static std::atomic<int> g_override_head{0};        // 1 = routing as separate launches whatever the batch size
 
-// Rows per unit: 16 (the weight-streaming kernels) while the average expert sees fewer than 16 rows; beyond that
-// (256 tokens at 128 experts and top-8: measured 378 against 387 us there, 449 against 488 us at 320 tokens, 512
-// against 717 us at 767) the tiled kernels, whose units hold 128 rows of one-term or 64 rows of two-term
-// activations.  The override forces one family or the other (16, or 128 = the tiled kernels).
+// Rows per unit: 16 (the weight-streaming kernels) while the average expert sees fewer than 16 rows; beyond that the
+// tiled kernels, whose units hold 128 rows of one-term or 64 rows of two-term activations.  The line is also where the
+// expert outputs change from f32 to bf16.  By time it could lie at about 13 rows (hidden 4096, 128 experts and top-8,
+// two terms, f32 outputs in both, 16-row / tiled: 192 tokens 296 / 300 us, 208 312 / 306, 224 344 / 313, 255 364 /
+// 333).  The override forces one family or the other (16, or 128 = the tiled kernels).
 int unit_rows_for(int n, int topk, int n_experts, bool two_term) {
     const int tiled = two_term ? 64 : 128;
     const int forced = g_override_unit_rows.load(std::memory_order_relaxed);
