@@ -1451,7 +1451,10 @@ int launch_permute(const int32_t* ids, int n, int topk, int n_experts, int32_t* 
     }
     const int nchunk = (n + 63) / 64;
     const size_t lds = perm_block_lds_bytes(n, n_experts);
-    if (n <= PM_SMALL_N && lds <= 60 * 1024) {
+    // one block while its masks, prefixes, counts and starts take at most 60 KiB: such calls need no scratch.  With the
+    // units' starts, E + 1 words more, 64 KiB are enough for every E up to PM_MAX_E.
+    static_assert(60 * 1024 + (PM_MAX_E + 1) * 4 <= 64 * 1024, "the block's tables fit the LDS of a plain launch");
+    if (n <= PM_SMALL_N && lds - (size_t)(n_experts + 1) * 4 <= 60 * 1024) {
         permute_small_kernel<<<1, 1024, lds, st>>>(a);
         return check_launch("permute_small");
     }

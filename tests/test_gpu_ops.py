@@ -438,6 +438,25 @@ def test_moe_permute_memcmp_vs_oracle(hip, oracle, n, k, e):
     assert np.array_equal(t["gather_src"], np.argsort(ids.ravel(), kind="stable"))
 
 
+@pytest.mark.parametrize("m,e,needs", [(513, 512, False), (577, 512, True), (640, 479, False), (640, 480, True),
+                                       (1024, 307, False), (1024, 308, True), (1025, 1, True)])
+def test_moe_permute_without_scratch(hip, oracle, m, e, needs):
+    """One block does the permutation, and no scratch is asked for, while masks, prefixes, counts and starts take 60 KiB:
+    12 bytes an expert and 64 assignments + 8 an expert + 4; at most 1024 assignments."""
+    assert needs == (m > 1024 or e * (12 * ((m + 63) // 64) + 8) + 4 > 60 * 1024)
+    ids = dev(hip, np.random.default_rng(m + e).integers(0, e, (m, 1)).astype(np.int32))
+    t = {k: torch.zeros(c, dtype=torch.int32, device=hip.device) for k, c in
+         (("counts", e), ("starts", e + 1), ("perm_map", m), ("gather_src", m), ("active", e), ("n_active", 1))}
+    rc = hip.lib.ferrite_moe_permute(ids.data_ptr(), m, 1, e, *(v.data_ptr() for v in t.values()), None, 0,
+                                     torch.cuda.current_stream(hip.device).cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == (3 if needs else 0)   # FERRITE_ERR_WORKSPACE, FERRITE_OK
+    if not needs:
+        o = oracle.moe_permute(ids.cpu().numpy(), e)
+        for key in ("counts", "starts", "perm_map", "gather_src", "active"):
+            assert np.array_equal(t[key].cpu().numpy(), o[key]), key
+
+
 def test_moe_permute_out_of_range_ids_drop_out(hip, oracle):  # dsv41_route.cu:253-261,300-303
     ids = np.array([[0, 7], [-1, 0], [2, 1]], np.int32)
     t = permute(hip, ids, 4)
