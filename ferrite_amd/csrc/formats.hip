@@ -167,6 +167,9 @@ extern "C" int ferrite_mxfp4_dequant(const uint8_t* w, const uint8_t* scale, int
     return check_launch("mxfp4_dequant");
 }
 
+// Blocks of 32 values a launch: four threads each, and a launch holds fewer than 2^32 threads.
+constexpr int64_t kMxQuantBlocks = int64_t(1) << 29;
+
 extern "C" int ferrite_mxfp4_quant(const void* x, int x_dtype, int64_t rows, int64_t cols, uint8_t* codes,
                                    uint8_t* scale, ferrite_stream_t stream) {
     if (rows < 0 || cols < 0 || cols % 32 != 0) return FERRITE_ERR_INVALID_ARG;
@@ -174,14 +177,17 @@ extern "C" int ferrite_mxfp4_quant(const void* x, int x_dtype, int64_t rows, int
     if (nblocks == 0) return FERRITE_OK;
     if (!x || !codes || !scale) return FERRITE_ERR_INVALID_ARG;
     if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(codes) & 15)) return FERRITE_DECLINED;
-    const unsigned grid = (unsigned)((nblocks * 4 + 255) / 256);
-    if (x_dtype == FERRITE_DT_F32)
-        mxfp4_quant_kernel<float><<<grid, 256, 0, as_stream(stream)>>>((const float*)x, nblocks, codes, scale);
-    else if (x_dtype == FERRITE_DT_BF16)
-        mxfp4_quant_kernel<uint16_t><<<grid, 256, 0, as_stream(stream)>>>((const uint16_t*)x, nblocks, codes, scale);
-    else
-        return FERRITE_ERR_INVALID_ARG;
-    return check_launch("mxfp4_quant");
+    if (x_dtype != FERRITE_DT_F32 && x_dtype != FERRITE_DT_BF16) return FERRITE_ERR_INVALID_ARG;
+    for (int64_t b0 = 0; b0 < nblocks; b0 += kMxQuantBlocks) {
+        const int64_t nb = nblocks - b0 < kMxQuantBlocks ? nblocks - b0 : kMxQuantBlocks;
+        const unsigned grid = (unsigned)((nb * 4 + 255) / 256);
+        if (x_dtype == FERRITE_DT_F32)
+            mxfp4_quant_kernel<float><<<grid, 256, 0, as_stream(stream)>>>((const float*)x + b0 * 32, nb, codes + b0 * 16, scale + b0);
+        else
+            mxfp4_quant_kernel<uint16_t><<<grid, 256, 0, as_stream(stream)>>>((const uint16_t*)x + b0 * 32, nb, codes + b0 * 16, scale + b0);
+        if (int rc = check_launch("mxfp4_quant")) return rc;
+    }
+    return FERRITE_OK;
 }
 
 extern "C" int ferrite_act_quant_fp8(const void* x, int x_dtype, int64_t rows, int cols, uint8_t* q, uint8_t* scale,
