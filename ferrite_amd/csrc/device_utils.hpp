@@ -44,8 +44,12 @@ __device__ __forceinline__ uint32_t e4m3_encode4_finite(float a, float b, float 
     return (uint32_t)w;
 }
 
-// What four codes leave over of the values they were made from: v - decode(code) * scale.  The product is exact (four
-// significant bits times a power of two), so one fused operation rounds as the subtraction alone does.
+// Blocks whose largest magnitude lies below this are the finite ones.  From 248 * 2^120 on, the midpoint of the codes 240 and
+// 256, code times scale is 2^128: the first term's product is infinite, and so is what it leaves over.
+constexpr float E4M3_FINITE_AMAX = 0x1.fp127f;
+
+// What four codes leave over of the values they were made from, in a finite block: v - decode(code) * scale.  The product is
+// exact (four significant bits times a power of two, below 2^128), so one fused operation rounds as the subtraction alone does.
 __device__ __forceinline__ void e4m3_residual4(uint32_t codes, float scale, float* v) {
     typedef float f2 __attribute__((ext_vector_type(2)));
     const f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, true);
@@ -110,7 +114,7 @@ __device__ __forceinline__ uint32_t encode_block32(float (&v)[32], uint8_t* __re
 #pragma unroll
     for (int i = 0; i < 32; ++i) amax = amax_nan(amax, v[i]);
     uint32_t out[8], sb;
-    if (amax < __builtin_inff()) {
+    if (amax < E4M3_FINITE_AMAX) {
         sb = block_scale_e8m0(amax);
         const float inv = u2f((254u - sb) << 23);   // 2^(127 - sb): exact reciprocal of the power-of-two scale
         const float sc = u2f(sb << 23);
@@ -119,7 +123,7 @@ __device__ __forceinline__ uint32_t encode_block32(float (&v)[32], uint8_t* __re
             out[i] = e4m3_encode4_finite(v[4 * i] * inv, v[4 * i + 1] * inv, v[4 * i + 2] * inv, v[4 * i + 3] * inv);
             if constexpr (kResidual) e4m3_residual4(out[i], sc, &v[4 * i]);
         }
-    } else {   // infinities or NaN in the block
+    } else {   // NaN or infinities in the block, or in what it leaves over
         amax = 0.0f;
 #pragma unroll
         for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));

@@ -483,7 +483,7 @@ __device__ __forceinline__ void gate_up_store(const MfmaArgs& a, const v4f (&acc
     }
     amax = block_amax(amax);
     QuantPair q, q2{};
-    if (a.limit >= 0.0f && !__any(!(amax < __builtin_inff()))) {   // wave-uniform
+    if (a.limit >= 0.0f && !__any(!(amax < E4M3_FINITE_AMAX))) {   // wave-uniform
         q = quant_pair_finite<kX2>(r0, r1, amax);
         if constexpr (kX2) {
             float amax2 = 0.0f;

@@ -539,6 +539,25 @@ def test_act_quant_blocks_with_nan_and_scale_edges(hip, oracle):
     assert np.array_equal(np.exp2(s2.astype(np.float64) - 127)[~nan_blocks], t2.astype(np.float64)[~nan_blocks])
 
 
+def test_act_quant_at_the_top_of_the_f32_range(hip, oracle):
+    """Block maxima from the last code below 2^128 to FLT_MAX.  From 248 * 2^120 on the code is 256 and code times scale is
+    infinite in f32: the second term is then made from what an infinite product leaves over.  Its scale is infinite, as the
+    oracle's, and its codes, which stand for nothing then, are all +-448."""
+    amax = np.concatenate([np.array([0x7f000000, 0x7f600000, 0x7f600001, 0x7f700000, 0x7f77ffff, 0x7f780000, 0x7f780001, 0x7f7c0000,
+                                     0x7f7fffff], np.uint32).view(np.float32), np.array([3.4e38, 3.3e38, 3.2e38], np.float32)])
+    rng = np.random.default_rng(13)
+    x = (rng.uniform(-1, 1, (2 * len(amax), 32)) * 2.0 ** rng.integers(90, 127, (2 * len(amax), 1))).astype(np.float32)
+    x[: len(amax), 7], x[len(amax):, 30] = amax, -amax
+    q1, s1, q2, s2 = (host(hip, t).ravel() for t in hip.act_quant_fp8_x2(torch.from_numpy(x).to(hip.device)))
+    o1, t1, o2, t2 = oracle.act_quant_fp8_x2(x)
+    assert np.array_equal(q1, o1) and np.array_equal(np.exp2(s1.astype(np.float64) - 127), t1.astype(np.float64))
+    over = np.tile(amax >= np.float32(248.0 * 2.0 ** 120), 2)
+    assert over.sum() == 12 and np.array_equal(np.isinf(t2), over)
+    assert (s2[over] == 255).all() and np.array_equal(np.exp2(s2[~over].astype(np.float64) - 127), t2[~over].astype(np.float64))
+    assert np.array_equal(q2.reshape(-1, 32)[~over], o2.reshape(-1, 32)[~over])
+    assert ((q2.reshape(-1, 32)[over] & 0x7f) == 0x7e).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_mxfp4_quant_ties_and_special_values_vs_oracle(hip, oracle, dtype):
     """Values one ulp around every tie and code of the e2m1 grid at several block scales, signed zeros, quotients that
