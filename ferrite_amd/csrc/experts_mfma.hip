@@ -15,6 +15,7 @@
 #include <hip/hip_ext.h>
 
 #include "internal.hpp"
+#include "launch_rules.hpp"
 #include "device_utils.hpp"
 #include "numerics.hpp"
 
@@ -1260,7 +1261,6 @@ __device__ __forceinline__ void st_pass(const StCtx<W, NT>& c, const StCtx<W, NT
 
 // A pass of a block: expert, first row, rows (0: the tables were not well formed, nothing is stored), item group and
 // units of the expert.
-constexpr int ST_CUS = 256, ST_MAX_PASSES = 128;
 struct StPass {
     int e, row0, nrows, ig, ne;
 };
@@ -1277,28 +1277,21 @@ __device__ __forceinline__ StPass st_lookup(const MfmaArgs& a, int n_units, int 
     return p;
 }
 
-// The passes of this block: block b works through passes xcd * per_xcd + slot, + slots, ... of its XCD's share, slot = b / 8.
-// kOne: the only one, into `one`; otherwise all of them, looked up at once, into `table`.  Returns their number.
-// groups comes in as a wave per item; several passes raise it as far as that leaves the rounds of passes the same, so
-// that the last round is not nearly empty (at 509 tokens of the decode shape 136 units x 6 groups are 3.2 rounds, x 7 are 3.7).
+// The passes of this block (stream_share).  kOne: the only one, into `one`; otherwise all of them, looked up at once, into
+// `table`.  Returns their number.  groups comes in as a wave per item.
 template <bool kOne>
 __device__ __forceinline__ int st_passes(const MfmaArgs& a, int items, int& groups, StPass* table, StPass& one) {
     const int n_units = min(*a.n_units, a.max_units);
     if (n_units <= 0) return 0;
-    const int slots = gridDim.x >> 3, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    if constexpr (!kOne) {
-        const int rounds = (n_units * groups + ST_CUS - 1) / ST_CUS;
-        groups = max(groups, min(rounds * ST_CUS / n_units, min(2 * groups, items)));
-    }
-    const int total = n_units * groups, per_xcd = (total + 7) >> 3;
-    const int hi = min(per_xcd, total - xcd * per_xcd);   // passes of this XCD
-    if (slot >= hi) return 0;
+    if constexpr (!kOne) groups = stream_raise(n_units, groups, items);
+    const StreamShare sh = stream_share(n_units * groups, gridDim.x, blockIdx.x);
+    if (sh.count <= 0) return 0;
     if constexpr (kOne) {
-        one = st_lookup(a, n_units, groups, xcd * per_xcd + slot);
+        one = st_lookup(a, n_units, groups, sh.first);
         return one.nrows > 0 ? 1 : 0;
     } else {
-        const int count = min((hi - slot + slots - 1) / slots, ST_MAX_PASSES);
-        for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup(a, n_units, groups, xcd * per_xcd + slot + i * slots);
+        const int count = min(sh.count, ST_MAX_PASSES);
+        for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup(a, n_units, groups, sh.first + i * sh.step);
         __syncthreads();
         return count;
     }
@@ -1433,7 +1426,6 @@ __global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, i
     offsets(c, p, gc, gs);
     StRegs<W, NT, D> r;
     st_start(c, l, lds, r);
-    const int apitch = scale_pitch(a.act_ld);
 #pragma unroll 1
     for (int i = 0; i < count; ++i) {
         StPass pn = p;
@@ -1560,11 +1552,6 @@ static bool stream_persistent(const ferrite_moe_shape& s, int n, int cap, int gr
     const double rows = (double)n * s.topk / s.n_experts, units = rows / cap + 0.5;
     const double hit = rows < 1.0 ? (double)n * s.topk : (double)s.n_experts;
     return (hit * (units > 1.0 ? units : 1.0) + (s.shared_inter > 0 ? (double)n / cap : 0.0)) * groups >= 2.5 * ST_CUS;
-}
-static unsigned stream_blocks(bool persistent, int max_units, int groups) {
-    if (!persistent) return (unsigned)(((size_t)max_units * groups + 7) / 8 * 8);
-    const size_t table = (size_t)ST_CUS * (ST_MAX_PASSES / 2);   // the kernel may double the groups
-    return (unsigned)(ST_CUS * (((size_t)max_units * groups + table - 1) / table));
 }
 constexpr int GU_WAVES = 4;
 constexpr int GU_WAVES_RESIDENT_X2 = 8;

@@ -1,5 +1,6 @@
-// Host build of csrc/numerics.hpp for the CPU tests (g++ -ffp-contract=off): the same text the device compiles.
-#include "../ferrite_amd/csrc/numerics.hpp"
+// Host build of csrc/numerics.hpp and csrc/launch_rules.hpp for the CPU tests (g++ -ffp-contract=off): the same text that
+// the device and the launchers compile.
+#include "../ferrite_amd/csrc/launch_rules.hpp"
 extern "C" {
 float shim_expf(float x) { return fe::fe_expf(x); }
 float shim_sigmoid(float x) { return fe::sigmoid_ref(x); }
@@ -10,4 +11,20 @@ float shim_e2m1_decode(unsigned c) { return fe::e2m1_decode(c); }
 float shim_ue8m0_decode(unsigned b) { return fe::ue8m0_decode(b); }
 unsigned shim_block_scale_e8m0(float amax) { return fe::block_scale_e8m0(amax); }
 void shim_expf_many(const float* x, float* y, long n) { for (long i = 0; i < n; ++i) y[i] = fe::fe_expf(x[i]); }
+int shim_stream_raise(int n_units, int groups, int items) { return fe::stream_raise(n_units, groups, items); }
+unsigned shim_stream_blocks(int several, int max_units, int groups) { return fe::stream_blocks(several != 0, max_units, groups); }
+// how often each of the passes 0 .. total - 1 is gone through; returns the largest number of passes of a block, -1 for one out of range
+int shim_stream_cover(int total, int blocks, int* times) {
+    int most = 0;
+    for (int b = 0; b < blocks; ++b) {
+        const fe::StreamShare s = fe::stream_share(total, blocks, b);
+        for (int i = 0; i < s.count; ++i) {
+            const int v = s.first + i * s.step;
+            if (v < 0 || v >= total) return -1;
+            ++times[v];
+        }
+        if (s.count > most) most = s.count;
+    }
+    return most;
+}
 }

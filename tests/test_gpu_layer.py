@@ -350,6 +350,28 @@ def test_streamed_passes_do_not_depend_on_their_split(hip, overrides, mode, n, h
         assert max_abs_rel(outs[(128, 3)], first) <= 1e-4
 
 
+def test_more_streamed_passes_than_a_block_per_cu_has_room_for(hip):
+    """4608 units of two-term activations x 8 item groups are more passes than the tables of 256 blocks hold: two rounds of blocks,
+    and the bits of a block per pass."""
+    from ferrite_amd.backend import OVERRIDE_PREFILL_TILE
+    cfg = synth.MoeConfig(32768, 128, 8, 8, 2048, 2048, 1, 1)
+    assert (cfg.n * 8 // 64 + 8 + cfg.n // 64) * (2048 // 32 // 8) > 256 * 128
+    inp = synth.make_inputs(cfg, seed=3)
+    layer = hip.load_moe_layer(inp, keep_checkpoint_layout=False)
+    x = hip.upload(inp.x)
+    outs = [torch.zeros_like(x) for _ in range(2)]
+    try:
+        for variant, out in zip((2, 3), outs):
+            hip.set_override(OVERRIDE_PREFILL_TILE, variant)
+            hip.moe_layer_dev_mxfp4(layer, x, out, MODE_MFMA_FP8_X2)
+            hip.sync()
+    finally:
+        hip.set_override(OVERRIDE_PREFILL_TILE, 0)
+        layer._ws.clear()
+    assert bool(torch.isfinite(outs[0]).all()) and bool((outs[0].abs().amax(1) > 0).all())
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("seed,n,hidden,inter,shared", [(6, 150, 256, 256, 128), (7, 700, 384, 256, 384),
                                                         (8, 1100, 512, 128, 0), (9, 520, 4096, 1536, 1536)])
 def test_two_term_64_row_units_agree_with_16_row_units(hip, oracle, overrides, seed, n, hidden, inter, shared):

@@ -1,6 +1,7 @@
 """CPU-side checks of the product: the C ABI library loads and exports every symbol the header declares, the
 op recorder behaves like the reference's (crates/ferrite-kernel/src/graph.rs:85-165), and the scalar numerics the
-kernels are built from (csrc/numerics.hpp, compiled for the host) agree with libm / the oracle bit for bit."""
+kernels are built from (csrc/numerics.hpp, compiled for the host) agree with libm / the oracle bit for bit, and the rules
+that launches follow (csrc/launch_rules.hpp) cover their work."""
 import ctypes as C
 import math
 import os
@@ -209,6 +210,7 @@ def shim(tmp_path_factory):
     lib.shim_e2m1_decode.argtypes = [C.c_uint]
     lib.shim_ue8m0_decode.argtypes = [C.c_uint]
     lib.shim_expf_many.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    lib.shim_stream_cover.argtypes = [C.c_int, C.c_int, C.c_void_p]
     return lib
 
 
@@ -281,3 +283,23 @@ def test_block_scale_is_the_rounded_quotient_s_exponent(shim):
         bits = (amax / np.float32(448.0)).view(np.uint32)
     want = np.maximum(((bits >> 23) & 0xff).astype(int) + ((bits & 0x7fffff) != 0), 1)
     assert [shim.shim_block_scale_e8m0(float(a)) for a in amax] == want.tolist()
+
+
+@pytest.mark.parametrize("groups,items", [(1, 2), (1, 8), (3, 20), (6, 48), (8, 64), (14, 112)])
+def test_streamed_passes_are_gone_through_once(shim, groups, items):
+    """Every pass of the streamed tiled kernels belongs to one block and fits its table of 128, whatever part of the units that a
+    launch is sized for is live; one block per CU as long as 128 passes per block suffice."""
+    for max_units in (1, 7, 42, 43, 128, 136, 300, 1023, 1408, 2340, 2341, 4096, 4097, 5000, 33000):
+        for n_units in sorted({1, max_units // 3 + 1, max_units - max_units // 8, max_units}):
+            for several in (0, 1):
+                g = shim.shim_stream_raise(n_units, groups, items) if several else groups
+                assert groups <= g <= max(groups, min(2 * groups, items))
+                blocks = shim.shim_stream_blocks(several, max_units, groups)
+                total = n_units * g
+                times = np.zeros(total, np.int32)
+                most = shim.shim_stream_cover(total, blocks, times.ctypes.data)
+                assert (times == 1).all() and blocks % 8 == 0
+                assert 0 < most <= (128 if several else 1)
+                if several:
+                    assert blocks == 256 * -(-max_units * groups // (256 * 128))
+                    assert -(-total // 256) == -(-n_units * groups // 256)
