@@ -383,7 +383,7 @@ struct MfmaArgs {
     const uint8_t* sh_scales;
     size_t codes_per_expert, scales_per_expert;
     const int32_t *unit_expert, *unit_row0, *unit_rows, *unit_first, *unit_count, *n_units;
-    int n, topk, n_experts, hidden, inter, shared_inter, act_ld, unit_cap, max_units;
+    int n, topk, n_experts, hidden, inter, shared_inter, act_ld, unit_cap, max_units, shared_units;
     int cached;                   // the layer's weights fit the memory-side cache (256 MB): plain loads in the streamed passes
     float limit;
 };
@@ -1259,39 +1259,45 @@ __device__ __forceinline__ void st_pass(const StCtx<W, NT>& c, const StCtx<W, NT
     st_step<3, true, P>(c, n, l, lds, kt + 3, r, acc);
 }
 
-// A pass of a block: expert, first row, rows (0: the tables were not well formed, nothing is stored), item group and
-// units of the expert.
+// A pass of a block: expert, first row, rows (0: the tables were not well formed, nothing is stored), units of the expert, and
+// the items from item0 up to item1, a wave for each.
 struct StPass {
-    int e, row0, nrows, ig, ne;
+    int e, row0, nrows, ne, item0, item1;
 };
 
-// Pass v of the launch, in the order of unit_block_work.
-__device__ __forceinline__ StPass st_lookup(const MfmaArgs& a, int n_units, int groups, int v) {
-    StPass p{0, 0, 0, 0, 0};
-    const int up = v / groups, first = a.unit_first[up], ne = a.unit_count[up];
-    if (first < 0 || ne < 1 || up < first || up >= first + ne || first + ne > n_units) return p;
-    const int vl = v - first * groups;
-    p.ig = vl / ne;
-    const int u = first + (vl - p.ig * ne), e = a.unit_expert[u], row0 = a.unit_row0[u], nrows = a.unit_rows[u];
-    if (unit_ok(a, e, row0, nrows)) { p.e = e; p.row0 = row0; p.nrows = nrows; p.ne = ne; }
-    return p;
+// Pass v of the launch, in the order of unit_block_work: items in runs of W for a block's only pass, in even parts otherwise.
+template <bool kDown, bool kOne, int W>
+__device__ __forceinline__ StPass st_lookup(const MfmaArgs& a, const StreamSplit& s, int v) {
+    StPass p{0, 0, 0, 0, 0, 0};
+    const int cut = s.routed * s.groups_r;
+    const bool shared = v >= cut;
+    const int groups = shared ? s.groups_s : s.groups_r, base = shared ? s.routed : 0, vs = shared ? v - cut : v;
+    const int up = base + vs / groups, first = a.unit_first[up], ne = a.unit_count[up];
+    if (first < base || ne < 1 || up < first || up >= first + ne || first + ne > base + (shared ? s.shared : s.routed)) return p;
+    const int vl = vs - (first - base) * groups, ig = vl / ne;
+    const int u = first + (vl - ig * ne), e = a.unit_expert[u], row0 = a.unit_row0[u], nrows = a.unit_rows[u];
+    if (!unit_ok(a, e, row0, nrows) || (e == a.n_experts) != shared) return p;
+    const int items = kDown ? a.hidden / 64 : (shared ? a.shared_inter : a.inter) / 32;
+    return StPass{e, row0, nrows, ne, kOne ? ig * W : ig * items / groups, kOne ? min((ig + 1) * W, items) : (ig + 1) * items / groups};
 }
 
 // The passes of this block (stream_share).  kOne: the only one, into `one`; otherwise all of them, looked up at once, into
-// `table`.  Returns their number.  groups comes in as a wave per item.
-template <bool kOne>
-__device__ __forceinline__ int st_passes(const MfmaArgs& a, int items, int& groups, StPass* table, StPass& one) {
+// `table`.  Returns their number.  groups_r and groups_s: a wave per item of the routed experts and of the shared one.
+template <bool kDown, bool kOne, int W>
+__device__ __forceinline__ int st_passes(const MfmaArgs& a, int groups_r, int groups_s, StPass* table, StPass& one) {
     const int n_units = min(*a.n_units, a.max_units);
     if (n_units <= 0) return 0;
-    if constexpr (!kOne) groups = stream_raise(n_units, groups, items);
-    const StreamShare sh = stream_share(n_units * groups, gridDim.x, blockIdx.x);
+    const int shared = min(a.shared_units, n_units);
+    StreamSplit s{n_units - shared, shared, groups_r, groups_s};
+    if constexpr (!kOne) s = stream_raise(s, kDown ? a.hidden / 64 : a.inter / 32, kDown ? a.hidden / 64 : a.shared_inter / 32);
+    const StreamShare sh = stream_share(stream_passes(s), gridDim.x, blockIdx.x);
     if (sh.count <= 0) return 0;
     if constexpr (kOne) {
-        one = st_lookup(a, n_units, groups, sh.first);
+        one = st_lookup<kDown, kOne, W>(a, s, sh.first);
         return one.nrows > 0 ? 1 : 0;
     } else {
         const int count = min(sh.count, ST_MAX_PASSES);
-        for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup(a, n_units, groups, sh.first + i * sh.step);
+        for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup<kDown, kOne, W>(a, s, sh.first + i * sh.step);
         __syncthreads();
         return count;
     }
@@ -1299,8 +1305,8 @@ __device__ __forceinline__ int st_passes(const MfmaArgs& a, int items, int& grou
 
 __device__ __forceinline__ StPass st_pass_at(const StPass* table, int i) {
     const StPass p = table[i];
-    return StPass{__builtin_amdgcn_readfirstlane(p.e), __builtin_amdgcn_readfirstlane(p.row0),
-                  __builtin_amdgcn_readfirstlane(p.nrows), __builtin_amdgcn_readfirstlane(p.ig), __builtin_amdgcn_readfirstlane(p.ne)};
+    return StPass{__builtin_amdgcn_readfirstlane(p.e),  __builtin_amdgcn_readfirstlane(p.row0),  __builtin_amdgcn_readfirstlane(p.nrows),
+                  __builtin_amdgcn_readfirstlane(p.ne), __builtin_amdgcn_readfirstlane(p.item0), __builtin_amdgcn_readfirstlane(p.item1)};
 }
 
 // The span of two planes that one buffer resource covers: plane p starts d[p] bytes after lo.
@@ -1342,16 +1348,14 @@ __device__ __forceinline__ StLane st_lane() {
     return l;
 }
 
-// The weights' side of a pass, an item of the unit's expert per wave: items ig * W .. of a block's only pass, the ig-th of
-// `groups` even parts otherwise.  Returns the wave's item, -1 for a wave without one (its loads return zeros).
-template <bool kDown, bool kOne, int P, int W, int NT>
-__device__ __forceinline__ int st_weights(StCtx<W, NT>& c, const MfmaArgs& a, const StPass& p, int groups, const StLane& l) {
+// The weights' side of a pass, an item of the unit's expert per wave.  Returns the wave's item, -1 for a wave without one (its
+// loads return zeros).
+template <bool kDown, int P, int W, int NT>
+__device__ __forceinline__ int st_weights(StCtx<W, NT>& c, const MfmaArgs& a, const StPass& p, const StLane& l) {
     const bool shared = p.e == a.n_experts;
-    const int inter = shared ? a.shared_inter : a.inter;
-    const int items = kDown ? a.hidden / 64 : inter / 32;
-    const int item = (kOne ? p.ig * W : p.ig * items / groups) + l.wave;
-    const bool live = item < (kOne ? items : (p.ig + 1) * items / groups) && p.nrows > 0;
-    c.KT = (kDown ? inter : a.hidden) / 128;
+    const int item = p.item0 + l.wave;
+    const bool live = item < p.item1 && p.nrows > 0;
+    c.KT = (!kDown ? a.hidden : shared ? a.shared_inter : a.inter) / 128;
     c.ntile = min(NT / P, (p.nrows + 15) >> 4);
     c.keep = a.cached || p.ne > 1;
     const int KT4 = (c.KT + 3) >> 2;
@@ -1375,7 +1379,7 @@ __device__ __forceinline__ void st_nothing(StCtx<W, NT>& n, const StCtx<W, NT>& 
 }
 
 template <int W, int NT, int P, int D, bool kOne>
-__global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, int groups, ActPlanes xin,
+__global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, int groups_r, int groups_s, ActPlanes xin,
                                                                    const int32_t* __restrict__ gather_src, ActPlanes act) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     using Cfg = StCfg<W, NT>;
@@ -1383,7 +1387,7 @@ __global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, i
     u4v* lds = reinterpret_cast<u4v*>(lds_raw);
     StPass* table = reinterpret_cast<StPass*>(lds_raw + Cfg::LDS_BYTES);
     StPass p;
-    const int count = st_passes<kOne>(a, a.act_ld / 32, groups, table, p);
+    const int count = st_passes<false, kOne, W>(a, groups_r, groups_s, table, p);
     if (count == 0) return;
     if constexpr (!kOne) p = st_pass_at(table, 0);
     const int H = a.hidden, nk = a.n * a.topk, topk = a.topk, tokens = a.n;
@@ -1422,7 +1426,7 @@ __global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, i
     for (int i = 0; i < Cfg::CF; ++i) gc[i] = gather(p, code_row(p, i));
 #pragma unroll
     for (int i = 0; i < Cfg::SF; ++i) gs[i] = gather(p, scale_row(p, i));
-    int item = st_weights<false, kOne, P>(c, a, p, groups, l);
+    int item = st_weights<false, P>(c, a, p, l);
     offsets(c, p, gc, gs);
     StRegs<W, NT, D> r;
     st_start(c, l, lds, r);
@@ -1439,7 +1443,7 @@ __global__ __launch_bounds__(W * 64, 1) void gate_up_stream_kernel(MfmaArgs a, i
             for (int q = 0; q < Cfg::CF; ++q) gc[q] = gather(pn, code_row(pn, q));
 #pragma unroll
             for (int q = 0; q < Cfg::SF; ++q) gs[q] = gather(pn, scale_row(pn, q));
-            item_n = st_weights<false, kOne, P>(n, a, pn, groups, l);
+            item_n = st_weights<false, P>(n, a, pn, l);
             offsets(n, pn, gc, gs);
         }
         v4f acc[4][RT];
@@ -1464,7 +1468,7 @@ __global__ __launch_bounds__(W * 64, 1) void down_stream_kernel(MfmaArgs a, int 
     u4v* lds = reinterpret_cast<u4v*>(lds_raw);
     StPass* table = reinterpret_cast<StPass*>(lds_raw + Cfg::LDS_BYTES);
     StPass p;
-    const int count = st_passes<kOne>(a, a.hidden / 64, groups, table, p);
+    const int count = st_passes<true, kOne, W>(a, groups, groups, table, p);
     if (count == 0) return;
     if constexpr (!kOne) p = st_pass_at(table, 0);
     const int H = a.hidden, apitch = scale_pitch(a.act_ld), act_ld = a.act_ld;
@@ -1487,7 +1491,7 @@ __global__ __launch_bounds__(W * 64, 1) void down_stream_kernel(MfmaArgs a, int 
             const int v = min(l.wave * Cfg::SF + i, NT - 1), col = v / P * 16 + (l.lane & 15);
             c.soff[i] = col < p.nrows ? as.at(v % P) + (uint32_t)col * (uint32_t)apitch + (uint32_t)((l.lane >> 4) * 4) : ST_OUT;
         }
-        return st_weights<true, kOne, P>(c, a, p, groups, l);
+        return st_weights<true, P>(c, a, p, l);
     };
     StCtx<W, NT> c, n;
     int item = context(c, p);
@@ -1546,12 +1550,16 @@ constexpr size_t ST_LDS = StCfg<ST_W, ST_NT>::LDS_BYTES + ST_MAX_PASSES * sizeof
 // Layer, us, a block per pass / several (two terms unless said): hidden 5120, 32 experts, 300 tokens (0.9 passes per CU)
 // 171 / 178, 500 (1.7) 232 / 240, 1000 (2.1) 332 / 332, one term (1.3) 258 / 267; hidden 4096, 128 experts, 300 (3.1) 333 / 321,
 // 2047 (7.8) 783 / 744, 4096 1375 / 1310.
-static bool stream_persistent(const ferrite_moe_shape& s, int n, int cap, int groups) {
+static bool stream_persistent(const ferrite_moe_shape& s, int n, int cap, int groups_r, int groups_s) {
     const int variant = g_prefill_variant.load(std::memory_order_relaxed);
     if (variant >= 2) return variant == 2;
     const double rows = (double)n * s.topk / s.n_experts, units = rows / cap + 0.5;
     const double hit = rows < 1.0 ? (double)n * s.topk : (double)s.n_experts;
-    return (hit * (units > 1.0 ? units : 1.0) + (s.shared_inter > 0 ? (double)n / cap : 0.0)) * groups >= 2.5 * ST_CUS;
+    return hit * (units > 1.0 ? units : 1.0) * groups_r + (s.shared_inter > 0 ? (double)n / cap : 0.0) * groups_s >= 2.5 * ST_CUS;
+}
+// The most units that a launch may have, in the passes that they make.
+static StreamSplit stream_most(const MfmaArgs& a, int groups_r, int groups_s) {
+    return StreamSplit{a.max_units - a.shared_units, a.shared_units, groups_r, groups_s};
 }
 constexpr int GU_WAVES = 4;
 constexpr int GU_WAVES_RESIDENT_X2 = 8;
@@ -1586,6 +1594,7 @@ static MfmaArgs make_args(const ferrite_moe_shape& s, const uint8_t* packed, int
     a.limit = s.swiglu_limit;
     a.unit_cap = units.unit_rows_cap;
     a.max_units = units.max_units;
+    a.shared_units = s.shared_inter > 0 ? (n + units.unit_rows_cap - 1) / units.unit_rows_cap : 0;
     a.cached = L.total <= (size_t)256 << 20;
     return a;
 }
@@ -1603,12 +1612,12 @@ int launch_gate_up_mfma(const ferrite_moe_shape& s, const uint8_t* packed, const
         if (units.unit_rows_cap != (x2 ? PF_ROWS_X2 : PF_ROWS)) return FERRITE_ERR_INVALID_ARG;
         const int variant = g_prefill_variant.load(std::memory_order_relaxed);
         int rc;
-        const int groups = (imax / 32 + ST_W - 1) / ST_W;
-        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups);
+        const int groups_r = (s.inter / 32 + ST_W - 1) / ST_W, groups_s = (s.shared_inter / 32 + ST_W - 1) / ST_W;
+        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups_r, groups_s);
         auto go = [&](auto limit, auto kernel) -> int {
             if ((rc = limit.ensure(ST_LDS))) return rc;
-            hipExtLaunchKernelGGL(kernel, dim3(stream_blocks(persistent, units.max_units, groups)), dim3(ST_W * 64), (uint32_t)ST_LDS, st,
-                                  k_start, k_stop, 0, a, groups, xin, gather_src, act);
+            hipExtLaunchKernelGGL(kernel, dim3(stream_blocks(persistent, stream_most(a, groups_r, groups_s))), dim3(ST_W * 64),
+                                  (uint32_t)ST_LDS, st, k_start, k_stop, 0, a, groups_r, groups_s, xin, gather_src, act);
             return check_launch("gate_up_stream");
         };
         auto stream = [&](auto planes, auto one) -> int {
@@ -1693,10 +1702,10 @@ int launch_down_mfma(const ferrite_moe_shape& s, const uint8_t* packed, const Ac
         float* yf = static_cast<float*>(y);
         int rc;
         const int groups = (s.hidden / 64 + ST_W - 1) / ST_W;
-        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups);
+        const bool persistent = stream_persistent(s, n, units.unit_rows_cap, groups, groups);
         auto go = [&](auto limit, auto kernel, auto* yp) -> int {
             if ((rc = limit.ensure(ST_LDS))) return rc;
-            kernel<<<stream_blocks(persistent, units.max_units, groups), ST_W * 64, ST_LDS, st>>>(a, groups, act, yp);
+            kernel<<<stream_blocks(persistent, stream_most(a, groups, groups)), ST_W * 64, ST_LDS, st>>>(a, groups, act, yp);
             return check_launch("down_stream");
         };
         auto stream_y = [&](auto planes, auto one, auto* yp) -> int {

@@ -11,8 +11,15 @@ float shim_e2m1_decode(unsigned c) { return fe::e2m1_decode(c); }
 float shim_ue8m0_decode(unsigned b) { return fe::ue8m0_decode(b); }
 unsigned shim_block_scale_e8m0(float amax) { return fe::block_scale_e8m0(amax); }
 void shim_expf_many(const float* x, float* y, long n) { for (long i = 0; i < n; ++i) y[i] = fe::fe_expf(x[i]); }
-int shim_stream_raise(int n_units, int groups, int items) { return fe::stream_raise(n_units, groups, items); }
-unsigned shim_stream_blocks(int several, int max_units, int groups) { return fe::stream_blocks(several != 0, max_units, groups); }
+// split: units and item groups as {routed, shared, groups_r, groups_s}
+void shim_stream_raise(int* split, int items_r, int items_s) {
+    const fe::StreamSplit s = fe::stream_raise(fe::StreamSplit{split[0], split[1], split[2], split[3]}, items_r, items_s);
+    split[2] = s.groups_r;
+    split[3] = s.groups_s;
+}
+unsigned shim_stream_blocks(int several, const int* split) {
+    return fe::stream_blocks(several != 0, fe::StreamSplit{split[0], split[1], split[2], split[3]});
+}
 // how often each of the passes 0 .. total - 1 is gone through; returns the largest number of passes of a block, -1 for one out of range
 int shim_stream_cover(int total, int blocks, int* times) {
     int most = 0;

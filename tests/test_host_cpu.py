@@ -210,6 +210,8 @@ def shim(tmp_path_factory):
     lib.shim_e2m1_decode.argtypes = [C.c_uint]
     lib.shim_ue8m0_decode.argtypes = [C.c_uint]
     lib.shim_expf_many.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    lib.shim_stream_raise.argtypes = [C.POINTER(C.c_int), C.c_int, C.c_int]
+    lib.shim_stream_blocks.argtypes = [C.c_int, C.POINTER(C.c_int)]
     lib.shim_stream_cover.argtypes = [C.c_int, C.c_int, C.c_void_p]
     return lib
 
@@ -285,21 +287,29 @@ def test_block_scale_is_the_rounded_quotient_s_exponent(shim):
     assert [shim.shim_block_scale_e8m0(float(a)) for a in amax] == want.tolist()
 
 
-@pytest.mark.parametrize("groups,items", [(1, 2), (1, 8), (3, 20), (6, 48), (8, 64), (14, 112)])
-def test_streamed_passes_are_gone_through_once(shim, groups, items):
+@pytest.mark.parametrize("items_r,items_s", [(2, 2), (8, 0), (20, 24), (48, 48), (44, 88), (32, 128), (128, 32), (64, 64), (112, 112)])
+def test_streamed_passes_are_gone_through_once(shim, items_r, items_s):
     """Every pass of the streamed tiled kernels belongs to one block and fits its table of 128, whatever part of the units that a
-    launch is sized for is live; one block per CU as long as 128 passes per block suffice."""
-    for max_units in (1, 7, 42, 43, 128, 136, 300, 1023, 1408, 2340, 2341, 4096, 4097, 5000, 33000):
-        for n_units in sorted({1, max_units // 3 + 1, max_units - max_units // 8, max_units}):
+    launch is sized for is live; one block per CU as long as 128 passes per block suffice.  Passes are counted by the items that the
+    unit's own expert has (eight a pass), so a wide shared expert adds none to the routed experts' units."""
+    gr, gs = -(-items_r // 8), -(-items_s // 8)
+    for routed in (1, 7, 42, 43, 128, 136, 300, 1023, 1408, 2340, 2341, 4096, 4097, 33000):
+        shared = -(-routed // 9) if items_s else 0
+        for live in sorted({1, routed // 3 + 1, routed - routed // 8, routed}):
             for several in (0, 1):
-                g = shim.shim_stream_raise(n_units, groups, items) if several else groups
-                assert groups <= g <= max(groups, min(2 * groups, items))
-                blocks = shim.shim_stream_blocks(several, max_units, groups)
-                total = n_units * g
+                split = (C.c_int * 4)(live, shared, gr, gs)
+                passes = live * gr + shared * gs
+                if several:
+                    shim.shim_stream_raise(split, items_r, items_s)
+                assert (live, shared) == (split[0], split[1])
+                for g, g0, items in ((split[2], gr, items_r), (split[3], gs, items_s)):
+                    assert g0 <= g <= max(g0, min(2 * g0, items) if several else g0)
+                blocks = shim.shim_stream_blocks(several, (C.c_int * 4)(routed, shared, gr, gs))
+                total = live * split[2] + shared * split[3]
+                assert -(-total // 256) == -(-passes // 256)
                 times = np.zeros(total, np.int32)
                 most = shim.shim_stream_cover(total, blocks, times.ctypes.data)
                 assert (times == 1).all() and blocks % 8 == 0
                 assert 0 < most <= (128 if several else 1)
                 if several:
-                    assert blocks == 256 * -(-max_units * groups // (256 * 128))
-                    assert -(-total // 256) == -(-n_units * groups // 256)
+                    assert blocks == 256 * -(-(routed * gr + shared * gs) // (256 * 128))
