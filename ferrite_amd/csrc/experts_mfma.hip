@@ -483,8 +483,11 @@ __device__ __forceinline__ void gate_up_store(const MfmaArgs& a, const v4f (&acc
         amax = amax_nan(amax_nan(amax, r0[v]), r1[v]);
     }
     amax = block_amax(amax);
+    const int c = lane & 15, g = lane >> 4;
     QuantPair q, q2{};
-    if (a.limit >= 0.0f && !__any(!(amax < E4M3_FINITE_AMAX))) {   // wave-uniform
+    // wave-uniform, and only the unit's own columns count: the 16-row kernels leave in the others what LDS held before, often
+    // NaN (32 tokens of the decode shape, one / two terms: 5.05 / 9.17 million vector instructions with all columns, 4.34 / 7.81)
+    if (a.limit >= 0.0f && !__any(c < nrows && !(amax < E4M3_FINITE_AMAX))) {
         q = quant_pair_finite<kX2>(r0, r1, amax);
         if constexpr (kX2) {
             float amax2 = 0.0f;
@@ -501,7 +504,6 @@ __device__ __forceinline__ void gate_up_store(const MfmaArgs& a, const v4f (&acc
         q = quant_pair_any(r0, r1);
         if constexpr (kX2) q2 = quant_pair_any(r0, r1);
     }
-    const int c = lane & 15, g = lane >> 4;
     if (c >= nrows) return;
     const size_t qoff = (size_t)(row0 + c) * a.act_ld + (size_t)item * 32 + g * 4;
     const size_t soff = (size_t)(row0 + c) * scale_pitch(a.act_ld) + scale_pos(item);
