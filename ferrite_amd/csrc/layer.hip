@@ -341,7 +341,7 @@ static int moe_layer_impl(const ferrite_moe_shape* shape, const ferrite_moe_weig
                              b + w.perm_scratch, w.perm_scratch_bytes, &units, has_shared, st)))
         return rc;
     if ((rc = mark(ev, 3, st))) return rc;
-    if ((rc = mark(ev, 4, st))) return rc;
+    if ((rc = mark(ev, 4, st))) return rc;   // nothing between the two: x was quantised with the routing
     }
     // 4-5. expert FFNs in grouped order, shared expert as the trailing rows
     if (mode == FERRITE_MODE_F32_CHECK) {

@@ -305,9 +305,11 @@ int ferrite_moe_block_mxfp4(const ferrite_moe_shape* shape, const ferrite_moe_we
 /* The same layer with HIP events recorded on `stream` at the stage boundaries, the counterpart of the
  * reference's FERRITE_TIMING probes (crates/ferrite-exec/src/lib.rs:1184-1299).  stage_events_host is a host
  * array of FERRITE_MOE_STAGE_EVENTS hipEvent_t handles (any may be NULL): [0] before the router GEMM, then
- * after: [1] router GEMM, [2] routing, [3] permutation, [4] activation quantisation (== [3] in f32 mode),
- * [5] gate/up GEMM + SwiGLU, [6] down GEMM, [7] combine; [8] and [9] bracket the gate/up kernel itself on the
- * device (start and end of its execution, without the launch gap that [4]..[5] includes; MFMA mode only).
+ * after: [1] router GEMM, [2] routing and, in the MFMA modes, activation quantisation (one launch), [3] permutation,
+ * [4] as [3], right behind it, [5] gate/up GEMM + SwiGLU, [6] down GEMM, [7] combine; [8] and [9] bracket the gate/up
+ * kernel itself on the device (start and end of its execution, without the launch gap that [4]..[5] includes; MFMA
+ * mode only).  Where one launch does everything in front of the experts (up to 256 tokens with packed weights), [1] is
+ * after all of it and [2] to [4] follow at once.
  * Not capturable. */
 #define FERRITE_MOE_STAGE_EVENTS 10
 int ferrite_moe_layer_mxfp4_timed(const ferrite_moe_shape* shape, const ferrite_moe_weights* w,

@@ -10,6 +10,7 @@ Bars, all as max|d| / max|ref| of the layer output:
   two-term MFMA mode against the f32 oracle         <= 2e-2  (the bar for bf16 / fp8 activations; observed ~2e-3)
   one-term MFMA mode against the f32 oracle         <= 8e-2  (three mantissa bits on x and on the SwiGLU output:
                                                              4-5 % by construction; asserted so it cannot grow)"""
+import ctypes
 import os
 
 import numpy as np
@@ -348,6 +349,33 @@ def test_streamed_passes_do_not_depend_on_their_split(hip, overrides, mode, n, h
         assert np.array_equal(outs[(128, 3)], first)
     else:
         assert max_abs_rel(outs[(128, 3)], first) <= 1e-4
+
+
+@pytest.mark.parametrize("n,mode", [(32, MODE_MFMA_FP8), (300, MODE_MFMA_FP8), (300, MODE_MFMA_FP8_X2), (300, MODE_F32_CHECK)])
+def test_timed_layer_records_its_stages_in_order(hip, n, mode):
+    """The timed call gives the untimed one's output and records the events in the order that the header states, one launch for
+    routing and quantisation: nothing runs between the permutation's event and the next one."""
+    cfg = synth.MoeConfig(n, 2048, 16, 4, 1024, 1024, 1, 1)
+    layer = hip.load_moe_layer(synth.make_inputs(cfg, seed=n))
+    x = torch.randn(n, cfg.hidden, device=hip.device)
+    out, timed = torch.empty_like(x), torch.empty_like(x)
+    hip.moe_layer_dev_mxfp4(layer, x, out, mode)
+    gaps = []
+    for _ in range(5):
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(10)]
+        for e in events:
+            e.record()
+        handles = (ctypes.c_void_p * 10)(*[e.cuda_event for e in events])
+        hip.moe_layer_dev_mxfp4(layer, x, timed, mode, stage_events=handles)
+        hip.sync()
+        torch.cuda.synchronize()
+        us = [events[i].elapsed_time(events[i + 1]) * 1e3 for i in range(7)]
+        assert min(us) >= 0.0 and sum(us) == pytest.approx(events[0].elapsed_time(events[7]) * 1e3, rel=1e-2)
+        gaps.append(us[3])
+        if mode != MODE_F32_CHECK:
+            assert 0.0 < events[8].elapsed_time(events[9]) * 1e3
+    assert torch.equal(out, timed)
+    assert min(gaps) < min(us[0], us[4])
 
 
 def test_more_streamed_passes_than_a_block_per_cu_has_room_for(hip):
