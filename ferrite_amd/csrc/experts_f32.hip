@@ -4,8 +4,6 @@
 //
 // Rows are addressed in the grouped order of the permutation: row g < n*topk is assignment gather_src[g]
 // (token = that / topk, expert = ids[that]); rows n*topk + t are the shared expert applied to token t.
-#include <math.h>
-
 #include "internal.hpp"
 #include "numerics.hpp"
 
@@ -316,29 +314,13 @@ __global__ __launch_bounds__(256) void combine_kernel(const YT* __restrict__ y, 
     }
 }
 
-// One pair of tiles per wave, or per block of four waves: where the former leaves some of the chip's 1024 SIMDs without work, and
-// where its last round of waves is so empty that rounds x blocks of 128 k per wave come out a tenth larger (a few thousand
-// waves; beyond that the rounds even out and the split only stages the activations four times as often).  The live units are
-// estimated.  Kernel, us, a wave / a block per pair: gate/up of hidden 2880, inter 480, 64 experts, 9 tokens 101 / 65, 64 tokens
-// 106 / 92; hidden 2880, 32 experts 75.3 / 63.9; on the other side hidden 2080, inter 736, 27 tokens 57.6 / 59.6, its down
-// 31.4 / 31.7; 64 experts, inter 1056 104.7 / 112.3; layer of hidden 1440, 64 experts, 64 tokens 87.8 / 92.9.
-static bool f32_split(const FxArgs& a, bool down) {
-    const double E = a.n_experts, hit = E * (1.0 - pow(1.0 - a.topk / E, a.n)), rows = a.n * (double)a.topk / hit;
-    const int step = down ? 32 : 16;
-    const double waves = hit * fmax(1.0, rows / 16.0 + 0.5) * (a.rows / step) + (a.sh_rows > 0 ? (a.n + 15) / 16 : 0) * (double)(a.sh_rows / step);
-    const int kblocks = (a.K + 127) / 128;
-    // whole rounds without the split, on the low side of the estimate; four times as many shorter ones fill up half of their last
-    const double whole = ceil(0.97 * waves / 1024.0) * kblocks, split = (4.0 * waves / 1024.0 + 0.5) * ((kblocks + 3) / 4);
-    return waves <= 4096.0 && split <= 0.9 * whole;
-}
-
 template <bool kGateUp>
 static int launch_experts_f32(FxArgs a, const UnitTables& units, hipStream_t st) {
     if (units.unit_rows_cap != 16) return FERRITE_ERR_INVALID_ARG;
     a.unit_expert = units.unit_expert; a.unit_row0 = units.unit_row0; a.unit_rows = units.unit_rows;
     a.n_units = units.n_units; a.max_units = units.max_units;
     const int pairs = (a.rows > a.sh_rows ? a.rows : a.sh_rows) / (kGateUp ? 16 : 32);
-    const bool split = (long)units.max_units * pairs <= 1024 || f32_split(a, !kGateUp);
+    const bool split = f32_split(a.n, a.topk, a.n_experts, units.max_units, a.rows, a.sh_rows, a.K, !kGateUp) != 0;
     a.groups = split ? pairs : (pairs + 3) / 4;
     const long blocks = (long)units.max_units * a.groups;
     if (blocks > 0x7fffffffL) return FERRITE_DECLINED;

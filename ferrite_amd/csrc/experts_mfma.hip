@@ -15,7 +15,6 @@
 #include <hip/hip_ext.h>
 
 #include "internal.hpp"
-#include "launch_rules.hpp"
 #include "device_utils.hpp"
 #include "numerics.hpp"
 

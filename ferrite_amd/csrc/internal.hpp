@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/ferrite_hip.h"
+#include "launch_rules.hpp"
 
 namespace fe {
 
@@ -28,13 +29,6 @@ struct UnitTables {
     int unit_rows_cap;     // rows per unit (column tile of the GEMM)
     int max_units;
 };
-
-inline int max_units_for(int n, int topk, int n_experts, int has_shared, int unit_rows) {
-    long assign = (long)n * topk;
-    long active_max = assign < n_experts ? assign : n_experts;
-    long u = assign / unit_rows + active_max + (has_shared ? (n + unit_rows - 1) / unit_rows : 0);
-    return (int)u;
-}
 
 // Rows per unit for a layer call: the tiled kernels (units of 128 rows, 64 with two-term activations) once the
 // average expert sees enough rows to fill them, 16-row units (weights streamed once per unit) below that.  A

@@ -11,6 +11,15 @@ float shim_e2m1_decode(unsigned c) { return fe::e2m1_decode(c); }
 float shim_ue8m0_decode(unsigned b) { return fe::ue8m0_decode(b); }
 unsigned shim_block_scale_e8m0(float amax) { return fe::block_scale_e8m0(amax); }
 void shim_expf_many(const float* x, float* y, long n) { for (long i = 0; i < n; ++i) y[i] = fe::fe_expf(x[i]); }
+int shim_max_units(int n, int topk, int n_experts, int shared, int unit_rows) {
+    return fe::max_units_for(n, topk, n_experts, shared > 0, unit_rows);
+}
+// the form that a layer's f32 gate/up (down = 0) and down GEMM take
+int shim_f32_split(int n, int hidden, int n_experts, int topk, int inter, int shared, int down) {
+    const int units = fe::max_units_for(n, topk, n_experts, shared > 0, 16);
+    if (down) return fe::f32_split(n, topk, n_experts, units, hidden, shared > 0 ? hidden : 0, inter, true);
+    return fe::f32_split(n, topk, n_experts, units, inter, shared, hidden, false);
+}
 // split: units and item groups as {routed, shared, groups_r, groups_s}
 void shim_stream_raise(int* split, int items_r, int items_s) {
     const fe::StreamSplit s = fe::stream_raise(fe::StreamSplit{split[0], split[1], split[2], split[3]}, items_r, items_s);

@@ -117,29 +117,24 @@ def test_layer_small_shapes_all_modes(hip, oracle, seed, n):
     check_mfma(hip, oracle, layer, inp, MODE_MFMA_FP8_X2, ref32)
 
 
-def max_units(n, topk, n_experts, shared):
-    """Units of up to 16 rows that a call may have (what grids are sized for)."""
-    return n * topk // 16 + min(n * topk, n_experts) + (-(-n // 16) if shared else 0)
-
-
-def f32_waves_share_a_pair(cfg):
-    """(gate/up, down): whether the four waves of a block share a pair of tiles in the f32 mode."""
-    units = max_units(cfg.n, cfg.topk, cfg.n_experts, cfg.shared_inter)
-    return units * (max(cfg.inter, cfg.shared_inter) // 16) <= 1024, units * (cfg.hidden // 32) <= 1024
+def f32_split(shim, cfg):
+    """(gate/up, down): why the four waves of a block share a pair of tiles in the f32 mode, by the launchers' own rule: 1 = too few
+    pairs for the SIMDs, 2 = a last round of waves that is nearly empty, 0 = they do not."""
+    return tuple(shim.shim_f32_split(cfg.n, cfg.hidden, cfg.n_experts, cfg.topk, cfg.inter, cfg.shared_inter, down) for down in (0, 1))
 
 
 @pytest.mark.parametrize("n,hidden,inter,shared,experts,topk,share", [
-    (1, 32, 32, 0, 8, 3, (True, True)), (5, 544, 96, 64, 8, 3, (True, True)), (40, 1056, 736, 32, 8, 3, (True, True)),
-    (3, 2080, 1120, 736, 8, 3, (True, True)), (130, 480, 160, 320, 8, 3, (True, True)),
-    (40, 2080, 736, 736, 32, 6, (False, False)), (24, 1056, 992, 96, 32, 4, (False, False)), (30, 160, 1504, 64, 32, 4, (False, True)),
-    (50, 4128, 224, 0, 32, 4, (True, False))])
-def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared, experts, topk, share):
+    (1, 32, 32, 0, 8, 3, (1, 1)), (5, 544, 96, 64, 8, 3, (1, 1)), (40, 1056, 736, 32, 8, 3, (1, 1)),
+    (3, 2080, 1120, 736, 8, 3, (1, 1)), (130, 480, 160, 320, 8, 3, (1, 1)),
+    (40, 2080, 736, 736, 32, 6, (0, 0)), (24, 1056, 992, 96, 32, 4, (0, 2)), (30, 160, 1504, 64, 32, 4, (0, 1)),
+    (50, 4128, 224, 0, 32, 4, (1, 0))])
+def test_f32_mode_tiles(hip, oracle, shim, n, hidden, inter, shared, experts, topk, share):
     """The f32 mode on sizes that are multiples of 32 only: reductions shorter than a block of 128, longer than the
     activation window and ragged in both, numbers of row tiles that are odd or no multiple of the four waves', a shared
     expert so short that whole blocks drop out, units of 1..16 rows, weights shared out to one wave per pair of tiles or
     to four; zero scales."""
     cfg = synth.MoeConfig(n, hidden, experts, topk, inter, shared, 4, 2)
-    assert f32_waves_share_a_pair(cfg) == share
+    assert f32_split(shim, cfg) == share
     inp = synth.make_inputs(cfg, seed=n + hidden)
     inp.gate_s.reshape(-1)[::7] = 0
     inp.down_s.reshape(-1)[::5] = 0
@@ -150,22 +145,12 @@ def test_f32_mode_tiles(hip, oracle, n, hidden, inter, shared, experts, topk, sh
     assert max_abs_rel(out, ref["out"]) <= TOL_F32
 
 
-def f32_splits_a_half_empty_round(n, topk, experts, kblocks, waves_per_unit, shared_waves):
-    """The second reason for four waves to share a pair: rounds of waves x blocks of 128 k, split against not, a tenth fewer."""
-    hit = experts * (1 - (1 - topk / experts) ** n)
-    waves = hit * max(1, n * topk / hit / 16 + 0.5) * waves_per_unit + -(-n // 16) * shared_waves
-    return waves <= 4096 and (4 * waves / 1024 + 0.5) * -(-kblocks // 4) <= 0.9 * np.ceil(0.97 * waves / 1024) * kblocks
-
-
-@pytest.mark.parametrize("n,hidden,inter,shared,experts,topk,splits", [
-    (9, 2080, 736, 736, 32, 6, (True, False)), (24, 2880, 736, 0, 32, 6, (True, False)), (5, 2080, 1504, 0, 32, 6, (False, True))])
-def test_f32_mode_split_of_a_half_empty_round(hip, oracle, n, hidden, inter, shared, experts, topk, splits):
+@pytest.mark.parametrize("n,hidden,inter,shared,experts,topk,share", [
+    (9, 2080, 736, 736, 32, 6, (2, 0)), (24, 2880, 736, 0, 32, 6, (2, 0)), (5, 2080, 1504, 0, 32, 6, (0, 2))])
+def test_f32_mode_split_of_a_half_empty_round(hip, oracle, shim, n, hidden, inter, shared, experts, topk, share):
     """More waves than SIMDs, but so few more that the waves of a block share a pair all the same: within the f32 bar."""
-    kb = lambda k: -(-k // 128)
-    assert splits == (f32_splits_a_half_empty_round(n, topk, experts, kb(hidden), inter // 16, shared // 16),
-                      f32_splits_a_half_empty_round(n, topk, experts, kb(inter), hidden // 32, hidden // 32 if shared else 0))
     cfg = synth.MoeConfig(n, hidden, experts, topk, inter, shared, 4, 2)
-    assert f32_waves_share_a_pair(cfg) != (True, True)
+    assert f32_split(shim, cfg) == share
     inp = synth.make_inputs(cfg, seed=n + hidden)
     layer = hip.load_moe_layer(inp, pack=False)
     ref = oracle.moe_ffn_mxfp4(inp, n_threads=8)
@@ -174,16 +159,17 @@ def test_f32_mode_split_of_a_half_empty_round(hip, oracle, n, hidden, inter, sha
     assert max_abs_rel(out, ref["out"]) <= TOL_F32
 
 
-@pytest.mark.parametrize("n,experts,topk,share", [(12, 8, 2, (True, True)), (40, 32, 4, (False, False))])
-def test_f32_mode_keeps_nan_where_it_belongs(hip, oracle, n, experts, topk, share):
+@pytest.mark.parametrize("n,hidden,inter,experts,topk,share", [(12, 1056, 992, 8, 2, (1, 1)), (40, 1056, 992, 32, 4, (0, 2)),
+                                                               (40, 2080, 736, 32, 6, (0, 0))])
+def test_f32_mode_keeps_nan_where_it_belongs(hip, oracle, shim, n, hidden, inter, experts, topk, share):
     """NaN scales (byte 255) in every matrix, at the ends of rows and of ragged blocks: NaN exactly where the oracle has it,
     everything else as close as ever.  A unit's rows share weight registers and MFMAs, its blocks LDS."""
-    cfg = synth.MoeConfig(n, 1056, experts, topk, 992, 96, 4, 2)
-    assert f32_waves_share_a_pair(cfg) == share
+    cfg = synth.MoeConfig(n, hidden, experts, topk, inter, 96, 4, 2)
+    assert f32_split(shim, cfg) == share
     inp = synth.make_inputs(cfg, seed=n)
     inp.down_s.reshape(experts, cfg.hidden, -1)[1, 5, 2] = 255
-    inp.down_s.reshape(experts, cfg.hidden, -1)[3, 1055, 30] = 255
-    inp.gate_s.reshape(experts, cfg.inter, -1)[2, 991, 32] = 255
+    inp.down_s.reshape(experts, cfg.hidden, -1)[3, hidden - 1, inter // 32 - 1] = 255
+    inp.gate_s.reshape(experts, cfg.inter, -1)[2, inter - 1, hidden // 32 - 1] = 255
     inp.up_s.reshape(experts, cfg.inter, -1)[4, 0, 0] = 255
     inp.sh_down_s.reshape(cfg.hidden, -1)[17, 2] = 255
     layer = hip.load_moe_layer(inp, pack=False)
@@ -378,12 +364,12 @@ def test_timed_layer_records_its_stages_in_order(hip, n, mode):
     assert min(gaps) < min(us[0], us[4])
 
 
-def test_more_streamed_passes_than_a_block_per_cu_has_room_for(hip):
+def test_more_streamed_passes_than_a_block_per_cu_has_room_for(hip, shim):
     """4608 units of two-term activations x 8 item groups are more passes than the tables of 256 blocks hold: two rounds of blocks,
     and the bits of a block per pass."""
     from ferrite_amd.backend import OVERRIDE_PREFILL_TILE
     cfg = synth.MoeConfig(32768, 128, 8, 8, 2048, 2048, 1, 1)
-    assert (cfg.n * 8 // 64 + 8 + cfg.n // 64) * (2048 // 32 // 8) > 256 * 128
+    assert shim.shim_max_units(cfg.n, 8, 8, 2048, 64) * (2048 // 32 // 8) > 256 * 128
     inp = synth.make_inputs(cfg, seed=3)
     layer = hip.load_moe_layer(inp, keep_checkpoint_layout=False)
     x = hip.upload(inp.x)
@@ -890,10 +876,10 @@ def test_layer_c3_skewed_scale(hip, oracle):
     assert 0.35 <= top <= 0.65, top
 
 
-def split_waves(cfg):
+def split_waves(shim, cfg):
     """Waves that share an item of gate/up and of down in the MFMA modes, 0 where the item is one wave's: up to four tokens,
     up to 640 items, and every wave needs a group of four k steps of the routed and of the shared reduction."""
-    units = max_units(cfg.n, cfg.topk, cfg.n_experts, cfg.shared_inter)
+    units = shim.shim_max_units(cfg.n, cfg.topk, cfg.n_experts, cfg.shared_inter, 16)
     groups = lambda k: -(-k // 512)
     gate_up = min(4, groups(cfg.hidden)) if units * (max(cfg.inter, cfg.shared_inter) // 32) <= 640 else 0
     down = min(4, groups(cfg.inter), groups(cfg.shared_inter or cfg.inter)) if units * (cfg.hidden // 64) <= 640 else 0
@@ -906,12 +892,12 @@ def split_waves(cfg):
     (5, 1024, 1024, 512, (0, 0)),
     (1, 2176, 512, 512, (4, 0)), (4, 2560, 512, 512, (4, 0)), (1, 3328, 512, 0, (4, 0)),      # 5, 5 and 7 groups on four waves
     (1, 1024, 2432, 1152, (2, 3)), (1, 1024, 1152, 2432, (2, 3)), (3, 1024, 1664, 640, (2, 2))])   # 5 | 3, 3 | 5, 4 | 2 groups
-def test_few_tokens_share_items_among_waves(hip, oracle, n, hidden, inter, shared, waves, mode):
+def test_few_tokens_share_items_among_waves(hip, oracle, shim, n, hidden, inter, shared, waves, mode):
     """A few tokens with a few hundred items: the waves of a block split an item's reduction.  Groups that do not divide
     among the waves, last groups of less than four k steps, routed and shared reductions of different lengths; five
     tokens do not split, nor do more than 640 items or reductions of a single group."""
     cfg = synth.MoeConfig(n, hidden, 8, 4, inter, shared, 4, 2)
-    assert split_waves(cfg) == waves
+    assert split_waves(shim, cfg) == waves
     inp = synth.make_inputs(cfg, seed=n)
     layer = hip.load_moe_layer(inp)
     check_mfma(hip, oracle, layer, inp, mode)
