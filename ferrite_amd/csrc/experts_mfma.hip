@@ -1292,12 +1292,12 @@ __device__ __forceinline__ int st_passes(const MfmaArgs& a, int groups_r, int gr
     StreamSplit s{n_units - shared, shared, groups_r, groups_s};
     if constexpr (!kOne) s = stream_raise(s, kDown ? a.hidden / 64 : a.inter / 32, kDown ? a.hidden / 64 : a.shared_inter / 32);
     const StreamShare sh = stream_share(stream_passes(s), gridDim.x, blockIdx.x);
-    if (sh.count <= 0) return 0;
+    if (sh.left <= 0) return 0;
     if constexpr (kOne) {
         one = st_lookup<kDown, kOne, W>(a, s, sh.first);
         return one.nrows > 0 ? 1 : 0;
     } else {
-        const int count = min(sh.count, ST_MAX_PASSES);
+        const int count = min(stream_count(sh), ST_MAX_PASSES);
         for (int i = threadIdx.x; i < count; i += blockDim.x) table[i] = st_lookup<kDown, kOne, W>(a, s, sh.first + i * sh.step);
         __syncthreads();
         return count;

@@ -58,13 +58,14 @@ inline unsigned stream_blocks(bool several, const StreamSplit& most) {
 // The passes of block b of `blocks`: first, first + step, ...  The hardware deals consecutive blocks round-robin over 8 XCDs;
 // the passes are cut into 8 contiguous ranges, one per XCD, and block b is number b / 8 of its XCD's.
 struct StreamShare {
-    int first, step, count;
+    int first, step, left;   // left: passes of the XCD's range from first on, <= 0 for none
 };
 FE_HD StreamShare stream_share(int total, int blocks, int b) {
-    const int per_xcd = (total + 7) >> 3, xcd = b & 7, slot = b >> 3, step = blocks >> 3;
-    const int left = total - xcd * per_xcd, range = left < per_xcd ? left : per_xcd;
-    return StreamShare{xcd * per_xcd + slot, step, slot < range ? (range - slot + step - 1) / step : 0};
+    const int per_xcd = (total + 7) >> 3, xcd = b & 7, slot = b >> 3;
+    const int left = total - xcd * per_xcd;
+    return StreamShare{xcd * per_xcd + slot, blocks >> 3, (left < per_xcd ? left : per_xcd) - slot};
 }
+FE_HD int stream_count(const StreamShare& s) { return s.left > 0 ? (s.left + s.step - 1) / s.step : 0; }
 
 // The f32 expert kernels: one pair of tiles per wave (0), or per block of four waves where the former leaves some of the chip's
 // 1024 SIMDs without work (1) and where its last round of waves is so empty that rounds x blocks of 128 k per wave come out a

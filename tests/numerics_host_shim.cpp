@@ -34,12 +34,13 @@ int shim_stream_cover(int total, int blocks, int* times) {
     int most = 0;
     for (int b = 0; b < blocks; ++b) {
         const fe::StreamShare s = fe::stream_share(total, blocks, b);
-        for (int i = 0; i < s.count; ++i) {
+        const int count = fe::stream_count(s);
+        for (int i = 0; i < count; ++i) {
             const int v = s.first + i * s.step;
             if (v < 0 || v >= total) return -1;
             ++times[v];
         }
-        if (s.count > most) most = s.count;
+        if (count > most) most = count;
     }
     return most;
 }
