@@ -71,7 +71,7 @@ FE_HD uint32_t e2m1_encode(float x) {
 
 // Four neighbouring lanes share a block, eight values each, so that a wave's loads and stores are whole lines.  The hardware
 // converts, rounding to nearest even, where the quotient by the power-of-two scale (an exact product) is finite: of the
-// seven ties 0.75, 1.75 and 3.5 would go up, so a value with at most three significant bits is moved towards zero by an ulp
+// seven ties 0.75, 1.75 and 3.5 would go up, so a value with at most four significant bits is moved towards zero by an ulp
 // or two first, which leaves the code of every one that is no tie as it is; adding zero drops the sign of a zero quotient.
 // Bound by the launch and HBM at the sizes of an expert (4096 x 1536 bf16: 12.6 MB in, 3.3 MB out); with seven compares and
 // a division per value and 64 bytes per thread it was 9.7 us of vector instructions, now 5.1.

@@ -73,6 +73,9 @@ struct ActPlanes {
 // route.hip
 int launch_matmul_exact(const void* x, int x_dtype, const float* w, const float* bias, float* out, int n, int k,
                         int o, hipStream_t st);
+// Routing and, with xq.q set, the quantisation of x [n][H] in the same launch.
+int launch_route(const float* logits, const float* bias, int n, int e, int topk, int n_group, int topk_group, float scaling,
+                 float* probs, float* ids_f32, int32_t* ids_i32, const void* x, int x_dtype, int H, const ActPlanes& xq, hipStream_t st);
 int launch_permute(const int32_t* ids, int n, int topk, int n_experts, int32_t* counts, int32_t* starts,
                    int32_t* perm_map, int32_t* gather_src, int32_t* active, int32_t* n_active, void* scratch,
                    size_t scratch_bytes, const UnitTables* units, int has_shared, hipStream_t st);
@@ -130,8 +133,6 @@ int launch_hc_post(const float* x, const float* residual, const float* post, con
 
 // formats.hip
 // q2 / scale2 (both or neither): the second term of a two-term quantisation, from the residual of the first.
-int launch_route(const float* logits, const float* bias, int n, int e, int topk, int n_group, int topk_group, float scaling,
-                 float* probs, float* ids_f32, int32_t* ids_i32, const void* x, int x_dtype, int H, const ActPlanes& xq, hipStream_t st);
 int launch_act_quant(const void* x, int x_dtype, int64_t rows, int cols, uint8_t* q, uint8_t* scale, uint8_t* q2,
                      uint8_t* scale2, hipStream_t st);
 

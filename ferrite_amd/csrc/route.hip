@@ -375,9 +375,9 @@ __global__ void swiglu_kernel(const float* __restrict__ gate_up, float limit, fl
 }
 
 // ------------------------------------------------------------------------------------------------
-// Routing: one wave per token.  sigmoid -> +bias -> (group top-2 sums -> keep topk_group groups) -> rank of
-// every candidate under (choice desc, index asc) by counting the candidates that beat it -> the topk lowest
-// ranks are the selection, in order -> renormalised weights from the raw sigmoid.
+// Routing: one wave per token.  sigmoid -> +bias -> (group top-2 sums -> keep topk_group groups) -> the topk-th
+// largest choice as a threshold, found bit by bit -> the candidates at or above it, ranked among themselves under
+// (choice desc, index asc), are the selection, in order -> renormalised weights from the raw sigmoid.
 // Semantics and operation order follow cpu.rs:546-569; ties -> lower index (cpu.rs:560).
 // ------------------------------------------------------------------------------------------------
 constexpr int RT_MAX_E = 512;
@@ -808,9 +808,8 @@ static inline size_t perm_block_lds_bytes(int n, int n_experts) {
     return (size_t)n_experts * nchunk * 12 + (size_t)(3 * n_experts + 2) * 4;
 }
 
-// The whole permutation by one workgroup (any multiple of 64 threads) or, with kWaveScope, by a single wave
-// of a larger workgroup.  lds: perm_block_lds_bytes.
-template <bool kCoherent, bool kWaveScope>
+// The whole permutation by one workgroup (any multiple of 64 threads).  lds: perm_block_lds_bytes.
+template <bool kCoherent>
 __device__ __forceinline__ void permute_in_block(const PermArgs& a, unsigned long long* lds) {
     const int E = a.n_experts, n = a.n, k = a.topk;
     const int nchunk = (n + 63) >> 6;
@@ -819,17 +818,16 @@ __device__ __forceinline__ void permute_in_block(const PermArgs& a, unsigned lon
     int32_t* cnt = offs + (size_t)E * nchunk;                            // [E]
     int32_t* starts_lds = cnt + E;                                       // [E+1]
     int32_t* first_lds = starts_lds + E + 1;                             // [E+1]
-    const int tid = kWaveScope ? (threadIdx.x & 63) : threadIdx.x, nthr = kWaveScope ? 64 : blockDim.x;
-    auto sync = [] { if constexpr (kWaveScope) wave_sync(); else __syncthreads(); };
+    const int tid = threadIdx.x, nthr = blockDim.x;
     auto id_at = [&](int i) -> int { return kCoherent ? load_coherent(a.ids + i) : a.ids[i]; };
     for (int i = tid; i < E * nchunk; i += nthr) mask[i] = 0ull;
-    sync();
+    __syncthreads();
     for (int i = tid; i < n * k; i += nthr) {
         int t = i / k;
         int e = id_at(i);
         if (e >= 0 && e < E) atomicOr(&mask[(size_t)e * nchunk + (t >> 6)], 1ull << (t & 63));
     }
-    sync();
+    __syncthreads();
     for (int e = tid; e < E; e += nthr) {
         int run = 0;
         for (int c = 0; c < nchunk; ++c) {
@@ -838,9 +836,9 @@ __device__ __forceinline__ void permute_in_block(const PermArgs& a, unsigned lon
         }
         cnt[e] = run;
     }
-    sync();
+    __syncthreads();
     if (tid < 64) perm_expert_scan(a, cnt, starts_lds, first_lds);
-    sync();
+    __syncthreads();
     perm_units(a, cnt, starts_lds, first_lds, tid, nthr);
     const int total = starts_lds[E];
     for (int i = tid; i < n * k; i += nthr) {
@@ -857,7 +855,7 @@ __device__ __forceinline__ void permute_in_block(const PermArgs& a, unsigned lon
 
 __global__ __launch_bounds__(1024) void permute_small_kernel(PermArgs a) {
     extern __shared__ unsigned long long pm_lds[];
-    permute_in_block<false, false>(a, pm_lds);
+    permute_in_block<false>(a, pm_lds);
 }
 
 // large-n phase A: one wave per 64-token chunk
@@ -1182,7 +1180,7 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
                     xrow = reinterpret_cast<const XT*>(row);
                 }
             }
-            for (int b = tid; b < H / 32; b += 512) {
+            for (int b = tid; b < H / 32; b += 512) {   // the row may be the normalised one in LDS
                 const size_t at = (size_t)t * scale_pitch(H) + scale_pos(b), qo = (size_t)t * H + b * 32;
                 if (a.xq.q2) {
                     const uint32_t sb = quant_block32_x2(xrow + b * 32, a.xq.q + qo, a.xq.q2 + qo);
@@ -1279,7 +1277,7 @@ __global__ __launch_bounds__(512) void moe_head_kernel(HeadArgs a) {
         if (lane == 0) perm_here = do_perm;
     }
     __syncthreads();
-    if (perm_here) permute_in_block<true, false>(a.perm, reinterpret_cast<unsigned long long*>(head_lds));
+    if (perm_here) permute_in_block<true>(a.perm, reinterpret_cast<unsigned long long*>(head_lds));
 }
 
 // tokens per block: two when one per block would not fit the chip's 256 CUs in one round
@@ -1364,7 +1362,7 @@ int launch_moe_head(const void* x, int x_dtype, const float* router_t, const flo
 
 // What every routing kernel here assumes of its parameters, for the stand-alone op and for the fused head alike:
 // argument errors first (the reference returns Err for them, cpu.rs:539-545), then the limits of these kernels
-// (LDS arrays of RT_MAX_E keys, RT_MAX_K selections, one lane per group) as FERRITE_DECLINED.
+// (eight slots of 64 experts and an LDS array of RT_MAX_E choices, RT_MAX_K selections, one lane per group) as FERRITE_DECLINED.
 int check_routing_params(int e, int topk, int n_group, int topk_group) {
     if (e <= 0 || topk <= 0 || topk > e) return FERRITE_ERR_INVALID_ARG;
     if (n_group > 1) {
