@@ -382,6 +382,7 @@ __global__ void swiglu_kernel(const float* __restrict__ gate_up, float limit, fl
 // ------------------------------------------------------------------------------------------------
 constexpr int RT_MAX_E = 512;
 constexpr int RT_MAX_K = 32;
+constexpr int RT_RANK_E = RT_MAX_K;   // experts up to which a token's are ranked against each other (route_wave_ni): RouteScratch::sel_key
 
 __device__ __forceinline__ uint32_t ordered_u32(float f) {
     uint32_t u = f2u(f);
@@ -441,6 +442,8 @@ __device__ __forceinline__ void group_top2(float& m1, float& m2, int lg) {
 // above it) instead of ranking every expert against every other, only the selected ones are ranked, and a group's two largest
 // meet by lane exchanges.  Against the ranking loops, us: head of one token 27.2 -> 25.7, 32 tokens 29.4 -> 27.6, 192 48.0 -> 45.5,
 // 200 tokens of 64 experts in one group 37.0 -> 25.9; moe_route_kernel, 4096 tokens x 128 experts 11.7 -> 8.3, 8192 x 256 50.5 -> 17.5.
+// Up to 32 experts the bits are more than the experts, and ranking stays (moe_route_kernel, 100 tokens, ranking / threshold: 8
+// experts 2.8 / 3.2, 16 3.1 / 3.4, 32 3.3 / 3.6, 48 3.5 / 3.6, 64 3.6 / 3.5).
 template <bool kCoherent, bool kOwn, int NI>
 __device__ __forceinline__ void route_wave_ni(const float* __restrict__ lg, float own, const float* __restrict__ bias, bool live,
                                            int e, int topk, int n_group, int topk_group, float scaling,
@@ -519,48 +522,62 @@ __device__ __forceinline__ void route_wave_ni(const float* __restrict__ lg, floa
     uint32_t key[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) key[i] = ok[i] ? ordered_u32(ch[i]) : 0u;
-    uint32_t thr = 0;   // the largest value that at least topk keys reach, or one that exactly topk reach
-    for (int bit = 31; bit >= 0; --bit) {
-        const uint32_t cand = thr | (1u << bit);
-        int cnt = 0;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) cnt += __popcll(__ballot(key[i] >= cand));
-        if (cnt >= topk) {
-            thr = cand;
-            if (cnt == topk) break;
-        }
-    }
-    // selected: every key above thr, and of those equal to it the first ones by index
-    int above = 0;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) above += __popcll(__ballot(key[i] > thr));
-    const unsigned long long below_me = (1ull << lane) - 1ull;
-    int ties = 0, m = 0;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const bool tie = key[i] == thr && key[i] != 0u;
-        const unsigned long long tmask = __ballot(tie);
-        const bool sel = key[i] > thr || (tie && ties + __popcll(tmask & below_me) < topk - above);
-        const unsigned long long smask = __ballot(sel);
-        if (sel) {
-            const int at = m + __popcll(smask & below_me);
-            const uint32_t j = lane + 64 * i;
-            // larger = earlier in the reference's sort (choice desc, index asc)
-            sc.sel_key[at] = ((unsigned long long)key[i] << 32) | (0xFFFFFFFFu - j);
-            sc.pre_sig[at] = sg[i];
-        }
-        ties += __popcll(tmask);
-        m += __popcll(smask);
-    }
-    wave_sync();
-    if (lane < m) {
-        const unsigned long long mine = sc.sel_key[lane];
+    if (NI == 1 && e <= RT_RANK_E) {   // every expert against every other
+        // larger = earlier in the reference's sort (choice desc, index asc)
+        const unsigned long long mine = key[0] != 0u ? ((unsigned long long)key[0] << 32) | (0xFFFFFFFFu - (uint32_t)lane) : 0ull;
+        if (lane < e) sc.sel_key[lane] = mine;
+        wave_sync();
         int rank = 0;
-        for (int r = 0; r < m; ++r) rank += sc.sel_key[r] > mine ? 1 : 0;
-        sc.sel_id[rank] = (int)(0xFFFFFFFFu - (uint32_t)mine);
-        sc.sel_sig[rank] = sc.pre_sig[lane];
+        for (int j2 = 0; j2 < e; ++j2) rank += sc.sel_key[j2] > mine ? 1 : 0;   // same address in every lane: an LDS broadcast
+        if (mine != 0ull && rank < topk) {
+            sc.sel_id[rank] = lane;
+            sc.sel_sig[rank] = sg[0];
+        }
+        wave_sync();
+    } else {
+        uint32_t thr = 0;   // the largest value that at least topk keys reach, or one that exactly topk reach
+        for (int bit = 31; bit >= 0; --bit) {
+            const uint32_t cand = thr | (1u << bit);
+            int cnt = 0;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) cnt += __popcll(__ballot(key[i] >= cand));
+            if (cnt >= topk) {
+                thr = cand;
+                if (cnt == topk) break;
+            }
+        }
+        // selected: every key above thr, and of those equal to it the first ones by index
+        int above = 0;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) above += __popcll(__ballot(key[i] > thr));
+        const unsigned long long below_me = (1ull << lane) - 1ull;
+        int ties = 0, m = 0;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const bool tie = key[i] == thr && key[i] != 0u;
+            const unsigned long long tmask = __ballot(tie);
+            const bool sel = key[i] > thr || (tie && ties + __popcll(tmask & below_me) < topk - above);
+            const unsigned long long smask = __ballot(sel);
+            if (sel) {
+                const int at = m + __popcll(smask & below_me);
+                const uint32_t j = lane + 64 * i;
+                // larger = earlier in the reference's sort (choice desc, index asc)
+                sc.sel_key[at] = ((unsigned long long)key[i] << 32) | (0xFFFFFFFFu - j);
+                sc.pre_sig[at] = sg[i];
+            }
+            ties += __popcll(tmask);
+            m += __popcll(smask);
+        }
+        wave_sync();
+        if (lane < m) {
+            const unsigned long long mine = sc.sel_key[lane];
+            int rank = 0;
+            for (int r = 0; r < m; ++r) rank += sc.sel_key[r] > mine ? 1 : 0;
+            sc.sel_id[rank] = (int)(0xFFFFFFFFu - (uint32_t)mine);
+            sc.sel_sig[rank] = sc.pre_sig[lane];
+        }
+        wave_sync();
     }
-    wave_sync();
     // cpu.rs:562-568: sum in selection order, then sig / (sum + f32::EPSILON) * scale
     const int slot = lane < RT_MAX_K ? lane : 0;
     const float my_sig = sc.sel_sig[slot];

@@ -283,10 +283,12 @@ def test_moe_route_ties_lower_index_first(hip, oracle):  # cpu.rs:560
 
 
 @pytest.mark.parametrize("e,k,ng,tg", [(512, 32, 8, 4), (160, 8, 8, 4), (96, 6, 8, 3), (64, 8, 64, 16), (128, 8, 2, 1), (256, 8, 2, 1),
-                                       (32, 8, 8, 4), (16, 16, 1, 1), (300, 7, 1, 1), (48, 4, 16, 2)])
+                                       (32, 8, 8, 4), (16, 16, 1, 1), (300, 7, 1, 1), (48, 4, 16, 2), (32, 32, 1, 1), (31, 6, 1, 1),
+                                       (33, 32, 1, 1), (8, 2, 4, 2), (24, 5, 8, 4)])
 def test_moe_route_groups_and_thresholds_vs_oracle(hip, oracle, e, k, ng, tg):
     """Groups that are aligned runs of 1 to 64 lanes, groups that are not, more than 64 experts a group; scores on a coarse grid,
-    so that many tie at the selection's threshold, in and across the 64-expert slots; infinite biases."""
+    so that many tie at the selection's threshold, in and across the 64-expert slots; infinite biases; both sides of the line
+    between ranking and the threshold (32 experts)."""
     rng = np.random.default_rng(e * 37 + ng)
     logits = (np.round(rng.normal(0, 1.5, (24, e)) * 2) / 2).astype(np.float32)
     logits[3] = 0.25
