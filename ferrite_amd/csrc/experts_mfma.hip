@@ -1852,9 +1852,11 @@ extern "C" int ferrite_moe_pack_weights(const ferrite_moe_shape* shape, const fe
         return rc;
     PackSrc gu{{w->gate_w, w->up_w}, {w->gate_s, w->up_s}, s.inter, s.hidden, 2, 32, (size_t)s.hidden / 32};
     PackSrc dn{{w->down_w, nullptr}, {w->down_s, nullptr}, s.hidden, s.inter, 1, 64, (size_t)s.inter / 32};
-    if ((rc = launch_pack(pack_job(gu, packed + L.gu_codes, packed + L.gu_scales), pack_job(dn, packed + L.dn_codes, packed + L.dn_scales),
-                          s.n_experts, st)))
-        return rc;
+    // gate/up of all experts first: a layer called right behind the packing reads them first, and what has just been written is
+    // read more slowly (first call, 32 tokens of the decode shape: gate/up 145 us with both groups of an expert side by side, 126 in
+    // this order; the call 275 / 253, as much as when other data has gone through the caches in between)
+    if ((rc = launch_pack(pack_job(gu, packed + L.gu_codes, packed + L.gu_scales), PackJob{}, s.n_experts, st))) return rc;
+    if ((rc = launch_pack(pack_job(dn, packed + L.dn_codes, packed + L.dn_scales), PackJob{}, s.n_experts, st))) return rc;
     if (s.shared_inter > 0) {
         PackSrc sgu{{w->sh_gate_w, w->sh_up_w}, {w->sh_gate_s, w->sh_up_s}, s.shared_inter, s.hidden, 2, 32,
                     (size_t)s.hidden / 32};
