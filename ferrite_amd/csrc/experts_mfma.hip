@@ -466,7 +466,7 @@ __device__ __forceinline__ QuantPair quant_pair_any(float (&r0)[4], float (&r1)[
 // Clamped SwiGLU of one item's 32 gate and up rows for the unit's tokens, quantised to e4m3 (one or two terms; the second
 // is the same quantiser on what the first leaves over).  Every lane of the wave must call this.
 // Vector instructions bound it: a wave of the tiled kernels has 32-64 values a lane to finish while nothing else runs on its
-// SIMD.  Finite values (any others in the wave take the general encoder) need no clamp to +-448, and the hardware
+// SIMD.  Finite values (any others in the unit's columns send the wave to the general encoder) need no clamp to +-448, and the hardware
 // decodes the first term.  Layer before -> after, us: 4096 tokens of the decode shape two terms 1472 -> 1443, one term 895 -> 886;
 // 509 tokens two terms 400 -> 395.
 template <bool kX2>
